@@ -80,6 +80,36 @@ def test_random_banks(quant, dtype, group, shape):
     assert torch.equal(qa, qb)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("group", [32, 64, 128])
+def test_division_free_form_equals_the_division(quant, dtype, group):
+    """The register kernels (no division) against the general kernel (the reference's division), which a start off the
+    16-byte grid selects: the same bytes, on random values, on coarse grids where weights fall on the rounding ties,
+    with tiny and huge ranges, infinities and NaN, and under odd clip factors."""
+    g = torch.Generator(device="cuda").manual_seed(group)
+    n = 64 * group
+    rnd = torch.randn(48, n, generator=g, device="cuda")
+    w = rnd * torch.logspace(-30, 4, 48, device="cuda")[:, None]
+    w[8:16] = torch.round(rnd[8:16] * 8) / 16             # grids: many exact ties
+    w[16:20] = torch.randint(-15, 16, (4, n), generator=g, device="cuda").float() * 0.03125
+    w[20] = 0.25
+    if dtype != torch.float16:
+        w[21] = rnd[21] * 1e30                            # past the register form's range
+        w[22] = rnd[22] * 1e-38
+    w[23, ::group], w[24, 5::group], w[25, 7::3 * group] = float("inf"), float("-inf"), float("nan")
+    w[26, :group] = float("nan")
+    w = w.to(dtype)
+    off = torch.empty(w.numel() + 8, dtype=dtype, device="cuda")
+    off[1:1 + w.numel()] = w.reshape(-1)
+    shifted = off[1:1 + w.numel()].view(w.shape)
+    assert shifted.data_ptr() % 16 and w.data_ptr() % 16 == 0
+    for clip in ((1.0, 0.95, 0.9, 0.85, 0.8), (0.0, 3.0, -1.0), (1e20, 1.0)):
+        a, b = quant.quantize_int4(w, group, clip), quant.quantize_int4(shifted, group, clip)
+        assert torch.equal(a["q"], b["q"])
+        for k in ("scale", "zero"):
+            assert torch.equal(a[k].view(torch.int16), b[k].view(torch.int16))
+
+
 def test_bad_group_is_an_assertion(quant):
     with pytest.raises(AssertionError):
         quant.quantize_int4(torch.randn(2, 48, device="cuda"), 64)
