@@ -1,6 +1,6 @@
 /* C-ABI of the fp32 path of the MoE layer: the reference run on fp32 tensors (its fp32 models; _gmm falls to its
  * per-group matmul loop for any non-bf16 tensor, smel/moe.py:58-72, and the tests compare at 1e-5,
- * tests/test_moe.py:10-36). Every product is an fp32 MFMA (v_mfma_f32_32x32x2_f32) with fp32 accumulation; int4 banks
+ * tests/test_moe.py:10-36). Every product is an fp32 MFMA (v_mfma_f32_16x16x4_f32) with fp32 accumulation; int4 banks
  * are dequantized to fp32 inside the GEMM (the reference's fp32 Int4Experts: w = q s + z in fp32, smel/quant.py:51-84).
  * Rows are in the sorted row space of smel_dispatch (include/smel_moe.h): the tile list {group, row0, row1, gk} and
  * the group kinds are the same as the bf16 GEMMs'. All pointers are device pointers; all matrices are row-major fp32
@@ -33,7 +33,7 @@ typedef struct smel_wset_f32 {
 } smel_wset_f32;
 
 /* ---- (A5/A6/A10/A11/A12) replaces _gmm, smel/moe.py:58-72 (per-group x_g @ w_g.T / x_g @ w_g), for fp32 tensors.
- * For each tile {g, row0, row1, gk} of tiles[0 .. n_tiles[0]) (any tile height: the block walks it in 64-row steps)
+ * For each tile {g, row0, row1, gk} of tiles[0 .. n_tiles[0]) (any tile height: the block walks it in 64- or 32-row steps)
  * whose kind (gk >> 16, gk = gkind[g] when gkind is given, else tile[3]) is in w->kinds, with W = matrix gk & 0xffff
  * of that kind:
  *   trans = 0:  C[r][n] = beta C[r][n] + alpha sum_k A[r][k] W[n][k]   (n < R, k < C: out = a W^T)
@@ -46,7 +46,8 @@ int smel_gmm_f32(const smel_wset_f32* w, int32_t trans, const int32_t* gkind, co
 /* ---- LoRA weight gradients (autograd of lora_linear / lora_gate_up, smel/lora.py:61-83, for fp32 tensors).
  * For each job j < n_jobs with rows [offsets[g], offsets[g+1]), g = job_group[j]:
  *   C_j[m][n] = alpha sum_r X[r][m] Y[r][n]   (m < M, n < N; C_j = C + j * c_stride, [M][N] row-major)
- * summed in row order within 16-row steps (a job with no rows writes zeros). X [rows][ldx], Y [rows][ldy]. */
+ * summed in a fixed order: eight interleaved streams of 4-row steps, then the streams in order (a job with no rows
+ * writes zeros). X [rows][ldx], Y [rows][ldy]. */
 int smel_wgrad_f32(const float* X, int64_t ldx, const float* Y, int64_t ldy, const int32_t* offsets,
                    const int32_t* job_group, int32_t n_jobs, int64_t M, int64_t N, float alpha, float* C,
                    int64_t c_stride, hipStream_t stream);

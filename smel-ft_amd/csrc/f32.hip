@@ -1,5 +1,5 @@
 // fp32 path of the MoE layer (include/smel_f32.h): the reference's layer on fp32 tensors, whose _gmm falls to a
-// per-group matmul loop for any non-bf16 tensor (smel/moe.py:58-72). Grouped GEMMs on v_mfma_f32_32x32x2_f32 over the
+// per-group matmul loop for any non-bf16 tensor (smel/moe.py:58-72). Grouped GEMMs on v_mfma_f32_16x16x4_f32 over the
 // same tile lists and group kinds as the bf16 GEMMs, LoRA weight gradients as row-group reductions on the same MFMA,
 // and the fp32 element-wise steps around them (gather, act-gate, combine, dX reduce, router selection and backward,
 // the Gemma router input, the shared-expert gate). Everything sums in a fixed order: no atomics.
@@ -11,22 +11,11 @@
 
 namespace {
 
-constexpr int FB = 64;        // output tile 64 x 64: 4 waves, each a 32 x 32 quadrant
-constexpr int FK = 16;        // k-step staged in LDS
-constexpr int FLD = FB + 4;   // LDS pitch (floats) of a [k][64] stage: the transposing stores hit distinct banks
+typedef float f32v4 __attribute__((ext_vector_type(4)));
 
-SMEL_DEV f32x16_t mfma_f32(float a, float b, const f32x16_t& c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// One staged k-step on a wave's quadrant (wm, wn): lane l supplies A[i = l % 32][k = 2 s + l / 32] and
-// B[k][j = l % 32]; both stages are [k][64] with the row (column) index contiguous.
-SMEL_DEV void mma_step(const float* __restrict__ As, const float* __restrict__ Bs, int wm, int wn, f32x16_t& acc) {
-  const int l = lane_id(), i = l & 31, kh = l >> 5;
-#pragma unroll
-  for (int s = 0; s < FK / 2; ++s)
-    acc = mfma_f32(As[(2 * s + kh) * FLD + 32 * wm + i], Bs[(2 * s + kh) * FLD + 32 * wn + i], acc);
-}
+// v_mfma_f32_16x16x4_f32: lane l supplies A[i = l % 16][k = l / 16] and B[k = l / 16][j = l % 16] and holds
+// D[4 (l / 16) + r][j = l % 16], r = 0..3
+SMEL_DEV f32v4 mfma4(float a, float b, const f32v4& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // ---------------------------------------------------------------------------------------------- weight matrices
 
@@ -42,6 +31,7 @@ struct WMat {
   int gpr;      // groups per row, C / group
   int group;
   int gshift;   // log2(group), or -1
+  uint32_t gmul;   // ceil(2^32 / group): col / group as one high product (while col group < 2^32)
   int rbf;
 };
 
@@ -88,6 +78,7 @@ SMEL_DEV bool resolve(const smel_wset_f32& w, int kind, int idx, WMat& m) {
   m.group = w.group > 0 ? w.group : 1;
   m.gpr = (int)(w.C / m.group);
   m.gshift = (m.group & (m.group - 1)) == 0 ? __builtin_ctz((unsigned)m.group) : -1;
+  m.gmul = 0xffffffffu / (uint32_t)m.group + 1u;
   m.rbf = w.q4_round_bf16;
   m.f = nullptr;
   m.q = nullptr;
@@ -107,19 +98,290 @@ SMEL_DEV bool resolve(const smel_wset_f32& w, int kind, int idx, WMat& m) {
   return m.f != nullptr;
 }
 
+// Eight consecutive weights from one 32-bit word of nibbles (even column in the low nibble of a byte), one scale / zero.
+SMEL_DEV void dq8(uint32_t w, float sc, float ze, int rbf, float* v) {
+  const uint32_t e = w & 0x0f0f0f0fu, o = (w >> 4) & 0x0f0f0f0fu;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v[2 * j] = fmaf((float)((e >> (8 * j)) & 0xffu), sc, ze);
+    v[2 * j + 1] = fmaf((float)((o >> (8 * j)) & 0xffu), sc, ze);
+  }
+  if (rbf) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = bf2f(f2bf(v[j]));
+  }
+}
+
 // ---------------------------------------------------------------------------------------------- grouped GEMM
-// Block = one tile of the list x 64 output columns; the tile's rows in 64-row chunks. Each k-step: every thread
-// loads 4 A values (row t / 4, k 4 (t % 4) ..) and 4 W values, stores them into the [k][64] stages, and the next
-// step's loads are issued before this step's MFMAs (two LDS stages, one barrier per step).
-// VEC: A rows and fp32 weights may be read as aligned float4 (lda, C multiples of 4, 16-byte aligned bases).
-template <int TRANS, bool VEC>
-__global__ __launch_bounds__(256) void gmm_f32_kernel(smel_wset_f32 w, const int32_t* __restrict__ gkind,
-                                                      const int32_t* __restrict__ tiles,
-                                                      const int32_t* __restrict__ n_tiles,
-                                                      const float* __restrict__ A, int64_t lda, float alpha,
-                                                      int beta1, float* __restrict__ C, int64_t ldc) {
-  __shared__ __align__(16) float As[2][FK * FLD];
-  __shared__ __align__(16) float Bs[2][FK * FLD];
+// What bounds it: the fp32 MFMA rate (64 FLOP per SIMD and clock), then the dequant of the weights beside it (about 3
+// VALU instructions per weight and 64-row tile). A block takes RB rows of one tile of the list (the tile in RB-row
+// steps) and NT output columns; per k-step of FK the operands go through two LDS stages (the next step's global loads
+// in flight during this step's MFMAs, one barrier per step). The rows run in 16-row slices, only as many as the tile
+// has: a frozen expert of 32 rows costs 2 slices (the 32x32 MFMA form computed 64 rows for it). A lane takes four
+// consecutive k of its row with one 16-byte LDS read and feeds them to four MFMAs (the order inside the sum over k is
+// free); a wave's NF column fragments interleave their columns (column = NF i + f), so that for W [K][N] one NF-float
+// read gives every fragment its value.
+// Two shapes (the rule is in smel_gmm_f32): 64 x 128 with the four waves side by side along the columns, and 32 x 64
+// with the four waves each on a quarter of the staged k, summed through LDS in wave order, for launches whose tiles
+// would leave most of the 256 CUs idle.
+// Measured, 1021 tokens top-8 of 256 experts (12 of them fp32), H 2048, I 512 (about 32 rows per expert): gate_up 991 ->
+// 445 us, down 462 -> 240, down backward 528 -> 274, gate_up backward 949 -> 485 (against 64 x 64 blocks of 32x32x2
+// MFMAs); the 16-row slices computed are 43 GFLOP of gate_up = 97 TFLOP/s of the 157 nominal. With the loop's barriers
+// waiting for global loads, or its load and store code behind branches, the same tiles took 560-620 us.
+// One k-step's operands of a thread on their way from global memory to LDS.
+struct StageRegs {
+  u32x4_t a[2];   // 8 values of an A row
+  u32x4_t b[4];   // a run of 16 weights: fp32 values, or the raw nibbles in b[0]
+  uint32_t bs, bz;   // and their bf16 scale and zero
+};
+
+struct GemmArgs {
+  const float* A;
+  int64_t lda;
+  float alpha;
+  int beta1;
+  float* C;
+  int64_t ldc;
+};
+
+// How a block reads its weights: runs of 16 nibbles (8 bytes, one scale / zero pair), fp32 in 16-byte loads, or element
+// by element (any alignment, any group; A too).
+// W_INT4R: W_INT4 with the dequantized values rounded to bf16.
+enum { W_INT4 = 0, W_F32 = 1, W_ANY = 2, W_INT4R = 3 };
+
+template <int TRANS, int RB, int NT, int KS, int FK>
+struct Gemm {
+  static constexpr int NWN = 4 / KS;            // waves along the columns
+  static constexpr int NF = NT / NWN / 16;      // 16-column fragments of a wave
+  static constexpr int RF = RB / 16;            // 16-row slices
+  static constexpr int KW = FK / KS;            // k of a step that one wave takes
+  static constexpr int PA = FK + 4;             // pitch of the [row][k] stages: 16-byte reads of 8 lanes on distinct banks
+  static constexpr int PB = TRANS ? NT : PA;    // W stage: [k][n] for TRANS, else [n][k]
+  static constexpr int SA = RB * PA, SB = TRANS ? FK * NT : NT * PA;
+  static constexpr int LDS_FLOATS = 2 * (SA + SB);
+  static_assert(RB * FK == 8 * 256 && NT * FK == 16 * 256, "staging split");
+  static_assert(KS == 1 || KS * RB * (NT + 4) <= LDS_FLOATS, "reduction buffer");
+
+  // NRF: the 16-row slices computed (those of the tile's rows; the others' rows are zeros in LDS)
+  template <int MODE, int NRF>
+  SMEL_DEV static void tile(float* __restrict__ lds, const GemmArgs& G, const WMat& m, int N, int K, int n0, int mr0,
+                            int mr1) {
+    constexpr bool INT4 = MODE == W_INT4 || MODE == W_INT4R;
+    const int t = threadIdx.x, l = lane_id(), wv = t >> 6, i = l & 15, kq = l >> 4;
+    const int wn = wv % NWN, wk = wv / NWN;
+    const int nk = (K + FK - 1) / FK;
+    // load coordinates: A row t / (FK / 8), 8 k; W: a run of 16 along the matrix's rows
+    const int am = t / (FK / 8), ak = 8 * (t % (FK / 8));
+    const int bo = TRANS ? t / (NT / 16) : t / (FK / 16);           // outer index: k (TRANS) or n
+    const int br = TRANS ? 16 * (t % (NT / 16)) : 16 * (t % (FK / 16));
+    const int WR = TRANS ? K : N, WC = TRANS ? N : K;
+    const float* const ab = G.A + (int64_t)mr0 * G.lda;
+    const rsrc_t ra = make_rsrc(ab, ((uint64_t)(mr1 - mr0 - 1) * G.lda + K) * 4);
+    const rsrc_t rw = INT4 ? make_rsrc(m.q, (uint64_t)WR * (m.C >> 1)) : make_rsrc(m.f, (uint64_t)WR * m.C * 4);
+    const rsrc_t rs = make_rsrc(m.s, INT4 ? (uint64_t)WR * m.gpr * 2 : 0);
+    const rsrc_t rz = make_rsrc(m.z, INT4 ? (uint64_t)WR * m.gpr * 2 : 0);
+    const uint32_t arow = am < mr1 - mr0 ? (uint32_t)(am * G.lda) : OOB;
+    auto load = [&](StageRegs& S, int k0) {
+      const int k = k0 + ak;
+      const int wr = TRANS ? k0 + bo : n0 + bo;   // matrix row and first column of the run
+      const int wc = TRANS ? n0 + br : k0 + br;
+      if (MODE == W_ANY) return;                  // loaded where it is stored
+#pragma unroll
+      for (int h = 0; h < 2; ++h) S.a[h] = ld16(ra, (arow != OOB && k + 4 * h < K) ? 4 * (arow + k + 4 * h) : OOB);
+      if (INT4) {   // C a multiple of 16, so a run is inside the matrix or past it
+        const bool ok = wr < WR && wc < WC;
+        const u32x2_t q = ld8(rw, ok ? (uint32_t)(wr * (m.C >> 1) + (wc >> 1)) : OOB);
+        S.b[0][0] = q[0], S.b[0][1] = q[1];
+        // past the matrix: zero nibbles under a zero scale and zero
+        const uint32_t go = ok ? 2u * (uint32_t)(wr * m.gpr + (int)__umulhi((uint32_t)wc, m.gmul)) : OOB;
+        S.bs = ld2(rs, go), S.bz = ld2(rz, go);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          S.b[j] = ld16(rw, (wr < WR && wc + 4 * j < WC) ? 4u * (uint32_t)(wr * m.C + wc + 4 * j) : OOB);
+      }
+    };
+    auto store = [&](StageRegs& S, int buf, int k0) {
+      float* const As = lds + buf * (SA + SB);
+      float* const Bs = As + SA;
+      float* const ap = As + am * PA + ak;
+      float* const bp = Bs + bo * PB + br;
+      if (MODE == W_ANY) {
+        const int wr = TRANS ? k0 + bo : n0 + bo, wc = TRANS ? n0 + br : k0 + br;
+#pragma unroll 1
+        for (int e = 0; e < 8; ++e) {
+          const int k = k0 + ak + e;
+          ap[e] = (am < mr1 - mr0 && k < K) ? ab[am * G.lda + k] : 0.f;
+        }
+#pragma unroll 1
+        for (int e = 0; e < 16; ++e) bp[e] = (wr < WR && wc + e < WC) ? w_at(m, wr, wc + e) : 0.f;
+        return;
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) *reinterpret_cast<u32x4_t*>(ap + 4 * h) = S.a[h];
+      if (INT4) {
+        float v[16];
+        const float sc = __uint_as_float(S.bs << 16), ze = __uint_as_float(S.bz << 16);
+        dq8(S.b[0][0], sc, ze, MODE == W_INT4R, v);
+        dq8(S.b[0][1], sc, ze, MODE == W_INT4R, v + 8);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<float4*>(bp + 4 * j) = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4_t*>(bp + 4 * j) = S.b[j];
+      }
+    };
+    f32v4 acc[NRF][NF] = {};
+    auto compute = [&](int buf) {
+      const float* const As = lds + buf * (SA + SB);
+      const float* const Bs = As + SA;
+#pragma unroll
+      for (int k16 = 0; k16 < KW; k16 += 16) {
+        const int kk = wk * KW + k16 + 4 * kq;
+        float b[4][NF];   // [k in the quad][fragment]
+        if (TRANS) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float* p = Bs + (kk + e) * PB + 16 * NF * wn + NF * i;
+            if (NF == 2) {
+              const float2 v = *reinterpret_cast<const float2*>(p);
+              b[e][0] = v.x, b[e][1] = v.y;
+            } else {
+              const float4 v = *reinterpret_cast<const float4*>(p);
+              b[e][0] = v.x, b[e][1] = v.y, b[e][2 % NF] = v.z, b[e][3 % NF] = v.w;
+            }
+          }
+        } else {
+#pragma unroll
+          for (int f = 0; f < NF; ++f) {
+            const float4 v = *reinterpret_cast<const float4*>(Bs + (16 * NF * wn + NF * i + f) * PB + kk);
+            b[0][f] = v.x, b[1][f] = v.y, b[2][f] = v.z, b[3][f] = v.w;
+          }
+        }
+#pragma unroll
+        for (int rf = 0; rf < NRF; ++rf) {
+          const float4 a = *reinterpret_cast<const float4*>(As + (16 * rf + i) * PA + kk);
+#pragma unroll
+          for (int f = 0; f < NF; ++f) acc[rf][f] = mfma4(a.x, b[0][f], acc[rf][f]);
+#pragma unroll
+          for (int f = 0; f < NF; ++f) acc[rf][f] = mfma4(a.y, b[1][f], acc[rf][f]);
+#pragma unroll
+          for (int f = 0; f < NF; ++f) acc[rf][f] = mfma4(a.z, b[2][f], acc[rf][f]);
+#pragma unroll
+          for (int f = 0; f < NF; ++f) acc[rf][f] = mfma4(a.w, b[3][f], acc[rf][f]);
+        }
+      }
+    };
+    // Global loads run two k-steps ahead of their use, in two register sets; the barriers wait for LDS only. One
+    // branch-free block per step, so that the next stage's dequant is issued between the MFMAs (two waves of a SIMD
+    // reach their MFMA and VALU phases together: apart, the phases would add up). Steps past K load and add zeros.
+    StageRegs S0, S1;
+    load(S0, 0);
+    load(S1, FK);
+    store(S0, 0, 0);
+    lds_barrier();
+    for (int kt = 0; kt < nk; kt += 2) {
+      load(S0, (kt + 2) * FK);
+      compute(0);
+      store(S1, 1, (kt + 1) * FK);
+      lds_barrier();
+      load(S1, (kt + 3) * FK);
+      compute(1);
+      store(S0, 0, (kt + 2) * FK);
+      lds_barrier();
+    }
+    if constexpr (KS == 1) {
+#pragma unroll
+      for (int rf = 0; rf < NRF; ++rf)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = mr0 + 16 * rf + 4 * kq + r;
+          if (row >= mr1) continue;
+          float* const p = G.C + (int64_t)row * G.ldc;
+#pragma unroll
+          for (int f = 0; f < NF; ++f) {
+            const int col = n0 + 16 * NF * wn + NF * i + f;
+            if (col < N) p[col] = G.beta1 ? p[col] + G.alpha * acc[rf][f][r] : G.alpha * acc[rf][f][r];
+          }
+        }
+    } else {   // the waves' k quarters, summed in wave order
+      constexpr int PR = NT + 4;
+#pragma unroll
+      for (int rf = 0; rf < NRF; ++rf)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int f = 0; f < NF; ++f) lds[(wk * RB + 16 * rf + 4 * kq + r) * PR + 16 * NF * wn + NF * i + f] = acc[rf][f][r];
+      lds_barrier();
+      for (int e = t; e < RB * NT; e += 256) {
+        const int rr = e / NT, cc = e % NT;
+        const int row = mr0 + rr, col = n0 + cc;
+        if (row >= mr1 || col >= N) continue;   // rows past NRF slices are past mr1
+        float v = lds[rr * PR + cc];
+#pragma unroll
+        for (int q = 1; q < KS; ++q) v += lds[(q * RB + rr) * PR + cc];
+        float* const p = G.C + (int64_t)row * G.ldc + col;
+        *p = G.beta1 ? *p + G.alpha * v : G.alpha * v;
+      }
+      lds_barrier();
+    }
+  }
+};
+
+template <int TRANS, int RB, int NT, int KS, int FK>
+__global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const int32_t* __restrict__ gkind,
+                                                         const int32_t* __restrict__ tiles,
+                                                         const int32_t* __restrict__ n_tiles, int vec, int qvec,
+                                                         GemmArgs G) {
+  using GM = Gemm<TRANS, RB, NT, KS, FK>;
+  __shared__ __align__(16) float lds[GM::LDS_FLOATS];
+  const int N = (int)(TRANS ? w.C : w.R), K = (int)(TRANS ? w.R : w.C);
+  // the column blocks of a tile run back to back on XCD tile % 8 (blocks go to the XCDs round robin): its A rows are
+  // read from that XCD's L2
+  const int ncol = (N + NT - 1) / NT, slot = blockIdx.x >> 3;
+  const int ti = (slot / ncol) * 8 + (blockIdx.x & 7), n0 = (slot % ncol) * NT;
+  if (ti >= n_tiles[0]) return;
+  const int g = tiles[4 * ti], r0 = tiles[4 * ti + 1], r1 = tiles[4 * ti + 2];
+  const int gk = gkind ? gkind[g] : tiles[4 * ti + 3];
+  const int kind = gk >> 16, idx = gk & 0xffff;
+  if (!((w.kinds >> kind) & 1)) return;
+  WMat m;
+  if (!resolve(w, kind, idx, m)) return;
+  // the tile's rows in RB-row steps; gridDim.z blocks share them
+  for (int mr0 = r0 + RB * (int)blockIdx.z; mr0 < r1; mr0 += RB * (int)gridDim.z) {
+    const int mr1 = min(r1, mr0 + RB);
+    const int nrf = (mr1 - mr0 + 15) >> 4;
+    if (!m.f && (vec & 1) && qvec && m.rbf) {
+      GM::template tile<W_INT4R, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
+    } else if (!m.f && (vec & 1) && qvec) {
+      if (nrf == 1) GM::template tile<W_INT4, 1>(lds, G, m, N, K, n0, mr0, mr1);
+      else if (nrf == 2) GM::template tile<W_INT4, 2>(lds, G, m, N, K, n0, mr0, mr1);
+      else if (GM::RF > 2 && nrf == 3) GM::template tile<W_INT4, GM::RF - 1>(lds, G, m, N, K, n0, mr0, mr1);
+      else GM::template tile<W_INT4, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
+    } else if (m.f && vec == 3) {
+      if (nrf == 1) GM::template tile<W_F32, 1>(lds, G, m, N, K, n0, mr0, mr1);
+      else if (nrf == 2) GM::template tile<W_F32, 2>(lds, G, m, N, K, n0, mr0, mr1);
+      else GM::template tile<W_F32, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
+    } else {
+      GM::template tile<W_ANY, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
+    }
+    lds_barrier();
+  }
+}
+
+// Few output columns (LoRA factors, the shared gate): one block per 16 rows of a tile, the 8 waves on interleaved
+// 16-wide runs of k, straight from global memory into registers (no staging: nothing is used twice), summed through
+// LDS in wave order. Bound: memory latency, which a wave meets K / 128 / UNR times. Columns of fragment f: NF i + f.
+template <int TRANS, int NF>
+__global__ __launch_bounds__(512) void gmm_f32_skinny_kernel(smel_wset_f32 w, const int32_t* __restrict__ gkind,
+                                                             const int32_t* __restrict__ tiles,
+                                                             const int32_t* __restrict__ n_tiles,
+                                                             const float* __restrict__ A, int64_t lda, int vec,
+                                                             float alpha, int beta1, float* __restrict__ C,
+                                                             int64_t ldc) {
+  constexpr int NT = 16 * NF, UNR = 4;
+  __shared__ float red[8][16][NT + 1];
   const int ti = blockIdx.x;
   if (ti >= n_tiles[0]) return;
   const int g = tiles[4 * ti], r0 = tiles[4 * ti + 1], r1 = tiles[4 * ti + 2];
@@ -128,144 +390,139 @@ __global__ __launch_bounds__(256) void gmm_f32_kernel(smel_wset_f32 w, const int
   if (!((w.kinds >> kind) & 1)) return;
   WMat m;
   if (!resolve(w, kind, idx, m)) return;
-  const int64_t N = TRANS ? w.C : w.R, K = TRANS ? w.R : w.C;
-  const int64_t n0 = (int64_t)blockIdx.y * FB;
-  if (n0 >= N) return;
-  const int t = threadIdx.x, wv = t >> 6, wm = wv & 1, wn = wv >> 1;
-  const int nk = (int)((K + FK - 1) / FK);
-  // this thread's load coordinates: A (and W for TRANS = 0) row t / 4, k quad t % 4; W for TRANS = 1: k t / 16,
-  // column quad t % 16
-  const int am = t >> 2, akq = 4 * (t & 3);
-  const int bk1 = t >> 4, bn1 = 4 * (t & 15);
-  const bool qvec = (w.C & 3) == 0 && (m.f ? VEC : true);
-  for (int mr0 = r0; mr0 < r1; mr0 += FB) {
-    const int mr1 = min(r1, mr0 + FB);
-    float ra[4], rb[4];
-    auto load = [&](int64_t k0) {
-      const int64_t row = mr0 + am, k = k0 + akq;
-      if (VEC && row < mr1 && k + 3 < K) {
-        const float4 v = *reinterpret_cast<const float4*>(A + row * lda + k);
-        ra[0] = v.x, ra[1] = v.y, ra[2] = v.z, ra[3] = v.w;
-      } else {
+  const int N = (int)(TRANS ? w.C : w.R), K = (int)(TRANS ? w.R : w.C);
+  const int t = threadIdx.x, l = lane_id(), wv = t >> 6, i = l & 15, kq = l >> 4;
+  const bool avec = vec & 1, wvec = (m.C & 3) == 0 && (m.f ? (vec & 2) != 0 : true);
+  for (int mr0 = r0 + 16 * (int)blockIdx.z; mr0 < r1; mr0 += 16 * (int)gridDim.z) {
+    const int row = mr0 + i;
+    const bool rok = row < r1;
+    const float* const ap = A + (int64_t)(rok ? row : mr0) * lda;
+    f32v4 acc[NF] = {};
+    for (int k0 = 16 * wv; k0 < K; k0 += 16 * 8 * UNR) {
+      float a[UNR][4], b[UNR][4][NF];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ra[i] = (row < mr1 && k + i < K) ? A[row * lda + k + i] : 0.f;
-      }
-      // weights: whole quads through w_quad when the matrix's rows are multiples of 4 (and, for fp32, its base
-      // 16-byte aligned: VEC), the guarded element path otherwise
-      if (TRANS == 0) {   // W [N][K]: row n0 + t / 4, k quad
-        const int n = (int)(n0 + am), kq = (int)k;
-        if (qvec && n < N && kq + 3 < K) {
-          w_quad(m, n, kq, rb);
+      for (int u = 0; u < UNR; ++u) {
+        const int k = k0 + 128 * u + 4 * kq;
+        if (avec && k + 3 < K) {
+          const float4 v = *reinterpret_cast<const float4*>(ap + k);
+          a[u][0] = v.x, a[u][1] = v.y, a[u][2] = v.z, a[u][3] = v.w;
         } else {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) rb[i] = (n < N && kq + i < K) ? w_at(m, n, kq + i) : 0.f;
+          for (int e = 0; e < 4; ++e) a[u][e] = k + e < K ? ap[k + e] : 0.f;
         }
-      } else {            // W [K][N]: row k0 + t / 16, column quad
-        const int kk = (int)(k0 + bk1), n = (int)(n0 + bn1);
-        if (qvec && kk < K && n + 3 < N) {
-          w_quad(m, kk, n, rb);
+        if (TRANS) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if (NF == 4 && wvec && k + e < K && NF * i + 3 < N) {
+              float v[4];
+              w_quad(m, k + e, 4 * i, v);
+#pragma unroll
+              for (int f = 0; f < NF; ++f) b[u][e][f] = v[f % 4];
+            } else {
+#pragma unroll
+              for (int f = 0; f < NF; ++f) b[u][e][f] = (k + e < K && NF * i + f < N) ? w_at(m, k + e, NF * i + f) : 0.f;
+            }
+          }
         } else {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) rb[i] = (kk < K && n + i < N) ? w_at(m, kk, n + i) : 0.f;
+          for (int f = 0; f < NF; ++f) {
+            const int n = NF * i + f;
+            if (wvec && n < N && k + 3 < K) {
+              float v[4];
+              w_quad(m, n, k, v);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) b[u][e][f] = v[e];
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) b[u][e][f] = (n < N && k + e < K) ? w_at(m, n, k + e) : 0.f;
+            }
+          }
         }
       }
-    };
-    auto store = [&](int buf) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) As[buf][(akq + i) * FLD + am] = ra[i];
-      if (TRANS == 0) {
+      for (int u = 0; u < UNR; ++u)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) Bs[buf][(akq + i) * FLD + am] = rb[i];
-      } else {
-        *reinterpret_cast<float4*>(&Bs[buf][bk1 * FLD + bn1]) = make_float4(rb[0], rb[1], rb[2], rb[3]);
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int f = 0; f < NF; ++f) acc[f] = mfma4(rok ? a[u][e] : 0.f, b[u][e][f], acc[f]);
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wv][4 * kq + r][NF * i + f] = acc[f][r];
+    __syncthreads();
+    for (int e = t; e < 16 * NT; e += 512) {
+      const int rr = e / NT, cc = e % NT;
+      if (mr0 + rr < r1 && cc < N) {
+        float v = red[0][rr][cc];
+#pragma unroll
+        for (int q = 1; q < 8; ++q) v += red[q][rr][cc];
+        float* const p = C + (int64_t)(mr0 + rr) * ldc + cc;
+        *p = beta1 ? *p + alpha * v : alpha * v;
       }
-    };
-    f32x16_t acc = {};
-    if (nk > 0) {
-      load(0);
-      store(0);
     }
     __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-      if (kt + 1 < nk) load((int64_t)(kt + 1) * FK);
-      mma_step(As[kt & 1], Bs[kt & 1], wm, wn, acc);
-      if (kt + 1 < nk) store((kt + 1) & 1);
-      __syncthreads();
-    }
-    const int l = lane_id();
-    const int64_t col = n0 + 32 * wn + (l & 31);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int64_t row = mr0 + 32 * wm + acc_row(r, l);
-      if (row < mr1 && col < N) {
-        float* p = C + row * ldc + col;
-        *p = beta1 ? *p + alpha * acc[r] : alpha * acc[r];
-      }
-    }
   }
 }
 
 // ---------------------------------------------------------------------------------------------- weight gradients
-// Block = (64 x 64 output tile, job); the job's rows are the contraction, 16 per staged step: X rows give the
-// [k][m] stage and Y rows the [k][n] stage directly (both row-contiguous).
-template <bool VEC>
-__global__ __launch_bounds__(256) void wgrad_f32_kernel(const float* __restrict__ X, int64_t ldx,
-                                                        const float* __restrict__ Y, int64_t ldy,
+// Block = (16 columns of the narrower side, 64 of the wider one, job); the job's rows are the contraction. The 8 waves
+// take interleaved row quads straight from global memory: lane (kq, i) reads S[row][s0 + i] and the 16 bytes
+// B[row][b0 + 4 i ..] of row = quad + kq, which feed four MFMAs (column 4 i + f in fragment f). The waves' sums are
+// added through LDS in wave order. Bound: memory latency of the row loop (rows / 32 quads per wave, UNR in flight).
+// S is X (SWAP 0: the output is [s][b]) or Y (SWAP 1: [b][s]).
+template <int SWAP>
+__global__ __launch_bounds__(512) void wgrad_f32_kernel(const float* __restrict__ S, int64_t lds_, int64_t ns,
+                                                        const float* __restrict__ B, int64_t ldb, int64_t nb,
                                                         const int32_t* __restrict__ offsets,
-                                                        const int32_t* __restrict__ job_group, int64_t M, int64_t N,
+                                                        const int32_t* __restrict__ job_group, int vec, int64_t N,
                                                         float alpha, float* __restrict__ C, int64_t c_stride) {
-  __shared__ __align__(16) float As[2][FK * FLD];
-  __shared__ __align__(16) float Bs[2][FK * FLD];
+  constexpr int UNR = 8;
+  __shared__ float red[8][16][65];
   const int j = blockIdx.y;
-  const int nbn = (int)((N + FB - 1) / FB);
-  const int64_t m0 = (int64_t)(blockIdx.x / nbn) * FB, n0 = (int64_t)(blockIdx.x % nbn) * FB;
+  const int nbb = (int)((nb + 63) / 64);
+  const int64_t s0 = (int64_t)(blockIdx.x / nbb) * 16, b0 = (int64_t)(blockIdx.x % nbb) * 64;
   const int g = job_group[j];
   const int64_t r0 = offsets[g], r1 = offsets[g + 1];
-  const int t = threadIdx.x, wv = t >> 6, wm = wv & 1, wn = wv >> 1;
-  const int kl = t >> 4, q4 = 4 * (t & 15);
-  const int nk = r1 > r0 ? (int)((r1 - r0 + FK - 1) / FK) : 0;
-  float ra[4], rb[4];
-  auto load = [&](int64_t k0) {
-    const int64_t r = r0 + k0 + kl;
-    const int64_t mm = m0 + q4, nn = n0 + q4;
-    if (VEC && r < r1 && mm + 3 < M) {
-      const float4 v = *reinterpret_cast<const float4*>(X + r * ldx + mm);
-      ra[0] = v.x, ra[1] = v.y, ra[2] = v.z, ra[3] = v.w;
-    } else {
+  const int t = threadIdx.x, l = lane_id(), wv = t >> 6, i = l & 15, kq = l >> 4;
+  const int64_t si = s0 + i, bi = b0 + 4 * i;
+  f32v4 acc[4] = {};
+  for (int64_t q0 = r0 + 4 * wv; q0 < r1; q0 += 32 * UNR) {
+    float a[UNR], b[UNR][4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) ra[i] = (r < r1 && mm + i < M) ? X[r * ldx + mm + i] : 0.f;
-    }
-    if (VEC && r < r1 && nn + 3 < N) {
-      const float4 v = *reinterpret_cast<const float4*>(Y + r * ldy + nn);
-      rb[0] = v.x, rb[1] = v.y, rb[2] = v.z, rb[3] = v.w;
-    } else {
+    for (int u = 0; u < UNR; ++u) {
+      const int64_t r = q0 + 32 * u + kq;
+      const bool ok = r < r1;
+      a[u] = (ok && si < ns) ? S[r * lds_ + si] : 0.f;
+      if (vec && ok && bi + 3 < nb) {
+        const float4 v = *reinterpret_cast<const float4*>(B + r * ldb + bi);
+        b[u][0] = v.x, b[u][1] = v.y, b[u][2] = v.z, b[u][3] = v.w;
+      } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) rb[i] = (r < r1 && nn + i < N) ? Y[r * ldy + nn + i] : 0.f;
+        for (int f = 0; f < 4; ++f) b[u][f] = (ok && bi + f < nb) ? B[r * ldb + bi + f] : 0.f;
+      }
     }
-  };
-  auto store = [&](int buf) {
-    *reinterpret_cast<float4*>(&As[buf][kl * FLD + q4]) = make_float4(ra[0], ra[1], ra[2], ra[3]);
-    *reinterpret_cast<float4*>(&Bs[buf][kl * FLD + q4]) = make_float4(rb[0], rb[1], rb[2], rb[3]);
-  };
-  f32x16_t acc = {};
-  if (nk > 0) {
-    load(0);
-    store(0);
+#pragma unroll
+    for (int u = 0; u < UNR; ++u)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) acc[f] = mfma4(a[u], b[u][f], acc[f]);
   }
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wv][4 * kq + r][4 * i + f] = acc[f][r];
   __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    if (kt + 1 < nk) load((int64_t)(kt + 1) * FK);
-    mma_step(As[kt & 1], Bs[kt & 1], wm, wn, acc);
-    if (kt + 1 < nk) store((kt + 1) & 1);
-    __syncthreads();
-  }
-  const int l = lane_id();
-  const int64_t col = n0 + 32 * wn + (l & 31);
-  float* Cj = C + (int64_t)j * c_stride;
+  float* const Cj = C + (int64_t)j * c_stride;
+  for (int e = t; e < 16 * 64; e += 512) {
+    const int ss = SWAP ? e % 16 : e / 64, bb = SWAP ? e / 16 : e % 64;
+    if (s0 + ss >= ns || b0 + bb >= nb) continue;
+    float v = red[0][ss][bb];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int64_t row = m0 + 32 * wm + acc_row(r, l);
-    if (row < M && col < N) Cj[row * N + col] = alpha * acc[r];
+    for (int q = 1; q < 8; ++q) v += red[q][ss][bb];
+    if (SWAP)
+      Cj[(b0 + bb) * N + s0 + ss] = alpha * v;
+    else
+      Cj[(s0 + ss) * N + b0 + bb] = alpha * v;
   }
 }
 
@@ -301,6 +558,34 @@ SMEL_DEV void act_grad32(float g, int act, float& a, float& da) {
   da = 0.5f * (1.0f + th) + 0.5f * g * (1.0f - th * th) * c * (1.0f + 3.0f * 0.044715f * g * g);
 }
 
+// The row kernels below take V = 4 columns per thread and access (16-byte loads and stores) where the row length, the
+// pitches and the bases allow it, V = 1 elsewhere; the same sums in the same order either way. They are bound by HBM;
+// 1021 tokens (8168 rows of 2048): combine and its backward 32 -> 24 us, dX reduce 37 -> 17 us with V = 4
+// against V = 1.
+template <int V>
+struct FVec {
+  float v[V];
+};
+template <int V>
+SMEL_DEV FVec<V> ldv(const float* p) {
+  FVec<V> r;
+  if constexpr (V == 4) {
+    const float4 x = *reinterpret_cast<const float4*>(p);
+    r.v[0] = x.x, r.v[1] = x.y, r.v[2] = x.z, r.v[3] = x.w;
+  } else {
+    r.v[0] = p[0];
+  }
+  return r;
+}
+template <int V>
+SMEL_DEV void stv(float* p, const FVec<V>& r) {
+  if constexpr (V == 4)
+    *reinterpret_cast<float4*>(p) = make_float4(r.v[0], r.v[1], r.v[2], r.v[3]);
+  else
+    p[0] = r.v[0];
+}
+
+template <int V>
 __global__ __launch_bounds__(256) void gather_rows_f32_kernel(const float* __restrict__ src, int64_t lds,
                                                               const int32_t* __restrict__ idx, int div,
                                                               const int32_t* __restrict__ n_valid, int64_t cols,
@@ -309,76 +594,104 @@ __global__ __launch_bounds__(256) void gather_rows_f32_kernel(const float* __res
   const int i = (n_valid && p >= n_valid[0]) ? -1 : idx[p];
   const float* s = i >= 0 ? src + (int64_t)(i / div) * lds : nullptr;
   float* o = out + p * cols;
-  for (int64_t c = threadIdx.x; c < cols; c += 256) o[c] = s ? s[c] : 0.f;
+  for (int64_t c = V * threadIdx.x; c < cols; c += 256 * V) stv<V>(o + c, s ? ldv<V>(s + c) : FVec<V>{});
 }
 
+template <int V>
 __global__ __launch_bounds__(256) void act_gate_f32_kernel(const float* __restrict__ h, int64_t ldh, int64_t I, int act,
                                                            float* __restrict__ a, int64_t lda) {
   const int64_t r = blockIdx.x;
-  for (int64_t j = threadIdx.x; j < I; j += 256) a[r * lda + j] = act32(h[r * ldh + j], act) * h[r * ldh + I + j];
+  for (int64_t j = V * threadIdx.x; j < I; j += 256 * V) {
+    const FVec<V> g = ldv<V>(h + r * ldh + j), u = ldv<V>(h + r * ldh + I + j);
+    FVec<V> o;
+#pragma unroll
+    for (int e = 0; e < V; ++e) o.v[e] = act32(g.v[e], act) * u.v[e];
+    stv<V>(a + r * lda + j, o);
+  }
 }
 
+template <int V>
 __global__ __launch_bounds__(256) void act_gate_bwd_f32_kernel(const float* __restrict__ h, int64_t ldh,
                                                                const float* __restrict__ da, int64_t ldda, int64_t I,
                                                                int act, float* __restrict__ dh, int64_t lddh) {
   const int64_t r = blockIdx.x;
-  for (int64_t j = threadIdx.x; j < I; j += 256) {
-    const float g = h[r * ldh + j], u = h[r * ldh + I + j], d = da[r * ldda + j];
-    float a, dg;
-    act_grad32(g, act, a, dg);
-    dh[r * lddh + j] = d * u * dg;
-    dh[r * lddh + I + j] = d * a;
+  for (int64_t j = V * threadIdx.x; j < I; j += 256 * V) {
+    const FVec<V> g = ldv<V>(h + r * ldh + j), u = ldv<V>(h + r * ldh + I + j), d = ldv<V>(da + r * ldda + j);
+    FVec<V> og, ou;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      float a, dg;
+      act_grad32(g.v[e], act, a, dg);
+      og.v[e] = d.v[e] * u.v[e] * dg;
+      ou.v[e] = d.v[e] * a;
+    }
+    stv<V>(dh + r * lddh + j, og);
+    stv<V>(dh + r * lddh + I + j, ou);
   }
 }
 
+template <int V>
 __global__ __launch_bounds__(256) void combine_f32_kernel(const float* __restrict__ ys, const float* __restrict__ topv,
                                                           const int32_t* __restrict__ inv, int K, int64_t H,
                                                           float* __restrict__ out) {
   const int64_t t = blockIdx.x;
-  for (int64_t c = threadIdx.x; c < H; c += 256) {
-    float acc = 0.f;
-    for (int k = 0; k < K; ++k) {
+  for (int64_t c = V * threadIdx.x; c < H; c += 256 * V) {
+    FVec<V> acc = {};
+#pragma unroll 8
+    for (int k = 0; k < K; ++k) {   // no branch: eight rows' loads in flight
       const int p = inv[t * K + k];
-      if (p >= 0) acc += ys[(int64_t)p * H + c] * topv[t * K + k];
+      const FVec<V> y = ldv<V>(ys + (int64_t)max(p, 0) * H + c);
+      const float w = topv[t * K + k];
+#pragma unroll
+      for (int e = 0; e < V; ++e) acc.v[e] = p >= 0 ? acc.v[e] + y.v[e] * w : acc.v[e];
     }
-    out[t * H + c] = acc;
+    stv<V>(out + t * H + c, acc);
   }
 }
 
+// One block per (token, slot): the row's gradient and its dot product with the row.
+template <int V>
 __global__ __launch_bounds__(256) void combine_bwd_f32_kernel(const float* __restrict__ ys,
                                                               const float* __restrict__ dout,
                                                               const float* __restrict__ topv,
                                                               const int32_t* __restrict__ inv, int K, int64_t H,
                                                               float* __restrict__ dys, float* __restrict__ dtopv) {
   __shared__ float red[4];
-  const int64_t t = blockIdx.x;
-  for (int k = 0; k < K; ++k) {
-    const int p = inv[t * K + k];   // block-uniform
-    float dot = 0.f;
-    if (p >= 0) {
-      const float tv = topv[t * K + k];
-      for (int64_t c = threadIdx.x; c < H; c += 256) {
-        const float d = dout[t * H + c];
-        dys[(int64_t)p * H + c] = tv * d;
-        dot += ys[(int64_t)p * H + c] * d;
+  const int64_t t = blockIdx.x, tk = t * K + blockIdx.y;
+  const int p = inv[tk];   // block-uniform
+  float dot = 0.f;
+  if (p >= 0) {
+    const float tv = topv[tk];
+    for (int64_t c = V * threadIdx.x; c < H; c += 256 * V) {
+      const FVec<V> d = ldv<V>(dout + t * H + c), y = ldv<V>(ys + (int64_t)p * H + c);
+      FVec<V> o;
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        o.v[e] = tv * d.v[e];
+        dot += y.v[e] * d.v[e];
       }
+      stv<V>(dys + (int64_t)p * H + c, o);
     }
-    dot = block_sum(dot, red);
-    if (threadIdx.x == 0) dtopv[t * K + k] = dot;
   }
+  dot = block_sum(dot, red);
+  if (threadIdx.x == 0) dtopv[tk] = dot;
 }
 
+template <int V>
 __global__ __launch_bounds__(256) void dx_reduce_f32_kernel(const float* __restrict__ dxs,
                                                             const int32_t* __restrict__ inv, int K, int64_t H,
                                                             float* __restrict__ dx) {
   const int64_t t = blockIdx.x;
-  for (int64_t c = threadIdx.x; c < H; c += 256) {
-    float acc = 0.f;
+  for (int64_t c = V * threadIdx.x; c < H; c += 256 * V) {
+    FVec<V> acc = {};
+#pragma unroll 8
     for (int k = 0; k < K; ++k) {
       const int p = inv[t * K + k];
-      if (p >= 0) acc += dxs[(int64_t)p * H + c];
+      const FVec<V> y = ldv<V>(dxs + (int64_t)max(p, 0) * H + c);
+#pragma unroll
+      for (int e = 0; e < V; ++e) acc.v[e] = p >= 0 ? acc.v[e] + y.v[e] : acc.v[e];
     }
-    dx[t * H + c] = acc;
+    stv<V>(dx + t * H + c, acc);
   }
 }
 
@@ -532,17 +845,22 @@ __global__ __launch_bounds__(256) void route_prenorm_bwd_f32_kernel(const float*
   }
 }
 
+template <int V>
 __global__ __launch_bounds__(256) void gate_mul_f32_kernel(const float* __restrict__ y, const float* __restrict__ s,
                                                            const float* __restrict__ base, int64_t H,
                                                            float* __restrict__ out) {
   const int64_t t = blockIdx.x;
   const float sg = sigmoid32(s[t]);
-  for (int64_t c = threadIdx.x; c < H; c += 256) {
-    const float v = y[t * H + c] * sg;
-    out[t * H + c] = base ? base[t * H + c] + v : v;
+  for (int64_t c = V * threadIdx.x; c < H; c += 256 * V) {
+    FVec<V> v = ldv<V>(y + t * H + c);
+    const FVec<V> b = base ? ldv<V>(base + t * H + c) : FVec<V>{};
+#pragma unroll
+    for (int e = 0; e < V; ++e) v.v[e] = base ? b.v[e] + v.v[e] * sg : v.v[e] * sg;
+    stv<V>(out + t * H + c, v);
   }
 }
 
+template <int V>
 __global__ __launch_bounds__(256) void gate_mul_bwd_f32_kernel(const float* __restrict__ y,
                                                                const float* __restrict__ s,
                                                                const float* __restrict__ dout, int64_t H,
@@ -551,10 +869,15 @@ __global__ __launch_bounds__(256) void gate_mul_bwd_f32_kernel(const float* __re
   const int64_t t = blockIdx.x;
   const float sg = sigmoid32(s[t]);
   float dot = 0.f;
-  for (int64_t c = threadIdx.x; c < H; c += 256) {
-    const float d = dout[t * H + c];
-    dy[t * H + c] = d * sg;
-    dot += d * y[t * H + c];
+  for (int64_t c = V * threadIdx.x; c < H; c += 256 * V) {
+    FVec<V> d = ldv<V>(dout + t * H + c);
+    const FVec<V> yv = ldv<V>(y + t * H + c);
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      dot += d.v[e] * yv.v[e];
+      d.v[e] *= sg;
+    }
+    stv<V>(dy + t * H + c, d);
   }
   dot = block_sum(dot, red);
   if (threadIdx.x == 0) ds[t] = dot * sg * (1.0f - sg);
@@ -588,17 +911,51 @@ extern "C" int smel_gmm_f32(const smel_wset_f32* w, int32_t trans, const int32_t
   SMEL_REQUIRE(!(w->kinds & (1 << SMEL_KIND_SEL)) || w->wsel, SMEL_EINVAL, "smel_gmm_f32: no selected weights");
   SMEL_REQUIRE(!(w->kinds & (1 << SMEL_KIND_SHARED)) || w->wsh, SMEL_EINVAL, "smel_gmm_f32: no shared weights");
   if (max_tiles == 0) return 0;
-  const bool vec = aligned16(A) && lda % 4 == 0 && w->C % 4 == 0 && (!w->wf || aligned16(w->wf)) &&
-                   (!w->wsel || aligned16(w->wsel)) && (!w->wsh || aligned16(w->wsh));
-  const dim3 grid((unsigned)max_tiles, (unsigned)((N + FB - 1) / FB));
+  // bit 0: A rows in 16-byte loads (32-bit offsets inside a tile); bit 1: every fp32 weight matrix too
+  const int vec = (aligned16(A) && lda % 4 == 0 && K % 4 == 0 && lda < (1 << 22) ? 1 : 0) |
+                  (w->C % 4 == 0 && w->R * w->C < (1 << 29) && (!w->wf || aligned16(w->wf)) && (!w->wsel || aligned16(w->wsel)) &&
+                           (!w->wsh || aligned16(w->wsh))
+                       ? 2
+                       : 0);
+  // 16 nibbles in one 8-byte load under one scale / zero pair
+  const int qvec = w->q4 && w->C % 16 == 0 && w->group % 16 == 0 && w->C * w->group < (1LL << 32) &&
+                   ((uintptr_t)w->q4 & 7) == 0 && ((uintptr_t)w->scale & 1) == 0 && ((uintptr_t)w->zero & 1) == 0;
   const int b1 = beta != 0.f;
-  if (trans == 0) {
-    if (vec) gmm_f32_kernel<0, true><<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, A, lda, alpha, b1, C, ldc);
-    else gmm_f32_kernel<0, false><<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, A, lda, alpha, b1, C, ldc);
-  } else {
-    if (vec) gmm_f32_kernel<1, true><<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, A, lda, alpha, b1, C, ldc);
-    else gmm_f32_kernel<1, false><<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, A, lda, alpha, b1, C, ldc);
+  const unsigned mt = (unsigned)max_tiles;
+  if (N <= 64) {   // at most one column block of the staged kernel: the whole K of a row tile in one block is the latency
+    const dim3 grid(mt, 1, 4);
+#define SKINNY(TR, NF) \
+  gmm_f32_skinny_kernel<TR, NF><<<grid, 512, 0, stream>>>(*w, gkind, tiles, n_tiles, A, lda, vec, alpha, b1, C, ldc)
+    if (trans == 0) {
+      if (N <= 16) SKINNY(0, 1);
+      else if (N <= 32) SKINNY(0, 2);
+      else SKINNY(0, 4);
+    } else {
+      if (N <= 16) SKINNY(1, 1);
+      else if (N <= 32) SKINNY(1, 2);
+      else SKINNY(1, 4);
+    }
+#undef SKINNY
+    return smel::launch_status();
   }
+  // two 64 x 128 blocks fit a CU: below that count the quarter tiles (32 x 64) fill more of the chip
+  const int64_t wide = max_tiles * ((N + 127) / 128);
+  const bool small = wide < 512;
+  const int64_t ncol = small ? (N + 63) / 64 : (N + 127) / 128;
+  const int64_t blocks = (max_tiles + 7) / 8 * 8 * ncol;
+  SMEL_REQUIRE(blocks < (1LL << 31), SMEL_EUNSUPPORTED, "smel_gmm_f32: too many blocks");
+  const dim3 grid((unsigned)blocks, 1, small ? 2 : 1);
+#define STAGED(TR, RB, NT, KS, FK)                                                                                \
+  gmm_f32_kernel<TR, RB, NT, KS, FK>                                                                              \
+      <<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, vec, qvec, GemmArgs{A, lda, alpha, b1, C, ldc})
+  if (trans == 0) {
+    if (small) STAGED(0, 32, 64, 4, 64);
+    else STAGED(0, 64, 128, 1, 32);
+  } else {
+    if (small) STAGED(1, 32, 64, 4, 64);
+    else STAGED(1, 64, 128, 1, 32);
+  }
+#undef STAGED
   return smel::launch_status();
 }
 
@@ -609,14 +966,18 @@ extern "C" int smel_wgrad_f32(const float* X, int64_t ldx, const float* Y, int64
   SMEL_REQUIRE(M > 0 && N > 0 && ldx >= M && ldy >= N && n_jobs >= 0 && n_jobs < 65536 && c_stride >= M * N,
                SMEL_EINVAL, "smel_wgrad_f32: bad sizes");
   if (n_jobs == 0) return 0;
-  const int64_t tiles = ((M + FB - 1) / FB) * ((N + FB - 1) / FB);
+  // the narrower side in 16-column slices, the wider one in 16-byte loads of 64 columns per block
+  const bool swap = N < M;
+  const int64_t ns = swap ? N : M, nb = swap ? M : N, lds_ = swap ? ldy : ldx, ldb = swap ? ldx : ldy;
+  const float *S = swap ? Y : X, *B = swap ? X : Y;
+  const int64_t tiles = ((ns + 15) / 16) * ((nb + 63) / 64);
   SMEL_REQUIRE(tiles < (1 << 30), SMEL_EINVAL, "smel_wgrad_f32: output too large");
-  const bool vec = aligned16(X) && aligned16(Y) && ldx % 4 == 0 && ldy % 4 == 0;
+  const int vec = aligned16(B) && ldb % 4 == 0;
   const dim3 grid((unsigned)tiles, (unsigned)n_jobs);
-  if (vec)
-    wgrad_f32_kernel<true><<<grid, 256, 0, stream>>>(X, ldx, Y, ldy, offsets, job_group, M, N, alpha, C, c_stride);
+  if (swap)
+    wgrad_f32_kernel<1><<<grid, 512, 0, stream>>>(S, lds_, ns, B, ldb, nb, offsets, job_group, vec, N, alpha, C, c_stride);
   else
-    wgrad_f32_kernel<false><<<grid, 256, 0, stream>>>(X, ldx, Y, ldy, offsets, job_group, M, N, alpha, C, c_stride);
+    wgrad_f32_kernel<0><<<grid, 512, 0, stream>>>(S, lds_, ns, B, ldb, nb, offsets, job_group, vec, N, alpha, C, c_stride);
   return smel::launch_status();
 }
 
@@ -625,7 +986,10 @@ extern "C" int smel_gather_rows_f32(const float* src, int64_t lds, const int32_t
   SMEL_REQUIRE(src && idx && out && div > 0 && n >= 0 && cols > 0 && lds >= cols && n < (1LL << 31), SMEL_EINVAL,
                "smel_gather_rows_f32: bad arguments");
   if (n == 0) return 0;
-  gather_rows_f32_kernel<<<(unsigned)n, 256, 0, stream>>>(src, lds, idx, div, n_valid, cols, out);
+  if (cols % 4 == 0 && lds % 4 == 0 && aligned16(src) && aligned16(out))
+    gather_rows_f32_kernel<4><<<(unsigned)n, 256, 0, stream>>>(src, lds, idx, div, n_valid, cols, out);
+  else
+    gather_rows_f32_kernel<1><<<(unsigned)n, 256, 0, stream>>>(src, lds, idx, div, n_valid, cols, out);
   return smel::launch_status();
 }
 
@@ -635,7 +999,10 @@ extern "C" int smel_act_gate_f32(const float* h, int64_t ldh, int64_t rows, int6
                    rows < (1LL << 31),
                SMEL_EINVAL, "smel_act_gate_f32: bad arguments");
   if (rows == 0) return 0;
-  act_gate_f32_kernel<<<(unsigned)rows, 256, 0, stream>>>(h, ldh, I, act, a, lda);
+  if (I % 4 == 0 && ldh % 4 == 0 && lda % 4 == 0 && aligned16(h) && aligned16(a))
+    act_gate_f32_kernel<4><<<(unsigned)rows, 256, 0, stream>>>(h, ldh, I, act, a, lda);
+  else
+    act_gate_f32_kernel<1><<<(unsigned)rows, 256, 0, stream>>>(h, ldh, I, act, a, lda);
   return smel::launch_status();
 }
 
@@ -645,7 +1012,10 @@ extern "C" int smel_act_gate_bwd_f32(const float* h, int64_t ldh, const float* d
                    (act == 0 || act == 1) && rows < (1LL << 31),
                SMEL_EINVAL, "smel_act_gate_bwd_f32: bad arguments");
   if (rows == 0) return 0;
-  act_gate_bwd_f32_kernel<<<(unsigned)rows, 256, 0, stream>>>(h, ldh, da, ldda, I, act, dh, lddh);
+  if (I % 4 == 0 && ldh % 4 == 0 && ldda % 4 == 0 && lddh % 4 == 0 && aligned16(h) && aligned16(da) && aligned16(dh))
+    act_gate_bwd_f32_kernel<4><<<(unsigned)rows, 256, 0, stream>>>(h, ldh, da, ldda, I, act, dh, lddh);
+  else
+    act_gate_bwd_f32_kernel<1><<<(unsigned)rows, 256, 0, stream>>>(h, ldh, da, ldda, I, act, dh, lddh);
   return smel::launch_status();
 }
 
@@ -654,7 +1024,10 @@ extern "C" int smel_combine_f32(const float* ys, const float* topv, const int32_
   SMEL_REQUIRE(ys && topv && inv && out && T >= 0 && K > 0 && K <= 64 && H > 0 && T < (1LL << 31), SMEL_EINVAL,
                "smel_combine_f32: bad arguments");
   if (T == 0) return 0;
-  combine_f32_kernel<<<(unsigned)T, 256, 0, stream>>>(ys, topv, inv, (int)K, H, out);
+  if (H % 4 == 0 && aligned16(ys) && aligned16(out))
+    combine_f32_kernel<4><<<(unsigned)T, 256, 0, stream>>>(ys, topv, inv, (int)K, H, out);
+  else
+    combine_f32_kernel<1><<<(unsigned)T, 256, 0, stream>>>(ys, topv, inv, (int)K, H, out);
   return smel::launch_status();
 }
 
@@ -663,7 +1036,10 @@ extern "C" int smel_combine_bwd_f32(const float* ys, const float* dout, const fl
   SMEL_REQUIRE(ys && dout && topv && inv && dys && dtopv && T >= 0 && K > 0 && K <= 64 && H > 0 && T < (1LL << 31),
                SMEL_EINVAL, "smel_combine_bwd_f32: bad arguments");
   if (T == 0) return 0;
-  combine_bwd_f32_kernel<<<(unsigned)T, 256, 0, stream>>>(ys, dout, topv, inv, (int)K, H, dys, dtopv);
+  if (H % 4 == 0 && aligned16(ys) && aligned16(dout) && aligned16(dys))
+    combine_bwd_f32_kernel<4><<<dim3((unsigned)T, (unsigned)K), 256, 0, stream>>>(ys, dout, topv, inv, (int)K, H, dys, dtopv);
+  else
+    combine_bwd_f32_kernel<1><<<dim3((unsigned)T, (unsigned)K), 256, 0, stream>>>(ys, dout, topv, inv, (int)K, H, dys, dtopv);
   return smel::launch_status();
 }
 
@@ -672,7 +1048,10 @@ extern "C" int smel_dx_reduce_f32(const float* dxs, const int32_t* inv, int64_t 
   SMEL_REQUIRE(dxs && inv && dx && T >= 0 && K > 0 && K <= 64 && H > 0 && T < (1LL << 31), SMEL_EINVAL,
                "smel_dx_reduce_f32: bad arguments");
   if (T == 0) return 0;
-  dx_reduce_f32_kernel<<<(unsigned)T, 256, 0, stream>>>(dxs, inv, (int)K, H, dx);
+  if (H % 4 == 0 && aligned16(dxs) && aligned16(dx))
+    dx_reduce_f32_kernel<4><<<(unsigned)T, 256, 0, stream>>>(dxs, inv, (int)K, H, dx);
+  else
+    dx_reduce_f32_kernel<1><<<(unsigned)T, 256, 0, stream>>>(dxs, inv, (int)K, H, dx);
   return smel::launch_status();
 }
 
@@ -727,7 +1106,10 @@ extern "C" int smel_gate_mul_f32(const float* y, const float* s, const float* ba
                                  hipStream_t stream) {
   SMEL_REQUIRE(y && s && out && T >= 0 && H > 0 && T < (1LL << 31), SMEL_EINVAL, "smel_gate_mul_f32: bad arguments");
   if (T == 0) return 0;
-  gate_mul_f32_kernel<<<(unsigned)T, 256, 0, stream>>>(y, s, base, H, out);
+  if (H % 4 == 0 && aligned16(y) && aligned16(out) && aligned16(base))
+    gate_mul_f32_kernel<4><<<(unsigned)T, 256, 0, stream>>>(y, s, base, H, out);
+  else
+    gate_mul_f32_kernel<1><<<(unsigned)T, 256, 0, stream>>>(y, s, base, H, out);
   return smel::launch_status();
 }
 
@@ -736,6 +1118,9 @@ extern "C" int smel_gate_mul_bwd_f32(const float* y, const float* s, const float
   SMEL_REQUIRE(y && s && dout && dy && ds && T >= 0 && H > 0 && T < (1LL << 31), SMEL_EINVAL,
                "smel_gate_mul_bwd_f32: bad arguments");
   if (T == 0) return 0;
-  gate_mul_bwd_f32_kernel<<<(unsigned)T, 256, 0, stream>>>(y, s, dout, H, dy, ds);
+  if (H % 4 == 0 && aligned16(y) && aligned16(dout) && aligned16(dy))
+    gate_mul_bwd_f32_kernel<4><<<(unsigned)T, 256, 0, stream>>>(y, s, dout, H, dy, ds);
+  else
+    gate_mul_bwd_f32_kernel<1><<<(unsigned)T, 256, 0, stream>>>(y, s, dout, H, dy, ds);
   return smel::launch_status();
 }

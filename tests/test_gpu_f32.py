@@ -86,6 +86,81 @@ def test_gmm_f32_against_fp64(trans, kind, pad):
     _check(Cd.cpu(), ref, "C", tol=1e-6)
 
 
+# (row counts of the groups, one matrix [R][C], int4 group): the tile shapes and load forms of smel_gmm_f32. The first
+# has enough tiles for the 64 x 128 blocks (every number of 16-row slices, N and K over an edge); the next ones the
+# 32 x 64 blocks (whole, with C not a multiple of 16, a group that is no power of two); then few output columns.
+_MANY = [1, 16, 17, 33, 48, 49, 64, 65, 100, 0, 130, 5] * 6
+GMM_SHAPES = [(_MANY, 840, 80, 16), ([40, 3, 70], 208, 144, 16), ([40, 3, 70], 132, 68, 4), ([65, 9], 192, 96, 48),
+              ([70, 20], 1, 300, 4), ([33], 8, 2048, 64), ([64, 1], 16, 37 * 2, 2), ([50], 24, 132, 4),
+              ([30, 17], 64, 512, 64)]
+
+
+@pytest.mark.parametrize("kind", ["int4", "int4_bf16", "fp32"])
+@pytest.mark.parametrize("trans", [0, 1])
+@pytest.mark.parametrize("shape", range(len(GMM_SHAPES)))
+def test_gmm_f32_shapes_against_fp64(shape, trans, kind):
+    """Every block shape and load form of smel_gmm_f32, forward and transposed, against the fp64 product; columns and
+    rows outside the result stay untouched. Bound: sums of K <= 2048 fp32 products (rounded to 2^-24 each, errors adding
+    as their square root against a sum that grows the same way) stay well inside 1e-6."""
+    from smel import _lib as L
+    from smel import moe_f32 as F
+    counts, Rw, Cw, group = GMM_SHAPES[shape]
+    if trans:
+        Rw, Cw = (Cw, Rw) if kind == "fp32" or Rw % group == 0 else (Cw, (Rw + group - 1) // group * group)
+    _say(f"gmm_f32 {Rw}x{Cw} trans={trans} kind={kind}")
+    torch.manual_seed(shape)
+    E, rows = len(counts), sum(counts)
+    if kind.startswith("int4"):
+        q = _int4_bank(E, Rw, Cw, group, shape)
+        W = R.dequant_int4(q["q"], q["scale"], q["zero"],
+                           torch.bfloat16 if kind == "int4_bf16" else torch.float32).double()
+        dq = {k: v.to(DEV) for k, v in q.items()}
+        w = F._ws(Rw, Cw, 1 << L.KIND_INT4, q4=L.ptr(dq["q"]), scale=L.ptr(dq["scale"]), zero=L.ptr(dq["zero"]))
+        w.group, w.q4_round_bf16 = group, int(kind == "int4_bf16")
+    else:
+        Wf = torch.randn(E, Rw, Cw) * 0.05
+        W, Wd = Wf.double(), Wf.to(DEV)
+        w = F._ws(Rw, Cw, 1 << L.KIND_BF16, wf=L.ptr(Wd))
+    K, N = (Rw, Cw) if trans else (Cw, Rw)
+    tl, _ = F.count_tiles(counts, L.KIND_INT4 if kind.startswith("int4") else L.KIND_BF16, DEV)
+    A, C0 = torch.randn(rows, K), torch.randn(rows + 1, N + 3)
+    Ad = A.to(DEV)
+    for beta in (0.0, 1.0):
+        Cd = C0.to(DEV)
+        F.gmm(w, trans, tl, Ad, K, Cd, N + 3, alpha=0.5, beta=beta)
+        ref = C0.double().clone()
+        ref[:rows, :N] *= beta
+        r = 0
+        for e, c in enumerate(counts):
+            ref[r:r + c, :N] += 0.5 * (A[r:r + c].double() @ (W[e] if trans else W[e].t()))
+            r += c
+        got = Cd.cpu()
+        _check(got[:rows, :N], ref[:rows, :N], "C", tol=1e-6)
+        assert torch.equal(got[:, N:], C0[:, N:]) and torch.equal(got[rows], C0[rows])
+
+
+@pytest.mark.parametrize("M,N", [(16, 200), (200, 16), (8, 36), (36, 33), (1, 64), (17, 65)])
+def test_wgrad_f32_shapes_against_fp64(M, N):
+    """smel_wgrad_f32 with either side the narrower one, sides off the block sizes, and row counts around the waves'
+    strides (one row to several rounds of 256)."""
+    from smel import moe_f32 as F
+    torch.manual_seed(M * N)
+    counts = [1, 255, 257, 900, 0, 31]
+    offs = torch.tensor([0] + list(itertools.accumulate(counts)), dtype=torch.int32)
+    X, Y = torch.randn(sum(counts), M), torch.randn(sum(counts), N + 4)
+    jobs = torch.arange(len(counts), dtype=torch.int32)
+    out = torch.full((len(counts), M, N), float("nan"), device=DEV)
+    Xd, Yd, od, jd = X.to(DEV), Y.to(DEV), offs.to(DEV), jobs.to(DEV)
+    F.wgrad(Xd, M, Yd, N + 4, od, jd, len(counts), M, N, 2.0, out)
+    for j in range(len(counts)):
+        r0, r1 = int(offs[j]), int(offs[j + 1])
+        ref = 2.0 * X[r0:r1].double().t() @ Y[r0:r1, :N].double()
+        if r1 == r0:
+            assert torch.equal(out[j].cpu(), torch.zeros(M, N))
+        else:
+            _check(out[j].cpu(), ref, f"job {j}", tol=1e-6)
+
+
 def test_wgrad_f32_against_fp64():
     """smel_wgrad_f32: per job, alpha X^T Y over its group's rows (an empty group writes zeros; M, N not multiples of
     64; rows not multiples of 16), against fp64."""
