@@ -43,13 +43,22 @@ int smel_ce_stats(const float* win_e, const float* win_s, int64_t nwin, int64_t 
 
 /* The gradient GEMM of vocabulary chunk number `chunk` (0, 1, ... in order) over its vc columns, with the head
  * transposed: WT [H][ldwt], column 0 = vocabulary id v0 (ldwt covers vc rounded up to 16 bytes). The chunk's columns
- * are split in two halves: acc [n][H] fp32 = (chunk == 0 ? 0 : r (acc + part[(chunk - 1) % 2])) + sum over the
- * first half of (P[v] 2^-shift) W[v], and part[chunk % 2] = the same sum over the second half (part: [2][n][H]
- * fp32; the gradient sum after the last chunk is acc + part[last % 2]). smel/loss.py:83-85
+ * are split in two halves: acc [n][H] fp32 = (chunk == 0 ? 0 : r acc) + sum over the first half of (P[v] 2^-shift) W[v],
+ * and part[chunk % 2] = (chunk == 0 ? 0 : r part[(chunk - 1) % 2]) + the same sum over the second half (part:
+ * [2][n][H] fp32; the gradient sum after the last chunk is acc + part[last % 2]). smel/loss.py:83-85
  * (`acc * r + p.to(h.dtype) @ W`), the product on MFMA. */
 int smel_ce_grad(const void* WT, int64_t ldwt, int64_t H, const void* P, int64_t ldp, int64_t vc,
                  const uint8_t* shift, int64_t ldn, const float* r, int64_t n, int32_t dtype, int32_t chunk,
                  float* acc, float* part, hipStream_t stream);
+
+/* The same product with the chunk's columns in `splits` parts (1..8), each with its own accumulator over the chunks:
+ * acc [splits][n][H] fp32, acc[s] = (chunk == 0 ? 0 : r acc[s]) + the sum over part s; the gradient sum after the last
+ * chunk is the sum of the parts. smel_ce_grad_splits: the number of parts that fills the GPU best for passes of n rows
+ * over chunks of vc columns (every chunk of a pass takes the same number). */
+int smel_ce_grad_splits(int64_t n, int64_t H, int64_t vc, int32_t dtype);
+int smel_ce_grad_split(const void* WT, int64_t ldwt, int64_t H, const void* P, int64_t ldp, int64_t vc,
+                       const uint8_t* shift, int64_t ldn, const float* r, int64_t n, int32_t dtype, int32_t chunk,
+                       int32_t splits, float* acc, hipStream_t stream);
 
 /* Per row: loss_rows = m ln 2 + log s - tz; with acc, g [n][ldg] in g_dtype = gscale ((acc + part) / s - td W[tgt])
  * (part: the last chunk's partial [n][H], may be null; no target row when tgt is outside [0, V)), the target row
@@ -58,6 +67,12 @@ int smel_ce_finish(const float* m, const float* s, const float* tz, const float*
                    const float* part, const void* W, int64_t ldw, const void* trows, const int64_t* tgt, int64_t V,
                    int64_t n, int64_t H, int32_t dtype, float gscale, void* g, int64_t ldg, int32_t g_dtype,
                    float* loss_rows, hipStream_t stream);
+
+/* The same with acc [splits][n][H] as smel_ce_grad_split leaves it, the parts added in order. */
+int smel_ce_finish_split(const float* m, const float* s, const float* tz, const float* td, const float* acc,
+                         int32_t splits, const void* W, int64_t ldw, const void* trows, const int64_t* tgt, int64_t V,
+                         int64_t n, int64_t H, int32_t dtype, float gscale, void* g, int64_t ldg, int32_t g_dtype,
+                         float* loss_rows, hipStream_t stream);
 
 /* total = (accumulate ? total : 0) + scale * sum of loss_rows, in fixed order (smel/loss.py:136-140). */
 int smel_ce_loss_sum(const float* loss_rows, int64_t n, float scale, int32_t accumulate, float* total,
@@ -70,6 +85,13 @@ int smel_ce_scale(void* x, int64_t n, int32_t dtype, const float* go, hipStream_
  * (made once per frozen head). */
 int smel_ce_transpose(const void* src, int64_t R, int64_t C, int64_t lds, void* dst, int64_t ldd, int32_t dtype,
                       hipStream_t stream);
+
+/* Rows of an int8 head (q [R][C], one scale per row in `dtype`, 0 bf16 or 2 fp16) as q * scale rounded once to `dtype`:
+ * rows [R][C] and, with wt, the same transposed: wt [C][ldt], columns R .. ldt - 1 zero. C a multiple of 8, rows and
+ * wt 16-byte aligned, ldt a multiple of 8. smel/quant.py:104-105 (dequant_int8_rows) and the head layout of
+ * smel_ce_grad in one pass. */
+int smel_ce_dequant8(const int8_t* q, const void* scale, int64_t R, int64_t C, int32_t dtype, void* rows, void* wt,
+                     int64_t ldt, hipStream_t stream);
 
 #ifdef __cplusplus
 }

@@ -10,12 +10,12 @@
 //   ce_stats   per row: chunk maximum E = max e, chunk sum, the running maximum nE = max(m, E) and sum
 //              s = s 2^(m - nE) + sum_w s_w 2^(e_w - nE), the accumulator's rescale r = 2^(m - nE), and per window
 //              the shift nE - e_w of its softmax terms. Every rescale is an exact power of two.
-//   ce_grad    (MFMA, 256 hidden x 256 token tile, 8 waves, the chunk's columns in two K halves):
-//              acc = r (acc + part_prev) + sum_v p'_v W_v over the first half, part = the second half's sum, with
+//   ce_grad    (MFMA, 256 hidden x 256 token tile, 8 waves, the chunk's columns in one to eight parts):
+//              acc_s = r acc_s + sum_v p'_v W_v over part s, with
 //              p' = p 2^-(shift): each 16-byte fragment of p is shifted in registers as it leaves LDS (bf16: one
 //              saturating 16-bit subtract of the exponent per value pair; fp16 / fp32: ldexp), so the products are
 //              the reference's `p.to(h.dtype) @ W` terms at the running maximum (smel/loss.py:85).
-//   ce_finish  per row: loss = nE ln 2 + log s - z_target, gradient row = (acc + part) / s - d_target W[target]
+//   ce_finish  per row: loss = nE ln 2 + log s - z_target, gradient row = sum_s acc_s / s - d_target W[target]
 //              (smel/loss.py:87-92), scaled and stored in the requested dtype; ce_loss_sum adds the rows' losses
 //              in fixed order.
 // The head operand of ce_grad is the head transposed ([H][V], one copy per frozen head, made by ce_transpose), so
@@ -271,24 +271,17 @@ struct LogitsArgs {
 
 constexpr int LG_NW = SMEL_CE_LG_NW, LG_NB = 8 / (LG_NW / 2);   // waves; token slices of 32 per wave
 
-template <int DT, bool CAP>
-__global__ __launch_bounds__(64 * LG_NW) __attribute__((amdgpu_waves_per_eu(LG_NW / 4, LG_NW / 4))) void
-ce_logits_kernel(LogitsArgs a) {
-  using R = Ring<SMEL_CE_LG_KB, LG_NB, SMEL_CE_LG_NST, LG_NW>;
-  static_assert(R::B_ROWS == 256, "256-row token tiles");
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[R::BYTES];
-  const int b = blockIdx.x, x = b % NXCD, jj = b / NXCD;
-  // blocks b, b + 8, ... run on one XCD: it takes vocabulary tiles x, x + 8, ... with all token tiles of each in a
-  // row, so one vocabulary tile's head rows are read from that XCD's L2 by all its token tiles
-  const int tt = jj % a.n_tt, vt = (jj / a.n_tt) * NXCD + x;
-  if (vt >= a.n_vt) return;
+// One tile: NB = LG_NB for 256 token rows, LG_NB / 2 for a tile that holds at most 128.
+template <int DT, bool CAP, int NB>
+SMEL_DEV void ce_logits_tile(const LogitsArgs& a, uint8_t* smem, int vt, int tt) {
+  using R = Ring<SMEL_CE_LG_KB, NB, SMEL_CE_LG_NST, LG_NW>;
   constexpr int E = ebytes<DT>();
   const int lane = lane_id(), h = lane >> 5, r32 = lane & 31;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = w & 1, wn = w >> 1;
   const int a0 = vt * VT, b0 = tt * 256;
   const int kbytes = a.K * E;
-  const int a_valid = min(VT, a.vc - a0), b_valid = min(256, a.n - b0);
+  const int a_valid = min(VT, a.vc - a0), b_valid = min(R::B_ROWS, a.n - b0);
   const rsrc_t ra = make_rsrc(static_cast<const uint8_t*>(a.W) + (int64_t)a0 * a.ldw * E,
                               (uint64_t)(a_valid - 1) * a.ldw * E + kbytes);
   const rsrc_t rb = make_rsrc(static_cast<const uint8_t*>(a.h) + (int64_t)b0 * a.ldh * E,
@@ -297,19 +290,19 @@ ce_logits_kernel(LogitsArgs a) {
   row_offsets<R>(aoff, w, lane, a_valid, (uint32_t)(a.ldw * E));
   row_offsets<R>(boff, w, lane, b_valid, (uint32_t)(a.ldh * E));
   // this lane's token rows' targets, loaded before the main loop (the epilogue would wait on them)
-  int tg[LG_NB];   // target - v0 - c0 (the window's first column), -1 when outside [0, 2^31)
+  int tg[NB];   // target - v0 - c0 (the window's first column), -1 when outside [0, 2^31)
 #pragma unroll
-  for (int n = 0; n < LG_NB; ++n) {
-    const int tok = b0 + 32 * LG_NB * wn + 32 * n + r32;
+  for (int n = 0; n < NB; ++n) {
+    const int tok = b0 + 32 * NB * wn + 32 * n + r32;
     const int64_t t = tok < a.n ? a.tgt[tok] - a.v0 - (a0 + 128 * wm) : -1;
     tg[n] = t >= 0 && t < INT32_MAX ? (int)t : -1;
   }
-  f32x16_t acc[4][LG_NB];
+  f32x16_t acc[4][NB];
 #pragma unroll
   for (int m = 0; m < 4; ++m)
 #pragma unroll
-    for (int n = 0; n < LG_NB; ++n) acc[m][n] = f32x16_t{};
-  nt_loop<DT, R, LG_NB>(acc, smem, ra, aoff, rb, boff, kbytes, 5 * (b / NXCD), [](int, bool) {},
+    for (int n = 0; n < NB; ++n) acc[m][n] = f32x16_t{};
+  nt_loop<DT, R, NB>(acc, smem, ra, aoff, rb, boff, kbytes, 5 * (int)(blockIdx.x / NXCD), [](int, bool) {},
                     [](int, int, const u32x4_t& v) { return v; });
   __syncthreads();   // every wave is done with the operand ring: the epilogue may use the LDS
 
@@ -325,7 +318,7 @@ ce_logits_kernel(LogitsArgs a) {
   // FULL: every column of the window lies in the chunk (all tiles but the chunk's last): no masking
   auto slice = [&](int n, auto full_tag) {
     constexpr bool FULL = decltype(full_tag)::value;
-    const int tok = b0 + 32 * LG_NB * wn + 32 * n + r32;
+    const int tok = b0 + 32 * NB * wn + 32 * n + r32;
     const bool tok_ok = tok < a.n;
     float mx = -INFINITY;
 #pragma unroll
@@ -374,7 +367,7 @@ ce_logits_kernel(LogitsArgs a) {
       }
     if constexpr (DT != 1) {
       if (a.P) {   // the slice's 32 token rows x 256 B: chunk k = 64 j + lane is row k / 16, 16-byte piece k % 16
-        const int tok_s = b0 + 32 * LG_NB * wn + 32 * n;
+        const int tok_s = b0 + 32 * NB * wn + 32 * n;
         uint8_t* pbase = static_cast<uint8_t*>(a.P) + ((int64_t)tok_s * a.ldp + c0) * E;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -394,7 +387,6 @@ ce_logits_kernel(LogitsArgs a) {
     const int tc64 = tok_ok ? tg[n] : -1;
     const bool here = tc64 >= 0 && tc64 < 128 && tc64 < ncol;
     if (__builtin_amdgcn_ballot_w64(here)) {
-      static_assert(LG_NW * 16384 <= R::BYTES, "per-wave staging / target scratch in the operand ring");
       float* zb = reinterpret_cast<float*>(smem + w * 16384) + r32 * 128;
 #pragma unroll
       for (int m = 0; m < 4; ++m)
@@ -412,56 +404,65 @@ ce_logits_kernel(LogitsArgs a) {
   };
   if (ncol >= 128) {
 #pragma unroll
-    for (int n = 0; n < LG_NB; ++n) slice(n, std::true_type{});
+    for (int n = 0; n < NB; ++n) slice(n, std::true_type{});
   } else {
 #pragma unroll
-    for (int n = 0; n < LG_NB; ++n) slice(n, std::false_type{});
+    for (int n = 0; n < NB; ++n) slice(n, std::false_type{});
   }
+}
+
+template <int DT, bool CAP>
+__global__ __launch_bounds__(64 * LG_NW) __attribute__((amdgpu_waves_per_eu(LG_NW / 4, LG_NW / 4))) void
+ce_logits_kernel(LogitsArgs a) {
+  using R = Ring<SMEL_CE_LG_KB, LG_NB, SMEL_CE_LG_NST, LG_NW>;
+  static_assert(R::B_ROWS == 256, "256-row token tiles");
+  static_assert(LG_NW * 16384 <= R::BYTES, "per-wave staging / target scratch in the operand ring");
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[R::BYTES];
+  const int b = blockIdx.x, x = b % NXCD, jj = b / NXCD;
+  // blocks b, b + 8, ... run on one XCD: it takes vocabulary tiles x, x + 8, ... with all token tiles of each in a
+  // row, so one vocabulary tile's head rows are read from that XCD's L2 by all its token tiles
+  const int tt = jj % a.n_tt, vt = (jj / a.n_tt) * NXCD + x;
+  if (vt >= a.n_vt) return;
+  if (a.n - 256 * tt > 128) ce_logits_tile<DT, CAP, LG_NB>(a, smem, vt, tt);
+  else ce_logits_tile<DT, CAP, LG_NB / 2>(a, smem, vt, tt);
 }
 
 // ------------------------------------------------------------------------------------------------ ce_grad
 // Tiles of 256 hidden x 256 token rows (the tile size sets the FLOPs per byte loaded, which bounds these GEMMs), the
-// chunk's K range split in two halves so that 4092 x 2048 outputs still give 256 workgroups: the first half adds
-// into the accumulator, acc = r (acc + part_prev) + sum_first_half, the second half writes its sum to a partial
-// buffer part[c % 2] (c = chunk index; the next chunk's first half folds it in, the finish adds the last one).
+// chunk's K range in `splits` parts so that the tiles of a pass fill the 256 CUs (grad_splits picks the number). Each
+// part keeps its own accumulator over the chunks, acc_s = r acc_s + its sum: one writer per element, no exchange between
+// parts; the finish adds the parts in order.
 struct GradArgs {
   const void* WT;        // transposed head [H][ldwt], column 0 = vocabulary id v0 of the chunk
   const void* P;         // softmax terms [n][ldp]
   const uint8_t* shift;  // [nwin][ldn]
   const float* r;        // accumulator rescale per row
-  float* acc;            // [n][H] fp32
-  float* part;           // [2][n][H] fp32 partials of the second halves
+  float* acc;            // part 0's accumulator [n][H] fp32
+  const float* prev;     // parts 1 ..: [splits - 1][n][H] as the chunk before left them
+  float* part;           //             and where this chunk's go (the same place, or another)
   int64_t ldwt, ldp, ldn;
-  int H, n, kbytes, first, parity;
+  int H, n, kbytes, first, splits;
   int n_ht, n_tt;        // 256-row hidden tiles, 256-row token tiles
 };
 
 constexpr int GR_NW = SMEL_CE_GR_NW, GR_NB = 8 / (GR_NW / 2);
 constexpr int GR_SP = 528;   // epilogue staging row pitch: 128 fp32 + 16 B (rows start on different banks)
 
-template <int DT>
-__global__ __launch_bounds__(64 * GR_NW) __attribute__((amdgpu_waves_per_eu(GR_NW / 4, GR_NW / 4))) void
-ce_grad_kernel(GradArgs a) {
-  using R = Ring<SMEL_CE_GR_KB, GR_NB, SMEL_CE_GR_NST, GR_NW>;
-  static_assert(R::B_ROWS == 256, "256-row token tiles");
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[R::BYTES > GR_NW * 32 * GR_SP ? R::BYTES : GR_NW * 32 * GR_SP];
-  // the list (half, token tile, hidden tile), XCD x a contiguous run of it: one XCD's tiles share their token
-  // tiles' softmax terms and the hidden tiles' head columns of one K half in its L2
-  const int n_tiles = a.n_ht * a.n_tt;
-  int item, unused;
-  if (!xcd_tile_chunk(2 * n_tiles, 1, item, unused)) return;
-  const int half = item / n_tiles, tile = item % n_tiles;
-  const int tt = tile / a.n_ht, ht = tile % a.n_ht;
+template <int DT, int NB>
+SMEL_DEV void ce_grad_tile(const GradArgs& a, uint8_t* smem, int split, int tt, int ht) {
+  using R = Ring<SMEL_CE_GR_KB, NB, SMEL_CE_GR_NST, GR_NW>;
   constexpr int E = ebytes<DT>();
   const int lane = lane_id(), h = lane >> 5, r32 = lane & 31;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = w & 1, wn = w >> 1;
   const int a0 = ht * 256, b0 = tt * 256;
-  const int a_valid = min(256, a.H - a0), b_valid = min(256, a.n - b0);
-  // the halves: k-steps [0, nk / 2) and [nk / 2, nk) of the chunk
-  const int nk = (a.kbytes + R::KB - 1) / R::KB;
-  const int klo = half ? (nk / 2) * R::KB : 0;
-  const int kbytes = half ? a.kbytes - klo : (nk / 2) * R::KB;
+  const int a_valid = min(256, a.H - a0), b_valid = min(R::B_ROWS, a.n - b0);
+  // Part s of the chunk in whole statistics windows, [nw s / splits, nw (s + 1) / splits): the loop below starts at a
+  // rotation and wraps to the part's first k-step, where the shifts of a window are only loaded if one begins.
+  constexpr int STEPS_PER_WIN = WIN * ebytes<DT>() / R::KB;
+  const int nw = (a.kbytes + STEPS_PER_WIN * R::KB - 1) / (STEPS_PER_WIN * R::KB);
+  const int klo = (int)((int64_t)nw * split / a.splits) * STEPS_PER_WIN * R::KB;
+  const int kbytes = min(a.kbytes, (int)((int64_t)nw * (split + 1) / a.splits) * STEPS_PER_WIN * R::KB) - klo;
   const rsrc_t ra = make_rsrc(static_cast<const uint8_t*>(a.WT) + (int64_t)a0 * a.ldwt * E,
                               (uint64_t)(a_valid - 1) * a.ldwt * E + a.kbytes);
   const rsrc_t rb = make_rsrc(static_cast<const uint8_t*>(a.P) + (int64_t)b0 * a.ldp * E,
@@ -473,19 +474,18 @@ ce_grad_kernel(GradArgs a) {
   for (int ii = 0; ii < R::VM_A; ++ii) aoff[ii] += (uint32_t)klo;   // an OOB offset stays past the buffer
 #pragma unroll
   for (int ii = 0; ii < R::VM_B; ++ii) boff[ii] += (uint32_t)klo;
-  f32x16_t acc[4][GR_NB];
+  f32x16_t acc[4][NB];
 #pragma unroll
   for (int m = 0; m < 4; ++m)
 #pragma unroll
-    for (int n = 0; n < GR_NB; ++n) acc[m][n] = f32x16_t{};
+    for (int n = 0; n < NB; ++n) acc[m][n] = f32x16_t{};
   // shifts of this lane's token rows: the window of k-step kk (of the chunk) is kk * KB / (WIN * E)
-  constexpr int STEPS_PER_WIN = WIN * E / R::KB;
   const int kbase = klo / R::KB;
-  const int tok0 = b0 + 32 * GR_NB * wn + r32;
-  uint32_t sh_cur[GR_NB], sh_next[GR_NB];
-  auto load_sh = [&](int win, uint32_t (&dst)[GR_NB]) {
+  const int tok0 = b0 + 32 * NB * wn + r32;
+  uint32_t sh_cur[NB], sh_next[NB];
+  auto load_sh = [&](int win, uint32_t (&dst)[NB]) {
 #pragma unroll
-    for (int n = 0; n < GR_NB; ++n) {
+    for (int n = 0; n < NB; ++n) {
       const int tok = tok0 + 32 * n;
       dst[n] = tok < a.n ? (uint32_t)a.shift[(int64_t)win * a.ldn + tok] : (uint32_t)SHIFT_ZERO;
     }
@@ -505,11 +505,11 @@ ce_grad_kernel(GradArgs a) {
     if (n == 0 && wj != cur_win) {
       cur_win = wj;
 #pragma unroll
-      for (int q = 0; q < GR_NB; ++q) sh_cur[q] = sh_next[q];
+      for (int q = 0; q < NB; ++q) sh_cur[q] = sh_next[q];
     }
     return shift_chunk<DT>(v, sh_cur[n]);
   };
-  nt_loop<DT, R, GR_NB>(acc, smem, ra, aoff, rb, boff, kbytes, 5 * (int)(blockIdx.x / NXCD), pre, fix);
+  nt_loop<DT, R, NB>(acc, smem, ra, aoff, rb, boff, kbytes, 5 * (int)(blockIdx.x / NXCD), pre, fix);
 
   // ---- epilogue: acc[m][n][r] = term of hidden column a0 + 128 wm + 32 m + 8 (r / 4) + 4 h + r % 4 and token
   // row tok0 + 32 n. Per token slice the wave stages its 32 rows x 128 columns in LDS (the ring is free) and writes
@@ -517,18 +517,18 @@ ce_grad_kernel(GradArgs a) {
   __syncthreads();
   uint8_t* stg = smem + w * (32 * GR_SP);
   const size_t nh = (size_t)a.n * a.H;
-  const float* prev = a.part + (size_t)(a.parity ^ 1) * nh;
-  float* mine = a.part + (size_t)a.parity * nh;
+  const float* prev = split ? a.prev + (split - 1) * nh : a.acc;
+  float* mine = split ? a.part + (split - 1) * nh : a.acc;
   const int col0 = a0 + 128 * wm;
 #pragma unroll
-  for (int n = 0; n < GR_NB; ++n) {
+  for (int n = 0; n < NB; ++n) {
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         *reinterpret_cast<f32x4_t*>(stg + r32 * GR_SP + (32 * m + 8 * q + 4 * h) * 4) =
             f32x4_t{acc[m][n][4 * q], acc[m][n][4 * q + 1], acc[m][n][4 * q + 2], acc[m][n][4 * q + 3]};
-    const int tok_s = b0 + 32 * GR_NB * wn + 32 * n;
+    const int tok_s = b0 + 32 * NB * wn + 32 * n;
 #pragma unroll
     for (int jj = 0; jj < 16; ++jj) {
       const int k = 64 * jj + lane, row = k >> 5, piece = k & 31;
@@ -536,20 +536,50 @@ ce_grad_kernel(GradArgs a) {
       f32x4_t v = *reinterpret_cast<const f32x4_t*>(stg + row * GR_SP + piece * 16);
       if (tok >= a.n || col >= a.H) continue;
       const size_t at = (size_t)tok * a.H + col;
-      if (half) {
-        *reinterpret_cast<f32x4_t*>(mine + at) = v;
-        continue;
-      }
       if (!a.first) {
         const float rr = a.r[tok];
-        const f32x4_t o = *reinterpret_cast<const f32x4_t*>(a.acc + at);
-        const f32x4_t pp = *reinterpret_cast<const f32x4_t*>(prev + at);
-        v = f32x4_t{fmaf(o[0] + pp[0], rr, v[0]), fmaf(o[1] + pp[1], rr, v[1]), fmaf(o[2] + pp[2], rr, v[2]),
-                    fmaf(o[3] + pp[3], rr, v[3])};
+        const f32x4_t o = *reinterpret_cast<const f32x4_t*>(prev + at);
+        v = f32x4_t{fmaf(o[0], rr, v[0]), fmaf(o[1], rr, v[1]), fmaf(o[2], rr, v[2]), fmaf(o[3], rr, v[3])};
       }
-      *reinterpret_cast<f32x4_t*>(a.acc + at) = v;
+      *reinterpret_cast<f32x4_t*>(mine + at) = v;
     }
   }
+}
+
+template <int DT>
+__global__ __launch_bounds__(64 * GR_NW) __attribute__((amdgpu_waves_per_eu(GR_NW / 4, GR_NW / 4))) void
+ce_grad_kernel(GradArgs a) {
+  using R = Ring<SMEL_CE_GR_KB, GR_NB, SMEL_CE_GR_NST, GR_NW>;
+  static_assert(R::B_ROWS == 256, "256-row token tiles");
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[R::BYTES > GR_NW * 32 * GR_SP ? R::BYTES : GR_NW * 32 * GR_SP];
+  // the list (part, token tile, hidden tile), XCD x a contiguous run of it: one XCD's tiles share their token
+  // tiles' softmax terms and the hidden tiles' head columns of one K part in its L2
+  const int n_tiles = a.n_ht * a.n_tt;
+  int item, unused;
+  if (!xcd_tile_chunk(a.splits * n_tiles, 1, item, unused)) return;
+  const int split = item / n_tiles, tile = item % n_tiles;
+  const int tt = tile / a.n_ht, ht = tile % a.n_ht;
+  if (a.n - 256 * tt > 128) ce_grad_tile<DT, GR_NB>(a, smem, split, tt, ht);
+  else ce_grad_tile<DT, GR_NB / 2>(a, smem, split, tt, ht);
+}
+
+// Number of K parts of a pass's gradient GEMM: the one with the shortest rounds(splits) x (k-steps of a part + what a
+// block costs beside them, about 10 steps for its first loads, epilogue and accumulator), one block per CU.
+// Measured (one chunk of 32768 columns): 777 x 2816 (44 tiles) with two parts 410 us, five 231 us; 4092 x 2048 (128 tiles)
+// keeps two, 597 us.
+constexpr int MAX_SPLITS = 8;
+int grad_splits(int64_t n, int64_t H, int64_t vc, int E) {
+  const int64_t tiles = ((H + 255) / 256) * ((n + 255) / 256), nk = (vc * E + SMEL_CE_GR_KB - 1) / SMEL_CE_GR_KB;
+  int best = 1;
+  int64_t cost = INT64_MAX;
+  for (int s = 1; s <= MAX_SPLITS; ++s) {
+    const int64_t c = ((tiles * s + 255) / 256) * ((nk + s - 1) / s + 10);
+    if (c < cost) {
+      cost = c;
+      best = s;
+    }
+  }
+  return best;
 }
 
 // ------------------------------------------------------------------------------------------------ small kernels
@@ -645,7 +675,8 @@ template <int DT, int GT>
 __global__ __launch_bounds__(256) void ce_finish_kernel(const float* __restrict__ m, const float* __restrict__ s,
                                                         const float* __restrict__ tz, const float* __restrict__ td,
                                                         const float* __restrict__ acc,
-                                                        const float* __restrict__ part, const void* __restrict__ W,
+                                                        const float* __restrict__ part, int n_part,
+                                                        const void* __restrict__ W,
                                                         int64_t ldw, const void* __restrict__ trows,
                                                         const int64_t* __restrict__ tgt, int64_t V, int64_t H,
                                                         float gscale, void* g, int64_t ldg, float* loss_rows,
@@ -665,9 +696,10 @@ __global__ __launch_bounds__(256) void ce_finish_kernel(const float* __restrict_
       const f32x4_t a0 = *reinterpret_cast<const f32x4_t*>(acc + row * H + c);
       const f32x4_t a1 = *reinterpret_cast<const f32x4_t*>(acc + row * H + c + 4);
       f32x4_t p0 = f32x4_t{0.f, 0.f, 0.f, 0.f}, p1 = p0;
-      if (part) {
-        p0 = *reinterpret_cast<const f32x4_t*>(part + row * H + c);
-        p1 = *reinterpret_cast<const f32x4_t*>(part + row * H + c + 4);
+      for (int q = 0; q < n_part; ++q) {
+        const float* pp = part + (q * (int64_t)gridDim.x + row) * H + c;
+        p0 += *reinterpret_cast<const f32x4_t*>(pp);
+        p1 += *reinterpret_cast<const f32x4_t*>(pp + 4);
       }
       const u32x4_t wv = ok ? *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(wsrc) + wrow + c)
                             : u32x4_t{0u, 0u, 0u, 0u};
@@ -684,7 +716,9 @@ __global__ __launch_bounds__(256) void ce_finish_kernel(const float* __restrict_
   }
   for (int64_t c = threadIdx.x; c < H; c += 256) {
     const float wv = ok ? ld_t<DT>(wsrc, wrow + c) : 0.f;
-    const float v = (acc[row * H + c] + (part ? part[row * H + c] : 0.f)) * inv - d * wv;
+    float pv = 0.f;
+    for (int q = 0; q < n_part; ++q) pv += part[(q * (int64_t)gridDim.x + row) * H + c];
+    const float v = (acc[row * H + c] + pv) * inv - d * wv;
     st_t<GT>(g, row * ldg + c, v * gscale);
   }
 }
@@ -735,6 +769,75 @@ __global__ __launch_bounds__(256) void ce_transpose_kernel(const uint8_t* __rest
     if (c < C && r < ldd)
       for (int b = 0; b < E; ++b) dst[(c * ldd + r) * E + b] = tile[rr][cc * E + b];
   }
+}
+
+// The transposed head in 16-byte accesses: a 64 x 64 tile (E = 2: 8 KB) through LDS, each thread 16 elements of a row
+// in and 16 of a column out. dst columns R .. ldd - 1 are zeroed (rows past R read as zeros).
+// INT8: the source is int8 rows with one scale per row (of the rows' dtype DT): each value is q * scale rounded once to
+// that dtype (the products of quant.py's dequant_int8_rows), written both row-major (rows, pitch C) and transposed (dst;
+// may be null: rows only).
+// Bound: HBM. A 32768 x 2816 chunk of an int8 head (92 MB in, 2 x 185 MB out): 100 us = 4.6 TB/s, where the conversion
+// in three element-wise passes and a byte-wise transpose took about 400 us (the transpose 134 us of it).
+template <int DT, bool INT8>
+__global__ __launch_bounds__(256) void ce_head_kernel(const void* __restrict__ src, const void* __restrict__ scale,
+                                                      int64_t R, int64_t C, int64_t lds, void* __restrict__ rows,
+                                                      void* __restrict__ dst, int64_t ldd) {
+  static_assert(DT != 1, "16-bit rows");
+  constexpr int P = 66;   // tile pitch in elements: a column's rows on distinct banks, pairs of rows side by side
+  __shared__ uint16_t tile[64 * P];
+  const int64_t r0 = (int64_t)blockIdx.x * 64, c0 = (int64_t)blockIdx.y * 64;
+  const int t = threadIdx.x, rr = t >> 2, cc = 16 * (t & 3);
+  const int64_t r = r0 + rr, c = c0 + cc;
+  uint32_t v[8];   // 16 values of row r, columns c ..
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = 0;
+  if (r < R) {
+    if constexpr (INT8) {
+      const float sc = ld_t<DT>(scale, r);
+      const int8_t* p = static_cast<const int8_t*>(src) + r * lds + c;
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {   // C is a multiple of 8
+        if (c + 8 * hf >= C) break;
+        const uint2 q = *reinterpret_cast<const uint2*>(p + 8 * hf);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t w = i < 2 ? q.x : q.y;
+          const float lo = (float)(int8_t)(w >> (16 * (i & 1))) * sc, hi = (float)(int8_t)(w >> (16 * (i & 1) + 8)) * sc;
+          if constexpr (DT == 0) v[4 * hf + i] = pack2bf(lo, hi);
+          else v[4 * hf + i] = pack2h(lo, hi);
+        }
+      }
+    } else {
+      const uint16_t* p = static_cast<const uint16_t*>(src) + r * lds + c;
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        if (c + 8 * hf >= C) break;
+        const u32x4_t q = *reinterpret_cast<const u32x4_t*>(p + 8 * hf);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[4 * hf + i] = q[i];
+      }
+    }
+    if (INT8 && rows) {
+      uint16_t* o = static_cast<uint16_t*>(rows) + r * C + c;
+      if (c < C) *reinterpret_cast<u32x4_t*>(o) = u32x4_t{v[0], v[1], v[2], v[3]};
+      if (c + 8 < C) *reinterpret_cast<u32x4_t*>(o + 8) = u32x4_t{v[4], v[5], v[6], v[7]};
+    }
+  }
+  if (!dst) return;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {   // transposed into the tile: [column][row]
+    tile[(cc + 2 * i) * P + rr] = (uint16_t)v[i];
+    tile[(cc + 2 * i + 1) * P + rr] = (uint16_t)(v[i] >> 16);
+  }
+  __syncthreads();
+  const int oc = t >> 2, orow = 16 * (t & 3);
+  if (c0 + oc >= C) return;
+  const uint32_t* tp = reinterpret_cast<const uint32_t*>(&tile[oc * P + orow]);
+  uint16_t* o = static_cast<uint16_t*>(dst) + (c0 + oc) * ldd + r0 + orow;
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf)   // ldd is a multiple of 8
+    if (r0 + orow + 8 * hf < ldd)
+      *reinterpret_cast<u32x4_t*>(o + 8 * hf) = u32x4_t{tp[4 * hf], tp[4 * hf + 1], tp[4 * hf + 2], tp[4 * hf + 3]};
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -818,16 +921,18 @@ extern "C" int smel_ce_stats(const float* win_e, const float* win_s, int64_t nwi
   return smel::launch_status();
 }
 
-extern "C" int smel_ce_grad(const void* WT, int64_t ldwt, int64_t H, const void* P, int64_t ldp, int64_t vc,
-                            const uint8_t* shift, int64_t ldn, const float* r, int64_t n, int32_t dtype, int32_t chunk,
-                            float* acc, float* part, hipStream_t stream) {
+namespace {
+int ce_grad(const void* WT, int64_t ldwt, int64_t H, const void* P, int64_t ldp, int64_t vc, const uint8_t* shift,
+            int64_t ldn, const float* r, int64_t n, int32_t dtype, int32_t chunk, int32_t splits, float* acc,
+            const float* prev, float* part, hipStream_t stream) {
   SMEL_REQUIRE(SMEL_DT_OK(dtype), SMEL_EINVAL, "ce_grad: dtype %d (0 bf16, 1 fp32, 2 fp16)", dtype);
   const int E = dtype == 1 ? 4 : 2;
   SMEL_REQUIRE(n >= 0 && vc >= 1 && H >= 1 && ldn >= n && chunk >= 0, SMEL_EINVAL, "ce_grad: bad sizes");
   if (n == 0) return 0;
-  SMEL_REQUIRE(WT && P && shift && acc && part && (chunk == 0 || r), SMEL_EINVAL, "ce_grad: null pointer");
+  SMEL_REQUIRE(splits >= 1 && splits <= MAX_SPLITS, SMEL_EINVAL, "ce_grad: %d parts (1..%d)", splits, MAX_SPLITS);
+  SMEL_REQUIRE(WT && P && shift && acc && (splits == 1 || (part && prev)) && (chunk == 0 || r), SMEL_EINVAL, "ce_grad: null pointer");
   const int64_t kbytes = (vc * E + 15) / 16 * 16;
-  SMEL_REQUIRE(H % 4 == 0 && aligned16(acc) && aligned16(part) && aligned16(WT) && aligned16(P) &&
+  SMEL_REQUIRE(H % 4 == 0 && aligned16(acc) && aligned16(part) && aligned16(prev) && aligned16(WT) && aligned16(P) &&
                    (ldwt * E) % 16 == 0 && (ldp * E) % 16 == 0 && ldp * E >= kbytes && ldwt * E >= kbytes,
                SMEL_EUNSUPPORTED, "ce_grad: rows must be 16-byte aligned runs covering the chunk (H=%lld)",
                (long long)H);
@@ -840,6 +945,7 @@ extern "C" int smel_ce_grad(const void* WT, int64_t ldwt, int64_t H, const void*
   a.shift = shift;
   a.r = r;
   a.acc = acc;
+  a.prev = prev;
   a.part = part;
   a.ldwt = ldwt;
   a.ldp = ldp;
@@ -848,10 +954,10 @@ extern "C" int smel_ce_grad(const void* WT, int64_t ldwt, int64_t H, const void*
   a.n = (int)n;
   a.kbytes = (int)kbytes;
   a.first = chunk == 0;
-  a.parity = chunk & 1;
+  a.splits = splits;
   a.n_ht = (int)((H + 255) / 256);
   a.n_tt = (int)((n + 255) / 256);
-  const int64_t items = 2 * (int64_t)a.n_ht * a.n_tt;
+  const int64_t items = splits * (int64_t)a.n_ht * a.n_tt;
   SMEL_REQUIRE(items < INT32_MAX, SMEL_EUNSUPPORTED, "ce_grad: grid too large");
   const dim3 g((unsigned)xcd_grid(items)), b(64 * GR_NW);
   if (dtype == 0) ce_grad_kernel<0><<<g, b, 0, stream>>>(a);
@@ -859,11 +965,35 @@ extern "C" int smel_ce_grad(const void* WT, int64_t ldwt, int64_t H, const void*
   else ce_grad_kernel<2><<<g, b, 0, stream>>>(a);
   return smel::launch_status();
 }
+}  // namespace
 
-extern "C" int smel_ce_finish(const float* m, const float* s, const float* tz, const float* td, const float* acc,
-                              const float* part, const void* W, int64_t ldw, const void* trows, const int64_t* tgt, int64_t V, int64_t n,
-                              int64_t H, int32_t dtype, float gscale, void* g, int64_t ldg, int32_t g_dtype,
-                              float* loss_rows, hipStream_t stream) {
+extern "C" int smel_ce_grad(const void* WT, int64_t ldwt, int64_t H, const void* P, int64_t ldp, int64_t vc,
+                            const uint8_t* shift, int64_t ldn, const float* r, int64_t n, int32_t dtype, int32_t chunk,
+                            float* acc, float* part, hipStream_t stream) {
+  SMEL_REQUIRE(part || n <= 0, SMEL_EINVAL, "ce_grad: null pointer");
+  const int64_t nh = n > 0 && H > 0 ? n * H : 0;
+  return ce_grad(WT, ldwt, H, P, ldp, vc, shift, ldn, r, n, dtype, chunk, 2, acc, part + ((chunk & 1) ^ 1) * nh,
+                 part + (chunk & 1) * nh, stream);
+}
+
+extern "C" int smel_ce_grad_splits(int64_t n, int64_t H, int64_t vc, int32_t dtype) {
+  if (n < 1 || H < 1 || vc < 1 || !SMEL_DT_OK(dtype)) return 1;
+  return grad_splits(n, H, vc, dtype == 1 ? 4 : 2);
+}
+
+extern "C" int smel_ce_grad_split(const void* WT, int64_t ldwt, int64_t H, const void* P, int64_t ldp, int64_t vc,
+                                  const uint8_t* shift, int64_t ldn, const float* r, int64_t n, int32_t dtype,
+                                  int32_t chunk, int32_t splits, float* acc, hipStream_t stream) {
+  SMEL_REQUIRE(acc || n <= 0, SMEL_EINVAL, "ce_grad: null pointer");
+  float* part = acc ? acc + (n > 0 && H > 0 ? n * H : 0) : nullptr;
+  return ce_grad(WT, ldwt, H, P, ldp, vc, shift, ldn, r, n, dtype, chunk, splits, acc, part, part, stream);
+}
+
+namespace {
+int ce_finish(const float* m, const float* s, const float* tz, const float* td, const float* acc, const float* part,
+              int32_t n_part, const void* W, int64_t ldw, const void* trows, const int64_t* tgt, int64_t V, int64_t n,
+              int64_t H, int32_t dtype, float gscale, void* g, int64_t ldg, int32_t g_dtype, float* loss_rows,
+              hipStream_t stream) {
   SMEL_REQUIRE(SMEL_DT_OK(dtype) && SMEL_DT_OK(g_dtype), SMEL_EINVAL, "ce_finish: dtype %d / %d", dtype, g_dtype);
   SMEL_REQUIRE(n >= 0 && H >= 1 && V >= 1, SMEL_EINVAL, "ce_finish: bad sizes");
   if (n == 0) return 0;
@@ -876,7 +1006,7 @@ extern "C" int smel_ce_finish(const float* m, const float* s, const float* tz, c
   const bool vec = acc && H % 8 == 0 && al16(acc) && al16(part) && al16(g) && ldg % 8 == 0 &&
                    (trows ? al16(trows) : (al16(W) && ldw % 8 == 0));
 #define SMEL_FIN(D, G) \
-  ce_finish_kernel<D, G><<<gr, b, 0, stream>>>(m, s, tz, td, acc, part, W, ldw, trows, tgt, V, H, gscale, g, ldg, \
+  ce_finish_kernel<D, G><<<gr, b, 0, stream>>>(m, s, tz, td, acc, part, n_part, W, ldw, trows, tgt, V, H, gscale, g, ldg, \
                                                loss_rows, vec)
 #define SMEL_FIN_G(D)            \
   if (g_dtype == 0) SMEL_FIN(D, 0); \
@@ -892,6 +1022,24 @@ extern "C" int smel_ce_finish(const float* m, const float* s, const float* tz, c
 #undef SMEL_FIN_G
 #undef SMEL_FIN
   return smel::launch_status();
+}
+}  // namespace
+
+extern "C" int smel_ce_finish(const float* m, const float* s, const float* tz, const float* td, const float* acc,
+                              const float* part, const void* W, int64_t ldw, const void* trows, const int64_t* tgt,
+                              int64_t V, int64_t n, int64_t H, int32_t dtype, float gscale, void* g, int64_t ldg,
+                              int32_t g_dtype, float* loss_rows, hipStream_t stream) {
+  return ce_finish(m, s, tz, td, acc, part, part ? 1 : 0, W, ldw, trows, tgt, V, n, H, dtype, gscale, g, ldg, g_dtype,
+                   loss_rows, stream);
+}
+
+extern "C" int smel_ce_finish_split(const float* m, const float* s, const float* tz, const float* td, const float* acc,
+                                    int32_t splits, const void* W, int64_t ldw, const void* trows, const int64_t* tgt,
+                                    int64_t V, int64_t n, int64_t H, int32_t dtype, float gscale, void* g, int64_t ldg,
+                                    int32_t g_dtype, float* loss_rows, hipStream_t stream) {
+  SMEL_REQUIRE(splits >= 1 && splits <= MAX_SPLITS, SMEL_EINVAL, "ce_finish: %d parts (1..%d)", splits, MAX_SPLITS);
+  return ce_finish(m, s, tz, td, acc, acc && n > 0 && H > 0 ? acc + n * H : nullptr, acc ? splits - 1 : 0, W, ldw, trows,
+                   tgt, V, n, H, dtype, gscale, g, ldg, g_dtype, loss_rows, stream);
 }
 
 extern "C" int smel_ce_loss_sum(const float* loss_rows, int64_t n, float scale, int32_t accumulate, float* total,
@@ -921,9 +1069,30 @@ extern "C" int smel_ce_transpose(const void* src, int64_t R, int64_t C, int64_t 
   const int64_t gx = (ldd + 63) / 64, gy = (C + 63) / 64;
   SMEL_REQUIRE(gx < INT32_MAX && gy < 65536, SMEL_EUNSUPPORTED, "ce_transpose: too large");
   const dim3 g((unsigned)gx, (unsigned)gy), b(256);
+  if (dtype != 1 && C % 8 == 0 && lds % 8 == 0 && ldd % 8 == 0 && aligned16(src) && aligned16(dst)) {
+    ce_head_kernel<0, false><<<g, b, 0, stream>>>(src, nullptr, R, C, lds, nullptr, dst, ldd);   // 16-bit patterns: any type
+    return smel::launch_status();
+  }
   const auto* s8 = static_cast<const uint8_t*>(src);
   auto* d8 = static_cast<uint8_t*>(dst);
   if (dtype == 1) ce_transpose_kernel<4><<<g, b, 0, stream>>>(s8, R, C, lds, d8, ldd);
   else ce_transpose_kernel<2><<<g, b, 0, stream>>>(s8, R, C, lds, d8, ldd);
+  return smel::launch_status();
+}
+
+extern "C" int smel_ce_dequant8(const int8_t* q, const void* scale, int64_t R, int64_t C, int32_t dtype, void* rows,
+                                void* wt, int64_t ldt, hipStream_t stream) {
+  SMEL_REQUIRE(dtype == 0 || dtype == 2, SMEL_EINVAL, "ce_dequant8: dtype %d (0 bf16, 2 fp16)", dtype);
+  SMEL_REQUIRE(R >= 0 && C >= 0 && (!wt || ldt >= R), SMEL_EINVAL, "ce_dequant8: bad sizes");
+  if (R == 0 || C == 0) return 0;
+  SMEL_REQUIRE(q && scale && rows, SMEL_EINVAL, "ce_dequant8: null pointer");
+  SMEL_REQUIRE(C % 8 == 0 && ((uintptr_t)q & 7) == 0 && aligned16(rows) && aligned16(wt) && (!wt || ldt % 8 == 0),
+               SMEL_EUNSUPPORTED, "ce_dequant8: rows of whole 8-element runs, 16-byte aligned outputs (C=%lld)",
+               (long long)C);
+  const int64_t gx = ((wt ? ldt : R) + 63) / 64, gy = (C + 63) / 64;
+  SMEL_REQUIRE(gx < INT32_MAX && gy < 65536, SMEL_EUNSUPPORTED, "ce_dequant8: too large");
+  const dim3 g((unsigned)gx, (unsigned)gy), b(256);
+  if (dtype == 0) ce_head_kernel<0, true><<<g, b, 0, stream>>>(q, scale, R, C, C, rows, wt, ldt);
+  else ce_head_kernel<2, true><<<g, b, 0, stream>>>(q, scale, R, C, C, rows, wt, ldt);
   return smel::launch_status();
 }

@@ -22,7 +22,7 @@ WSET_EXT2 = 2        # smel_wset.flags: the LoRA K-extension of the gate_up proj
 WSET_XCD_CHUNK = 4   # smel_wset.flags: group-ordered tile list, a contiguous chunk of it per XCD
 WSET_MERGE_SHORT = 8 # smel_wset.flags: gate_up forward, a full int4 tile also takes the group's short last tile
 WSET_MERGED_LIST = 16 # smel_wset.flags: gate_up forward on smel_dispatch's merged tile list (int4 tiles up to 160 rows)
-ABI_VERSION = 23
+ABI_VERSION = 24
 
 vp, i64, i32, f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_float
 
@@ -156,6 +156,11 @@ SIGNATURES = {
     "smel_ce_stats": (i32, [vp, vp, i64, i64, i64, vp, vp, vp, vp, vp]),
     "smel_ce_grad": (i32, [vp, i64, i64, vp, i64, i64, vp, i64, vp, i64, i32, i32, vp, vp, vp]),
     "smel_ce_finish": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, vp, vp, i64, i64, i64, i32, f32, vp, i64, i32, vp, vp]),
+    "smel_ce_grad_splits": (i32, [i64, i64, i64, i32]),
+    "smel_ce_grad_split": (i32, [vp, i64, i64, vp, i64, i64, vp, i64, vp, i64, i32, i32, i32, vp, vp]),
+    "smel_ce_finish_split": (i32, [vp, vp, vp, vp, vp, i32, vp, i64, vp, vp, i64, i64, i64, i32, f32, vp, i64, i32, vp,
+                                   vp]),
+    "smel_ce_dequant8": (i32, [vp, vp, i64, i64, i32, vp, vp, i64, vp]),
     "smel_ce_loss_sum": (i32, [vp, i64, f32, i32, vp, vp]),
     "smel_ce_scale": (i32, [vp, i64, i32, vp, vp]),
     "smel_ce_transpose": (i32, [vp, i64, i64, i64, vp, i64, i32, vp]),

@@ -8,15 +8,16 @@ Structure here:
     of exponentials, the softmax terms written in the rows' dtype, the target's logit), ``smel_ce_stats`` folds the
     windows into each row's running maximum and sum (every rescale an exact power of two) and ``smel_ce_grad`` runs
     the gradient GEMM p W on MFMA, shifting each fragment of p to the running maximum as it is loaded and adding into
-    the fp32 accumulator rescaled by the same power of two (the chunk's columns in two halves, the second half's sum
-    kept apart and folded in by the next chunk); ``smel_ce_finish`` writes the loss rows and the gradient rows
-    (acc / s - d W[target], scaled), ``smel_ce_loss_sum`` their sum;
+    an fp32 accumulator rescaled by the same power of two (the chunk's columns in one to eight parts, each with an
+    accumulator of its own); ``smel_ce_finish`` writes the loss rows and the gradient rows
+    (sum of the parts / s - d W[target], scaled), ``smel_ce_loss_sum`` their sum;
   * the gradient GEMM reads the head transposed ([H][V]): a dense head whose dtype is the rows' is transposed once
     and kept with the head (it is frozen); other heads (int8, or another dtype) are converted per vocabulary chunk,
     as the reference's ``rows()`` does, and that chunk is transposed;
   * vocabulary chunks are ``vocab_chunk`` rounded up to 256 columns (the logits tile), and a pass takes at most
     ``token_chunk`` rows, so token_chunk x vocab_chunk bounds its buffers as in the reference (the softmax terms of a
-    pass take rows x chunk values of the rows' dtype); a caller that leaves token_chunk at its default gets passes of
+    pass take rows x chunk values of the rows' dtype); a pass of fewer rows takes chunks of more columns under the same
+    bound where the head is read in place; a caller that leaves token_chunk at its default gets passes of
     up to 4096 rows (256 MB of bf16 terms at vocab_chunk 32768), where the GEMMs' row tiles fill the GPU. The rows are
     independent, so the results are those of the reference's chunking either way.
 The gradient is computed in the forward (lm_head is frozen) and handed back by the backward, as in the reference.
@@ -42,15 +43,15 @@ class _DefaultTokenChunk(int):
 TOKEN_CHUNK_DEFAULT = _DefaultTokenChunk(1024)
 
 
-def _rows_per_pass(N: int, token_chunk) -> int:
-    """Token rows of one pass: at most ``token_chunk`` (it bounds a pass's buffers, the softmax terms
+def _max_rows(token_chunk) -> int:
+    """Token rows a pass may take: at most ``token_chunk`` (it bounds a pass's buffers, the softmax terms
     [rows][vocab_chunk] and about 12 H bytes per row), or up to ROWS_PER_PASS when the caller left the default."""
     tc = int(token_chunk)
     if tc <= 0:
         raise ValueError(f"chunked_ce: token_chunk must be positive, got {tc}")
     if isinstance(token_chunk, _DefaultTokenChunk):
         tc = max(tc, ROWS_PER_PASS)
-    return min(N, tc)
+    return tc
 
 
 def _round_up(x: int, m: int) -> int:
@@ -85,6 +86,10 @@ class _DenseRows:
             return None
         return w
 
+    def kernel_rows(self, v0: int, v1: int, dtype, transposed: bool):
+        """(rows [vc, H], the same transposed [H, vc rounded up to 8] or None) of a chunk in ``dtype``."""
+        return _rows_and_transpose(self.span(v0, v1, dtype).contiguous(), transposed)
+
     def moved(self, device):
         return _DenseRows(self.w.to(device))
 
@@ -107,8 +112,31 @@ class _Int8Rows:
     def native(self, dtype):
         return None
 
+    def kernel_rows(self, v0: int, v1: int, dtype, transposed: bool):
+        """As _DenseRows.kernel_rows; 16-bit rows are dequantized and transposed in one launch."""
+        q, scale = self.q["q"][v0:v1], self.q["scale"][v0:v1]
+        H = q.shape[1]
+        if dtype == torch.float32 or H % 8 or q.dtype != torch.int8 or not q.is_contiguous() or q.data_ptr() % 8:
+            return _rows_and_transpose(dequant_int8_rows(q, scale, dtype).contiguous(), transposed)
+        scale = scale.to(dtype).contiguous()
+        vc = v1 - v0
+        W = torch.empty(vc, H, dtype=dtype, device=q.device)
+        WT = torch.empty(H, _round_up(vc, 8), dtype=dtype, device=q.device) if transposed else None
+        L.call("smel_ce_dequant8", L.ptr(q), L.ptr(scale), vc, H, _DT[dtype], L.ptr(W), L.ptr(WT),
+               WT.stride(0) if transposed else 0, L.stream())
+        return W, WT
+
     def moved(self, device):
         return _Int8Rows({k: v.to(device) for k, v in self.q.items()})
+
+
+def _rows_and_transpose(W: torch.Tensor, transposed: bool):
+    if not transposed:
+        return W, None
+    V, H = W.shape
+    wt = torch.empty(H, _round_up(V, 8), dtype=W.dtype, device=W.device)
+    L.call("smel_ce_transpose", L.ptr(W), V, H, W.stride(0), L.ptr(wt), wt.stride(0), _DT[W.dtype], L.stream())
+    return W, wt
 
 
 class LMHead:
@@ -160,10 +188,19 @@ class LMHead:
         return out
 
     # ---- what the kernels read
-    def _kernel_chunks(self):
-        """Vocabulary chunks of the kernels: vocab_chunk rounded up to whole logits tiles."""
-        step = _round_up(max(1, min(self.vocab_chunk, self.vocab)), TILE_V)
+    def _kernel_chunks(self, cols: int | None = None):
+        """Vocabulary chunks of the kernels: ``cols`` (default vocab_chunk) rounded up to whole logits tiles."""
+        step = _round_up(max(1, min(max(cols or 0, self.vocab_chunk), self.vocab)), TILE_V)
         return [(v0, min(self.vocab, v0 + step)) for v0 in range(0, self.vocab, step)], step
+
+    def _pass_chunks(self, rows: int, max_rows: int, dtype):
+        """The chunks of a pass of ``rows`` rows where a pass may take ``max_rows``: a head read in place takes as many
+        columns as keep rows x columns at max_rows x vocab_chunk (the bound of a pass's softmax terms), so that short
+        passes fill the GPU; a head converted chunk by chunk stays at vocab_chunk, which bounds the converted rows."""
+        cols = self.vocab_chunk
+        if self._src.native(dtype) is not None:
+            cols = min(self.vocab, cols * max(1, max_rows // max(1, rows)))
+        return self._kernel_chunks(cols)
 
     def _transposed(self, w: torch.Tensor) -> torch.Tensor:
         """The head [V, H] transposed to [H, Vp] (Vp = V rounded up to 8, zero columns past V), made once."""
@@ -171,9 +208,7 @@ class LMHead:
         got = self._wt.get(w.dtype)
         if got is not None and got[0] == key:
             return got[1]
-        V, H = w.shape
-        wt = torch.empty(H, _round_up(V, 8), dtype=w.dtype, device=w.device)
-        L.call("smel_ce_transpose", L.ptr(w), V, H, w.stride(0), L.ptr(wt), wt.stride(0), _DT[w.dtype], L.stream())
+        _, wt = _rows_and_transpose(w, True)
         self._wt[w.dtype] = (key, wt)
         return wt
 
@@ -182,34 +217,35 @@ class LMHead:
 
 
 class _Pass:
-    """Scratch of one pass over n token rows: per-row state, window statistics, softmax terms, accumulator."""
+    """Scratch of one pass over n token rows: per-row state, window statistics, softmax terms, accumulators (one per
+    part of the gradient GEMM's contraction)."""
 
-    def __init__(self, n: int, H: int, vcp: int, dtype, need_grad: bool, device):
+    def __init__(self, n: int, H: int, chunks, dtype, need_grad: bool, device):
         f = lambda *s: torch.empty(*s, dtype=torch.float32, device=device)
+        self.chunks, vcp = chunks
         nwin = vcp // WIN
         self.n = n
         self.m, self.s, self.tz, self.td, self.r, self.loss = (f(n) for _ in range(6))
         self.win_e, self.win_s = f(nwin, n), f(nwin, n)
         self.shift = torch.empty(nwin, n, dtype=torch.uint8, device=device)
         self.P = torch.empty(n, vcp, dtype=dtype, device=device) if need_grad else None
-        self.acc = f(n, H) if need_grad else None
-        self.part = f(2, n, H) if need_grad else None     # the second K halves' partials, by chunk parity
-        self.last = 0                                       # chunks of the last sweep
+        self.splits = L.load().smel_ce_grad_splits(n, H, vcp, _DT[dtype])
+        self.acc = f(self.splits, n, H) if need_grad else None
 
 
 def _sweep(h, head: LMHead, tgt, need_grad: bool, ps: _Pass, m0=None):
-    """One pass over the vocabulary for the rows h [n, H]: the per-row state and (need_grad) the accumulator."""
+    """One pass over the vocabulary for the rows h [n, H]: the per-row state and (need_grad) the accumulators."""
     n, H = h.shape
     dt, st, p = _DT[h.dtype], L.stream(), L.ptr
     L.call("smel_ce_begin", p(ps.m), p(ps.s), p(ps.tz), p(ps.td), p(m0), n, st)
     native = head._src.native(h.dtype)
-    chunks, _ = head._kernel_chunks()
-    for i, (v0, v1) in enumerate(chunks):
+    for i, (v0, v1) in enumerate(ps.chunks):
         vc = v1 - v0
+        WT = None
         if native is not None:
             W, ldw = native[v0:v1], native.stride(0)
         else:
-            W = head.rows(v0, v1, h.dtype).contiguous()
+            W, WT = head._src.kernel_rows(v0, v1, h.dtype, need_grad)
             ldw = W.stride(0)
         nwin = _round_up(vc, TILE_V) // WIN
         P = ps.P if need_grad else None
@@ -218,15 +254,9 @@ def _sweep(h, head: LMHead, tgt, need_grad: bool, ps: _Pass, m0=None):
         L.call("smel_ce_stats", p(ps.win_e), p(ps.win_s), nwin, n, n, p(ps.m), p(ps.s), p(ps.shift), p(ps.r), st)
         if need_grad:
             if native is not None:
-                wt = head._transposed(native)
-                WT, ldwt = wt[:, v0:], wt.stride(0)
-            else:
-                WT = torch.empty(H, _round_up(vc, 8), dtype=h.dtype, device=h.device)
-                L.call("smel_ce_transpose", p(W), vc, H, ldw, p(WT), WT.stride(0), dt, st)
-                ldwt = WT.stride(0)
-            L.call("smel_ce_grad", p(WT), ldwt, H, p(ps.P), ps.P.stride(0), vc, p(ps.shift), n, p(ps.r), n, dt,
-                   i, p(ps.acc), p(ps.part), st)
-    ps.last = len(chunks) - 1
+                WT = head._transposed(native)[:, v0:]
+            L.call("smel_ce_grad_split", p(WT), WT.stride(0), H, p(ps.P), ps.P.stride(0), vc, p(ps.shift), n, p(ps.r), n,
+                   dt, i, ps.splits, p(ps.acc), st, tag="smel_ce_grad")
 
 
 def _finish(h, head: LMHead, tgt, ps: _Pass, need_grad: bool, gscale: float = 1.0, g=None):
@@ -245,10 +275,9 @@ def _finish(h, head: LMHead, tgt, ps: _Pass, need_grad: bool, gscale: float = 1.
             trows = head.rows_at(torch.where(ok, tgt, torch.zeros_like(tgt)), h.dtype).contiguous()
         if g is None:
             g = torch.empty(n, H, dtype=torch.float32, device=h.device)
-    part = ps.part[ps.last % 2] if need_grad else None
-    L.call("smel_ce_finish", p(ps.m), p(ps.s), p(ps.tz), p(ps.td), p(ps.acc), p(part), p(W), ldw, p(trows), p(tgt),
-           head.vocab, n, H, dt, float(gscale), p(g), g.stride(0) if g is not None else 0,
-           _DT[g.dtype] if g is not None else 0, p(ps.loss), L.stream())
+    L.call("smel_ce_finish_split", p(ps.m), p(ps.s), p(ps.tz), p(ps.td), p(ps.acc) if need_grad else None, ps.splits,
+           p(W), ldw, p(trows), p(tgt), head.vocab, n, H, dt, float(gscale), p(g), g.stride(0) if g is not None else 0,
+           _DT[g.dtype] if g is not None else 0, p(ps.loss), L.stream(), tag="smel_ce_finish")
     return g
 
 
@@ -269,9 +298,8 @@ def _loss_sum(ps: _Pass, total: torch.Tensor, scale: float, accumulate: bool):
 def _one_chunk(h, head: LMHead, tgt, need_grad, two_pass: bool):
     h, tgt = _prep(h, tgt)
     n, H = h.shape
-    _, vcp = head._kernel_chunks()
     total = torch.empty((), dtype=torch.float32, device=h.device)
-    ps = _Pass(n, H, vcp, h.dtype, need_grad, h.device)
+    ps = _Pass(n, H, head._kernel_chunks(), h.dtype, need_grad, h.device)
     m0 = None
     if two_pass:
         _sweep(h, head, tgt, False, ps)
@@ -304,17 +332,17 @@ class _ChunkedCE(torch.autograd.Function):
     written into one output during the forward and returned, times the incoming gradient, by the backward."""
 
     @staticmethod
-    def forward(ctx, h, head, tgt, denom, rows, need_grad):
+    def forward(ctx, h, head, tgt, denom, rows, max_rows, need_grad):
         h, tgt = _prep(h, tgt)
         N, H = h.shape
-        _, vcp = head._kernel_chunks()
         grad = torch.empty_like(h) if need_grad else None
         total = torch.empty((), dtype=torch.float32, device=h.device)
-        ps = _Pass(rows, H, vcp, h.dtype, need_grad, h.device)
+        ps = None
         for t0 in range(0, N, rows):
             t1 = min(N, t0 + rows)
-            if t1 - t0 != ps.n:
-                ps = _Pass(t1 - t0, H, vcp, h.dtype, need_grad, h.device)
+            if ps is None or t1 - t0 != ps.n:
+                ps = None   # the pass before gives its scratch back first
+                ps = _Pass(t1 - t0, H, head._pass_chunks(t1 - t0, max_rows, h.dtype), h.dtype, need_grad, h.device)
             _sweep(h[t0:t1], head, tgt[t0:t1], need_grad, ps)
             _finish(h[t0:t1], head, tgt[t0:t1], ps, need_grad, 1.0 / denom, grad[t0:t1] if need_grad else None)
             _loss_sum(ps, total, 1.0 / denom, t0 > 0)
@@ -327,7 +355,7 @@ class _ChunkedCE(torch.autograd.Function):
         ctx.grad = None
         go = go.to(device=g.device, dtype=torch.float32).contiguous()
         L.call("smel_ce_scale", L.ptr(g), g.numel(), _DT[g.dtype], L.ptr(go), L.stream())
-        return g, None, None, None, None, None
+        return g, None, None, None, None, None, None
 
 
 def chunked_ce(h, head: LMHead, tgt, denom: float, token_chunk: int = TOKEN_CHUNK_DEFAULT, need_grad: bool = True):
@@ -335,7 +363,8 @@ def chunked_ce(h, head: LMHead, tgt, denom: float, token_chunk: int = TOKEN_CHUN
     tgt: [N] long. A pass over the vocabulary takes at most ``token_chunk`` rows when the caller sets it."""
     if h.shape[0] == 0:
         return h.sum() * 0.0
-    rows = _rows_per_pass(h.shape[0], token_chunk)
+    max_rows = _max_rows(token_chunk)
+    rows = min(h.shape[0], max_rows)
     grad = need_grad and h.requires_grad
     with torch.set_grad_enabled(grad and torch.is_grad_enabled()):
-        return _ChunkedCE.apply(h, head, tgt, float(denom), rows, grad)
+        return _ChunkedCE.apply(h, head, tgt, float(denom), rows, max_rows, grad)

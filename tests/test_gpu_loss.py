@@ -200,6 +200,78 @@ def test_several_row_passes(lm):
     assert abs(l_many.item() - float(l64)) / abs(float(l64)) < 1e-3
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("n", [1, 128, 129, 257, 384, 385])
+def test_row_tiles_and_parts(lm, n, dtype):
+    """Row counts around the 128- and 256-row tiles, with the gradient's contraction in several parts and a vocabulary of
+    several chunks where the pass takes them (vocab_chunk 512), against the fp64 oracle: fp32 rows to 1e-4, 16-bit rows
+    within their rounding (the softmax terms and the logits each rounded once: 2 x 2^-8, bf16)."""
+    loss_mod, _ = lm
+    torch.manual_seed(n)
+    H, V = 328, 6007
+    h = (torch.randn(n, H, device="cuda") * 0.5).to(dtype)
+    W = (torch.randn(V, H, device="cuda") * 0.1).to(dtype)
+    tgt = torch.randint(0, V, (n,), device="cuda")
+    l64, g64 = LR.full_ce(h, W, tgt, 0.0, denom=n)
+    for kw in ({"vocab_chunk": 512}, {}):
+        for tc in ({}, {"token_chunk": 200}):
+            x = h.clone().requires_grad_(True)
+            loss = loss_mod.chunked_ce(x, loss_mod.LMHead(weight=W, **kw), tgt, denom=n, **tc)
+            loss.backward()
+            rel = float((x.grad.double().cpu() - g64).norm() / g64.norm())
+            print(f"CE n={n} {dtype} {kw} {tc}: loss {loss.item():.6f} grad rel {rel:.2e}", flush=True)
+            assert abs(loss.item() - float(l64)) < (1e-4 if dtype == torch.float32 else 2e-3) * abs(float(l64))
+            assert rel < (1e-4 if dtype == torch.float32 else 1e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,H", [(1, 8), (63, 72), (129, 64), (700, 328)])
+def test_int8_rows_and_transpose_bits(lm, V, H, dtype):
+    """smel_ce_dequant8 against dequant_int8_rows bit for bit, the transposed copy's padding columns zero, and the
+    16-byte transpose of a dense head against torch's."""
+    loss_mod, quant = lm
+    from smel import _lib as L
+    torch.manual_seed(V)
+    q = {"q": torch.randint(-127, 128, (V, H), dtype=torch.int8, device="cuda"),
+         "scale": (torch.rand(V, device="cuda") * 0.01).to(torch.bfloat16)}
+    ref = quant.dequant_int8_rows(q["q"], q["scale"], dtype)
+    Vp = (V + 7) // 8 * 8
+    rows, wt = torch.empty_like(ref), torch.full((H, Vp), 7.0, dtype=dtype, device="cuda")
+    sc = q["scale"].to(dtype)
+    L.call("smel_ce_dequant8", L.ptr(q["q"]), L.ptr(sc), V, H, loss_mod._DT[dtype], L.ptr(rows), L.ptr(wt), Vp, L.stream())
+    assert torch.equal(rows.view(torch.int16), ref.view(torch.int16))
+    assert torch.equal(wt[:, :V], ref.t()) and not wt[:, V:].any()
+    _, wt2 = loss_mod._rows_and_transpose(ref, True)
+    assert torch.equal(wt2, wt)
+
+
+def test_two_half_form_equals_two_parts(lm):
+    """smel_ce_grad / smel_ce_finish (two halves, the second one's accumulator alternating between two buffers) against
+    smel_ce_grad_split / _finish_split with two parts, over three chunks: bitwise."""
+    from smel import _lib as L
+    torch.manual_seed(3)
+    n, H, vc, p = 200, 136, 768, L.ptr
+    f = lambda *s: torch.empty(*s, device="cuda")
+    P = torch.rand(n, vc, device="cuda").bfloat16()
+    WT = torch.randn(H, vc, device="cuda").bfloat16()
+    shift = torch.randint(0, 4, (vc // 128, n), dtype=torch.uint8, device="cuda")
+    r = torch.full((n,), 0.5, device="cuda")
+    acc, part, acc2 = f(n, H), f(2, n, H), f(2, n, H)
+    for c in range(3):
+        L.call("smel_ce_grad", p(WT), vc, H, p(P), vc, vc, p(shift), n, p(r), n, 0, c, p(acc), p(part), L.stream())
+        L.call("smel_ce_grad_split", p(WT), vc, H, p(P), vc, vc, p(shift), n, p(r), n, 0, c, 2, p(acc2), L.stream())
+    assert torch.equal(acc, acc2[0]) and torch.equal(part[0], acc2[1])
+    m, s, tz, td, l1, l2 = (torch.ones(n, device="cuda") for _ in range(6))
+    tgt = torch.randint(0, 10, (n,), device="cuda")
+    trows = torch.randn(n, H, device="cuda").bfloat16()
+    g1, g2 = f(n, H), f(n, H)
+    L.call("smel_ce_finish", p(m), p(s), p(tz), p(td), p(acc), p(part[0]), None, 0, p(trows), p(tgt), 10, n, H, 0, 0.5,
+           p(g1), H, 1, p(l1), L.stream())
+    L.call("smel_ce_finish_split", p(m), p(s), p(tz), p(td), p(acc2), 2, None, 0, p(trows), p(tgt), 10, n, H, 0, 0.5,
+           p(g2), H, 1, p(l2), L.stream())
+    assert torch.equal(g1, g2) and torch.equal(l1, l2)
+
+
 def test_token_chunk_bounds_pass_memory(lm):
     """token_chunk x vocab_chunk bounds a pass's scratch, as the reference promises for its peak memory: with
     token_chunk=256 over 4096 rows, one call allocates at most one 256-row pass (softmax terms 256 x vocab_chunk
