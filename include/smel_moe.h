@@ -73,6 +73,10 @@ typedef struct smel_wset {
  * group's last tile of at most 32 rows); each is one tile (one weight stream and dequant), and no block idles.
  * Without it a tile of the list has at most 128 rows (rows past 128 are not computed). */
 #define SMEL_WSET_MERGED_LIST 16
+/* SMEL_WSET_TILE32 (smel_gmm_fwd, smel_gmm_bwd): the tile list's tiles hold at most 32 rows (smel_dispatch with m_tile
+ * 32): kernels with a quarter of the LDS and registers per block run more blocks per CU. Excludes the merged forms.
+ * Rows of a tile past 32 are not computed. */
+#define SMEL_WSET_TILE32 32
 
 const char* smel_last_error(void);
 int smel_abi_version(void);

@@ -25,29 +25,41 @@
 
 namespace {
 
-constexpr int MT = 128;
 constexpr int KT = 64;
 constexpr int NB = 256;            // output columns per block
-constexpr int A_BYTES = MT * KT * 2;         // A rows of one stage
+// Rows of a tile and what follows from them: MT 128 for ordinary tile lists (two blocks per CU), MT 32 for lists whose
+// tiles hold at most 32 rows (SMEL_WSET_TILE32): a quarter of the LDS and one 32-row slice of accumulators, so that
+// more blocks share a CU.
 // scale/zero of one stage: 4 waves x 64 rows x (scale, zero) fp32, per group (two groups per wave when the int4 group
 // is 32 wide: SZ2)
 constexpr int z_bytes(bool sz2) { return 4 * 512 * (sz2 ? 2 : 1); }
-constexpr int q_stage(bool sz2) { return A_BYTES + z_bytes(sz2); }
-// 4 stages; the epilogue's staged tile (4 x A_BYTES) and its 512-B row table fit inside
-constexpr int smem_bytes(bool sz2) { return 4 * q_stage(sz2); }
-static_assert(smem_bytes(false) <= 80 * 1024 && 4 * A_BYTES + 512 <= smem_bytes(false), "two blocks per CU");
-
-// Vector-memory operations per wave in each issue group of the main loops; the issue code below is written with
-// these counts and every wait is computed from them (vmcnt retires in issue order).
-constexpr int VM_A = A_BYTES / (4 * 1024);                 // A rows of a stage: 1-KB LDS-DMA wave-loads, 4 waves
-constexpr int VM_Q = 2;                                     // int4: 16-B words of the two column pairs
-constexpr int vm_sz(bool sz2) { return sz2 ? 4 : 2; }       // int4: 256-B scale/zero runs, per group
-constexpr int vm_q4(bool sz2) { return VM_Q + vm_sz(sz2) + VM_A; }
-constexpr int VM_B = 2 * 4;                                 // bf16: 2 substeps x 4 column fragments
-// int4: steps j+1 and j+2 may be in flight while step j computes; bf16: issue order ... W(j+1), A(j+3), so before
-// step j only A(j+2) may be
-constexpr int q4_wait(bool sz2) { return 2 * vm_q4(sz2); }
-constexpr int BF_WAIT = VM_A;
+// int4: A rows of a stage (1-KB LDS-DMA wave-loads, 4 waves), 16-B words of the two column pairs, 256-B scale/zero runs
+// per group; bf16 weights: 2 substeps x 4 column fragments. The vector-memory operations per wave in each issue group
+// of the main loops; the issue code below is written with these counts and every wait is computed from them (vmcnt
+// retires in issue order).
+constexpr int VM_Q = 2;
+constexpr int vm_sz(bool sz2) { return sz2 ? 4 : 2; }
+constexpr int VM_B = 2 * 4;
+template <int MT_>
+struct Cfg {
+  static constexpr int MT = MT_;
+  static constexpr int A_BYTES = MT_ * KT * 2;         // A rows of one stage
+  static constexpr int q_stage(bool sz2) { return A_BYTES + z_bytes(sz2); }
+  // LoRA rows: a dh chunk [MT][136] and two planes of bt [32][136]
+  static constexpr int LR_BYTES = (MT_ + 2 * 32) * (128 + 8) * 2;
+  // 4 stages; the epilogue's staged tile (4 x A_BYTES), its row table and the LoRA rows' chunks fit inside
+  static constexpr int smem_bytes(bool sz2) {
+    return 4 * q_stage(sz2) > LR_BYTES ? 4 * q_stage(sz2) : (LR_BYTES + 1023) / 1024 * 1024;
+  }
+  static_assert(4 * A_BYTES + 4 * MT_ <= smem_bytes(false), "the row table fits behind the staged tile");
+  static constexpr int VM_A = A_BYTES / (4 * 1024);
+  static constexpr int vm_q4(bool sz2) { return VM_Q + vm_sz(sz2) + VM_A; }
+  // int4: steps j+1 and j+2 may be in flight while step j computes; bf16: issue order ... W(j+1), A(j+3), so before
+  // step j only A(j+2) may be
+  static constexpr int q4_wait(bool sz2) { return 2 * vm_q4(sz2); }
+  static constexpr int BF_WAIT = VM_A;
+};
+static_assert(Cfg<128>::smem_bytes(false) <= 80 * 1024, "two blocks per CU");
 
 struct BwdArgs {
   smel_wset w;
@@ -92,16 +104,18 @@ SMEL_DEV void ld4_lds(rsrc_t r, const void* lds, uint32_t off) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)(lds), 4, off, 0, 0, 0);
 }
 
-template <int EPI, bool Q4, int NS, bool SZ2, bool FAST>
+template <int EPI, bool Q4, int NS, bool SZ2, bool FAST, int MT_>
 SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows, int nb, uint8_t* smem) {
+  using CF = Cfg<MT_>;
+  constexpr int MT = MT_, A_BYTES = CF::A_BYTES, VM_A = CF::VM_A, BF_WAIT = CF::BF_WAIT;
   // LDS rings of 4 stages. int4: [A rows 16 KB | scale/zero pairs of 4 waves x 64 rows (x 2 groups for SZ2), 2 KB
   // (4 KB)]; bf16: A rows. The weights go to registers. The epilogue reuses the first 64 KB.
-  constexpr int QS = q_stage(SZ2), ZW = SZ2 ? 1024 : 512;   // stage bytes, scale/zero bytes per wave
+  constexpr int QS = CF::q_stage(SZ2), ZW = SZ2 ? 1024 : 512;   // stage bytes, scale/zero bytes per wave
   auto St = [&](int st) {
     return reinterpret_cast<uint16_t*>(smem + st * (Q4 ? QS : A_BYTES));
   };
   auto Zt = [&](int st) { return smem + st * QS + A_BYTES; };
-  auto Et = [&](int m) { return reinterpret_cast<uint16_t*>(smem + m * A_BYTES); };
+  auto Et = [&](int m) { return reinterpret_cast<uint16_t*>(smem + m * (32 * NB * 2)); };   // 32 staged rows
   const int tid = threadIdx.x, l = lane_id(), kq = l >> 4, li = l & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int Kd = a.Kd, N = a.N;
@@ -291,7 +305,7 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
     u32x4_t qa[VM_Q], qb[VM_Q], qc[VM_Q], qe[VM_Q];
     u32x4_t* const qs[4] = {qa, qb, qc, qe};
     auto step = [&](int j, int st) {
-      wait_vm_lds<q4_wait(SZ2)>();
+      wait_vm_lds<CF::q4_wait(SZ2)>();
       __builtin_amdgcn_s_barrier();
       issue_lds(j + 3, (st + 3) & 3, qs[(st + 3) & 3]);
       compute(st, qs[st]);
@@ -415,7 +429,7 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
           for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
-              const int row = xr + 64 * h, p = p0 + q;
+              const int row = xr + 64 * h, p = p0 + q;   // rows past MT are past nrows
               const uint32_t o =
                   (row < nrows && p < P) ? (uint32_t)(((row * P + p) * planes + c) * 128 + 4 * xj) : OOB;
               x[h][q][0] = ld16(rp, o);
@@ -433,9 +447,10 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          *reinterpret_cast<u32x4_t*>(X + (xr + 64 * h) * 32 * planes + 32 * c + xj) =
-              u32x4_t{pack2bf(v[h][0], v[h][1]), pack2bf(v[h][2], v[h][3]), pack2bf(v[h][4], v[h][5]),
-                      pack2bf(v[h][6], v[h][7])};
+          if (xr + 64 * h < MT)
+            *reinterpret_cast<u32x4_t*>(X + (xr + 64 * h) * 32 * planes + 32 * c + xj) =
+                u32x4_t{pack2bf(v[h][0], v[h][1]), pack2bf(v[h][2], v[h][3]), pack2bf(v[h][4], v[h][5]),
+                        pack2bf(v[h][6], v[h][7])};
       }
       __syncthreads();
     }
@@ -508,7 +523,7 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
   const float* const wmap = reinterpret_cast<const float*>(rowmap);
   // 32 threads per row, 8 rows per pass; the saved (g, u) of PB passes are loaded before any of them is used, so the
   // stores of one batch never wait for the loads of the next row.
-  constexpr int PB = 8;
+  constexpr int PB = MT / 8 < 8 ? MT / 8 : 8;
   const int act = a.act;
   {
     for (int rb = tid >> 5; rb < nrows; rb += 8 * PB) {
@@ -581,7 +596,8 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
   constexpr int DP = 128 + 8;                         // LDS row pitch (bf16): 272 B
   uint16_t* const D = reinterpret_cast<uint16_t*>(smem);   // dh chunk [128][DP]
   uint16_t* const Bs = D + MT * DP;                         // bt chunk [planes][32][DP]
-  static_assert(MT * DP * 2 + 2 * 32 * DP * 2 <= smem_bytes(false), "LoRA-row chunks fit in the ring");
+  static_assert(MT * DP * 2 + 2 * 32 * DP * 2 <= CF::smem_bytes(false), "LoRA-row chunks fit in the ring");
+  constexpr int GI = MT / 16;   // dh rows of a thread
   const rsrc_t rd = make_rsrc(a.out + (int64_t)row0 * a.ldo, (uint64_t)nrows * a.ldo * 2);
   const rsrc_t rb0 = make_rsrc(bt, (uint64_t)32 * I2 * 2);
   const rsrc_t rb1 = make_rsrc(gplanes > 1 ? bt + pstride : bt, gplanes > 1 ? (uint64_t)32 * I2 * 2 : 0);
@@ -591,7 +607,7 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
   auto piece_col = [&](int q) { return (q >= 2 ? I : 0) + nb * NB + 128 * (q & 1) + 8 * gch; };
   // the bt rows of all 4 chunks before the barrier (they do not depend on this block's stores), the dh rows of all
   // 4 chunks right after it: one memory round trip for the whole projection
-  u32x4_t pd[4][8], pb[4][2][2];
+  u32x4_t pd[4][GI], pb[4][2][2];
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -606,14 +622,14 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < GI; ++i) {
       const int row = grow + 16 * i;
       pd[q][i] = ld16(rd, piece_ok(q) && row < nrows ? (uint32_t)(row * a.ldo + piece_col(q)) * 2 : OOB);
     }
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4_t*>(D + (grow + 16 * i) * DP + 8 * gch) = pd[q][i];
+    for (int i = 0; i < GI; ++i) *reinterpret_cast<u32x4_t*>(D + (grow + 16 * i) * DP + 8 * gch) = pd[q][i];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       *reinterpret_cast<u32x4_t*>(Bs + (grow + 16 * i) * DP + 8 * gch) = pb[q][0][i];
@@ -644,17 +660,21 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
   }
 }
 
-template <int EPI, bool Q4, bool SZ2, bool FAST>
+template <int EPI, bool Q4, bool SZ2, bool FAST, int MT_>
 SMEL_DEV void run_tile_ns(const BwdArgs& a, int kind, int idx, int row0, int nrows, int nb, uint8_t* smem) {
-  switch ((nrows + 31) >> 5) {
-    case 1: run_tile<EPI, Q4, 1, SZ2, FAST>(a, kind, idx, row0, nrows, nb, smem); break;
-    case 2: run_tile<EPI, Q4, 2, SZ2, FAST>(a, kind, idx, row0, nrows, nb, smem); break;
-    case 3: run_tile<EPI, Q4, 3, SZ2, FAST>(a, kind, idx, row0, nrows, nb, smem); break;
-    default: run_tile<EPI, Q4, 4, SZ2, FAST>(a, kind, idx, row0, nrows, nb, smem); break;
+  if constexpr (MT_ == 32) {
+    run_tile<EPI, Q4, 1, SZ2, FAST, MT_>(a, kind, idx, row0, nrows, nb, smem);
+  } else {
+    switch ((nrows + 31) >> 5) {
+      case 1: run_tile<EPI, Q4, 1, SZ2, FAST, MT_>(a, kind, idx, row0, nrows, nb, smem); break;
+      case 2: run_tile<EPI, Q4, 2, SZ2, FAST, MT_>(a, kind, idx, row0, nrows, nb, smem); break;
+      case 3: run_tile<EPI, Q4, 3, SZ2, FAST, MT_>(a, kind, idx, row0, nrows, nb, smem); break;
+      default: run_tile<EPI, Q4, 4, SZ2, FAST, MT_>(a, kind, idx, row0, nrows, nb, smem); break;
+    }
   }
 }
 
-template <int EPI, bool SZ2>
+template <int EPI, bool SZ2, int MT_>
 SMEL_DEV void gmm_bwd_body(const BwdArgs& a, uint8_t* smem) {
   int tile, nb;
   if (!((a.w.flags & SMEL_WSET_XCD_CHUNK) ? xcd_tile_chunk(a.n_tiles[0], a.nblk, tile, nb)
@@ -663,30 +683,41 @@ SMEL_DEV void gmm_bwd_body(const BwdArgs& a, uint8_t* smem) {
   const int4 t = a.tiles[tile];
   const int gk = a.gkind ? a.gkind[t.x] : t.w;   // the tile list may carry the group kind itself
   const int kind = gk >> 16, idx = gk & 0xffff;
-  const int nrows = min(t.z - t.y, MT);
+  const int nrows = min(t.z - t.y, MT_);
   if (nrows <= 0) return;
   if (kind == SMEL_KIND_INT4) {
     if (a.w.flags & SMEL_WSET_FAST_DQ)
-      run_tile_ns<EPI, true, SZ2, true>(a, kind, idx, t.y, nrows, nb, smem);
+      run_tile_ns<EPI, true, SZ2, true, MT_>(a, kind, idx, t.y, nrows, nb, smem);
     else
-      run_tile_ns<EPI, true, SZ2, false>(a, kind, idx, t.y, nrows, nb, smem);
+      run_tile_ns<EPI, true, SZ2, false, MT_>(a, kind, idx, t.y, nrows, nb, smem);
   } else {
-    run_tile_ns<EPI, false, false, false>(a, kind, idx, t.y, nrows, nb, smem);
+    run_tile_ns<EPI, false, false, false, MT_>(a, kind, idx, t.y, nrows, nb, smem);
   }
 }
 
 template <int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gmm_bwd_kernel(BwdArgs a) {
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[smem_bytes(false)];
-  gmm_bwd_body<EPI, false>(a, smem);
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[Cfg<128>::smem_bytes(false)];
+  gmm_bwd_body<EPI, false, 128>(a, smem);
 }
 
 // An int4 group of 32 columns (the 64 columns of a wave span two scale/zero groups): the larger ring allows one
 // block per CU.
 template <int EPI>
 __global__ __launch_bounds__(256) void gmm_bwd_kernel_sz2(BwdArgs a) {
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[smem_bytes(true)];
-  gmm_bwd_body<EPI, true>(a, smem);
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[Cfg<128>::smem_bytes(true)];
+  gmm_bwd_body<EPI, true, 128>(a, smem);
+}
+
+// Tile lists of at most 32 rows a tile: 128 registers a wave and at most 26 KB of LDS a block, four blocks per CU. Bound
+// by the weight stream and its dequant (about 40 us each for a 256-expert gate_up bank). Same values, bit for bit, as
+// gmm_bwd_kernel on the same rows. Measured (Qwen shape, 517 tokens: 16 rows per expert; two blocks per CU -> four):
+// down backward 82 -> 72 us, gate_up backward 96 -> 86 us.
+template <int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void
+gmm_bwd_kernel32(BwdArgs a) {
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[Cfg<32>::smem_bytes(false)];
+  gmm_bwd_body<EPI, false, 32>(a, smem);
 }
 
 }  // namespace
@@ -767,6 +798,11 @@ extern "C" int smel_gmm_bwd_lr(const smel_wset* w, const int32_t* gkind, const i
       gmm_bwd_kernel_sz2<1><<<grid, 256, 0, stream>>>(a);
     else
       gmm_bwd_kernel_sz2<0><<<grid, 256, 0, stream>>>(a);
+  } else if (w->flags & SMEL_WSET_TILE32) {
+    if (epilogue == 1)
+      gmm_bwd_kernel32<1><<<grid, 256, 0, stream>>>(a);
+    else
+      gmm_bwd_kernel32<0><<<grid, 256, 0, stream>>>(a);
   } else {
     if (epilogue == 1)
       gmm_bwd_kernel<1><<<grid, 256, 0, stream>>>(a);

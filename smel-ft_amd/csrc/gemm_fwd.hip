@@ -26,20 +26,26 @@
 
 namespace {
 
-constexpr int MT = 128;            // rows of a tile of the tile list
-constexpr int MT_MERGED = 160;     // rows of a merged tile: a full tile + a last tile of <= 32 rows
 constexpr int KT = 64;
+// Rows of a tile and what follows from them. Two kernels: MT 128 for ordinary tile lists (merged tiles of 160 rows
+// among them; 80 KB of A stages, two blocks and 2 waves per SIMD), and MT 32 for lists whose tiles hold at most 32 rows
+// (SMEL_WSET_TILE32): 16 KB of stages and a single 32-row slice of accumulators, so that more blocks share a CU.
 // An A stage holds MT_MERGED rows (row r at r * KT bf16, no padding; the four stages are contiguous). The gate_up
-// epilogue keeps the g and u tiles of 160 x 128 in them; the down epilogue its output tile. A tile of at most MT rows
-// leaves rows MT.. of every stage alone: the down projection keeps its LoRA rows (stages 0 and 1) and its rows'
-// output slots (stage 2) there.
-constexpr int STAGE = MT_MERGED * KT;   // bf16 elements of a stage
-constexpr int SPARE = MT * KT;          // first element of a stage's rows past MT
+// epilogue keeps the g and u tiles of MT_MERGED x 128 in them; the down epilogue its output tile. With MT 128 a tile of
+// at most MT rows leaves rows MT.. of every stage alone: the down projection keeps its LoRA rows (stages 0 and 1) and
+// its rows' output slots (stage 2) there; with MT 32 they have LDS of their own.
+template <int MT_>
+struct Cfg {
+  static constexpr int MT = MT_;
+  static constexpr int MT_MERGED = MT_ == 128 ? 160 : MT_;   // a merged tile: a full tile + a last tile of <= 32 rows
+  static constexpr int STAGE = MT_MERGED * KT;               // bf16 elements of a stage
+  static constexpr int SPARE = MT_ * KT;                     // first element of a stage's rows past MT
+};
 
 // Vector-memory operations per wave in each issue group of the main loops; the issue code below is written with
 // these counts and every wait is computed from them (vmcnt retires in issue order).
-// A rows of a stage: 1-KB LDS-DMA wave-loads of 8 rows; with 4 waves, 4 per wave cover 128 rows, 5 cover 160.
-constexpr int vm_a(int ns) { return ns > 4 ? 5 : 4; }
+// A rows of a stage: 1-KB LDS-DMA wave-loads of 8 rows; with 4 waves, 4 per wave cover 128 rows, 5 cover 160, 1 covers 32.
+constexpr int vm_a(int mt, int ns) { return ns > 4 ? 5 : mt / 32; }
 constexpr int VM_Q = 2;                           // int4: one 16-B word per weight fragment, 2 fragments
 constexpr int VM_SZ = 2;                          // int4: a scale/zero run (16 B) or pair (4 B), per fragment
 constexpr int VM_B = 2 * 4;                       // bf16: 4 substep chunks per fragment, 2 fragments
@@ -74,11 +80,12 @@ struct FwdArgs {
   bool lr_on;
 };
 
-template <int EPI, bool Q4, int NS, bool FAST>
+template <int EPI, bool Q4, int NS, bool FAST, int MT_>
 SMEL_DEV void run_tile(const FwdArgs& a, int kind, int idx, int row0, int nrows, int nb, uint16_t* S0, uint16_t* S1,
                        uint16_t* S2, uint16_t* S3, int* rowmap, uint16_t* X) {
+  constexpr int MT = MT_, MT_MERGED = Cfg<MT_>::MT_MERGED, STAGE = Cfg<MT_>::STAGE;
   static_assert(NS * 32 <= MT_MERGED, "the tile's rows fit the A stages");
-  constexpr int VMA = vm_a(NS);               // A wave-loads per wave and stage
+  constexpr int VMA = vm_a(MT, NS);               // A wave-loads per wave and stage
   constexpr int BF_WAIT = VMA;                // bf16: issue order ... B(j+1), A(j+3): before step j only A(j+2)
   const int tid = threadIdx.x, l = lane_id(), hi = l >> 5, r32 = l & 31;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -136,7 +143,7 @@ SMEL_DEV void run_tile(const FwdArgs& a, int kind, int idx, int row0, int nrows,
     const int P = a.lr.parts;
     const rsrc_t rp = make_rsrc(a.lr.part + (int64_t)row0 * P * 32, (uint64_t)nrows * P * 128);
 #pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {   // 256 threads x 8 values x 2 passes = 128 rows x 32
+    for (int pass = 0; pass < (MT + 63) / 64; ++pass) {   // 256 threads x 8 values a pass = 64 rows x 32
       const int row = (tid >> 2) + 64 * pass, k0 = 8 * (tid & 3);
       float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       for (int p = 0; p < P; ++p) {
@@ -149,7 +156,7 @@ SMEL_DEV void run_tile(const FwdArgs& a, int kind, int idx, int row0, int nrows,
         }
       }
       const u32x4_t h = u32x4_t{pack2bf(v[0], v[1]), pack2bf(v[2], v[3]), pack2bf(v[4], v[5]), pack2bf(v[6], v[7])};
-      *reinterpret_cast<u32x4_t*>(X + pass * STAGE + (row & 63) * 32 + k0) = h;
+      if (row < MT) *reinterpret_cast<u32x4_t*>(X + pass * STAGE + (row & 63) * 32 + k0) = h;
       if (nb == 0 && a.lr.ext_out && row < nrows)
         *reinterpret_cast<u32x4_t*>(a.lr.ext_out + (int64_t)(row0 + row) * 32 + k0) = h;
     }
@@ -596,24 +603,51 @@ SMEL_DEV void run_tile(const FwdArgs& a, int kind, int idx, int row0, int nrows,
   }
 }
 
-template <int EPI, bool Q4, bool FAST>
+template <int EPI, bool Q4, bool FAST, int MT_>
 SMEL_DEV void run_tile_ns(const FwdArgs& a, int kind, int idx, int row0, int nrows, int nb, uint16_t* S0,
                           uint16_t* S1, uint16_t* S2, uint16_t* S3, int* rowmap, uint16_t* X) {
-  switch ((nrows + 31) >> 5) {
-    case 1: run_tile<EPI, Q4, 1, FAST>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X); break;
-    case 2: run_tile<EPI, Q4, 2, FAST>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X); break;
-    case 3: run_tile<EPI, Q4, 3, FAST>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X); break;
-    case 4: run_tile<EPI, Q4, 4, FAST>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X); break;
-    default:   // 5 slices: only a merged int4 tile (fast dequant form) has more rows
-      if constexpr (Q4 && FAST)
-        run_tile<EPI, Q4, 5, FAST>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X);
-      break;
+  if constexpr (MT_ == 32) {
+    run_tile<EPI, Q4, 1, FAST, MT_>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X);
+  } else {
+    switch ((nrows + 31) >> 5) {
+      case 1: run_tile<EPI, Q4, 1, FAST, MT_>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X); break;
+      case 2: run_tile<EPI, Q4, 2, FAST, MT_>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X); break;
+      case 3: run_tile<EPI, Q4, 3, FAST, MT_>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X); break;
+      case 4: run_tile<EPI, Q4, 4, FAST, MT_>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X); break;
+      default:   // 5 slices: only a merged int4 tile (fast dequant form) has more rows
+        if constexpr (Q4 && FAST)
+          run_tile<EPI, Q4, 5, FAST, MT_>(a, kind, idx, row0, nrows, nb, S0, S1, S2, S3, rowmap, X);
+        break;
+    }
+  }
+}
+
+template <int EPI>
+SMEL_DEV void gmm_fwd_body32(const FwdArgs& a, uint16_t* S0, uint16_t* S1, uint16_t* S2, uint16_t* S3, int* rowmap,
+                             uint16_t* X) {
+  int tile, nb;
+  const int n_t = a.n_tiles[0];
+  if (!((a.w.flags & SMEL_WSET_XCD_CHUNK) ? xcd_tile_chunk(n_t, a.nblk, tile, nb) : xcd_tile(n_t, a.nblk, tile, nb)))
+    return;
+  const int4 t = a.tiles[tile];
+  const int gk = a.gkind ? a.gkind[t.x] : t.w;
+  const int kind = gk >> 16, idx = gk & 0xffff;
+  const int nrows = min(t.z - t.y, 32);
+  if (nrows <= 0) return;
+  if (kind == SMEL_KIND_INT4) {
+    if (a.w.flags & SMEL_WSET_FAST_DQ)
+      run_tile_ns<EPI, true, true, 32>(a, kind, idx, t.y, nrows, nb, S0, S1, S2, S3, rowmap, X);
+    else
+      run_tile_ns<EPI, true, false, 32>(a, kind, idx, t.y, nrows, nb, S0, S1, S2, S3, rowmap, X);
+  } else {
+    run_tile_ns<EPI, false, false, 32>(a, kind, idx, t.y, nrows, nb, S0, S1, S2, S3, rowmap, X);
   }
 }
 
 template <int EPI>
 SMEL_DEV void gmm_fwd_body(const FwdArgs& a, uint16_t* S0, uint16_t* S1, uint16_t* S2, uint16_t* S3, int* rowmap,
                            uint16_t* X) {
+  constexpr int MT = 128, MT_MERGED = Cfg<128>::MT_MERGED;
   int tile, nb;
   const int n_t = a.n_tiles[0];
   if (!((a.w.flags & SMEL_WSET_XCD_CHUNK) ? xcd_tile_chunk(n_t, a.nblk, tile, nb) : xcd_tile(n_t, a.nblk, tile, nb)))
@@ -644,11 +678,11 @@ SMEL_DEV void gmm_fwd_body(const FwdArgs& a, uint16_t* S0, uint16_t* S1, uint16_
   if (nrows <= 0) return;
   if (kind == SMEL_KIND_INT4) {
     if (a.w.flags & SMEL_WSET_FAST_DQ)
-      run_tile_ns<EPI, true, true>(a, kind, idx, t.y, nrows, nb, S0, S1, S2, S3, rowmap, X);
+      run_tile_ns<EPI, true, true, 128>(a, kind, idx, t.y, nrows, nb, S0, S1, S2, S3, rowmap, X);
     else
-      run_tile_ns<EPI, true, false>(a, kind, idx, t.y, nrows, nb, S0, S1, S2, S3, rowmap, X);
+      run_tile_ns<EPI, true, false, 128>(a, kind, idx, t.y, nrows, nb, S0, S1, S2, S3, rowmap, X);
   } else {
-    run_tile_ns<EPI, false, false>(a, kind, idx, t.y, min(nrows, MT), nb, S0, S1, S2, S3, rowmap, X);
+    run_tile_ns<EPI, false, false, 128>(a, kind, idx, t.y, min(nrows, MT), nb, S0, S1, S2, S3, rowmap, X);
   }
 }
 
@@ -657,6 +691,7 @@ SMEL_DEV void gmm_fwd_body(const FwdArgs& a, uint16_t* S0, uint16_t* S1, uint16_
 // rows; a merged tile of more is an int4 tile, without either).
 template <int EPI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gmm_fwd_kernel(FwdArgs a) {
+  constexpr int STAGE = Cfg<128>::STAGE, SPARE = Cfg<128>::SPARE;
   __shared__ __attribute__((aligned(1024))) uint16_t ring[4 * STAGE];
   uint16_t* const S0 = ring;
   if constexpr (EPI == 0)
@@ -664,6 +699,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                       reinterpret_cast<int*>(S0 + 2 * STAGE + SPARE), S0 + SPARE);
   else
     gmm_fwd_body<EPI>(a, S0, S0 + STAGE, S0 + 2 * STAGE, S0 + 3 * STAGE, nullptr, nullptr);
+}
+
+// Tile lists of at most 32 rows a tile: 128 registers a wave and at most 26 KB of LDS a block, four blocks per CU. Bound
+// by the weight stream and its dequant (about 40 us each for a 256-expert gate_up bank). Same values, bit for bit, as
+// gmm_fwd_kernel on the same rows. Measured (Qwen shape, 517 tokens: 16 rows per expert; two blocks per CU -> four):
+// gate_up 97 -> 90 us (forward only: 90 -> 76), down 56 -> 54 us; 23 tokens: gate_up 64 -> 48, down 30 -> 28 us.
+template <int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void
+gmm_fwd_kernel32(FwdArgs a) {
+  constexpr int STAGE = Cfg<32>::STAGE;
+  __shared__ __attribute__((aligned(1024))) uint16_t ring[4 * STAGE];
+  __shared__ __attribute__((aligned(16))) uint16_t X[EPI == 0 ? 32 * 32 : 8];
+  __shared__ int rowmap[32];
+  uint16_t* const S0 = ring;
+  gmm_fwd_body32<EPI>(a, S0, S0 + STAGE, S0 + 2 * STAGE, S0 + 3 * STAGE, rowmap, X);
 }
 
 }  // namespace
@@ -697,6 +747,8 @@ extern "C" int smel_gmm_fwd_lr(const smel_wset* w, const int32_t* gkind, const i
                SMEL_EINVAL,
                "gmm_fwd: a merged tile list (SMEL_WSET_MERGED_LIST) on an int4 bank needs its fast dequant form and K "
                "a multiple of 64");
+  SMEL_REQUIRE(!(w->flags & SMEL_WSET_TILE32) || !(w->flags & (SMEL_WSET_MERGED_LIST | SMEL_WSET_MERGE_SHORT)),
+               SMEL_EINVAL, "gmm_fwd: SMEL_WSET_TILE32 excludes merged tiles");
   SMEL_REQUIRE(!a_gather || order || TK == 0, SMEL_EINVAL, "gmm_fwd: gather needs order");
   SMEL_REQUIRE(act == 0 || act == 1, SMEL_EINVAL, "gmm_fwd: act %d", act);
   SMEL_REQUIRE(a_rows >= 0 && a_rows * lda * 2 < (1ll << 31), SMEL_EUNSUPPORTED, "gmm_fwd: A larger than 2 GiB");
@@ -732,10 +784,16 @@ extern "C" int smel_gmm_fwd_lr(const smel_wset* w, const int32_t* gkind, const i
   a.K = (int)w->C;
   a.nblk = (int)(epilogue == 1 ? (w->R / 2 + 127) / 128 : (w->R + 255) / 256);
   const unsigned grid = (unsigned)(xcd_grid(max_tiles) * a.nblk);
-  if (epilogue == 1)
+  if (w->flags & SMEL_WSET_TILE32) {
+    if (epilogue == 1)
+      gmm_fwd_kernel32<1><<<grid, 256, 0, stream>>>(a);
+    else
+      gmm_fwd_kernel32<0><<<grid, 256, 0, stream>>>(a);
+  } else if (epilogue == 1) {
     gmm_fwd_kernel<1><<<grid, 256, 0, stream>>>(a);
-  else
+  } else {
     gmm_fwd_kernel<0><<<grid, 256, 0, stream>>>(a);
+  }
   return smel::launch_status();
 }
 

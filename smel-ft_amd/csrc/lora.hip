@@ -218,9 +218,10 @@ __global__ __launch_bounds__(512) void lora_ext_kernel(const int4* __restrict__ 
   const rsrc_t ra = make_rsrc(A, (uint64_t)a_rows * lda * 2);
   const int nk = (Kd + 63) / 64;
   for (int item = blockIdx.x; item < 4 * total; item += gridDim.x) {
-    const int4 t = lt[item >> 2];
+    // slice-major: tiles of one slice each (short lists, last tiles) would otherwise leave three blocks of four idle
+    const int m = item / total;
+    const int4 t = lt[item - m * total];
     const int kind = t.w >> 16, idx = t.w & 0xffff;
-    const int m = item & 3;
     const int nrows = min(t.z - t.y, 128);
     if (m * 32 >= nrows) continue;   // uniform over the block
     const uint16_t* wc = kind == SMEL_KIND_SEL ? wsel + (int64_t)idx * 32 * Kd : wsh;

@@ -31,6 +31,7 @@ from .quant import dequant_int4, quantize_int4
 
 M_TILE = 128      # rows per GEMM tile (the tile list of smel_dispatch)
 M_MERGED = 160    # rows of a merged gate_up forward tile (a full tile + an int4 expert's last tile of <= 32 rows)
+M_SHORT = 32      # rows per tile of a short list (_tile_rows)
 EXT = 32          # width of one plane of the LoRA K-extension
 MAX_LORA_RANK = 32
 
@@ -791,6 +792,16 @@ def _prep_lora(ex: LayerExperts, lora_ex, lora_sh, with_shared: bool, H: int, de
     return lb_ex, lb_sh
 
 
+def _tile_rows(TK: int, E: int, lora: bool) -> int:
+    """Rows per tile of a layer's lists. With few rows per expert nearly every tile is one 32-row slice, whose blocks
+    are bound by latency and by the last, partial round of blocks: the 32-row kernels (SMEL_WSET_TILE32) keep twice as
+    many on a CU. The line lies where experts of more than 32 rows, whose weights a short list streams and dequantizes
+    twice, cost as much: measured (Qwen shape, top-8 of 256, sum of launches) 517 tokens forward 190 -> 175 us, 768
+    194 -> 187, 1024 209 -> 214; forward and backward 517 tokens 522 -> 493 us, 640 514 -> 486, 1024 538 -> 555; under
+    Zipf routing (half of the rows on 12 LoRA experts) 300 tokens 497 -> 456, 517 524 -> 517, 700 551 -> 580."""
+    return M_SHORT if TK <= (18 if lora else 26) * E else M_TILE
+
+
 def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool, shared, lora_ex, lora_sh,
                       need_grad: bool, c: _Ctx, prep=None, shared_rows=None, counted_ws=None, ext_pre=None):
     """Dispatch + expert GEMMs + combine. ``shared`` = (gate_up, down, sgate fp32 [T], gate_up^T, down^T) or None
@@ -807,13 +818,14 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
     TK = T * K
     rows_sh = T if shared is not None else 0
     M = TK + rows_sh
-    maxt = L.load().smel_dispatch_max_tiles(TK, E, rows_sh, M_TILE)
+    mt = _tile_rows(TK, E, lora_ex is not None or lora_sh is not None)
+    maxt = L.load().smel_dispatch_max_tiles(TK, E, rows_sh, mt)
     i32 = lambda *s: torch.empty(*s, dtype=torch.int32, device=dev)
     counts, offsets, order, inv = i32(E), i32(E + 1), i32(max(TK, 1)), i32(max(TK, 1))
     tiles, tiles_g, ntiles, err = i32(maxt * 4), i32(maxt * 4), i32(1), i32(1)
     # the gate_up forward's merged tile list: an int4 expert's last tile of <= 32 rows joins its full tile
     fz = ex.frozen
-    merge = _MERGE_SHORT and isinstance(fz, Int4Experts) and H % 64 == 0 and fz.fast_dq("gu")
+    merge = mt == M_TILE and _MERGE_SHORT and isinstance(fz, Int4Experts) and H % 64 == 0 and fz.fast_dq("gu")
     tiles_m, ntiles_m = (i32(maxt * 4), i32(1)) if merge else (None, None)
     dws = counted_ws if counted_ws is not None else i32(max(1, L.load().smel_dispatch_ws_size(TK, E)))
     if prep is None:   # LoRA layouts on a side stream, overlapping the dispatch
@@ -823,7 +835,7 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
         prep = (fork, bufs)
     gk_groups = ex.gkind(shared is not None, dev)
     L.call("smel_dispatch_counted" if counted_ws is not None else "smel_dispatch", L.ptr(topi_ids), int(ids_i64), T, K,
-           E, rows_sh, M_TILE, L.ptr(gk_groups), L.ptr(counts), L.ptr(offsets), L.ptr(order), L.ptr(inv), L.ptr(tiles),
+           E, rows_sh, mt, L.ptr(gk_groups), L.ptr(counts), L.ptr(offsets), L.ptr(order), L.ptr(inv), L.ptr(tiles),
            L.ptr(tiles_g), L.ptr(ntiles), L.ptr(err), M_MERGED if merge else 0, L.ptr(tiles_m), L.ptr(ntiles_m),
            L.ptr(dws), st, tag="smel_dispatch")
     gk = None   # the tile list carries each tile's group kind
@@ -854,7 +866,8 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
     # group order, a chunk per XCD (an expert's tiles share its weights in L2); the down GEMMs the long-tiles-first
     # order (short tiles fill the last round)
     w_gu = _wset(ex, "gu", sel_gu, sh_gu, g(lb_ex, "fwd_gu"), g(lb_sh, "fwd_gu"), planes=planes)
-    w_gu.flags |= L.WSET_MERGED_LIST if merge else L.WSET_XCD_CHUNK
+    short = L.WSET_TILE32 if mt == M_SHORT else 0
+    w_gu.flags |= short | (L.WSET_MERGED_LIST if merge else L.WSET_XCD_CHUNK)
     # the down LoRA's rows come from the gate_up epilogue (per-column-block partials of h A_dn^T), summed and stored
     # by the down GEMM: no separate projection launch
     lr = None
@@ -872,6 +885,7 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
         ext_dn = _lora_ext(tl, actb, I, M, 0, order, TK, K, lb_ex, lb_sh, "a_dn", I, 1, M, dev, st)
     Y = bf(M, H)
     w_dn = _wset(ex, "dn", sel_dn, sh_dn, g(lb_ex, "fwd_dn"), g(lb_sh, "fwd_dn"))
+    w_dn.flags |= short
     # the down forward on the same merged list when its bank is in the fast form too (and I a multiple of 64)
     merge_dn = merge and I % 64 == 0 and fz.fast_dq("dn")
     if merge_dn:
@@ -886,7 +900,7 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
         sgate, ysh = shared_rows
     L.call("smel_combine", L.ptr(Y), L.ptr(topv), L.ptr(inv), L.ptr(sgate), L.ptr(ysh), T, K, H, L.ptr(out), st)
     # everything the backward needs
-    c.T, c.H, c.I, c.E, c.K, c.TK, c.M, c.maxt = T, H, I, E, K, TK, M, maxt
+    c.T, c.H, c.I, c.E, c.K, c.TK, c.M, c.maxt, c.short = T, H, I, E, K, TK, M, maxt, short
     c.ex, c.shared_w = ex, (sh_gu_t, sh_dn_t) if shared is not None else None
     sel_t = ex.packed_sel_t() if (need_grad and sel_gu is not None) else None
     c.tensors = dict(x=x, topv=topv, sgate=sgate, counts=counts, offsets=offsets, order=order, inv=inv, tiles=tiles,
@@ -925,6 +939,7 @@ def _backward_pipeline(c: _Ctx, dout: torch.Tensor, router=None, shared_split=No
     dh = bf(M, 2 * I)
     dwp = torch.empty(M, nblk, dtype=torch.float32, device=dev)
     w_dn = _wset(ex, "dn", t["sel_dn"], sh_dn, g(lb_ex, "at_dn"), g(lb_sh, "at_dn"), t=True)
+    w_dn.flags |= c.short
     # with the LoRA rows from this GEMM's epilogue: DXA = s [dg B_g, du B_u] as per-column-block partials
     lrows = _bwd_lora_rows(lb_ex, lb_sh, nblk, M, planes, dev) if any_lora and _BWD_LORA_ROWS else None
     lr = ctypes.byref(lrows[0]) if lrows is not None else None
@@ -989,7 +1004,7 @@ def _backward_pipeline(c: _Ctx, dout: torch.Tensor, router=None, shared_split=No
     # (4) gate_up backward: per-slot dx rows
     dxs = bf(M, H)
     w_gu = _wset(ex, "gu", t["sel_gu"], sh_gu, g(lb_ex, "at_gu"), g(lb_sh, "at_gu"), t=True, planes=planes)
-    w_gu.flags |= L.WSET_XCD_CHUNK
+    w_gu.flags |= L.WSET_XCD_CHUNK | c.short
     L.call("smel_gmm_bwd_lr", ctypes.byref(w_gu), L.ptr(gk), L.ptr(t["tiles_g"]), L.ptr(ntiles), maxt, L.ptr(dh),
            2 * I, M, 0, L.ptr(order), TK, K, None if lrows is not None else L.ptr(ext_dxa), 0, _ACT[ex.act], None, None,
            None, L.ptr(dxs), H, None, lr, st, tag="gemm_gu_bwd")

@@ -617,6 +617,23 @@ def test_merged_short_tiles_bitwise(name, monkeypatch):
         assert torch.equal(a["grads"][k], b["grads"][k]), k
 
 
+@pytest.mark.parametrize("name", sorted(LAYERS))
+def test_short_tiles_bitwise(name, monkeypatch):
+    """The 32-row kernels (SMEL_WSET_TILE32, chosen for few rows per expert) accumulate every row as the 128-row kernels
+    do, whatever tiles the rows are in: y, dX and the LoRA gradients of a layer are bitwise equal on either list."""
+    import smel.moe as M
+    _say(f"short tiles {name}")
+    out = []
+    for mt in (M.M_SHORT, M.M_TILE):
+        monkeypatch.setattr(M, "_tile_rows", lambda *a, mt=mt: mt)
+        out.append(run_layer(name, seed=2))
+    a, b = out
+    assert torch.equal(a["y"].view(torch.int16), b["y"].view(torch.int16))
+    assert torch.equal(a["dx"].view(torch.int16), b["dx"].view(torch.int16))
+    for k in b["grads"]:
+        assert torch.equal(a["grads"][k], b["grads"][k]), k
+
+
 @pytest.mark.parametrize("name", ["r16", "r24_mixed", "c1"])
 def test_shared_lora_rows_on_side_stream_bitwise(name, monkeypatch):
     """The fused shared expert's gate_up LoRA rows projected on a side stream beside the router (SMEL_FWD_EXT_SIDE,
