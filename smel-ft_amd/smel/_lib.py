@@ -248,7 +248,51 @@ def ptr(t: torch.Tensor | None):
 
 
 def stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current HIP stream's handle on the current device."""
+    return _raw_stream(_device()) if _raw_stream is not None else torch.cuda.current_stream().cuda_stream
+
+
+# the handle alone, without building a torch.cuda.Stream object per launch (about 5 us); None on a torch without them
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None)
+if _device is None:
+    _raw_stream = None
+
+
+class Carve:
+    """One device allocation cut into buffers: ``take(bytes)`` plans a 256-byte aligned buffer, ``alloc()`` makes the
+    memory (on the current stream). A pass needs some thirty small buffers; each allocation of its own costs the host
+    as much as a launch. The buffers keep the memory alive."""
+
+    __slots__ = ("n", "t")
+
+    def __init__(self):
+        self.n, self.t = 0, None
+
+    def take(self, nbytes: int) -> "Buf":
+        b = Buf(self, self.n)
+        self.n += (max(int(nbytes), 1) + 255) & ~255
+        return b
+
+    def alloc(self, device) -> "Carve":
+        self.t = torch.empty(max(self.n, 256), dtype=torch.uint8, device=device)
+        return self
+
+
+class Buf:
+    """A buffer of a Carve; ``ptr`` takes it like a tensor."""
+
+    __slots__ = ("c", "off")
+
+    def __init__(self, c: Carve, off: int):
+        self.c, self.off = c, off
+
+    def data_ptr(self) -> int:
+        return self.c.t.data_ptr() + self.off
+
+    def tensor(self, dtype, n: int) -> torch.Tensor:
+        """The buffer's first n values as a tensor."""
+        return self.c.t[self.off:self.off + n * dtype.itemsize].view(dtype)
 
 
 def require_device(*ts):

@@ -19,6 +19,8 @@ shared expert in fp32 before the single rounding; gradients are accumulated in f
 from __future__ import annotations
 
 import ctypes
+import functools
+import math
 import os
 from collections import OrderedDict
 
@@ -328,8 +330,15 @@ def _dense_tiles(T: int, device):
         for i in range(n):
             t[i, 0], t[i, 1], t[i, 2], t[i, 3] = 0, i * M_TILE, min(T, (i + 1) * M_TILE), L.KIND_SHARED << 16
         _dense_tiles_cache[key] = (t.reshape(-1).to(device), torch.tensor([n], dtype=torch.int32, device=device),
-                                   n, torch.tensor([L.KIND_SHARED << 16], dtype=torch.int32, device=device))
-    return _dense_tiles_cache[key]
+                                   n, torch.tensor([L.KIND_SHARED << 16], dtype=torch.int32, device=device),
+                                   torch.zeros(2, dtype=torch.int32).to(device))
+    return _dense_tiles_cache[key][:4]
+
+
+def _dense_zeros(T: int, device) -> torch.Tensor:
+    """Two zeros kept with the tile list of the same rows."""
+    _dense_tiles(T, device)
+    return _dense_tiles_cache[(T, str(device))][4]
 
 
 def _router_ext_weight(gate_w: torch.Tensor, sg_w: torch.Tensor | None, store: dict | None = None) -> PackedW:
@@ -394,25 +403,33 @@ def _side_stream(dev, i: int) -> torch.cuda.Stream:
 
 
 class _Fork:
-    """``with _Fork(dev, i) as s:`` launches on side stream i after the current stream's work so far; ``join()``
-    makes the current (main) stream wait for everything launched there."""
+    """``with _Fork(dev, i) as st:`` launches on side stream i (handle ``st``) after the current stream's work so far;
+    ``join()`` makes the current (main) stream wait for everything launched there. Launches take the handle, so torch's
+    current stream is switched only while launches are timed (their events go to it)."""
 
     def __init__(self, dev, i: int, on: bool = None):
-        self.main = torch.cuda.current_stream(dev)
-        self.side = _side_stream(dev, i) if (i in _SIDE_ON if on is None else on) else self.main
-        if self.side is not self.main:
+        if i in _SIDE_ON if on is None else on:
+            self.main = torch.cuda.current_stream(dev)
+            self.side = _side_stream(dev, i)
             self.side.wait_stream(self.main)
-        self._ctx = torch.cuda.stream(self.side)
+            self.st = self.side.cuda_stream
+        else:
+            self.side, self.st = None, L.stream()
+        self._ctx = None
 
     def __enter__(self):
-        self._ctx.__enter__()
-        return self.side
+        if self.side is not None and L._timing is not None:
+            self._ctx = torch.cuda.stream(self.side)
+            self._ctx.__enter__()
+        return self.st
 
     def __exit__(self, *exc):
-        return self._ctx.__exit__(*exc)
+        if self._ctx is not None:
+            ctx, self._ctx = self._ctx, None
+            return ctx.__exit__(*exc)
 
     def join(self):
-        if self.side is not self.main:
+        if self.side is not None:
             self.main.wait_stream(self.side)
 
 
@@ -421,62 +438,68 @@ class _LoRABufs:
     gate_up side has ``planes`` 32-wide planes (a_gu, bt_gu: plane-major, one [n][32][K] matrix per plane; at_gu:
     [n][planes][H][32])."""
 
-    def __init__(self, lora, n: int, H: int, I: int, device, planes: int = 1, prep: bool = True):
+    def __init__(self, lora, n: int, H: int, I: int, planes: int, mem: L.Carve):
         self.scale = float(lora.scale)
         self.r = lora.r
         self.planes = planes
         self.H, self.I = H, I
-        e = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device=device)
+        e = lambda *s: mem.take(2 * math.prod(s))
         self.fwd_gu, self.fwd_dn = e(n, 2 * I, EXT), e(n, H, EXT)
         self.a_gu, self.a_dn = e(planes, n, EXT, H), e(n, EXT, I)
         self.bt_dn, self.bt_gu = e(n, EXT, H), e(planes, n, EXT, 2 * I)
         self.at_gu, self.at_dn = e(n, planes, H, EXT), e(n, I, EXT)
-        self.factors = [getattr(lora, k).detach().float().contiguous() for k in
-                        ("A_gate", "B_gate", "A_up", "B_up", "A_down", "B_down")]
+        self.plane_bytes = {"a_gu": 2 * n * EXT * H, "bt_gu": 2 * n * EXT * 2 * I}
+        self.factors = [p if p.dtype == torch.float32 and p.is_contiguous() else p.detach().float().contiguous()
+                        for p in (_factor(lora, k) for k in _PREP_NAMES)]
         self.n = n
-        if prep:
-            _prep_sets([self])
 
     def lora_set(self) -> L.LoraSet:
-        s = L.LoraSet(*[L.ptr(p) for p in self.factors], self.n, self.r)
-        for k in ("fwd_gu", "fwd_dn", "a_gu", "a_dn", "bt_dn", "bt_gu", "at_gu", "at_dn"):
-            setattr(s, k, L.ptr(getattr(self, k)))
-        return s
+        return L.LoraSet(*[p.data_ptr() for p in self.factors], self.n, self.r,
+                         *[getattr(self, k).data_ptr() for k in _LAYOUTS])
 
 
-def _prep_sets(bufs) -> None:
+_PREP_NAMES = ("A_gate", "B_gate", "A_up", "B_up", "A_down", "B_down")
+_LAYOUTS = ("fwd_gu", "fwd_dn", "a_gu", "a_dn", "bt_dn", "bt_gu", "at_gu", "at_dn")
+
+
+def _factor(lora, name: str):
+    """A factor of a LoRA set, past torch's module attribute lookup where it is a plain parameter."""
+    p = lora._parameters.get(name)
+    return p if p is not None else getattr(lora, name)
+
+
+def _lora_bufs(sets, H: int, planes: int, dev, st):
+    """The bf16 layouts of LoRA sets [(lora or None, n, I), ...] in one allocation and one launch (None for None)."""
+    mem = L.Carve()
+    bufs = [_LoRABufs(m, n, H, I, planes, mem) if m is not None else None for m, n, I in sets]
+    if any(b is not None for b in bufs):
+        mem.alloc(dev)
+        _prep_sets(bufs, st)
+    return bufs
+
+
+def _prep_sets(bufs, st) -> None:
     """smel_lora_prep_sets: the bf16 layouts of one or two LoRA sets (same shapes and planes) in one launch."""
     bufs = [b for b in bufs if b is not None]
-    if not bufs:
-        return
     arr = (L.LoraSet * len(bufs))(*[b.lora_set() for b in bufs])
     b0 = bufs[0]
-    L.call("smel_lora_prep_sets", arr, len(bufs), b0.planes, b0.H, b0.I, L.stream(), tag="smel_lora_prep")
+    L.call("smel_lora_prep_sets", arr, len(bufs), b0.planes, b0.H, b0.I, st, tag="smel_lora_prep")
 
 
-_PLANE_MAJOR = ("a_gu", "bt_gu")   # layouts with a leading plane dimension (lora_ext operands)
-
-
-def _lora_ext(tl, A, lda, a_rows, gather, order, TK, K, lb_ex, lb_sh, name: str, Kd: int, planes: int, M: int, dev,
-              st, ext=None, row0: int = 0):
-    """ext rows [M][32 * planes] of one direction: smel_lora_ext once per plane (``name`` = the layout the rows are
-    projected on; the down side's layouts have one plane). ``tl`` = (tiles, n_tiles, max_tiles, gkind). ``ext`` = a
-    buffer to fill instead of a new one, the tiles' row r going to its row row0 + r."""
+def _lora_ext(tl, A, lda, a_rows, gather, order, TK, K, lb_ex, lb_sh, name: str, Kd: int, planes: int, ext, st,
+              row0: int = 0):
+    """ext rows [M][32 * planes] of one direction into the buffer ``ext`` (the tiles' row r to its row row0 + r):
+    smel_lora_ext once per plane (``name`` = the layout the rows are projected on; the down side's layouts have one
+    plane). ``tl`` = (tiles, n_tiles, max_tiles, gkind)."""
     tiles, ntiles, maxt, gk = tl
-    if ext is None:
-        ext = torch.empty(M, EXT * planes, dtype=torch.bfloat16, device=dev)
     base = ext.data_ptr() + 2 * row0 * EXT * planes
     s_ex = lb_ex.scale if lb_ex is not None else 0.0
     s_sh = lb_sh.scale if lb_sh is not None else 0.0
     for c in range(planes):
-        def w(lb):
-            if lb is None:
-                return None
-            t = getattr(lb, name)
-            return t[c] if name in _PLANE_MAJOR else t
+        def w(lb):   # plane c of the plane-major layouts
+            return None if lb is None else getattr(lb, name).data_ptr() + c * lb.plane_bytes.get(name, 0)
         L.call("smel_lora_ext", L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(gk), L.ptr(A), lda, a_rows, gather,
-               L.ptr(order), TK, K, L.ptr(w(lb_ex)), L.ptr(w(lb_sh)), Kd, s_ex, s_sh, base + 2 * EXT * c,
-               EXT * planes, st)
+               L.ptr(order), TK, K, w(lb_ex), w(lb_sh), Kd, s_ex, s_sh, base + 2 * EXT * c, EXT * planes, st)
     return ext
 
 
@@ -492,34 +515,31 @@ def _token_tiles(T: int, E: int, dev):
     return cache[key]
 
 
-def _shared_lora_ext(x, K: int, E: int, bufs, dev):
+def _shared_lora_ext(x, K: int, E: int, bufs, dev, st):
     """The gate_up LoRA projection of the fused shared expert's rows [TK, TK + T) (x in token order, no routing
     needed) into a new ext buffer of all TK + T rows; the routed rows are filled after the dispatch."""
     lb_ex, lb_sh = bufs
     T, H = x.shape
     planes = (lb_ex or lb_sh).planes
     ext = torch.empty(T * K + T, EXT * planes, dtype=torch.bfloat16, device=dev)
-    return _lora_ext(_token_tiles(T, E, dev), x, H, T, 0, None, 0, 1, None, lb_sh, "a_gu", H, planes, T, dev,
-                     L.stream(), ext=ext, row0=T * K)
+    return _lora_ext(_token_tiles(T, E, dev), x, H, T, 0, None, 0, 1, None, lb_sh, "a_gu", H, planes, ext, st,
+                     row0=T * K)
 
 
-def _bwd_lora_rows(lb_ex, lb_sh, nblk: int, M: int, planes: int, dev):
+def _bwd_lora_rows(lb_ex, lb_sh, nblk: int, planes: int, part):
     """smel_bwd_lora_rows for the down backward (producer) and the gate_up backward (consumer), with its fp32 partial
-    buffer [M][nblk][planes][32]."""
-    part = torch.empty(M, nblk, planes, EXT, dtype=torch.float32, device=dev)
-    lr = L.BwdLoraRows(L.ptr(lb_ex.bt_gu) if lb_ex is not None else None,
-                       L.ptr(lb_sh.bt_gu) if lb_sh is not None else None,
-                       lb_ex.scale if lb_ex is not None else 0.0, lb_sh.scale if lb_sh is not None else 0.0,
-                       lb_ex.n if lb_ex is not None else 0, planes, L.ptr(part), nblk)
-    return lr, part
+    buffer ``part`` [M][nblk][planes][32]."""
+    return L.BwdLoraRows(L.ptr(lb_ex.bt_gu) if lb_ex is not None else None,
+                         L.ptr(lb_sh.bt_gu) if lb_sh is not None else None,
+                         lb_ex.scale if lb_ex is not None else 0.0, lb_sh.scale if lb_sh is not None else 0.0,
+                         lb_ex.n if lb_ex is not None else 0, planes, L.ptr(part), nblk)
 
 
-def _lora_rows_sum(tl, lr, lb_ex, lb_sh, M: int, planes: int, dev, st):
-    """bf16 rows [M][32 planes] of the LoRA tiles from the partials of ``lr`` (for the LoRA gradients)."""
+def _lora_rows_sum(tl, lr, lb_ex, lb_sh, ext, st):
+    """bf16 rows [M][32 planes] of the LoRA tiles into ``ext`` from the partials of ``lr`` (for the LoRA gradients)."""
     tiles, ntiles, maxt, gk = tl
-    ext = torch.empty(M, EXT * planes, dtype=torch.bfloat16, device=dev)
     L.call("smel_lora_rows_sum", L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(gk), int(lb_ex is not None),
-           int(lb_sh is not None), lr.part, lr.parts, planes, L.ptr(ext), st, tag="smel_lora_rows")
+           int(lb_sh is not None), lr.part, lr.parts, lr.planes, L.ptr(ext), st, tag="smel_lora_rows")
     return ext
 
 
@@ -665,20 +685,21 @@ class _RouteFn(torch.autograd.Function):
         dl = torch.empty(T, Epad, dtype=torch.bfloat16, device=dev)
         L.call("smel_route_bwd", L.ptr(dwp), 1, None, L.ptr(probs), L.ptr(topi32), None, None, 0, T, K, E, T * K,
                L.ptr(dl), Epad, None, None, L.stream())
-        dx = _router_dx(dl, wr, T)
+        dx = _router_dx(dl, wr, T, dev, L.stream())
         return dx, None, None
 
 
-def _router_dx(dl: torch.Tensor, wr: PackedW, T: int, dx: torch.Tensor | None = None) -> torch.Tensor:
+def _router_dx(dl, wr: PackedW, T: int, dev, st, dx=None):
+    """dx [T, H] (a new tensor, or the buffer given) = dl [T][wr.R] times the router weight."""
     H = wr.C
-    tiles, ntiles, maxt, gk = _dense_tiles(T, dl.device)
+    tiles, ntiles, maxt, gk = _dense_tiles(T, dev)
     if dx is None:
-        dx = torch.empty(T, H, dtype=torch.bfloat16, device=dl.device)
+        dx = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
     w = L.WSet()
     w.wsh = L.ptr(wr.t)
     w.R, w.C, w.group = wr.R, H, 32
-    L.call("smel_gmm_bwd", ctypes.byref(w), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(dl), dl.shape[1], T, 0,
-           None, 0, 1, None, 0, 0, None, None, None, L.ptr(dx), H, None, L.stream(), tag="gemm_router_bwd")
+    L.call("smel_gmm_bwd", ctypes.byref(w), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(dl), wr.R, T, 0,
+           None, 0, 1, None, 0, 0, None, None, None, L.ptr(dx), H, None, st, tag="gemm_router_bwd")
     return dx
 
 
@@ -729,7 +750,7 @@ class _RouteGemma4Fn(torch.autograd.Function):
         dw = dtopv.float().contiguous()
         L.call("smel_route_bwd", L.ptr(dw), 1, None, L.ptr(probs), L.ptr(topi32), None, None, 0, T, K, E, T * K,
                L.ptr(dl), wr.R, None, L.ptr(pes), L.stream())
-        dxn = _router_dx(dl, wr, T)
+        dxn = _router_dx(dl, wr, T, dev, L.stream())
         dh = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
         L.call("smel_route_gemma4_prenorm_bwd", L.ptr(h), L.ptr(scale), L.ptr(rstd), L.ptr(dxn), T, H, L.ptr(dh),
                L.stream())
@@ -778,18 +799,15 @@ def _expert_I(ex: LayerExperts) -> int:
     return (ex.frozen.dn["q"].shape[2] * 2) if isinstance(ex.frozen, Int4Experts) else ex.frozen.down.shape[2]
 
 
-def _prep_lora(ex: LayerExperts, lora_ex, lora_sh, with_shared: bool, H: int, dev):
-    """The bf16 LoRA layouts of the selected experts and the shared MLP (lora_prep launches on the current stream),
-    with the gate_up planes both sets need."""
+def _prep_lora(ex: LayerExperts, lora_ex, lora_sh, with_shared: bool, H: int, dev, st):
+    """The bf16 LoRA layouts of the selected experts and the shared MLP (a lora_prep launch on stream ``st``), with the
+    gate_up planes both sets need."""
     I = _expert_I(ex)
     has_sel = ex.sel_ids is not None and len(ex._slot)
     use_ex = lora_ex if (lora_ex is not None and has_sel) else None
     use_sh = lora_sh if (lora_sh is not None and with_shared) else None
     planes = _lora_planes(use_ex, use_sh)
-    lb_ex = _LoRABufs(use_ex, len(ex._slot), H, I, dev, planes, prep=False) if use_ex is not None else None
-    lb_sh = _LoRABufs(use_sh, 1, H, I, dev, planes, prep=False) if use_sh is not None else None
-    _prep_sets([lb_ex, lb_sh])   # both sets in one launch
-    return lb_ex, lb_sh
+    return _lora_bufs([(use_ex, len(ex._slot), I), (use_sh, 1, I)], H, planes, dev, st)
 
 
 def _tile_rows(TK: int, E: int, lora: bool) -> int:
@@ -820,19 +838,31 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
     M = TK + rows_sh
     mt = _tile_rows(TK, E, lora_ex is not None or lora_sh is not None)
     maxt = L.load().smel_dispatch_max_tiles(TK, E, rows_sh, mt)
-    i32 = lambda *s: torch.empty(*s, dtype=torch.int32, device=dev)
-    counts, offsets, order, inv = i32(E), i32(E + 1), i32(max(TK, 1)), i32(max(TK, 1))
-    tiles, tiles_g, ntiles, err = i32(maxt * 4), i32(maxt * 4), i32(1), i32(1)
     # the gate_up forward's merged tile list: an int4 expert's last tile of <= 32 rows joins its full tile
     fz = ex.frozen
     merge = mt == M_TILE and _MERGE_SHORT and isinstance(fz, Int4Experts) and H % 64 == 0 and fz.fast_dq("gu")
-    tiles_m, ntiles_m = (i32(maxt * 4), i32(1)) if merge else (None, None)
-    dws = counted_ws if counted_ws is not None else i32(max(1, L.load().smel_dispatch_ws_size(TK, E)))
     if prep is None:   # LoRA layouts on a side stream, overlapping the dispatch
         fork = _Fork(dev, 2)
         with fork:
-            bufs = _prep_lora(ex, lora_ex, lora_sh, shared is not None, H, dev)
+            bufs = _prep_lora(ex, lora_ex, lora_sh, shared is not None, H, dev, fork.st)
         prep = (fork, bufs)
+    fork, (lb_ex, lb_sh) = prep
+    any_lora = lb_ex is not None or lb_sh is not None
+    planes = (lb_ex or lb_sh).planes if any_lora else 1
+    I = _expert_I(ex)
+    # what the backward reads again in one allocation, the rest (given back when this returns) in another
+    keep, tmp = L.Carve(), L.Carve()
+    counts, offsets, order, inv = keep.take(4 * E), keep.take(4 * (E + 1)), keep.take(4 * TK), keep.take(4 * TK)
+    tiles, tiles_g, ntiles, err = keep.take(16 * maxt), keep.take(16 * maxt), keep.take(4), keep.take(4)
+    ext_gu = ext_pre if ext_pre is not None else (keep.take(2 * M * EXT * planes) if any_lora else None)
+    ext_dn = keep.take(2 * M * EXT) if any_lora else None
+    tiles_m, ntiles_m = (tmp.take(16 * maxt), tmp.take(4)) if merge else (None, None)
+    dws = counted_ws if counted_ws is not None else tmp.take(4 * max(1, L.load().smel_dispatch_ws_size(TK, E)))
+    parts = int(L.load().smel_gmm_fwd_nblocks(2 * I, 1))
+    xpart = tmp.take(4 * M * parts * EXT) if any_lora and _FWD_LORA_ROWS else None
+    Y = tmp.take(2 * M * H)
+    keep.alloc(dev)
+    tmp.alloc(dev)
     gk_groups = ex.gkind(shared is not None, dev)
     L.call("smel_dispatch_counted" if counted_ws is not None else "smel_dispatch", L.ptr(topi_ids), int(ids_i64), T, K,
            E, rows_sh, mt, L.ptr(gk_groups), L.ptr(counts), L.ptr(offsets), L.ptr(order), L.ptr(inv), L.ptr(tiles),
@@ -842,24 +872,18 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
     sel_gu = sel_dn = None
     if ex.sel_ids is not None and len(ex._slot):
         sel_gu, sel_dn = ex.packed_sel()
-    I = _expert_I(ex)
     sh_gu = sh_dn = sgate = sh_gu_t = sh_dn_t = None
     if shared is not None:
         sh_gu, sh_dn, sgate, sh_gu_t, sh_dn_t = shared
-    fork, (lb_ex, lb_sh) = prep
     fork.join()
-    any_lora = lb_ex is not None or lb_sh is not None
-    planes = (lb_ex or lb_sh).planes if any_lora else 1
     g = lambda b, n: getattr(b, n) if b is not None else None
     bf = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device=dev)
     tl = (tiles, ntiles, maxt, gk)
-    ext_gu = ext_dn = None
     if any_lora and ext_pre is not None:   # the shared rows are done: the selected experts' rows only
-        ext_gu = ext_pre
         if lb_ex is not None:
-            _lora_ext(tl, x, H, T, 1, order, TK, K, lb_ex, None, "a_gu", H, planes, M, dev, st, ext=ext_gu)
+            _lora_ext(tl, x, H, T, 1, order, TK, K, lb_ex, None, "a_gu", H, planes, ext_gu, st)
     elif any_lora:
-        ext_gu = _lora_ext(tl, x, H, T, 1, order, TK, K, lb_ex, lb_sh, "a_gu", H, planes, M, dev, st)
+        _lora_ext(tl, x, H, T, 1, order, TK, K, lb_ex, lb_sh, "a_gu", H, planes, ext_gu, st)
     actb = bf(M, I)
     hsave = bf(M, 2 * I) if need_grad else None
     # the gate_up forward takes the merged list (tile t on XCD t % 8, the merged tiles first) or else the tiles in
@@ -871,10 +895,7 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
     # the down LoRA's rows come from the gate_up epilogue (per-column-block partials of h A_dn^T), summed and stored
     # by the down GEMM: no separate projection launch
     lr = None
-    if any_lora and _FWD_LORA_ROWS:
-        parts = int(L.load().smel_gmm_fwd_nblocks(2 * I, 1))
-        xpart = torch.empty(M, parts, EXT, dtype=torch.float32, device=dev)
-        ext_dn = bf(M, EXT)
+    if xpart is not None:
         lr = L.FwdLoraRows(L.ptr(g(lb_ex, "a_dn")), L.ptr(g(lb_sh, "a_dn")), lb_ex.scale if lb_ex is not None else 0.0,
                            lb_sh.scale if lb_sh is not None else 0.0, L.ptr(xpart), parts, L.ptr(ext_dn))
     L.call("smel_gmm_fwd_lr", ctypes.byref(w_gu), L.ptr(gk), L.ptr(tiles_m if merge else tiles_g),
@@ -882,8 +903,7 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
            L.ptr(order), TK, K, L.ptr(ext_gu), 1, _ACT[ex.act], L.ptr(actb), I, L.ptr(hsave),
            ctypes.byref(lr) if lr is not None else None, st, tag="gemm_gu_fwd")
     if any_lora and lr is None:   # the down LoRA's rows as a projection launch of the gate_up output
-        ext_dn = _lora_ext(tl, actb, I, M, 0, order, TK, K, lb_ex, lb_sh, "a_dn", I, 1, M, dev, st)
-    Y = bf(M, H)
+        _lora_ext(tl, actb, I, M, 0, order, TK, K, lb_ex, lb_sh, "a_dn", I, 1, ext_dn, st)
     w_dn = _wset(ex, "dn", sel_dn, sh_dn, g(lb_ex, "fwd_dn"), g(lb_sh, "fwd_dn"))
     w_dn.flags |= short
     # the down forward on the same merged list when its bank is in the fast form too (and I a multiple of 64)
@@ -930,47 +950,46 @@ def _backward_pipeline(c: _Ctx, dout: torch.Tensor, router=None, shared_split=No
     sh_gu, sh_dn = c.shared_w if c.shared_w is not None else (None, None)
     order, tiles, ntiles, gk = t["order"], t["tiles"], t["ntiles"], t["gk"]
     tl = (tiles, ntiles, maxt, gk)
-    # (1) LoRA down-projection of dout for the down backward: DB = s dout B_d (not yet scaled by the row weight)
-    ext_db = None
-    if any_lora:
-        ext_db = _lora_ext(tl, dout, H, T, 1, order, TK, K, lb_ex, lb_sh, "bt_dn", H, 1, M, dev, st)
-    # (2) down backward + SiLU-gate backward + d(row weight) partials
     nblk = L.load().smel_gmm_bwd_nblocks(I)
-    dh = bf(M, 2 * I)
-    dwp = torch.empty(M, nblk, dtype=torch.float32, device=dev)
+    rows_lr = any_lora and _BWD_LORA_ROWS   # the gate_up LoRA's rows from the down backward's epilogue
+    tmp = L.Carve()   # every scratch buffer of the backward
+    ext_db, ext_dxa = (tmp.take(2 * M * EXT), tmp.take(2 * M * EXT * planes)) if any_lora else (None, None)
+    dh, dxs, dwp = tmp.take(4 * M * I), tmp.take(2 * M * H), tmp.take(4 * M * nblk)
+    part = tmp.take(4 * M * nblk * planes * EXT) if rows_lr else None
+    dl, dxr = (tmp.take(2 * T * router[2].R), tmp.take(2 * T * H)) if router is not None else (None, None)
+    tmp.alloc(dev)
+    # (1) LoRA down-projection of dout for the down backward: DB = s dout B_d (not yet scaled by the row weight)
+    if any_lora:
+        _lora_ext(tl, dout, H, T, 1, order, TK, K, lb_ex, lb_sh, "bt_dn", H, 1, ext_db, st)
+    # (2) down backward + SiLU-gate backward + d(row weight) partials
     w_dn = _wset(ex, "dn", t["sel_dn"], sh_dn, g(lb_ex, "at_dn"), g(lb_sh, "at_dn"), t=True)
     w_dn.flags |= c.short
     # with the LoRA rows from this GEMM's epilogue: DXA = s [dg B_g, du B_u] as per-column-block partials
-    lrows = _bwd_lora_rows(lb_ex, lb_sh, nblk, M, planes, dev) if any_lora and _BWD_LORA_ROWS else None
-    lr = ctypes.byref(lrows[0]) if lrows is not None else None
+    lrows = _bwd_lora_rows(lb_ex, lb_sh, nblk, planes, part) if rows_lr else None
+    lr = ctypes.byref(lrows) if lrows is not None else None
     L.call("smel_gmm_bwd_lr", ctypes.byref(w_dn), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(dout), H, T, 1,
            L.ptr(order), TK, K, L.ptr(ext_db), 1, _ACT[ex.act], L.ptr(t["hsave"]), L.ptr(t["topv"]), L.ptr(t["sgate"]),
            L.ptr(dh), 2 * I, L.ptr(dwp), lr, st, tag="gemm_dn_bwd")
     # (3) LoRA B^T projection of dh for the gate_up backward: DXA = s [dg B_g, du B_u] (without the partials)
-    ext_dxa = None
     if any_lora and _BWD_ONE_SIDE and lrows is None:
-        ext_dxa = _lora_ext(tl, dh, 2 * I, M, 0, order, TK, K, lb_ex, lb_sh, "bt_gu", 2 * I, planes, M, dev, st)
+        _lora_ext(tl, dh, 2 * I, M, 0, order, TK, K, lb_ex, lb_sh, "bt_gu", 2 * I, planes, ext_dxa, st)
     # (5, side stream 0) router backward (fused layer) or d topv (routed_experts): needs only dwp, so it overlaps
     # steps (3) and (4)
-    dxr = None
     dtopv = None
     side_r = _Fork(dev, 0)
     if router is not None:
         probs, topi32, wr = router
-        Epad = wr.R
-        dl = bf(T, Epad)
-        dxr = bf(T, H)
-        with side_r:
+        with side_r as sst:
             dwp_sh, nblk_sh = (shared_split[0], shared_split[1]) if shared_split is not None else (None, 0)
             L.call("smel_route_bwd", L.ptr(dwp), nblk, L.ptr(t["inv"]), L.ptr(probs), L.ptr(topi32),
-                   L.ptr(t["sgate"]), L.ptr(dwp_sh), nblk_sh, T, K, E, TK, L.ptr(dl), Epad, None, None, L.stream())
-            _router_dx(dl, wr, T, dxr)
+                   L.ptr(t["sgate"]), L.ptr(dwp_sh), nblk_sh, T, K, E, TK, L.ptr(dl), wr.R, None, None, sst)
+            _router_dx(dl, wr, T, dev, sst, dxr)
     else:
         dtopv = torch.empty(T, K, dtype=torch.float32, device=dev)
-        with side_r:
-            L.call("smel_dtopv", L.ptr(dwp), nblk, L.ptr(t["inv"]), TK, L.ptr(dtopv), L.stream())
+        with side_r as sst:
+            L.call("smel_dtopv", L.ptr(dwp), nblk, L.ptr(t["inv"]), TK, L.ptr(dtopv), sst)
     if any_lora and not _BWD_ONE_SIDE and lrows is None:
-        ext_dxa = _lora_ext(tl, dh, 2 * I, M, 0, order, TK, K, lb_ex, lb_sh, "bt_gu", 2 * I, planes, M, dev, st)
+        _lora_ext(tl, dh, 2 * I, M, 0, order, TK, K, lb_ex, lb_sh, "bt_gu", 2 * I, planes, ext_dxa, st)
     # (6, side stream 1, or after the router backward on stream 0) LoRA factor gradients: one launch for the four
     # products, written into parameter-shaped fp32 tensors; every operand is ready here, so it overlaps the gate_up
     # backward
@@ -981,35 +1000,30 @@ def _backward_pipeline(c: _Ctx, dout: torch.Tensor, router=None, shared_split=No
         groups = _lora_groups(ex, lb_sh is not None, n_sel, dev)
         sets = ((c.lora_ex if lb_ex is not None else None), (c.lora_sh if lb_sh is not None else None))
         gx, gs = (_alloc_lora_grads(m, dev) for m in sets)
-        if lrows is not None:
-            ext_dxa = torch.empty(M, EXT * planes, dtype=torch.bfloat16, device=dev)   # filled on the side stream
-        jobs, nj = _wgrad_jobs(H, I, (gx, gs), sets, (ext_dxa, t["x"], T, 1, 0), (t["ext_gu"], dh, M, 0, 0),
-                               (ext_db, t["act"], M, 0, 1), (t["ext_dn"], dout, T, 1, 1), planes)
+        jobs, nj = _wgrad_jobs(H, I, (gx, gs), sets, (ext_dxa, t["x"], H, T, 1, 0), (t["ext_gu"], dh, 2 * I, M, 0, 0),
+                               (ext_db, t["act"], I, M, 0, 1), (t["ext_dn"], dout, H, T, 1, 1), planes)
         # rows of all LoRA groups: a token routes at most min(K, n_sel) slots to selected experts, + the shared rows
         max_rows = (min(K, n_sel) * T if lb_ex is not None else 0) + (T if lb_sh is not None else 0)
         ws = _wgrad_ws(jobs, nj, groups.numel(), max_rows, dev)
         side_w = side_r if _BWD_ONE_SIDE else _Fork(dev, 1)
-        with side_w:
+        with side_w as sst:
             if lrows is not None:
-                L.call("smel_lora_rows_sum", L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(gk), int(lb_ex is not None),
-                       int(lb_sh is not None), L.ptr(lrows[1]), nblk, planes, L.ptr(ext_dxa), L.stream(),
-                       tag="smel_lora_rows")
+                _lora_rows_sum(tl, lrows, lb_ex, lb_sh, ext_dxa, sst)
             L.call("smel_lora_wgrad", jobs, nj, L.ptr(groups), groups.numel(), n_sel, L.ptr(t["offsets"]), E, T, TK,
-                   K, L.ptr(order), L.ptr(t["topv"]), L.ptr(t["sgate"]), max_rows, L.ptr(ws), ws.numel(), L.stream(),
+                   K, L.ptr(order), L.ptr(t["topv"]), L.ptr(t["sgate"]), max_rows, L.ptr(ws), ws.numel(), sst,
                    tag="lora_wgrad")
         if gx is not None:
             grads["ex"] = gx
         if gs is not None:
             grads["sh"] = gs
     # (4) gate_up backward: per-slot dx rows
-    dxs = bf(M, H)
     w_gu = _wset(ex, "gu", t["sel_gu"], sh_gu, g(lb_ex, "at_gu"), g(lb_sh, "at_gu"), t=True, planes=planes)
     w_gu.flags |= L.WSET_XCD_CHUNK | c.short
     L.call("smel_gmm_bwd_lr", ctypes.byref(w_gu), L.ptr(gk), L.ptr(t["tiles_g"]), L.ptr(ntiles), maxt, L.ptr(dh),
            2 * I, M, 0, L.ptr(order), TK, K, None if lrows is not None else L.ptr(ext_dxa), 0, _ACT[ex.act], None, None,
            None, L.ptr(dxs), H, None, lr, st, tag="gemm_gu_bwd")
     side_r.join()
-    dx = bf(T, H)
+    dx = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
     dxsh = shared_split[2] if shared_split is not None else None
     L.call("smel_dx_reduce", L.ptr(dxs), L.ptr(dxr), L.ptr(t["inv"]), int(t["sgate"] is not None), L.ptr(dxsh), T,
            K, H, L.ptr(dx), st)
@@ -1022,7 +1036,7 @@ _LORA_NAMES = ("A_gate", "B_gate", "A_up", "B_up", "A_down", "B_down")
 
 
 def _lora_leaves(lora):
-    return [getattr(lora, n) for n in _LORA_NAMES] if lora is not None else []
+    return [_factor(lora, n) for n in _LORA_NAMES] if lora is not None else []
 
 
 def _shape_grads(grads: dict, tag: str, lora, squeeze: bool = False):
@@ -1039,8 +1053,8 @@ def _alloc_lora_grads(lora, device):
     weight-gradient kernel), or None without the set."""
     if lora is None:
         return None
-    return {n: torch.empty(getattr(lora, n).shape, dtype=torch.float32, device=device)
-            for n in _LORA_NAMES if getattr(lora, n).requires_grad}
+    ps = [(n, _factor(lora, n)) for n in _LORA_NAMES]
+    return {n: torch.empty(p.shape, dtype=torch.float32, device=device) for n, p in ps if p.requires_grad}
 
 
 def _wgrad_ws(jobs, n_jobs: int, n_lora: int, max_rows: int, device) -> torch.Tensor:
@@ -1049,45 +1063,60 @@ def _wgrad_ws(jobs, n_jobs: int, n_lora: int, max_rows: int, device) -> torch.Te
     return torch.empty(max(n, 1), dtype=torch.float32, device=device)
 
 
-def _wgrad_jobs(H, I, grads, sets, j_agu, j_bgu, j_adn, j_bdn, planes: int = 1):
-    """The smel_wg_job list of a backward: dA and dB of gate/up, dA and dB of down. Each j_* = (L rows, Rm, Rm rows,
-    r_gather, use_w). Destinations: class 0 = the selected experts' ExpertsLoRA (slot = its index), class 1 = the
-    shared MLPLoRA. With one gate_up plane a gate/up product is one job whose result splits in two halves (ranks
-    0..15 / 16..31; the B factors' columns 0..I-1 / I..2I-1); with two planes it is one job per plane (L = that
-    plane's 32 columns of the 64-wide ext rows; the up B job reads the up half of dh only). Returns (jobs, count)."""
-    gate_up = []   # (L byte offset, ldl, Rm byte offset, Q, [(half, param, p0, q0, nq, col_major)])
+@functools.lru_cache(maxsize=64)
+def _wgrad_plan(H: int, I: int, planes: int, present: tuple):
+    """The parts of a backward's smel_wg_job list that only shapes decide: (job bytes, per job (source index, L byte
+    offset, Rm byte offset), [(pointer word, class, parameter name)]). ``present`` = per class (rank, slots, names of
+    the parameters with a gradient). With one gate_up plane a gate/up product is one job whose result splits in two
+    halves (ranks 0..15 / 16..31; the B factors' columns 0..I-1 / I..2I-1); with two planes it is one job per plane (L =
+    that plane's 32 columns of the 64-wide ext rows; the up B job reads the up half of dh only)."""
+    gate_up = []   # (source, L byte offset, ldl, Rm byte offset, Q, [(half, param, p0, q0, nq, col_major)])
     if planes == 1:
-        gate_up.append((j_agu, 0, EXT, 0, H, [(0, "A_gate", 0, 0, H, False), (1, "A_up", EXT // 2, 0, H, False)]))
-        gate_up.append((j_bgu, 0, EXT, 0, 2 * I,
-                        [(0, "B_gate", 0, 0, I, True), (1, "B_up", EXT // 2, I, I, True)]))
+        gate_up.append((0, 0, EXT, 0, H, [(0, "A_gate", 0, 0, H, False), (1, "A_up", EXT // 2, 0, H, False)]))
+        gate_up.append((1, 0, EXT, 0, 2 * I, [(0, "B_gate", 0, 0, I, True), (1, "B_up", EXT // 2, I, I, True)]))
     else:
         w = 2 * EXT
-        gate_up.append((j_agu, 0, w, 0, H, [(0, "A_gate", 0, 0, H, False)]))
-        gate_up.append((j_agu, 2 * EXT, w, 0, H, [(0, "A_up", 0, 0, H, False)]))
-        gate_up.append((j_bgu, 0, w, 0, I, [(0, "B_gate", 0, 0, I, True)]))
-        gate_up.append((j_bgu, 2 * EXT, w, 2 * I, I, [(0, "B_up", 0, 0, I, True)]))
-    specs = gate_up + [(j_adn, 0, EXT, 0, I, [(0, "A_down", 0, 0, I, False)]),
-                       (j_bdn, 0, EXT, 0, H, [(0, "B_down", 0, 0, H, True)])]
+        gate_up.append((0, 0, w, 0, H, [(0, "A_gate", 0, 0, H, False)]))
+        gate_up.append((0, 2 * EXT, w, 0, H, [(0, "A_up", 0, 0, H, False)]))
+        gate_up.append((1, 0, w, 0, I, [(0, "B_gate", 0, 0, I, True)]))
+        gate_up.append((1, 2 * EXT, w, 2 * I, I, [(0, "B_up", 0, 0, I, True)]))
+    specs = gate_up + [(2, 0, EXT, 0, I, [(0, "A_down", 0, 0, I, False)]), (3, 0, EXT, 0, H, [(0, "B_down", 0, 0, H, True)])]
     jobs = (L.WgJob * len(specs))()
-    for J, ((Lb, Rm, rows, gather, use_w), l_off, ldl, r_off, Q, dests) in zip(jobs, specs):
-        J.L, J.Rm = Lb.data_ptr() + l_off, Rm.data_ptr() + r_off
-        J.ldl, J.ldr, J.r_rows, J.r_gather, J.use_w, J.Q = ldl, Rm.shape[1], rows, gather, use_w, Q
-        for cls in range(2):
-            g, m = grads[cls], sets[cls]
-            if g is None:
-                continue
-            lead = 1 if cls == 0 else 0
+    srcs, dests_at = [], []
+    for i, (J, (src, l_off, ldl, r_off, Q, dests)) in enumerate(zip(jobs, specs)):
+        J.ldl, J.Q = ldl, Q
+        srcs.append((src, l_off, r_off))
+        for cls, (r, slots, names) in enumerate(present):
             for h, name, p0, q0, nq, col_major in dests:
-                t = g.get(name)
-                if t is None:
+                if name not in names:
                     continue
                 d = J.dest[cls][h]
-                d.ptr = L.ptr(t)
-                d.s_idx = t.stride(0) if lead else 0
                 # A factors [.., r, Q] (p rows, q contiguous); B factors [.., Q, r] (q rows, p contiguous)
-                d.s_p, d.s_q = (1, t.stride(lead)) if col_major else (t.stride(lead), 1)
-                d.p0, d.np, d.q0, d.nq = p0, m.r, q0, nq
-    return jobs, len(specs)
+                d.s_idx = r * nq if slots else 0
+                d.s_p, d.s_q = (1, r) if col_major else (nq, 1)
+                d.p0, d.np, d.q0, d.nq = p0, r, q0, nq
+                at = i * ctypes.sizeof(L.WgJob) + L.WgJob.dest.offset + (2 * cls + h) * ctypes.sizeof(L.WgDest)
+                dests_at.append(((at + L.WgDest.ptr.offset) // 8, cls, name))
+    return bytes(jobs), tuple(srcs), tuple(dests_at)
+
+
+def _wgrad_jobs(H, I, grads, sets, j_agu, j_bgu, j_adn, j_bdn, planes: int = 1):
+    """The smel_wg_job list of a backward: dA and dB of gate/up, dA and dB of down. Each j_* = (L rows, Rm, Rm columns,
+    Rm rows, r_gather, use_w). Destinations (contiguous tensors of _alloc_lora_grads): class 0 = the selected experts'
+    ExpertsLoRA (slot = its index), class 1 = the shared MLPLoRA. Returns (jobs, count)."""
+    present = tuple((m.r, cls == 0, frozenset(g)) if g is not None else (0, False, frozenset())
+                    for cls, (g, m) in enumerate(zip(grads, sets)))
+    tmpl, srcs, dests = _wgrad_plan(H, I, planes, present)
+    jobs = (L.WgJob * len(srcs)).from_buffer_copy(tmpl)
+    ops = [(Lb.data_ptr(), Rm.data_ptr(), cols, rows, gather, use_w)
+           for Lb, Rm, cols, rows, gather, use_w in (j_agu, j_bgu, j_adn, j_bdn)]
+    for J, (src, l_off, r_off) in zip(jobs, srcs):
+        lp, rp, J.ldr, J.r_rows, J.r_gather, J.use_w = ops[src]
+        J.L, J.Rm = lp + l_off, rp + r_off
+    words = (ctypes.c_uint64 * (len(tmpl) // 8)).from_buffer(jobs)
+    for at, cls, name in dests:
+        words[at] = grads[cls][name].data_ptr()
+    return jobs, len(srcs)
 
 
 class _MoELayerFn(torch.autograd.Function):
@@ -1103,24 +1132,30 @@ class _MoELayerFn(torch.autograd.Function):
         has_sh = plan["shared"] is not None
         split = has_sh and plan["split_shared"]
         fuse = has_sh and not split
-        probs = torch.empty(T, E, dtype=torch.float32, device=dev)
-        topv = torch.empty(T, K, dtype=torch.bfloat16, device=dev)
-        topv32 = torch.empty(T, K, dtype=torch.float32, device=dev)   # fp32 of topv: the combine weight
-        topi = torch.empty(T, K, dtype=torch.int64, device=dev)
-        topi32 = torch.empty(T, K, dtype=torch.int32, device=dev)
-        sgate = torch.empty(T, dtype=torch.float32, device=dev) if has_sh else None
+        keep, tmp = L.Carve(), L.Carve()   # read again by the backward, and not
+        # topv32: fp32 of topv, the combine weight
+        topv32, topi32 = keep.take(4 * T * K), keep.take(4 * T * K)
+        sgate = keep.take(4 * T) if has_sh else None
+        if stats is None:
+            probs, topv, topi = keep.take(4 * T * E), tmp.take(2 * T * K), tmp.take(8 * T * K)
+        else:   # the hook's tensors
+            probs = torch.empty(T, E, dtype=torch.float32, device=dev)
+            topv = torch.empty(T, K, dtype=torch.bfloat16, device=dev)
+            topi = torch.empty(T, K, dtype=torch.int64, device=dev)
+        lg = tmp.take(2 * T * L.load().smel_route_ld(E, int(has_sh)))
+        # the router also counts the dispatch's per-block histograms of its picks into the dispatch workspace
+        dws = tmp.take(4 * max(1, L.load().smel_dispatch_ws_size(T * K, E)))
+        keep.alloc(dev)
+        tmp.alloc(dev)
         sgw = plan["shared"][2] if has_sh else None
-        lg = torch.empty(T, L.load().smel_route_ld(E, int(has_sh)), dtype=torch.bfloat16, device=dev)
         # LoRA layouts (and the shared rows' LoRA projection) overlap the router and the dispatch
         side_ext = _FWD_EXT_SIDE and fuse and plan["lora_sh"] is not None
         fork = _Fork(dev, 2, on=True if side_ext else None)
         ext_pre = None
-        with fork:
-            bufs = _prep_lora(plan["ex"], plan["lora_ex"], plan["lora_sh"] if fuse else None, fuse, H, dev)
+        with fork as sst:
+            bufs = _prep_lora(plan["ex"], plan["lora_ex"], plan["lora_sh"] if fuse else None, fuse, H, dev, sst)
             if side_ext and bufs[1] is not None:
-                ext_pre = _shared_lora_ext(x, K, E, bufs, dev)
-        # the router also counts the dispatch's per-block histograms of its picks into the dispatch workspace
-        dws = torch.empty(max(1, L.load().smel_dispatch_ws_size(T * K, E)), dtype=torch.int32, device=dev)
+                ext_pre = _shared_lora_ext(x, K, E, bufs, dev, sst)
         L.call("smel_route_counted", L.ptr(x), L.ptr(plan["gate_w"]), L.ptr(sgw), T, H, E, K, L.ptr(probs),
                L.ptr(topv), L.ptr(topv32), L.ptr(topi), L.ptr(topi32), L.ptr(sgate), L.ptr(lg), L.ptr(dws), L.stream(),
                tag="smel_route")
@@ -1132,7 +1167,7 @@ class _MoELayerFn(torch.autograd.Function):
         if split:
             pgu, pdn, _, Is, pgu_t, pdn_t = plan["shared"]
             lsh = plan["lora_sh"]
-            lb_sh = _LoRABufs(lsh, 1, H, Is, dev, _lora_planes(lsh)) if lsh is not None else None
+            lb_sh = _lora_bufs([(lsh, 1, Is)], H, _lora_planes(lsh), dev, L.stream())[0]
             ysh, sv = _dense_mlp_fwd(x, pgu, pdn, lb_sh, "silu", tag="gemm_shared")
             shared_rows = (sgate, ysh)
             c.split = (sv, pgu_t, pdn_t, lsh, sgate)
@@ -1174,7 +1209,7 @@ class _RoutedFn(torch.autograd.Function):
         tv = topv.detach().float().contiguous()   # fp32 combine weights: the reference's topv.float() (:252)
         need = ctx.needs_input_grad[0] or ctx.needs_input_grad[1] or any(ctx.needs_input_grad[5:])
         out = _forward_pipeline(x, ex, K, tv, topi.contiguous(), topi.dtype == torch.int64, None, lora, None, need, c)
-        _ID_CHECK.record(c.tensors["err"])
+        _ID_CHECK.record(c.tensors["err"].tensor(torch.int32, 1))
         if need:
             ctx.c = c
         ctx.topv_dtype = topv.dtype
@@ -1269,15 +1304,19 @@ def _dense_mlp_fwd(x, w_gu: PackedW, w_dn: PackedW, lb, act_name: str, tag: str 
     planes = lb.planes if lb is not None else 1
     sv = _DenseSaved()
     sv.x, sv.lb, sv.ext_gu, sv.ext_dn = x, lb, None, None
+    keep = L.Carve()
+    sv.actb, sv.hsave = keep.take(2 * T * Is), keep.take(4 * T * Is)
     if lb is not None:
-        sv.ext_gu = _lora_ext(tl, x, H, T, 0, None, 0, 1, None, lb, "a_gu", H, planes, T, dev, st)
-    sv.actb, sv.hsave = bf(T, Is), bf(T, 2 * Is)
+        sv.ext_gu, sv.ext_dn = keep.take(2 * T * EXT * planes), keep.take(2 * T * EXT)
+    keep.alloc(dev)
+    if lb is not None:
+        _lora_ext(tl, x, H, T, 0, None, 0, 1, None, lb, "a_gu", H, planes, sv.ext_gu, st)
     wg = _dense_wset(w_gu, g("fwd_gu"), planes)
     L.call("smel_gmm_fwd", ctypes.byref(wg), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(x), H, T, 0,
            None, 0, 1, L.ptr(sv.ext_gu), 1, _ACT[act_name], L.ptr(sv.actb), Is, L.ptr(sv.hsave), st,
            tag=tag + "_gu_fwd")
     if lb is not None:
-        sv.ext_dn = _lora_ext(tl, sv.actb, Is, T, 0, None, 0, 1, None, lb, "a_dn", Is, 1, T, dev, st)
+        _lora_ext(tl, sv.actb, Is, T, 0, None, 0, 1, None, lb, "a_dn", Is, 1, sv.ext_dn, st)
     y = bf(T, H)
     wd = _dense_wset(w_dn, g("fwd_dn"))
     L.call("smel_gmm_fwd", ctypes.byref(wd), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(sv.actb), Is, T, 0,
@@ -1301,20 +1340,24 @@ def _dense_mlp_bwd(sv: _DenseSaved, dy, w_gu_t: PackedW, w_dn_t: PackedW, lora, 
     bf = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device=dev)
     g = lambda n: getattr(lb, n) if lb is not None else None
     planes = lb.planes if lb is not None else 1
-    ext_db = ext_dxa = None
-    if lb is not None:
-        ext_db = _lora_ext(tl, dy, H, T, 0, None, 0, 1, None, lb, "bt_dn", H, 1, T, dev, st)
     nblk = L.load().smel_gmm_bwd_nblocks(Is)
-    dh = bf(T, 2 * Is)
+    rows_lr = lb is not None and _BWD_LORA_ROWS
+    tmp = L.Carve()
+    dh = tmp.take(4 * T * Is)
+    ext_db, ext_dxa = (tmp.take(2 * T * EXT), tmp.take(2 * T * EXT * planes)) if lb is not None else (None, None)
+    part = tmp.take(4 * T * nblk * planes * EXT) if rows_lr else None
+    tmp.alloc(dev)
     dwp = torch.empty(T, nblk, dtype=torch.float32, device=dev)
+    if lb is not None:
+        _lora_ext(tl, dy, H, T, 0, None, 0, 1, None, lb, "bt_dn", H, 1, ext_db, st)
     wd = _dense_wset(w_dn_t, g("at_dn"))
-    lrows = _bwd_lora_rows(None, lb, nblk, T, planes, dev) if lb is not None and _BWD_LORA_ROWS else None
-    lr = ctypes.byref(lrows[0]) if lrows is not None else None
+    lrows = _bwd_lora_rows(None, lb, nblk, planes, part) if rows_lr else None
+    lr = ctypes.byref(lrows) if lrows is not None else None
     L.call("smel_gmm_bwd_lr", ctypes.byref(wd), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(dy), H, T, 0,
            None, 0, 1, L.ptr(ext_db), 1, _ACT[act_name], L.ptr(sv.hsave), None, L.ptr(row_w), L.ptr(dh), 2 * Is,
            L.ptr(dwp), lr, st, tag=tag + "_dn_bwd")
     if lb is not None and lrows is None:
-        ext_dxa = _lora_ext(tl, dh, 2 * Is, T, 0, None, 0, 1, None, lb, "bt_gu", 2 * Is, planes, T, dev, st)
+        _lora_ext(tl, dh, 2 * Is, T, 0, None, 0, 1, None, lb, "bt_gu", 2 * Is, planes, ext_dxa, st)
     dx = bf(T, H)
     wg = _dense_wset(w_gu_t, g("at_gu"), planes)
     L.call("smel_gmm_bwd_lr", ctypes.byref(wg), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(dh), 2 * Is, T,
@@ -1323,15 +1366,14 @@ def _dense_mlp_bwd(sv: _DenseSaved, dy, w_gu_t: PackedW, w_dn_t: PackedW, lora, 
     grads = None
     if lb is not None:
         if lrows is not None:   # the LoRA gradients take the same rows the gate_up backward summed
-            ext_dxa = _lora_rows_sum(tl, lrows[0], None, lb, T, planes, dev, st)
-        zero = torch.zeros(2, dtype=torch.int32, device=dev)     # offsets of zero experts
-        groups = torch.zeros(1, dtype=torch.int32, device=dev)   # group 0 >= E = 0: rows [0, T)
+            _lora_rows_sum(tl, lrows, None, lb, ext_dxa, st)
+        zero = _dense_zeros(T, dev)   # offsets [0, 0] of zero experts; group 0 >= E = 0: rows [0, T)
         gs = _alloc_lora_grads(lora, dev)
         # the down projection's products take the row weight (dh already carries it)
-        jobs, nj = _wgrad_jobs(H, Is, (None, gs), (None, lora), (ext_dxa, x, T, 0, 0), (sv.ext_gu, dh, T, 0, 0),
-                               (ext_db, sv.actb, T, 0, 1), (sv.ext_dn, dy, T, 0, 1), planes)
+        jobs, nj = _wgrad_jobs(H, Is, (None, gs), (None, lora), (ext_dxa, x, H, T, 0, 0), (sv.ext_gu, dh, 2 * Is, T, 0, 0),
+                               (ext_db, sv.actb, Is, T, 0, 1), (sv.ext_dn, dy, H, T, 0, 1), planes)
         ws = _wgrad_ws(jobs, nj, 1, T, dev)
-        L.call("smel_lora_wgrad", jobs, nj, L.ptr(groups), 1, 0, L.ptr(zero), 0, T, 0, 1, None, None, L.ptr(row_w),
+        L.call("smel_lora_wgrad", jobs, nj, L.ptr(zero), 1, 0, L.ptr(zero), 0, T, 0, 1, None, None, L.ptr(row_w),
                T, L.ptr(ws), ws.numel(), st, tag="lora_wgrad")
         grads = gs
     return dx, grads, dwp, nblk
@@ -1344,7 +1386,7 @@ class _MLPFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w_gu2, w_dn2, lora, act_name, *leaves):
-        lb = _LoRABufs(lora, 1, x.shape[1], w_dn2[0].C, x.device, _lora_planes(lora)) if lora is not None else None
+        lb = _lora_bufs([(lora, 1, w_dn2[0].C)], x.shape[1], _lora_planes(lora), x.device, L.stream())[0]
         y, sv = _dense_mlp_fwd(x, w_gu2[0], w_dn2[0], lb, act_name)
         ctx.sv, ctx.w, ctx.lora, ctx.act_name = sv, (w_gu2[1], w_dn2[1]), lora, act_name
         return y
