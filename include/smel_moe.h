@@ -77,6 +77,10 @@ typedef struct smel_wset {
  * 32): kernels with a quarter of the LDS and registers per block run more blocks per CU. Excludes the merged forms.
  * Rows of a tile past 32 are not computed. */
 #define SMEL_WSET_TILE32 32
+/* SMEL_WSET_COL_CHUNK (smel_gmm_fwd, smel_gmm_bwd, any tile list): the (column block, tile) pairs in column-block order,
+ * a contiguous run of them per XCD: each XCD reads an eighth of the weights and all rows (few rows against the weight's:
+ * a dense MLP on a short sequence), instead of all weights and an eighth of the rows. Excludes SMEL_WSET_XCD_CHUNK. */
+#define SMEL_WSET_COL_CHUNK 64
 
 const char* smel_last_error(void);
 int smel_abi_version(void);

@@ -211,6 +211,17 @@ SMEL_DEV bool xcd_tile_chunk(int n_tiles, int nblk, int& tile, int& nb) {
   nb = j % nblk;
   return true;
 }
+// xcd_col_chunk: the (column block, tile) pairs in column-block order, XCD x a contiguous run of them: an XCD reads an
+// eighth of the weights and every tile's A rows, where the other two mappings read an eighth of the rows and all weights.
+SMEL_DEV bool xcd_col_chunk(int n_tiles, int nblk, int& tile, int& nb) {
+  const int b = blockIdx.x;
+  const int chunk = (n_tiles * nblk + NXCD - 1) / NXCD;
+  const int j = b / NXCD, item = b % NXCD * chunk + j;
+  if (j >= chunk || item >= n_tiles * nblk) return false;
+  nb = item / n_tiles;
+  tile = item % n_tiles;
+  return true;
+}
 SMEL_DEV bool xcd_tile(int n_tiles, int nblk, int& tile, int& nb) {
   const int b = blockIdx.x;
   const int x = b % NXCD, j = b / NXCD;
@@ -219,6 +230,13 @@ SMEL_DEV bool xcd_tile(int n_tiles, int nblk, int& tile, int& nb) {
   tile = t;
   nb = j % nblk;
   return true;
+}
+
+// The mapping a weight set's flags ask for.
+SMEL_DEV bool xcd_map(int flags, int n_tiles, int nblk, int& tile, int& nb) {
+  if (flags & SMEL_WSET_COL_CHUNK) return xcd_col_chunk(n_tiles, nblk, tile, nb);
+  if (flags & SMEL_WSET_XCD_CHUNK) return xcd_tile_chunk(n_tiles, nblk, tile, nb);
+  return xcd_tile(n_tiles, nblk, tile, nb);
 }
 
 // ------------------------------------------------------------------------------------------------ row mapping

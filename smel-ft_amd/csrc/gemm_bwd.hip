@@ -677,9 +677,7 @@ SMEL_DEV void run_tile_ns(const BwdArgs& a, int kind, int idx, int row0, int nro
 template <int EPI, bool SZ2, int MT_>
 SMEL_DEV void gmm_bwd_body(const BwdArgs& a, uint8_t* smem) {
   int tile, nb;
-  if (!((a.w.flags & SMEL_WSET_XCD_CHUNK) ? xcd_tile_chunk(a.n_tiles[0], a.nblk, tile, nb)
-                                          : xcd_tile(a.n_tiles[0], a.nblk, tile, nb)))
-    return;
+  if (!xcd_map(a.w.flags, a.n_tiles[0], a.nblk, tile, nb)) return;
   const int4 t = a.tiles[tile];
   const int gk = a.gkind ? a.gkind[t.x] : t.w;   // the tile list may carry the group kind itself
   const int kind = gk >> 16, idx = gk & 0xffff;
@@ -745,6 +743,8 @@ extern "C" int smel_gmm_bwd_lr(const smel_wset* w, const int32_t* gkind, const i
   SMEL_REQUIRE(epilogue == 0 || (epilogue == 1 && hsave && dwp && (topv || TK == 0)), SMEL_EINVAL,
                "gmm_bwd: epilogue %d needs hsave, dwp and topv", epilogue);
   SMEL_REQUIRE(!a_gather || order || TK == 0, SMEL_EINVAL, "gmm_bwd: gather needs order");
+  SMEL_REQUIRE(!(w->flags & SMEL_WSET_COL_CHUNK) || !(w->flags & SMEL_WSET_XCD_CHUNK), SMEL_EINVAL,
+               "gmm_bwd: SMEL_WSET_COL_CHUNK excludes SMEL_WSET_XCD_CHUNK");
   SMEL_REQUIRE(!(w->flags & SMEL_WSET_EXT2) || epilogue == 0, SMEL_EINVAL,
                "gmm_bwd: a two-plane LoRA extension belongs to the gate_up backward (epilogue 0)");
   SMEL_REQUIRE(act == 0 || act == 1, SMEL_EINVAL, "gmm_bwd: act %d", act);

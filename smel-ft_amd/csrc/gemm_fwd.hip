@@ -627,8 +627,7 @@ SMEL_DEV void gmm_fwd_body32(const FwdArgs& a, uint16_t* S0, uint16_t* S1, uint1
                              uint16_t* X) {
   int tile, nb;
   const int n_t = a.n_tiles[0];
-  if (!((a.w.flags & SMEL_WSET_XCD_CHUNK) ? xcd_tile_chunk(n_t, a.nblk, tile, nb) : xcd_tile(n_t, a.nblk, tile, nb)))
-    return;
+  if (!xcd_map(a.w.flags, n_t, a.nblk, tile, nb)) return;
   const int4 t = a.tiles[tile];
   const int gk = a.gkind ? a.gkind[t.x] : t.w;
   const int kind = gk >> 16, idx = gk & 0xffff;
@@ -650,8 +649,7 @@ SMEL_DEV void gmm_fwd_body(const FwdArgs& a, uint16_t* S0, uint16_t* S1, uint16_
   constexpr int MT = 128, MT_MERGED = Cfg<128>::MT_MERGED;
   int tile, nb;
   const int n_t = a.n_tiles[0];
-  if (!((a.w.flags & SMEL_WSET_XCD_CHUNK) ? xcd_tile_chunk(n_t, a.nblk, tile, nb) : xcd_tile(n_t, a.nblk, tile, nb)))
-    return;
+  if (!xcd_map(a.w.flags, n_t, a.nblk, tile, nb)) return;
   const int4 t = a.tiles[tile];
   const int gk = a.gkind ? a.gkind[t.x] : t.w;   // the tile list may carry the group kind itself
   const int kind = gk >> 16, idx = gk & 0xffff;
@@ -747,6 +745,8 @@ extern "C" int smel_gmm_fwd_lr(const smel_wset* w, const int32_t* gkind, const i
                SMEL_EINVAL,
                "gmm_fwd: a merged tile list (SMEL_WSET_MERGED_LIST) on an int4 bank needs its fast dequant form and K "
                "a multiple of 64");
+  SMEL_REQUIRE(!(w->flags & SMEL_WSET_COL_CHUNK) || !(w->flags & (SMEL_WSET_XCD_CHUNK | SMEL_WSET_MERGE_SHORT)),
+               SMEL_EINVAL, "gmm_fwd: SMEL_WSET_COL_CHUNK excludes SMEL_WSET_XCD_CHUNK and SMEL_WSET_MERGE_SHORT");
   SMEL_REQUIRE(!(w->flags & SMEL_WSET_TILE32) || !(w->flags & (SMEL_WSET_MERGED_LIST | SMEL_WSET_MERGE_SHORT)),
                SMEL_EINVAL, "gmm_fwd: SMEL_WSET_TILE32 excludes merged tiles");
   SMEL_REQUIRE(!a_gather || order || TK == 0, SMEL_EINVAL, "gmm_fwd: gather needs order");

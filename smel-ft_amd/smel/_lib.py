@@ -23,6 +23,7 @@ WSET_XCD_CHUNK = 4   # smel_wset.flags: group-ordered tile list, a contiguous ch
 WSET_MERGE_SHORT = 8 # smel_wset.flags: gate_up forward, a full int4 tile also takes the group's short last tile
 WSET_MERGED_LIST = 16 # smel_wset.flags: gate_up forward on smel_dispatch's merged tile list (int4 tiles up to 160 rows)
 WSET_TILE32 = 32     # smel_wset.flags: a tile list of at most 32 rows a tile
+WSET_COL_CHUNK = 64  # smel_wset.flags: column blocks, not tiles, are spread over the XCDs
 ABI_VERSION = 24
 
 vp, i64, i32, f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_float

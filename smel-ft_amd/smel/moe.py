@@ -321,14 +321,15 @@ def _bf16(t: torch.Tensor) -> torch.Tensor:
 _dense_tiles_cache = {}
 
 
-def _dense_tiles(T: int, device):
-    """Tile list of one dense group of T rows (group 0), for the router-backward GEMM."""
-    key = (T, str(device))
+def _dense_tiles(T: int, device, rows: int = M_TILE):
+    """Tile list of one dense group of T rows (group 0) in tiles of ``rows`` rows, for the router-backward GEMM and the
+    dense MLP."""
+    key = (T, str(device), rows)
     if key not in _dense_tiles_cache:
-        n = (T + M_TILE - 1) // M_TILE
+        n = (T + rows - 1) // rows
         t = torch.zeros(max(n, 1), 4, dtype=torch.int32)
         for i in range(n):
-            t[i, 0], t[i, 1], t[i, 2], t[i, 3] = 0, i * M_TILE, min(T, (i + 1) * M_TILE), L.KIND_SHARED << 16
+            t[i, 0], t[i, 1], t[i, 2], t[i, 3] = 0, i * rows, min(T, (i + 1) * rows), L.KIND_SHARED << 16
         _dense_tiles_cache[key] = (t.reshape(-1).to(device), torch.tensor([n], dtype=torch.int32, device=device),
                                    n, torch.tensor([L.KIND_SHARED << 16], dtype=torch.int32, device=device),
                                    torch.zeros(2, dtype=torch.int32).to(device))
@@ -338,7 +339,7 @@ def _dense_tiles(T: int, device):
 def _dense_zeros(T: int, device) -> torch.Tensor:
     """Two zeros kept with the tile list of the same rows."""
     _dense_tiles(T, device)
-    return _dense_tiles_cache[(T, str(device))][4]
+    return _dense_tiles_cache[(T, str(device), M_TILE)][4]
 
 
 def _router_ext_weight(gate_w: torch.Tensor, sg_w: torch.Tensor | None, store: dict | None = None) -> PackedW:
@@ -1290,6 +1291,41 @@ class _DenseSaved:
     __slots__ = ("x", "actb", "hsave", "ext_gu", "ext_dn", "lb")
 
 
+# (rows of a tile, a lone block's time against the 128-row tile's forward and backward, blocks that share a CU)
+_DENSE_TILES = ((128, 1.0, 1.0, 2), (96, 0.86, 0.86, 2), (64, 0.73, 0.73, 2), (M_SHORT, 0.75, 0.64, 4))
+
+
+def _dense_rows(T: int, nblk: int, fwd: bool) -> int:
+    """Rows of a dense group's tiles for a GEMM of ``nblk`` column blocks over T rows: the height with the shortest
+    launch. A block's time is set by the bytes its CU takes in per k-step (the weights' and the rows'), so a lone block of
+    a lower tile is faster, until its blocks need another turn of the 256 CUs: blocks sharing a CU take 1.6 times a lone
+    block's time in pairs (up to 2.1 times for four of the 32-row kernels'). Measured (hidden 2816, intermediate 2112,
+    rank 16; us by rows of a tile, 128 / 96 / 64 / 32): down backward at 1531 rows 76 / 66 / 55 / 52, gate_up forward
+    57 / 64 / 59 / 77, down forward 39 / 34 / 43 / 49; gate_up forward at 4096 rows 133 / 121 / 147 / 171, at 517 52 / 45
+    / 39 / 38."""
+    def cost(rows, tf, tb, share):
+        n = -(-(-(-T // rows) * nblk) // 256)   # blocks of a CU
+        full, rest = divmod(n, share)
+        f = (1.6, 2.1)[share // 4] * full + (0.0, 1.0, 1.6, 1.9)[rest]
+        return (tf if fwd else tb) * f
+    return min(_DENSE_TILES, key=lambda t: cost(*t))[0]
+
+
+def _dense_list(T: int, N: int, fwd: bool, epilogue: int, w: L.WSet, dev):
+    """The tile list of a dense group's GEMM with N output columns (weight rows forward, weight columns backward), and
+    its flags in ``w``. Up to twice as many rows as columns the column blocks are spread over the XCDs instead of the
+    tiles (SMEL_WSET_COL_CHUNK): past L2 go then the weights once and the rows eight times, not the other way round
+    (gate_up forward of 1531 rows of 2816, 4224 columns: 80 -> 57 us; at 4096 rows on 96-row tiles 139 -> 121)."""
+    lib = L.load()
+    nblk = int(lib.smel_gmm_fwd_nblocks(N, epilogue) if fwd else lib.smel_gmm_bwd_nblocks(N))
+    rows = _dense_rows(T, nblk, fwd)
+    if rows == M_SHORT:
+        w.flags |= L.WSET_TILE32
+    if T <= 2 * N:
+        w.flags |= L.WSET_COL_CHUNK
+    return _dense_tiles(T, dev, rows)
+
+
 def _dense_mlp_fwd(x, w_gu: PackedW, w_dn: PackedW, lb, act_name: str, tag: str = "gemm_mlp"):
     """Gated MLP y = down(act(gate(x)) * up(x)) (+ LoRA on all three as the K-extension) as one dense group of the
     grouped GEMMs (rows = tokens). Returns (y [T, H] bf16, _DenseSaved)."""
@@ -1312,6 +1348,7 @@ def _dense_mlp_fwd(x, w_gu: PackedW, w_dn: PackedW, lb, act_name: str, tag: str 
     if lb is not None:
         _lora_ext(tl, x, H, T, 0, None, 0, 1, None, lb, "a_gu", H, planes, sv.ext_gu, st)
     wg = _dense_wset(w_gu, g("fwd_gu"), planes)
+    tiles, ntiles, maxt, gk = _dense_list(T, 2 * Is, True, 1, wg, dev)
     L.call("smel_gmm_fwd", ctypes.byref(wg), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(x), H, T, 0,
            None, 0, 1, L.ptr(sv.ext_gu), 1, _ACT[act_name], L.ptr(sv.actb), Is, L.ptr(sv.hsave), st,
            tag=tag + "_gu_fwd")
@@ -1319,6 +1356,7 @@ def _dense_mlp_fwd(x, w_gu: PackedW, w_dn: PackedW, lb, act_name: str, tag: str 
         _lora_ext(tl, sv.actb, Is, T, 0, None, 0, 1, None, lb, "a_dn", Is, 1, sv.ext_dn, st)
     y = bf(T, H)
     wd = _dense_wset(w_dn, g("fwd_dn"))
+    tiles, ntiles, maxt, gk = _dense_list(T, H, True, 0, wd, dev)
     L.call("smel_gmm_fwd", ctypes.byref(wd), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(sv.actb), Is, T, 0,
            None, 0, 1, L.ptr(sv.ext_dn), 0, _ACT[act_name], L.ptr(y), H, None, st, tag=tag + "_dn_fwd")
     return y, sv
@@ -1351,6 +1389,7 @@ def _dense_mlp_bwd(sv: _DenseSaved, dy, w_gu_t: PackedW, w_dn_t: PackedW, lora, 
     if lb is not None:
         _lora_ext(tl, dy, H, T, 0, None, 0, 1, None, lb, "bt_dn", H, 1, ext_db, st)
     wd = _dense_wset(w_dn_t, g("at_dn"))
+    tiles, ntiles, maxt, gk = _dense_list(T, Is, False, 1, wd, dev)
     lrows = _bwd_lora_rows(None, lb, nblk, planes, part) if rows_lr else None
     lr = ctypes.byref(lrows) if lrows is not None else None
     L.call("smel_gmm_bwd_lr", ctypes.byref(wd), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(dy), H, T, 0,
@@ -1360,6 +1399,7 @@ def _dense_mlp_bwd(sv: _DenseSaved, dy, w_gu_t: PackedW, w_dn_t: PackedW, lora, 
         _lora_ext(tl, dh, 2 * Is, T, 0, None, 0, 1, None, lb, "bt_gu", 2 * Is, planes, ext_dxa, st)
     dx = bf(T, H)
     wg = _dense_wset(w_gu_t, g("at_gu"), planes)
+    tiles, ntiles, maxt, gk = _dense_list(T, H, False, 0, wg, dev)
     L.call("smel_gmm_bwd_lr", ctypes.byref(wg), L.ptr(gk), L.ptr(tiles), L.ptr(ntiles), maxt, L.ptr(dh), 2 * Is, T,
            0, None, 0, 1, None if lrows is not None else L.ptr(ext_dxa), 0, 0, None, None, None, L.ptr(dx), H, None,
            lr, st, tag=tag + "_gu_bwd")

@@ -777,6 +777,42 @@ def test_route_api_backward():
     assert_close_bf16(xg.grad.cpu(), xo.grad, "dx", rel=3e-2, cos=0.999)
 
 
+@pytest.mark.parametrize("T", [1, 33, 97, 300])
+@pytest.mark.parametrize("r", [8, 24])
+def test_dense_tile_heights_bitwise(T, r, monkeypatch):
+    """The dense MLP's GEMMs on tiles of 128, 96, 64 and 32 rows, spread over the XCDs by tiles or by column blocks (a
+    last column block cut short in every GEMM): each row's sums are the same, so y, dX and the LoRA gradients are
+    bitwise equal."""
+    import smel.moe as M
+    from smel import _lib as L
+    from smel.lora import MLPLoRA
+    H, Is = 320, 608
+    _say(f"dense tile heights T{T} r{r}")
+    g = torch.Generator(device=DEV).manual_seed(T)
+    rn = lambda *s, std=0.05: (torch.randn(*s, generator=g, device=DEV) * std).to(torch.bfloat16)
+    x, wg, wu, wd, gy = rn(T, H, std=1.0), rn(Is, H), rn(Is, H), rn(H, Is), rn(T, H)
+    torch.manual_seed(r)
+    lora = MLPLoRA(H, Is, r, 2.0 * r).to(DEV)
+    with torch.no_grad():
+        for n in ("B_gate", "B_up", "B_down"):
+            getattr(lora, n).normal_(0, 0.05)
+    runs = []
+    for rows in (128, 96, 64, 32):
+        for col in (0, L.WSET_COL_CHUNK):
+            def lst(T_, N, fwd, epi, w, dev):
+                w.flags |= col | (L.WSET_TILE32 if rows == 32 else 0)
+                return M._dense_tiles(T_, dev, rows)
+            monkeypatch.setattr(M, "_dense_list", lst)
+            xg = x.clone().requires_grad_(True)
+            lora.zero_grad()
+            y = M.mlp_lora(xg, wg, wu, wd, lora, "gelu_tanh")
+            y.backward(gy)
+            runs.append([y.detach(), xg.grad] + [p.grad.clone() for p in lora.parameters()])
+    for other in runs[1:]:
+        for a, b in zip(runs[0], other):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("act_name,T,H,Is,r", [("silu", 300, 256, 128, 8), ("gelu_tanh", 257, 512, 192, 16),
                                                ("silu", 64, 128, 64, 0), ("gelu_tanh", 190, 256, 128, 32),
                                                ("silu", 140, 128, 64, 20)])
