@@ -126,7 +126,8 @@ SMEL_DEV void dq8(uint32_t w, float sc, float ze, int rbf, float* v) {
 // would leave most of the 256 CUs idle.
 // Measured, 1021 tokens top-8 of 256 experts (12 of them fp32), H 2048, I 512 (about 32 rows per expert): gate_up 991 ->
 // 445 us, down 462 -> 240, down backward 528 -> 274, gate_up backward 949 -> 485 (against 64 x 64 blocks of 32x32x2
-// MFMAs); the 16-row slices computed are 43 GFLOP of gate_up = 97 TFLOP/s of the 157 nominal. With the loop's barriers
+// MFMAs; int4 tiles on whole k-steps now run as Split below); the 16-row slices computed are 43 GFLOP of gate_up = 97
+// TFLOP/s of the 157 nominal. With the loop's barriers
 // waiting for global loads, or its load and store code behind branches, the same tiles took 560-620 us.
 // One k-step's operands of a thread on their way from global memory to LDS.
 struct StageRegs {
@@ -329,6 +330,209 @@ struct Gemm {
   }
 };
 
+// ---------------------------------------------------------------------------------------------- int4 tiles on bf16 MFMAs
+// fp32 products of int4 tiles from 16-bit matrix instructions without losing bits: every fp32 value is the sum of three
+// bf16 values (x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1); the differences are exact and 3 x 8 bits hold
+// all 24), a bf16 x bf16 product is exact in fp32, and of the nine products the three below 2^-25 of the largest are
+// left out: x w = x0 w0 + (x0 w1 + x1 w0) + (x0 w2 + x1 w1 + x2 w0). Six v_mfma_f32_16x16x32_bf16 take 96 cycles for the
+// 32 k that eight v_mfma_f32_16x16x4_f32 take 256 for, and they round the sum six times instead of eight to 32 times, so
+// the error against 64 bits is smaller than the fp32 instruction's. Weights rounded to bf16 (RBF) are one value: three products.
+// Values that do not split (infinities, NaN, numbers that round up to infinity) leave a non-finite sum: such a tile is
+// computed again by the fp32 instruction, which decides what the result is.
+// What bounds it: the VALU work of dequant and splitting, about 8 instructions per weight and pass (with every load of
+// the loop out of range 255 of gate_up's 315 us remain; a cheaper-looking split by two-term dot products, two
+// instructions less per value, took the same time). So no weight is split twice in a pass of up to 48 rows: a wave takes
+// all 128 columns of the block for its quarter of the k-steps (every fourth step of 32), straight from global memory into
+// registers without a barrier, and the waves' sums are added through LDS in wave order. Only the block's scales and
+// zeros (packed) wait in LDS. Measured (1021 tokens top-8 of 256 experts, H 2048, I 512; fp32 instruction -> split):
+// gate_up 450 -> 310 us, down 243 -> 186, down backward 276 -> 183, gate_up backward 496 -> 321.
+// x and y as three bf16 values each, packed (the differences are exact).
+SMEL_DEV void split3(float x, float y, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
+  p0 = pack2bf(x, y);
+  x -= bf_lo(p0), y -= bf_hi(p0);
+  p1 = pack2bf(x, y);
+  x -= bf_lo(p1), y -= bf_hi(p1);
+  p2 = pack2bf(x, y);
+}
+
+SMEL_DEV f32v4 mfma32b(const u32x4_t& a, const u32x4_t& b, const f32v4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0,
+                                                 0, 0);
+}
+
+template <int TRANS>
+struct Split {
+  using GM = Gemm<TRANS, 64, 128, 1, 32>;
+  static constexpr int NF = 8, NT = 128, MAXRF = 3;
+  static constexpr int PR = NT + 4;   // pitch of the reduction rows
+  static_assert(4 * 16 * PR <= GM::LDS_FLOATS, "reduction buffer");
+
+  // groups of one k row (TRANS) or of one output row that the block's panel of scales holds
+  SMEL_DEV static int panel_groups(const WMat& m, int N, int n0) {
+    return TRANS ? (min(n0 + NT, N) - 1) / m.group - n0 / m.group + 1 : m.gpr;
+  }
+  // (vec and qvec hold) whole k-steps, a lane's 8 weights under one scale / zero pair, the panel inside the LDS
+  SMEL_DEV static bool fits(const WMat& m, int N, int K, int n0) {
+    return K % 32 == 0 && m.group % 32 == 0 && (int64_t)panel_groups(m, N, n0) * (TRANS ? K : NT) <= GM::LDS_FLOATS;
+  }
+
+  template <int NRF, bool RBF>
+  SMEL_DEV static void tile(float* __restrict__ lds, const GemmArgs& G, const WMat& m, int N, int K, int n0, int mr0,
+                            int mr1) {
+    const int t = threadIdx.x, l = lane_id(), i = l & 15, kq = l >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nk = K / 32, nfw = min(NT, N - n0);
+    const int half = m.C >> 1, WR = TRANS ? K : N;
+    const rsrc_t ra = make_rsrc(G.A + (int64_t)mr0 * G.lda, ((uint64_t)(mr1 - mr0 - 1) * G.lda + K) * 4);
+    const rsrc_t rw = make_rsrc(m.q, (uint64_t)WR * half);
+    uint32_t arow[NRF];
+#pragma unroll
+    for (int rf = 0; rf < NRF; ++rf) {
+      const int r = 16 * rf + i;
+      arow[rf] = r < mr1 - mr0 ? 4u * (uint32_t)(r * (int)G.lda + 8 * kq) : OOB;
+    }
+    // column 8 i + f of the block is fragment f of lane i; rows of the matrix past its last read as zeros
+    const uint32_t wb = TRANS ? (8 * i < nfw ? (uint32_t)(8 * kq * half + ((n0 + 8 * i) >> 1)) : OOB)
+                              : (uint32_t)((n0 + 8 * i) * half + 4 * kq);
+    u32x4_t araw[NRF][2];   // 8 k of the lane's row per 16-row slice
+    uint32_t q[8], qn[8];   // 64 nibbles
+    auto load_a = [&](int step) {
+#pragma unroll
+      for (int rf = 0; rf < NRF; ++rf)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          araw[rf][h] = ld16(ra, step < nk && arow[rf] != OOB ? arow[rf] + 128u * step + 16 * h : OOB);
+    };
+    auto load_q = [&](uint32_t* o, int step) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        o[j] = ld4(rw, step < nk && wb != OOB
+                           ? wb + (uint32_t)(j * half) + (TRANS ? (uint32_t)(32 * step * half) : 16u * step)
+                           : OOB);
+    };
+    load_a(wv);
+    load_q(q, wv);
+    // scale | zero << 16 of the block's weights: [group][column] or, TRANS, [group][k]
+    uint32_t* const P = reinterpret_cast<uint32_t*>(lds);
+    const int ng = panel_groups(m, N, n0), g0 = TRANS ? n0 / m.group : 0;
+    const int outer = TRANS ? K : NT;
+    {
+      const int gs = ng <= 1 ? 0 : 32 - __builtin_clz((unsigned)(ng - 1));   // consecutive threads: a row's groups
+      const rsrc_t rs = make_rsrc(m.s, (uint64_t)WR * m.gpr * 2), rz = make_rsrc(m.z, (uint64_t)WR * m.gpr * 2);
+#pragma unroll 8
+      for (int e = t; e < outer << gs; e += 256) {
+        const int o = e >> gs, g = e & ((1 << gs) - 1);
+        const uint32_t off = 2u * (uint32_t)((TRANS ? o : n0 + o) * m.gpr + g0 + g);
+        const uint32_t s = ld2(rs, off), z = ld2(rz, off);
+        if (g < ng) P[g * outer + o] = s | (z << 16);
+      }
+    }
+    lds_barrier();
+    const uint32_t* const pl = P + (TRANS ? ((n0 + min(8 * i, nfw - 1)) / m.group - g0) * K + 8 * kq : 8 * i);
+    f32v4 acc[NRF][NF] = {};
+    for (int step = wv; step < nk; step += 4) {   // no barrier: each wave its own steps
+      u32x4_t a0[NRF], a1[NRF], a2[NRF];
+#pragma unroll
+      for (int rf = 0; rf < NRF; ++rf)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          uint32_t p0, p1, p2;
+          split3(__uint_as_float(araw[rf][j >> 1][2 * (j & 1)]), __uint_as_float(araw[rf][j >> 1][2 * (j & 1) + 1]), p0,
+                 p1, p2);
+          a0[rf][j] = p0, a1[rf][j] = p1, a2[rf][j] = p2;
+        }
+      __builtin_amdgcn_sched_barrier(0);
+      load_a(step + 4);
+      load_q(qn, step + 4);
+      __builtin_amdgcn_sched_barrier(0);
+      const uint32_t* const sp = pl + (TRANS ? 32 * step : 32 * step / m.group * NT);
+      const u32x4_t z0 = *reinterpret_cast<const u32x4_t*>(sp), z1 = *reinterpret_cast<const u32x4_t*>(sp + 4);
+      // TRANS: nibble f of every row's word; the even ones first, then the odd ones shifted into their bytes
+      uint32_t nib8[8];
+      u32x4_t b[2][3];
+      auto weights = [&](int f, u32x4_t* o) {   // fragment f's 8 weights, split
+        float w[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {   // TRANS: row j's nibble f; else row f's nibble j
+          const int wd = TRANS ? j : f, nb = TRANS ? f : j;
+          if (TRANS ? (f == 0 || f == 1) : j < 2)
+            nib8[TRANS ? j : j & 1] = (nb & 1 ? q[wd] >> 4 : q[wd]) & 0x0f0f0f0fu;
+          const uint32_t sz = wd < 4 ? z0[wd & 3] : z1[wd & 3];
+          const uint32_t n4 = nib8[TRANS ? j : j & 1];
+          w[j] = fmaf(nb < 2 ? ub0(n4) : nb < 4 ? ub1(n4) : nb < 6 ? ub2(n4) : ub3(n4), bf_lo(sz), bf_hi(sz));
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          uint32_t p0, p1 = 0, p2 = 0;
+          if constexpr (RBF) p0 = pack2bf(w[2 * j], w[2 * j + 1]);
+          else split3(w[2 * j], w[2 * j + 1], p0, p1, p2);
+          o[0][j] = p0, o[1][j] = p1, o[2][j] = p2;
+        }
+      };
+      // fragments in the order 0 2 4 6 1 3 5 7; the next one's weights are made between this one's MFMAs, and the fence
+      // keeps the later ones out of registers that are not there
+      weights(0, b[0]);
+#pragma unroll
+      for (int o = 0; o < NF; ++o) {
+        const int f = o < 4 ? 2 * o : 2 * o - 7, fn = o + 1 < 4 ? 2 * o + 2 : 2 * o - 5;
+        __builtin_amdgcn_sched_barrier(0);
+        auto mm = [&](const u32x4_t* a, const u32x4_t& bb) {
+#pragma unroll
+          for (int rf = 0; rf < NRF; ++rf) acc[rf][f] = mfma32b(a[rf], bb, acc[rf][f]);
+        };
+        const u32x4_t* const c = b[o & 1];
+        mm(a2, c[0]);   // the small products first
+        if constexpr (!RBF) {
+          mm(a1, c[1]);
+          mm(a0, c[2]);
+        }
+        mm(a1, c[0]);
+        if constexpr (!RBF) mm(a0, c[1]);
+        mm(a0, c[0]);
+        if (o + 1 < NF) weights(fn, b[(o + 1) & 1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = qn[j];
+    }
+    float bad = 0.f;   // NaN once any sum is infinite or NaN
+#pragma unroll
+    for (int rf = 0; rf < NRF; ++rf)
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bad = fmaf(acc[rf][f][r], 0.f, bad);
+    if (__syncthreads_or(bad != 0.f)) {
+      GM::template tile<RBF ? W_INT4R : W_INT4, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
+      lds_barrier();
+      return;
+    }
+#pragma unroll
+    for (int rf = 0; rf < NRF; ++rf) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          *reinterpret_cast<f32v4*>(lds + (16 * wv + 4 * kq + r) * PR + 8 * i + 4 * h) =
+              f32v4{acc[rf][4 * h][r], acc[rf][4 * h + 1][r], acc[rf][4 * h + 2][r], acc[rf][4 * h + 3][r]};
+      lds_barrier();
+      const int cc = t & (NT - 1), row0 = mr0 + 16 * rf;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int rr = (t >> 7) + 2 * j;
+        float v = lds[rr * PR + cc];
+#pragma unroll
+        for (int q = 1; q < 4; ++q) v += lds[(16 * q + rr) * PR + cc];
+        if (row0 + rr < mr1 && cc < nfw) {
+          float* const p = G.C + (int64_t)(row0 + rr) * G.ldc + n0 + cc;
+          *p = G.beta1 ? *p + G.alpha * v : G.alpha * v;
+        }
+      }
+      lds_barrier();
+    }
+  }
+};
+
 template <int TRANS, int RB, int NT, int KS, int FK>
 __global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const int32_t* __restrict__ gkind,
                                                          const int32_t* __restrict__ tiles,
@@ -348,6 +552,21 @@ __global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const 
   if (!((w.kinds >> kind) & 1)) return;
   WMat m;
   if (!resolve(w, kind, idx, m)) return;
+  if constexpr (NT == Split<TRANS>::NT) {
+    if (!m.f && (vec & 1) && qvec && Split<TRANS>::fits(m, N, K, n0)) {
+      // the tile's 16-row slices in passes of up to three, as even as they go
+      const int ns = (r1 - r0 + 15) >> 4, np = (ns + Split<TRANS>::MAXRF - 1) / Split<TRANS>::MAXRF;
+      for (int p = blockIdx.z; p < np; p += gridDim.z) {
+        const int s0 = p * ns / np, s1 = (p + 1) * ns / np;
+        const int mr0 = r0 + 16 * s0, mr1 = min(r1, r0 + 16 * s1);
+        if (m.rbf) Split<TRANS>::template tile<3, true>(lds, G, m, N, K, n0, mr0, mr1);
+        else if (s1 - s0 == 1) Split<TRANS>::template tile<1, false>(lds, G, m, N, K, n0, mr0, mr1);
+        else if (s1 - s0 == 2) Split<TRANS>::template tile<2, false>(lds, G, m, N, K, n0, mr0, mr1);
+        else Split<TRANS>::template tile<3, false>(lds, G, m, N, K, n0, mr0, mr1);
+      }
+      return;
+    }
+  }
   // the tile's rows in RB-row steps; gridDim.z blocks share them
   for (int mr0 = r0 + RB * (int)blockIdx.z; mr0 < r1; mr0 += RB * (int)gridDim.z) {
     const int mr1 = min(r1, mr0 + RB);

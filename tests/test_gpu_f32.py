@@ -139,6 +139,52 @@ def test_gmm_f32_shapes_against_fp64(shape, trans, kind):
         assert torch.equal(got[:, N:], C0[:, N:]) and torch.equal(got[rows], C0[rows])
 
 
+# (output columns, K, int4 group) of the tiles whose fp32 products run as bf16 parts: K of one step of 32 to more than a
+# round of four waves, columns over an edge of 128, one to many groups; counts over every number of 16-row slices of a pass
+SPLIT_COUNTS = [1, 16, 17, 33, 48, 49, 64, 65, 97, 128, 130, 0] * 6
+
+
+@pytest.mark.parametrize("kind", ["int4", "int4_bf16"])
+@pytest.mark.parametrize("trans,N,K,group", [(0, 901, 32, 32), (0, 901, 192, 96), (0, 1024, 320, 64), (1, 960, 32, 32),
+                                             (1, 960, 160, 96), (1, 1088, 288, 64)])
+def test_gmm_f32_split_int4_tiles(trans, N, K, group, kind):
+    """Rows of very different sizes, and rows with values that do not split into bf16 parts (infinities, NaN, the largest
+    finite number), against the fp64 product. Bound of a finite row: at most 6 K / 32 + 5 <= 65 roundings of 2^-24 of the
+    running sum, adding as their square root (5e-7 of the result's typical size |A row| std(W)), with a factor of 4 for
+    the largest of a million results; a row that is not finite has the fp64 product's infinities and NaN."""
+    from smel import _lib as L
+    from smel import moe_f32 as F
+    _say(f"gmm_f32 split N={N} K={K} g={group} trans={trans} kind={kind}")
+    torch.manual_seed(N + K)
+    counts, Rw, Cw = SPLIT_COUNTS, (K if trans else N), (N if trans else K)
+    E, rows = len(counts), sum(counts)
+    q = _int4_bank(E, Rw, Cw, group, 3)
+    W = R.dequant_int4(q["q"], q["scale"], q["zero"],
+                       torch.bfloat16 if kind == "int4_bf16" else torch.float32).double()
+    dq = {k: v.to(DEV) for k, v in q.items()}
+    w = F._ws(Rw, Cw, 1 << L.KIND_INT4, q4=L.ptr(dq["q"]), scale=L.ptr(dq["scale"]), zero=L.ptr(dq["zero"]))
+    w.group, w.q4_round_bf16 = group, int(kind == "int4_bf16")
+    tl, _ = F.count_tiles(counts, L.KIND_INT4, DEV)
+    A = torch.randn(rows, K) * torch.exp2(torch.randint(-60, 60, (rows, 1)).float())
+    for i, v in enumerate((float("inf"), float("-inf"), float("nan"), 3.4028234e38)):
+        A[torch.arange(100 + i, rows, 997), i] = v
+    Ad, Cd = A.to(DEV), torch.full((rows, N), 7.0, device=DEV)
+    F.gmm(w, trans, tl, Ad, K, Cd, N, alpha=0.5, beta=0.0)
+    got = Cd.cpu().double()
+    off = 0
+    for e, c in enumerate(counts):
+        ref = 0.5 * (A[off:off + c].double() @ (W[e] if trans else W[e].t()))
+        g = got[off:off + c]
+        fin = ref.isfinite()
+        assert torch.equal(fin, g.isfinite()), f"expert {e}"
+        assert torch.equal(torch.nan_to_num(ref[~fin], nan=1.5, posinf=2.5, neginf=3.5),
+                           torch.nan_to_num(g[~fin], nan=1.5, posinf=2.5, neginf=3.5)), f"expert {e}"
+        size = (A[off:off + c].double() ** 2).sum(1, keepdim=True).sqrt() * W[e].std()
+        ok = fin.all(1)
+        assert ((g - ref).abs() <= 2e-6 * size)[ok].all(), f"expert {e}: {((g - ref).abs() / size)[ok].max():.2e}"
+        off += c
+
+
 @pytest.mark.parametrize("M,N", [(16, 200), (200, 16), (8, 36), (36, 33), (1, 64), (17, 65)])
 def test_wgrad_f32_shapes_against_fp64(M, N):
     """smel_wgrad_f32 with either side the narrower one, sides off the block sizes, and row counts around the waves'
