@@ -206,6 +206,59 @@ __global__ __launch_bounds__(256) void route_logits_kernel(const uint16_t* __res
   }
 }
 
+// The same logits, bit for bit (each is one accumulator's MFMAs in k order in both kernels), for few tokens: a wave takes
+// 16 tokens x 16 columns straight from global memory into registers, so that 16 times as many CUs pull rows as 64 x 96
+// blocks give work to. Bound by memory latency, which a wave meets H / 512 times (16 steps of 32 load while 16 are
+// used); its 32 rows for 256 MFMA columns make it the worse one once every CU has rows enough (see launch_logits).
+constexpr int RS_U = 16;
+__global__ __launch_bounds__(64) void route_logits_few_kernel(const uint16_t* __restrict__ x,
+                                                              const uint16_t* __restrict__ gw,
+                                                              const uint16_t* __restrict__ sg, int T, int H, int E,
+                                                              int ldl, uint16_t* __restrict__ logits,
+                                                              int32_t* __restrict__ zero_ws, int zero_n) {
+  const int l = threadIdx.x, kq = l >> 4, li = l & 15;
+  if (zero_ws) {
+    const int nblk = gridDim.x * gridDim.y, b = blockIdx.y * gridDim.x + blockIdx.x;
+    for (int i = b * 64 + l; i < zero_n; i += nblk * 64) zero_ws[i] = 0;
+  }
+  const int t0 = blockIdx.x * 16, c0 = blockIdx.y * 16;
+  const int E32 = (E + 31) / 32 * 32;
+  const int n = H / 32, c = c0 + li, tok = t0 + li;
+  const bool gate = c0 < E32;   // uniform: the 16 columns are gate rows (or padding), or the shared gate and padding
+  const rsrc_t rx = make_rsrc(x, (uint64_t)T * H * 2);
+  const rsrc_t rw = gate ? make_rsrc(gw, (uint64_t)E * H * 2) : make_rsrc(sg ? sg : gw, sg ? (uint64_t)H * 2 : 0);
+  const uint32_t xo = tok < T ? (uint32_t)tok * H * 2 + 16 * kq : OOB;
+  const uint32_t wo = gate ? (c < E ? (uint32_t)c * H * 2 + 16 * kq : OOB) : ((sg && c == E32) ? 16u * kq : OOB);
+  u32x4_t A[2][RS_U], B[2][RS_U];
+  auto load = [&](int s, int set) {
+#pragma unroll
+    for (int u = 0; u < RS_U; ++u) {
+      const bool in = s + u < n;
+      A[set][u] = ld16(rx, in ? xo + 64u * (s + u) : OOB);
+      B[set][u] = ld16(rw, in ? wo + 64u * (s + u) : OOB);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x4_t acc = f32x4_t{};
+  auto compute = [&](int set) {   // steps past H add zeros
+#pragma unroll
+    for (int u = 0; u < RS_U; ++u) acc = mfma16r(A[set][u], B[set][u], acc);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  load(0, 0);
+  for (int s = 0; s < n; s += 2 * RS_U) {
+    load(s + RS_U, 1);
+    compute(0);
+    load(s + 2 * RS_U, 0);
+    compute(1);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int t = t0 + 4 * kq + r;
+    if (t < T && c < ldl) logits[(int64_t)t * ldl + c] = f2bf(acc[r]);
+  }
+}
+
 // ---- selection: one wave per token over its bf16 logits row (probs, top-k, renorm; shared-gate sigmoid).
 template <int NPL>
 __global__ __launch_bounds__(256) void route_select(const uint16_t* __restrict__ logits, int ldl, int T, int E, int K,
@@ -392,8 +445,17 @@ __global__ __launch_bounds__(256) void dtopv_kernel(const float* __restrict__ dw
   out[p] = v;
 }
 
+// Few tokens (up to 2.5 waves of 16 x 16 logits per CU) take the kernel without staging. Measured with the selection,
+// H 2048, 256 experts and the shared gate (64 x 96 blocks -> waves of 16 x 16): 1 token 18.3 -> 9.2 us, 23 20.4 -> 11.7,
+// 256 21.4 -> 14.5, 512 21.5 -> 18.2, 640 21.4 -> 19.6; 768 21.5 -> 22.1, 1024 21.6 -> 26.3.
+constexpr int64_t ROUTE_FEW = 640;
 void launch_logits(hipStream_t stream, const uint16_t* x, const uint16_t* gw, const uint16_t* sg, int T, int H, int E,
                    int ldl, uint16_t* logits, int32_t* zero_ws = nullptr, int zero_n = 0) {
+  const dim3 few((unsigned)((T + 15) / 16), (unsigned)((ldl + 15) / 16));
+  if ((int64_t)few.x * few.y <= ROUTE_FEW) {
+    route_logits_few_kernel<<<few, 64, 0, stream>>>(x, gw, sg, T, H, E, ldl, logits, zero_ws, zero_n);
+    return;
+  }
   const dim3 grid((unsigned)((T + RT - 1) / RT), (unsigned)((ldl + RC - 1) / RC));
   route_logits_kernel<<<grid, 256, 0, stream>>>(x, gw, sg, T, H, E, ldl, logits, zero_ws, zero_n);
 }

@@ -360,6 +360,33 @@ def test_route_fused(T, H, E, K, shared):
         assert torch.allclose(sgate.cpu(), ref, rtol=1e-2, atol=1e-3)
 
 
+@pytest.mark.parametrize("T,H,E,K,shared", [(1300, 2048, 256, 8, True), (1600, 64, 100, 4, False), (700, 576, 512, 8, True),
+                                            (10400, 320, 8, 2, False)])
+def test_route_few_tokens_bitwise(T, H, E, K, shared):
+    """Few tokens take the logits kernel without staging: every output of a token is the same, bit for bit, as in a call
+    of many tokens (k rounds of one step to more than four, columns and tokens off the 16)."""
+    from smel import _lib as L
+    _say(f"route few T{T} H{H} E{E}")
+    g = torch.Generator(device=DEV).manual_seed(T)
+    rn = lambda *s, std: (torch.randn(*s, generator=g, device=DEV) * std).to(torch.bfloat16)
+    x, gw, sg = rn(T, H, std=1.0), rn(E, H, std=0.05), rn(H, std=0.05)
+    ld = L.load().smel_route_ld(E, int(shared))
+
+    def run(xs):
+        n = xs.shape[0]
+        o = [torch.full(sh, 0, dtype=dt, device=DEV) for sh, dt in
+             (((n, E), torch.float32), ((n, K), torch.bfloat16), ((n, K), torch.float32), ((n, K), torch.int64),
+              ((n, K), torch.int32), ((n,), torch.float32), ((n, ld), torch.bfloat16))]
+        L.call("smel_route", L.ptr(xs), L.ptr(gw), L.ptr(sg) if shared else None, n, H, E, K, *[L.ptr(t) for t in o],
+               L.stream())
+        return o
+
+    many = run(x)
+    for t0, n in ((0, 1), (5, 17), (T - 40, 40), (3, 160)):
+        for a, b in zip(run(x[t0:t0 + n].contiguous()), many):
+            assert torch.equal(a, b[t0:t0 + n])
+
+
 @pytest.mark.parametrize("T,H,E,K,shared", [(4092, 2048, 256, 8, True), (77, 128, 16, 3, False),
                                            (1300, 256, 512, 8, True)])
 def test_route_counted_then_dispatch_counted(T, H, E, K, shared):
