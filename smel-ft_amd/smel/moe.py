@@ -461,11 +461,12 @@ class _LoRABufs:
 
 _PREP_NAMES = ("A_gate", "B_gate", "A_up", "B_up", "A_down", "B_down")
 _LAYOUTS = ("fwd_gu", "fwd_dn", "a_gu", "a_dn", "bt_dn", "bt_gu", "at_gu", "at_dn")
+_NO_PARAMETERS = {}   # of a LoRA set that is no torch module: its factors are plain attributes
 
 
 def _factor(lora, name: str):
     """A factor of a LoRA set, past torch's module attribute lookup where it is a plain parameter."""
-    p = lora._parameters.get(name)
+    p = getattr(lora, "_parameters", _NO_PARAMETERS).get(name)
     return p if p is not None else getattr(lora, name)
 
 

@@ -149,3 +149,21 @@ def test_block_build_and_adapter_roundtrip(tmp_path):
     for k in sd0:
         assert torch.equal(sd0[k], sd1[k]), k
     assert BlockLoRA.build({1: [0]}, 32, 16, 24, r=4, alpha=8.0, shared=False).get(1).shared is None
+
+
+def test_layer_reads_factors_of_any_lora_object():
+    """The layer's factor lookup: parameters of a module, the computed weights of a parametrized one, and plain
+    attributes of an object that is no module."""
+    from types import SimpleNamespace
+
+    from smel.moe import _LORA_NAMES, _lora_leaves
+    sh = MLPLoRA(64, 48, r=4, alpha=8.0)
+    assert all(a is getattr(sh, n) for a, n in zip(_lora_leaves(sh), _LORA_NAMES))
+    plain = SimpleNamespace(scale=sh.scale, r=sh.r, **{n: getattr(sh, n).detach() for n in NAMES})
+    assert all(a is getattr(plain, n) for a, n in zip(_lora_leaves(plain), _LORA_NAMES))
+
+    class Double(torch.nn.Module):
+        def forward(self, w):
+            return 2 * w
+    torch.nn.utils.parametrize.register_parametrization(sh, "B_up", Double())
+    assert [torch.equal(a, getattr(sh, n)) for a, n in zip(_lora_leaves(sh), _LORA_NAMES)] == [True] * 6
