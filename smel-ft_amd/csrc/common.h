@@ -36,6 +36,23 @@ SMEL_DEV float wave_max(float v) {
   for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
   return v;
 }
+// Largest of v over the wave, uniform: DPP moves run in the vector ALU (six of about 8 cycles), where a shuffle is a round
+// trip through the LDS unit (six of about 64). Lanes without a source read 0.
+SMEL_DEV uint32_t wave_max_u32(uint32_t v) {
+#define SMEL_DPP_MAX(ctrl, rows) \
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false))
+  SMEL_DPP_MAX(0x111, 0xf);   // row_shr:1, 2, 4, 8: lane 15 of each row of 16 holds the row's
+  SMEL_DPP_MAX(0x112, 0xf);
+  SMEL_DPP_MAX(0x114, 0xf);
+  SMEL_DPP_MAX(0x118, 0xf);
+  SMEL_DPP_MAX(0x142, 0xa);   // row_bcast:15 into rows 1 and 3
+  SMEL_DPP_MAX(0x143, 0xc);   // row_bcast:31 into rows 2 and 3
+#undef SMEL_DPP_MAX
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// v of lane k (k uniform), uniform
+SMEL_DEV int lane_get(int v, int k) { return __builtin_amdgcn_readlane(v, k); }
+SMEL_DEV float lane_get(float v, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k)); }
 // sum over the 32 lanes that share lane/32 (the two halves of a wave reduce independently)
 SMEL_DEV float half_sum(float v) {
 #pragma unroll

@@ -53,33 +53,29 @@ SMEL_DEV void select_topk(Get logit, int E, int K, int64_t t, float* __restrict_
     const uint32_t ord = (b & 0x8000u) ? (~b & 0xffffu) : (b | 0x8000u);
     key[j] = e < E ? (ord << 16) | (0xffffu - (uint32_t)e) : 0u;
   }
-  float pk[16];
-  int ik[16];
-  float psum = 0.f;
+  // A round is a serial chain, and the selection little else: with the maximum by DPP moves instead of shuffles and a
+  // pick kept by its lane instead of in arrays it went from 7.5 to 6.0 us for 23 tokens, from 10.6 to 9.5 us for 4092.
+  float p = 0.f, psum = 0.f;   // lane k keeps pick k
+  int i = 0;
   for (int k = 0; k < K; ++k) {
     uint32_t best = key[0];
 #pragma unroll
     for (int j = 1; j < NPL; ++j) best = max(best, key[j]);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) best = max(best, (uint32_t)__shfl_xor((int)best, o, 64));
+    best = wave_max_u32(best);
     const int bi = (int)(0xffffu - (best & 0xffffu));
 #pragma unroll
     for (int j = 0; j < NPL; ++j)
       if (bi == l + 64 * j) key[j] = 0u;
     const uint32_t ob = best >> 16;
     const float bv = __uint_as_float(((ob & 0x8000u) ? (ob & 0x7fffu) : (~ob & 0xffffu)) << 16);
-    ik[k] = bi;
-    pk[k] = expf(bv - m) * inv_s;   // the same expression as probs[t][bi]
-    psum += pk[k];
+    const float pk = expf(bv - m) * inv_s;   // the same expression as probs[t][bi]
+    psum += pk;
+    if (l == k) {
+      p = pk;
+      i = bi;
+    }
   }
   if (l < K) {
-    float p = 0.f;
-    int i = 0;
-    for (int k = 0; k < K; ++k)
-      if (k == l) {
-        p = pk[k];
-        i = ik[k];
-      }
     if (topv_f32) {
       topv_f32[t * K + l] = pes ? (p / psum) * bf2f(pes[i]) : p / psum;   // route_gemma4: fp32, x per-expert scale
     } else {
@@ -293,6 +289,10 @@ void launch_select(hipStream_t stream, const uint16_t* logits, int ldl, int T, i
 //   renorm:  topv_k = p_k / S  ->  dp_k = (dtopv_k - sum_j dtopv_j topv_j) / S
 //   softmax: dlogit_e = p_e (dp_e - sum_k dp_k p_{i_k}),  dp_e = 0 off the top-k
 //   shared gate: dlogit_sg = (sum_j dwp[TK+t][j]) * sg (1 - sg)
+// Bound by latency: the uniform values go through scalar registers (lane_get) instead of LDS shuffles, and the loads that
+// need no other go out together: 517 tokens 7.6 -> 5.7 us.
+// NPL: probabilities a lane holds in registers (experts past 64 NPL are read again where they are used)
+template <int NPL>
 __global__ __launch_bounds__(256) void route_bwd(const float* __restrict__ dwp, int nblk,
                                                  const int32_t* __restrict__ inv, const float* __restrict__ probs,
                                                  const int32_t* __restrict__ topi32, const float* __restrict__ sgate,
@@ -303,45 +303,53 @@ __global__ __launch_bounds__(256) void route_bwd(const float* __restrict__ dwp, 
   const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= T) return;
   const int l = lane_id();
-  // per-k quantities, lane k holds slot k
+  // per-k quantities, lane k holds slot k; loads that need no other go out together (the chain is two round trips)
   float dtv = 0.f, p = 0.f;
   int idx = -1;
+  float pr[NPL];
+#pragma unroll
+  for (int j = 0; j < NPL; ++j) pr[j] = l + 64 * j < E ? probs[t * E + l + 64 * j] : 0.f;
   if (l < K) {
     // -1 for a slot the dispatch dropped (id out of range); no inv = dwp rows are the slots themselves
     const int row = inv ? inv[t * K + l] : (int)(t * K + l);
+    idx = topi32[t * K + l];
+    if (idx < 0 || idx >= E) idx = -1;
+    p = probs[t * E + max(idx, 0)];
+    if (idx < 0) p = 0.f;
     if (row >= 0)
       for (int j = 0; j < nblk; ++j) dtv += dwp[(int64_t)row * nblk + j];
-    idx = topi32[t * K + l];
-    if (idx >= 0 && idx < E) p = probs[t * E + idx];
-    else idx = -1;
     if (dtopv_out) dtopv_out[t * K + l] = dtv;
     if (pes && idx >= 0) dtv *= bf2f(pes[idx]);   // route_gemma4's topv = renorm * per_expert_scale[i]
   }
   // S = sum_k p_k ; topv_k = p_k / S (recomputed in fp32, not the bf16-rounded copy)
   float S = 0.f, dot = 0.f;
-  for (int k = 0; k < K; ++k) S += __shfl(p, k, 64);
+  for (int k = 0; k < K; ++k) S += lane_get(p, k);
   const float tv = (l < K) ? p / S : 0.f;
-  for (int k = 0; k < K; ++k) dot += __shfl(dtv * tv, k, 64);
+  for (int k = 0; k < K; ++k) dot += lane_get(dtv * tv, k);
   const float dp = (l < K) ? (dtv - dot) / S : 0.f;
   float pdp = 0.f;   // sum_k dp_k p_k
-  for (int k = 0; k < K; ++k) pdp += __shfl(dp * p, k, 64);
-  // every lane gets the K (id, dp) pairs before any lane-divergent code (a shuffle only reads active lanes)
+  for (int k = 0; k < K; ++k) pdp += lane_get(dp * p, k);
+  // the K (id, dp) pairs, uniform
   int ik[16];
   float dk[16];
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
-    ik[k] = k < K ? __shfl(idx, k, 64) : -1;
-    dk[k] = k < K ? __shfl(dp, k, 64) : 0.f;
+    ik[k] = k < K ? lane_get(idx, k) : -1;
+    dk[k] = k < K ? lane_get(dp, k) : 0.f;
   }
-  for (int e = l; e < ldl; e += 64) {
-    float g = 0.f;
-    if (e < E) {
-      float dpe = 0.f;
+  auto expert = [&](int e, float pe) {
+    float dpe = 0.f;
 #pragma unroll
-      for (int k = 0; k < 16; ++k)
-        if (ik[k] == e) dpe = dk[k];
-      g = probs[t * E + e] * (dpe - pdp);
-    } else if (e == E && sgate) {
+    for (int k = 0; k < 16; ++k)
+      if (ik[k] == e) dpe = dk[k];
+    if (e < E) dlogits[t * ldl + e] = f2bf(pe * (dpe - pdp));
+  };
+#pragma unroll
+  for (int j = 0; j < NPL; ++j) expert(l + 64 * j, pr[j]);
+  for (int e = l + 64 * NPL; e < E; e += 64) expert(e, probs[t * E + e]);
+  for (int e = E + l; e < ldl; e += 64) {
+    float g = 0.f;
+    if (e == E && sgate) {
       float ds = 0.f;
       if (dwp_sh)   // the shared expert ran as its own GEMMs: its row-weight partials, [T][nblk_sh]
         for (int j = 0; j < nblk_sh; ++j) ds += dwp_sh[t * nblk_sh + j];
@@ -539,9 +547,13 @@ extern "C" int smel_route_bwd(const float* dwp, int64_t nblk, const int32_t* inv
   if (T == 0) return 0;
   SMEL_REQUIRE(dwp && probs && topi32 && dlogits, SMEL_EINVAL, "route_bwd: null pointer");
   SMEL_REQUIRE(inv || TK == T * K, SMEL_EINVAL, "route_bwd: without inv, dwp rows are the T*K slots");
-  route_bwd<<<(unsigned)((T + 3) / 4), 256, 0, stream>>>(dwp, (int)nblk, inv, probs, topi32, sgate, dwp_sh,
-                                                         (int)nblk_sh, (int)T, (int)K, (int)E, (int)TK, dlogits,
-                                                         (int)ldl, dtopv_out, per_expert_scale);
+  const unsigned grid = (unsigned)((T + 3) / 4);
+  if (E <= 256)
+    route_bwd<4><<<grid, 256, 0, stream>>>(dwp, (int)nblk, inv, probs, topi32, sgate, dwp_sh, (int)nblk_sh, (int)T,
+                                           (int)K, (int)E, (int)TK, dlogits, (int)ldl, dtopv_out, per_expert_scale);
+  else
+    route_bwd<8><<<grid, 256, 0, stream>>>(dwp, (int)nblk, inv, probs, topi32, sgate, dwp_sh, (int)nblk_sh, (int)T,
+                                           (int)K, (int)E, (int)TK, dlogits, (int)ldl, dtopv_out, per_expert_scale);
   return smel::launch_status();
 }
 

@@ -1076,3 +1076,39 @@ def test_layer_skewed_parity_and_determinism():
     assert_close_bf16(outs[0][1], dx, "dx")
     for k, v in grads.items():
         assert_close_bf16(outs[0][2][k], v, k)
+
+
+@pytest.mark.parametrize("E,K,shared", [(1, 1, 0), (63, 8, 1), (256, 8, 1), (257, 16, 0), (512, 8, 1), (577, 16, 1)])
+def test_route_bwd_against_fp64(E, K, shared):
+    """smel_route_bwd at the edges of the probabilities a lane holds in registers (256, 512) and past them, against its
+    formula in float64: each value within a bf16 rounding, plus fp32 rounding of the sums it is the difference of."""
+    L = _lib()
+    T, nblk, ldl = 9, 3, (E + shared + 31) // 32 * 32
+    g = torch.Generator().manual_seed(E)
+    probs = torch.softmax(torch.randn(T, E, generator=g), 1)
+    topi = torch.topk(probs, K, dim=1).indices.int()
+    if K > 1:
+        topi[2, 0] = -1   # a slot whose id is out of range gives nothing
+    dwp = torch.randn(T * K + T, nblk, generator=g)
+    sg = torch.rand(T, generator=g)
+    d = {k: v.to(DEV).contiguous() for k, v in dict(probs=probs, topi=topi, dwp=dwp, sg=sg).items()}
+    out = torch.full((T, ldl), 7.0, dtype=torch.bfloat16, device=DEV)
+    dt = torch.empty(T, K, device=DEV)
+    L.call("smel_route_bwd", L.ptr(d["dwp"]), nblk, None, L.ptr(d["probs"]), L.ptr(d["topi"]),
+           L.ptr(d["sg"]) if shared else None, None, 0, T, K, E, T * K, L.ptr(out), ldl, L.ptr(dt), None, L.stream())
+    p, w = probs.double(), dwp.double()
+    ok = topi >= 0
+    pk = p.gather(1, topi.clamp_min(0).long()) * ok
+    dtv = w[:T * K].sum(1).view(T, K)
+    S = pk.sum(1, keepdim=True)
+    dp = (dtv - (dtv * pk / S).sum(1, keepdim=True)) / S
+    dpe = torch.zeros(T, E, dtype=torch.float64).scatter_add_(1, topi.clamp_min(0).long(), dp * ok)
+    ref = torch.zeros(T, ldl, dtype=torch.float64)
+    ref[:, :E] = p * (dpe - (dp * pk).sum(1, keepdim=True))
+    if shared:
+        s = sg.double()
+        ref[:, E] = w[T * K:].sum(1) * s * (1 - s)
+    got = out.cpu().double()
+    scale = (p.amax(1, keepdim=True) * dp.abs().amax(1, keepdim=True))
+    assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-6 * (scale + 1)).all()
+    assert (dt.cpu().double() - dtv).abs().max() < 1e-5
