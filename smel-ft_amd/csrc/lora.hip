@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void lora_prep_kernel(PrepArgs pa) {
 // ext[row * ldx + 0:32] = bf16(scale * A_src[src(row)] . wcat^T) for the rows of SEL / SHARED tiles (one 32-wide
 // plane per call). Persistent: one block per CU first builds, in LDS, the list of this call's tiles that carry a LoRA
 // (the tile list holds each tile's kind; all tile entries are loaded at once, one memory latency), then takes the
-// (LoRA tile, 32-row slice) items blockIdx.x, blockIdx.x + gridDim.x, ... A slice's 8 waves take the 64-wide k-steps
+// (LoRA tile, slice of 32 or 16 rows) items blockIdx.x, blockIdx.x + gridDim.x, ... A slice's 8 waves take the 64-wide k-steps
 // j = w, w + 8, ..., issuing all loads of up to XPRE of their steps before the MFMAs (one memory latency per XPRE
 // steps, not one per step); the partial sums are added in wave order through LDS. The 16x16x32 MFMA layout lets four
 // lanes share a row, so each load takes 64 contiguous bytes of 16 rows (32 bytes of 32 rows with 32x32x16).
@@ -167,6 +167,88 @@ constexpr int XPRE = 4;
 constexpr int XT_PER = 8;              // tile entries each thread scans
 constexpr int XLT = 512 * XT_PER;      // tiles one call may hold
 
+// Rows m0 .. m0 + 16 NF - 1 of tile t (its kind in the fourth field) by a block of XW waves.
+template <int NF>
+SMEL_DEV void ext_slice(float* red, const int4& t, int m0, const uint16_t* __restrict__ A, int64_t lda, int64_t a_rows,
+                        int a_gather, const int32_t* __restrict__ order, int TK, int topk,
+                        const uint16_t* __restrict__ wsel, const uint16_t* __restrict__ wsh, int Kd, float ssel, float ssh,
+                        uint16_t* __restrict__ ext, int ldx) {
+  const int l = lane_id(), w = threadIdx.x >> 6, kq = l >> 4, li = l & 15;
+  const rsrc_t ra = make_rsrc(A, (uint64_t)a_rows * lda * 2);
+  const int nk = (Kd + 63) / 64;
+  const int kind = t.w >> 16, idx = t.w & 0xffff;
+  const int nrows = min(t.z - t.y, 128);
+  if (m0 >= nrows) return;   // uniform over the block
+  const uint16_t* wc = kind == SMEL_KIND_SEL ? wsel + (int64_t)idx * 32 * Kd : wsh;
+  const float scale = kind == SMEL_KIND_SEL ? ssel : ssh;
+  // v_mfma_f32_16x16x32_bf16: lane (kq, i) holds row 16 fr + i of the slice and factor row 16 fc + i, k = 32 s +
+  // 8 kq + [0, 8) of each 64-wide step, so a load takes 64 contiguous bytes of 16 rows (4 lanes per row)
+  const rsrc_t rb = make_rsrc(wc, (uint64_t)32 * Kd * 2);
+  uint32_t ao[NF], bo[2];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const int row = m0 + 16 * f + li;
+    ao[f] = OOB;
+    if (row < nrows) {
+      const int grow = t.y + row;
+      ao[f] = (uint32_t)(a_gather ? row_token(grow, order, TK, topk) : grow) * (uint32_t)lda * 2 + 16 * kq;
+    }
+  }
+#pragma unroll
+  for (int f = 0; f < 2; ++f) bo[f] = (uint32_t)(16 * f + li) * Kd * 2 + 16 * kq;
+  f32x4_t acc[NF][2];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) acc[f][0] = acc[f][1] = f32x4_t{};
+  for (int j0 = w; j0 < nk; j0 += XW * XPRE) {
+    u32x4_t av[XPRE][NF][2], bv[XPRE][2][2];   // [step][fragment][substep]
+    // the factor rows first: they do not wait for the row's token (a gathered row's address does)
+#pragma unroll
+    for (int p = 0; p < XPRE; ++p)
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) {
+        const int kk = (j0 + XW * p) * 64 + 32 * s2;
+        const bool ok = kk + 32 <= Kd;   // Kd % 32 == 0: a 32-wide substep is all in or all out
+#pragma unroll
+        for (int f = 0; f < 2; ++f) bv[p][f][s2] = ld16(rb, ok ? bo[f] + kk * 2 : OOB);
+      }
+#pragma unroll
+    for (int p = 0; p < XPRE; ++p)
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) {
+        const int kk = (j0 + XW * p) * 64 + 32 * s2;
+        const bool ok = kk + 32 <= Kd;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) av[p][f][s2] = ld16(ra, (ok && ao[f] != OOB) ? ao[f] + kk * 2 : OOB);
+      }
+    __builtin_amdgcn_sched_barrier(0);   // every load of the batch is issued before the first MFMA waits
+#pragma unroll
+    for (int p = 0; p < XPRE; ++p)
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+        for (int fr = 0; fr < NF; ++fr)
+#pragma unroll
+          for (int fc = 0; fc < 2; ++fc) acc[fr][fc] = mfma16x(av[p][fr][s2], bv[p][fc][s2], acc[fr][fc]);
+  }
+  // element q = 8 fr + 4 fc + r of a lane: row 16 fr + 4 kq + r of the slice, factor row (ext column) 16 fc + i
+#pragma unroll
+  for (int q = 0; q < 8 * NF; ++q)
+    red[(w * 8 * NF + q) * 64 + l] = acc[q >> 3][(q >> 2) & 1][q & 3];   // lane-contiguous
+  lds_barrier();
+  // each wave sums NF elements over the waves, in wave order, and stores those values
+  static_assert(XW == 8, "NF accumulator elements per wave");
+#pragma unroll
+  for (int rr = 0; rr < NF; ++rr) {
+    const int q = NF * w + rr;
+    float v = red[q * 64 + l];
+#pragma unroll
+    for (int ww = 1; ww < XW; ++ww) v += red[(ww * 8 * NF + q) * 64 + l];
+    const int orow = m0 + 16 * (q >> 3) + 4 * kq + (q & 3);
+    if (orow < nrows) ext[(int64_t)(t.y + orow) * ldx + 16 * ((q >> 2) & 1) + li] = f2bf(scale * v);
+  }
+  lds_barrier();   // red is reused by the next item
+}
+
 __global__ __launch_bounds__(512) void lora_ext_kernel(const int4* __restrict__ tiles, const int32_t* __restrict__ n_tiles,
                                                        const int32_t* __restrict__ gkind, const uint16_t* __restrict__ A,
                                                        int64_t lda, int64_t a_rows, int a_gather,
@@ -177,7 +259,7 @@ __global__ __launch_bounds__(512) void lora_ext_kernel(const int4* __restrict__ 
   __shared__ float red[XW * 64 * 16];
   __shared__ int4 lt[XLT];   // the call's LoRA tiles (whole entries: no second load per item)
   __shared__ int wcnt[XT_PER][XW];
-  const int tid = threadIdx.x, l = lane_id(), w = tid >> 6, kq = l >> 4, li = l & 15;
+  const int tid = threadIdx.x, l = lane_id(), w = tid >> 6;
   // ---- the LoRA tiles of this call, in tile order
   const int nt = min(n_tiles[0], max_tiles);
   bool fl[XT_PER];
@@ -215,81 +297,20 @@ __global__ __launch_bounds__(512) void lora_ext_kernel(const int4* __restrict__ 
   }
   __syncthreads();
   // ---- (tile, slice) items
-  const rsrc_t ra = make_rsrc(A, (uint64_t)a_rows * lda * 2);
-  const int nk = (Kd + 63) / 64;
-  for (int item = blockIdx.x; item < 4 * total; item += gridDim.x) {
+  // Slices of 32 rows, or of 16 where even those leave CUs idle (short sequences, dense MLPs): an item is bound by the
+  // bytes its CU takes in, the factor's and the rows'. Each row's sums are the same either way, bit for bit. Measured (32
+  // -> 16 rows): 1531 rows of 2816 and 2112 columns 14.5 -> 11.8 us a launch, the layer of 517 tokens (29 tiles) 11.9 ->
+  // 10.2, 12 experts of 256 rows 19.9 -> 16.5. From there on 16-row items would need a second turn of the CUs.
+  const bool half = 8 * total <= (int)gridDim.x;
+  const int items = (half ? 8 : 4) * total;
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
     // slice-major: tiles of one slice each (short lists, last tiles) would otherwise leave three blocks of four idle
     const int m = item / total;
     const int4 t = lt[item - m * total];
-    const int kind = t.w >> 16, idx = t.w & 0xffff;
-    const int nrows = min(t.z - t.y, 128);
-    if (m * 32 >= nrows) continue;   // uniform over the block
-    const uint16_t* wc = kind == SMEL_KIND_SEL ? wsel + (int64_t)idx * 32 * Kd : wsh;
-    const float scale = kind == SMEL_KIND_SEL ? ssel : ssh;
-    // v_mfma_f32_16x16x32_bf16: lane (kq, i) holds row 16 fr + i of the slice and factor row 16 fc + i, k = 32 s +
-    // 8 kq + [0, 8) of each 64-wide step, so a load takes 64 contiguous bytes of 16 rows (4 lanes per row)
-    const rsrc_t rb = make_rsrc(wc, (uint64_t)32 * Kd * 2);
-    uint32_t ao[2], bo[2];
-#pragma unroll
-    for (int f = 0; f < 2; ++f) {
-      const int row = m * 32 + 16 * f + li;
-      ao[f] = OOB;
-      if (row < nrows) {
-        const int grow = t.y + row;
-        ao[f] = (uint32_t)(a_gather ? row_token(grow, order, TK, topk) : grow) * (uint32_t)lda * 2 + 16 * kq;
-      }
-      bo[f] = (uint32_t)(16 * f + li) * Kd * 2 + 16 * kq;
-    }
-    f32x4_t acc[2][2];
-#pragma unroll
-    for (int f = 0; f < 2; ++f) acc[f][0] = acc[f][1] = f32x4_t{};
-    for (int j0 = w; j0 < nk; j0 += XW * XPRE) {
-      u32x4_t av[XPRE][2][2], bv[XPRE][2][2];   // [step][fragment][substep]
-      // the factor rows first: they do not wait for the row's token (a gathered row's address does)
-#pragma unroll
-      for (int p = 0; p < XPRE; ++p)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const int kk = (j0 + XW * p) * 64 + 32 * s2;
-          const bool ok = kk + 32 <= Kd;   // Kd % 32 == 0: a 32-wide substep is all in or all out
-#pragma unroll
-          for (int f = 0; f < 2; ++f) bv[p][f][s2] = ld16(rb, ok ? bo[f] + kk * 2 : OOB);
-        }
-#pragma unroll
-      for (int p = 0; p < XPRE; ++p)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const int kk = (j0 + XW * p) * 64 + 32 * s2;
-          const bool ok = kk + 32 <= Kd;
-#pragma unroll
-          for (int f = 0; f < 2; ++f) av[p][f][s2] = ld16(ra, (ok && ao[f] != OOB) ? ao[f] + kk * 2 : OOB);
-        }
-      __builtin_amdgcn_sched_barrier(0);   // every load of the batch is issued before the first MFMA waits
-#pragma unroll
-      for (int p = 0; p < XPRE; ++p)
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-          for (int fr = 0; fr < 2; ++fr)
-#pragma unroll
-            for (int fc = 0; fc < 2; ++fc) acc[fr][fc] = mfma16x(av[p][fr][s2], bv[p][fc][s2], acc[fr][fc]);
-    }
-    // element q = 8 fr + 4 fc + r of a lane: row 16 fr + 4 kq + r of the slice, factor row (ext column) 16 fc + i
-#pragma unroll
-    for (int q = 0; q < 16; ++q) red[(w * 16 + q) * 64 + l] = acc[q >> 3][(q >> 2) & 1][q & 3];   // lane-contiguous
-    lds_barrier();
-    // wave w sums elements 2w and 2w + 1 over the waves, in wave order, and stores those values
-    static_assert(2 * XW == 16, "two accumulator elements per wave");
-#pragma unroll
-    for (int rr = 0; rr < 2; ++rr) {
-      const int q = 2 * w + rr;
-      float v = red[q * 64 + l];
-#pragma unroll
-      for (int ww = 1; ww < XW; ++ww) v += red[(ww * 16 + q) * 64 + l];
-      const int orow = m * 32 + 16 * (q >> 3) + 4 * kq + (q & 3);
-      if (orow < nrows) ext[(int64_t)(t.y + orow) * ldx + 16 * ((q >> 2) & 1) + li] = f2bf(scale * v);
-    }
-    lds_barrier();   // red is reused by the next item
+    if (half)
+      ext_slice<1>(red, t, 16 * m, A, lda, a_rows, a_gather, order, TK, topk, wsel, wsh, Kd, ssel, ssh, ext, ldx);
+    else
+      ext_slice<2>(red, t, 32 * m, A, lda, a_rows, a_gather, order, TK, topk, wsel, wsh, Kd, ssel, ssh, ext, ldx);
   }
 }
 

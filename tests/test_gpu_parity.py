@@ -1112,3 +1112,25 @@ def test_route_bwd_against_fp64(E, K, shared):
     scale = (p.amax(1, keepdim=True) * dp.abs().amax(1, keepdim=True))
     assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-6 * (scale + 1)).all()
     assert (dt.cpu().double() - dtv).abs().max() < 1e-5
+
+
+@pytest.mark.parametrize("tiles,last", [(1, 1), (1, 16), (2, 17), (31, 33), (32, 128), (32, 15), (33, 1), (64, 127)])
+@pytest.mark.parametrize("Kd", [32, 2112])
+def test_lora_ext_slices(tiles, last, Kd):
+    """smel_lora_ext on lists that take 16-row slices (few tiles against the CUs) and 32-row slices, with ragged last
+    tiles: the fp32 product rounded once, and the rows past the last tile's left alone."""
+    L = _lib()
+    T = (tiles - 1) * 128 + last
+    g = torch.Generator().manual_seed(tiles + Kd)
+    x = torch.randn(T, Kd, generator=g).to(torch.bfloat16)
+    a = torch.randn(32, Kd, generator=g).to(torch.bfloat16)
+    t = torch.tensor([[0, 128 * i, min(T, 128 * i + 128), L.KIND_SHARED << 16] for i in range(tiles)], dtype=torch.int32)
+    xd, ad, td, nd = x.to(DEV), a.to(DEV), t.to(DEV), torch.tensor([tiles], dtype=torch.int32, device=DEV)
+    ext = torch.full((T + 40, 32), 7.0, dtype=torch.bfloat16, device=DEV)
+    L.call("smel_lora_ext", L.ptr(td), L.ptr(nd), tiles, None, L.ptr(xd), Kd, T, 0, None, 0, 1, None, L.ptr(ad), Kd, 1.0,
+           0.5, L.ptr(ext), 32, L.stream())
+    got = ext.cpu().double()
+    ref = 0.5 * x.double() @ a.double().t()
+    # one bf16 rounding, and Kd fp32 sums of products of standard normals
+    assert ((got[:T] - ref).abs() <= 2.0 ** -8 * ref.abs() + Kd * 2.0 ** -22).all()
+    assert (got[T:] == 7.0).all()
