@@ -50,6 +50,20 @@ SMEL_DEV uint32_t wave_max_u32(uint32_t v) {
 #undef SMEL_DPP_MAX
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
+// Inclusive sums over the lanes of a row of 16, and over the wave, by DPP moves
+SMEL_DEV int row_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  return v;
+}
+SMEL_DEV int wave_scan(int v) {
+  v = row_scan(v);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
 // v of lane k (k uniform), uniform
 SMEL_DEV int lane_get(int v, int k) { return __builtin_amdgcn_readlane(v, k); }
 SMEL_DEV float lane_get(float v, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k)); }

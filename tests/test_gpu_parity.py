@@ -544,6 +544,12 @@ def test_dispatch_bitexact(T, K, E, shared, kind):
             assert (cover == 1).all()
 
 
+@pytest.mark.parametrize("slots", [1023, 1025, 8 * 1024, 8 * 1024 + 1, 16 * 1024, 56 * 1024 + 1])
+def test_dispatch_histogram_groups(slots):
+    """The fused scan and scatter at the edges of the groups of eight histograms it reads (bit for bit)."""
+    test_dispatch_bitexact(slots, 1, 130, False, "uniform")
+
+
 def test_dispatch_flags_bad_ids():
     _say("dispatch bad ids")
     topi = torch.tensor([[0, 3], [9, 1], [2, -1]], dtype=torch.int64)
