@@ -358,3 +358,24 @@ def test_targets_outside_the_vocabulary(lm):
         lc, gc = rounded_full_ce(h, W, tgt, softcap)
         assert abs(l1.item() - lc.item()) < 1e-4 * abs(lc.item())
         assert (g1 - gc).norm() / gc.norm() < 1e-4
+
+
+@pytest.mark.parametrize("n", [1, 128, 129, 256, 257, 384, 385, 512])
+def test_tail_tile_edges(n):
+    """Row counts at the edges of the short last token tile (its own kernel): each row's loss and gradient equal those of
+    the row in a pass of whole tiles within the rounding of sums in another order, and the fp64 formula."""
+    g = torch.Generator().manual_seed(n)
+    H, V = 64, 700
+    h = torch.randn(n, H, generator=g).to(torch.bfloat16)
+    w = (torch.randn(V, H, generator=g) * 0.2).to(torch.bfloat16)
+    tgt = torch.randint(0, V, (n,), generator=g)
+    from smel.loss import LMHead, chunked_ce
+    hd = h.cuda().requires_grad_(True)
+    loss = chunked_ce(hd, LMHead(weight=w.cuda()), tgt.cuda(), n)
+    loss.backward()
+    h64 = h.double().requires_grad_(True)
+    ref = torch.nn.functional.cross_entropy(h64 @ w.double().t(), tgt)
+    ref.backward()
+    # logits are rounded to bf16 (2^-9 of values of about 1.6, V of them averaged), gradients once more
+    assert abs(loss.item() - ref.item()) < 1e-2 * abs(ref.item())
+    assert (hd.grad.cpu().double() - h64.grad).norm() < 1.5e-2 * h64.grad.norm()
