@@ -173,10 +173,10 @@ SMEL_DEV void row_offsets(uint32_t (&off)[VM], int w, int lane, int valid, uint3
 // The main loop over kbytes (a multiple of 16) of every row, in the k-step order rot, rot + 1, ..., nk - 1, 0, ...,
 // rot - 1: a tile's sum over k is then taken in an order fixed by `rot`, and tiles running side by side with different
 // rotations read different 128-byte columns of their rows at any moment (with row pitches that are multiples of
-// 2 KB, the rows of one column all fall on one L2 channel). `pre(kk, first)` runs before the operand loads of the
-// step after the current one are issued (kk = that step's k-step index; first: before the loop, for the first
-// step) and may issue its own loads: they retire before the next step's wait. `fix(n, kk, v)` transforms a B fragment
-// of tile column n in k-step kk as it leaves LDS.
+// 2 KB, the rows of one column all fall on one L2 channel). `pre(now, next)` runs at the start of k-step `now` (-1:
+// before the loop), before the operand loads of a later step are issued; `next` is the k-step that follows it (-1 after
+// the last). Loads it issues for `next` retire before that step's wait. `fix(n, v)` transforms a B fragment of tile
+// column n in k-step `now` as it leaves LDS.
 template <int DT, class R, int NB, class Pre, class Fix>
 SMEL_DEV void nt_loop(f32x16_t (&acc)[4][NB], uint8_t* smem, rsrc_t ra, const uint32_t (&aoff)[R::VM_A], rsrc_t rb,
                       const uint32_t (&boff)[R::VM_B], int kbytes, int rot, Pre&& pre, Fix&& fix) {
@@ -211,7 +211,7 @@ SMEL_DEV void nt_loop(f32x16_t (&acc)[4][NB], uint8_t* smem, rsrc_t ra, const ui
   uint32_t pcb[R::NSUB];
 #pragma unroll
   for (int s = 0; s < R::NSUB; ++s) pcb[s] = (uint32_t)r32 * KB + 16u * (uint32_t)R::phys(R::NSUB * h + s, r32);
-  pre(kstep(0), true);
+  pre(-1, kstep(0));
 #pragma unroll
   for (int s = 0; s < NST - 1; ++s)
     if (s < nk) issue(s);
@@ -223,9 +223,8 @@ SMEL_DEV void nt_loop(f32x16_t (&acc)[4][NB], uint8_t* smem, rsrc_t ra, const ui
     else wait_vm_lds<0>();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    if (j + 1 < nk) pre(kstep(j + 1), false);
+    pre(kstep(j), j + 1 < nk ? kstep(j + 1) : -1);
     if (j + NST - 1 < nk) issue(j + NST - 1);
-    const int kk = kstep(j);
     const uint8_t* A = smem + (j % NST) * R::STAGE + wm * 128 * KB;
     const uint8_t* B = smem + (j % NST) * R::STAGE + R::A_BYTES + wn * 32 * NB * KB;
     // fragments in two register sets: those of substep s + 1 are read from LDS before the MFMAs of substep s are
@@ -245,7 +244,7 @@ SMEL_DEV void nt_loop(f32x16_t (&acc)[4][NB], uint8_t* smem, rsrc_t ra, const ui
       __builtin_amdgcn_sched_barrier(0);
       u32x4_t bx[NB];
 #pragma unroll
-      for (int n = 0; n < NB; ++n) bx[n] = fix(n, kk, bf[cur][n]);
+      for (int n = 0; n < NB; ++n) bx[n] = fix(n, bf[cur][n]);
 #pragma unroll
       for (int m = 0; m < 4; ++m)
 #pragma unroll
@@ -302,8 +301,8 @@ SMEL_DEV void ce_logits_tile(const LogitsArgs& a, uint8_t* smem, int vt, int tt)
   for (int m = 0; m < 4; ++m)
 #pragma unroll
     for (int n = 0; n < NB; ++n) acc[m][n] = f32x16_t{};
-  nt_loop<DT, R, NB>(acc, smem, ra, aoff, rb, boff, kbytes, 5 * (int)(blockIdx.x / NXCD), [](int, bool) {},
-                    [](int, int, const u32x4_t& v) { return v; });
+  nt_loop<DT, R, NB>(acc, smem, ra, aoff, rb, boff, kbytes, 5 * (int)(blockIdx.x / NXCD), [](int, int) {},
+                    [](int, const u32x4_t& v) { return v; });
   __syncthreads();   // every wave is done with the operand ring: the epilogue may use the LDS
 
   // ---- epilogue. acc[m][n][r] = z at vocabulary column c0 + 32 m + 8 (r / 4) + 4 h + r % 4 of token row
@@ -460,7 +459,7 @@ SMEL_DEV void ce_grad_tile(const GradArgs& a, uint8_t* smem, int split, int tt, 
   const int a0 = ht * 256, b0 = tt * 256;
   const int a_valid = min(256, a.H - a0), b_valid = min(R::B_ROWS, a.n - b0);
   // Part s of the chunk in whole statistics windows, [nw s / splits, nw (s + 1) / splits): the loop below starts at a
-  // rotation and wraps to the part's first k-step, where the shifts of a window are only loaded if one begins.
+  // rotation and wraps to the part's first k-step, and a window's shifts are loaded where one begins.
   constexpr int STEPS_PER_WIN = WIN * ebytes<DT>() / R::KB;
   const int nw = (a.kbytes + STEPS_PER_WIN * R::KB - 1) / (STEPS_PER_WIN * R::KB);
   const int klo = (int)((int64_t)nw * split / a.splits) * STEPS_PER_WIN * R::KB;
@@ -484,33 +483,26 @@ SMEL_DEV void ce_grad_tile(const GradArgs& a, uint8_t* smem, int split, int tt, 
   // shifts of this lane's token rows: the window of k-step kk (of the chunk) is kk * KB / (WIN * E)
   const int kbase = klo / R::KB;
   const int tok0 = b0 + 32 * NB * wn + r32;
-  uint32_t sh_cur[NB], sh_next[NB];
-  auto load_sh = [&](int win, uint32_t (&dst)[NB]) {
+  typedef uint32_t shifts_t __attribute__((ext_vector_type(NB)));
+  auto load_sh = [&](int kg) {
+    shifts_t v;   // rows past n take the last one's (their terms read as zeros): no select waits for the loads
 #pragma unroll
-    for (int n = 0; n < NB; ++n) {
-      const int tok = tok0 + 32 * n;
-      dst[n] = tok < a.n ? (uint32_t)a.shift[(int64_t)win * a.ldn + tok] : (uint32_t)SHIFT_ZERO;
-    }
+    for (int n = 0; n < NB; ++n)
+      v[n] = a.shift[(int64_t)(kg / STEPS_PER_WIN) * a.ldn + min(tok0 + 32 * n, a.n - 1)];
+    return v;
   };
-  int cur_win = 0;
-  auto pre = [&](int kk, bool first) {   // the shifts of k-step kk's window, loaded where a window starts
-    const int kg = kbase + kk;
-    if (first) {
-      cur_win = kg / STEPS_PER_WIN;
-      load_sh(cur_win, sh_cur);
-    } else if (kg % STEPS_PER_WIN == 0) {
-      load_sh(kg / STEPS_PER_WIN, sh_next);
+  // sh_cur takes the current step's window before sh_next is loaded for the next step's: two steps in a row may each
+  // begin a window (a chunk's last window of a single k-step, then the wrap to the part's first).
+  shifts_t sh_cur{}, sh_next{};
+  auto pre = [&](int now, int next) {
+    if (now < 0) {
+      sh_next = load_sh(kbase + next);
+      return;
     }
+    sh_cur = sh_next;   // of the window last begun, `now`'s
+    if (next >= 0 && (kbase + next) % STEPS_PER_WIN == 0) sh_next = load_sh(kbase + next);
   };
-  auto fix = [&](int n, int kk, const u32x4_t& v) {
-    const int wj = (kbase + kk) / STEPS_PER_WIN;
-    if (n == 0 && wj != cur_win) {
-      cur_win = wj;
-#pragma unroll
-      for (int q = 0; q < NB; ++q) sh_cur[q] = sh_next[q];
-    }
-    return shift_chunk<DT>(v, sh_cur[n]);
-  };
+  auto fix = [&](int n, const u32x4_t& v) { return shift_chunk<DT>(v, sh_cur[n]); };
   nt_loop<DT, R, NB>(acc, smem, ra, aoff, rb, boff, kbytes, 5 * (int)(blockIdx.x / NXCD), pre, fix);
 
   // ---- epilogue: acc[m][n][r] = term of hidden column a0 + 128 wm + 32 m + 8 (r / 4) + 4 h + r % 4 and token

@@ -245,6 +245,64 @@ def test_int8_rows_and_transpose_bits(lm, V, H, dtype):
     assert torch.equal(wt2, wt)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("vc", [4097, 4160, 4128, 4161, 4224])
+def test_gradient_windows_keep_their_shifts(lm, vc, dtype):
+    """The gradient product against fp64 where neighbouring windows' shifts differ by up to twelve powers of two and the last
+    window holds one k-step (vc % 128 in 1..64 for 16-bit rows, 1..32 for fp32) or more, for every number of parts: a
+    block's k loop is rotated, so that it takes the last window's step right before the part's first."""
+    from smel import _lib as L
+    torch.manual_seed(vc)
+    n, H, p = 512, 2048, L.ptr
+    vcp = (vc + 255) // 256 * 256
+    P = torch.zeros(n, vcp, device="cuda")
+    P[:, :vc] = torch.rand(n, vc, device="cuda") * 0.5 + 0.5
+    WT = torch.zeros(H, vcp, device="cuda")
+    WT[:, :vc] = torch.randn(H, vc, device="cuda")
+    P, WT = P.to(dtype), WT.to(dtype)
+    nwin = vcp // 128
+    r = torch.ones(n, device="cuda")
+    shift = ((torch.arange(nwin, device="cuda") * 5 + 3) % 13).to(torch.uint8)   # the last window's is no part's first
+    sh = shift[:, None].expand(nwin, n).contiguous()
+    scale = torch.ldexp(torch.ones(nwin, device="cuda", dtype=torch.float64), -shift.int()).repeat_interleave(128)
+    ref = (P.double() * scale) @ WT.double().t()
+    for splits in range(1, 9):
+        acc = torch.empty(splits, n, H, device="cuda")
+        L.call("smel_ce_grad_split", p(WT), vcp, H, p(P), vcp, vc, p(sh), n, p(r), n, L_DT[dtype], 0, splits, p(acc),
+               L.stream())
+        # fp32 sums of about 4000 terms in some order: 2^-24 sqrt(4000) = 4e-6 of the result; the shifted terms stay exact
+        # (an fp16 term of 0.5 at the largest shift is 2^-13)
+        err = ((acc.double().sum(0) - ref).norm() / ref.norm()).item()
+        assert err < 1e-5, (splits, err)
+
+
+L_DT = {torch.bfloat16: 0, torch.float32: 1, torch.float16: 2}
+
+
+@pytest.mark.parametrize("tail_level", [6.0, -6.0])
+@pytest.mark.parametrize("V", [4097, 4160])
+def test_short_last_window_of_the_vocabulary(lm, V, tail_level):
+    """A vocabulary whose last window holds one k-step, its logits 6 above or below all others: the column of the gradient
+    that only those rows of the head reach, against fp64."""
+    loss_mod, _ = lm
+    torch.manual_seed(V)
+    n, H, m = 512, 2048, V - 4096
+    h = torch.randn(n, H, device="cuda") * 0.1
+    h[:, 0], h[:, 1] = 1.0, 0.0
+    W = torch.randn(V, H, device="cuda") * 0.02
+    W[:, :2] = 0.0
+    W[4096:, 0], W[4096:, 1] = tail_level, 4.0
+    h, W = h.bfloat16(), W.bfloat16()
+    tgt = torch.randint(0, 4096, (n,), device="cuda")
+    x = h.clone().requires_grad_(True)
+    loss_mod.chunked_ce(x, loss_mod.LMHead(weight=W), tgt, denom=1.0).backward()
+    p = torch.softmax(h.double() @ W.double().t(), -1)
+    ref = 4.0 * p[:, 4096:].sum(-1)
+    # a logit near 6 is rounded to bf16 steps of 2^-5 (half of one: 1.6 % of its term), the others' errors average out;
+    # terms and the gradient round once more (2^-9 each)
+    assert ((x.grad[:, 1].double() - ref).abs() <= 0.025 * ref).all()
+
+
 def test_two_half_form_equals_two_parts(lm):
     """smel_ce_grad / smel_ce_finish (two halves, the second one's accumulator alternating between two buffers) against
     smel_ce_grad_split / _finish_split with two parts, over three chunks: bitwise."""
