@@ -405,8 +405,9 @@ def _side_stream(dev, i: int) -> torch.cuda.Stream:
 
 class _Fork:
     """``with _Fork(dev, i) as st:`` launches on side stream i (handle ``st``) after the current stream's work so far;
-    ``join()`` makes the current (main) stream wait for everything launched there. Launches take the handle, so torch's
-    current stream is switched only while launches are timed (their events go to it)."""
+    ``join()`` makes the current (main) stream wait for everything launched there. Launches take the handle, and torch's
+    current stream is switched only while launches are timed (their events go to it): torch operations whose results the
+    launches read, and their buffers' allocation, come before the fork is made."""
 
     def __init__(self, dev, i: int, on: bool = None):
         if i in _SIDE_ON if on is None else on:
@@ -470,19 +471,21 @@ def _factor(lora, name: str):
     return p if p is not None else getattr(lora, name)
 
 
-def _lora_bufs(sets, H: int, planes: int, dev, st):
-    """The bf16 layouts of LoRA sets [(lora or None, n, I), ...] in one allocation and one launch (None for None)."""
+def _lora_bufs(sets, H: int, planes: int, dev):
+    """The buffers of the bf16 layouts of LoRA sets [(lora or None, n, I), ...] in one allocation (None for None), and
+    their factors as contiguous fp32 on the current stream; _prep_sets fills the layouts."""
     mem = L.Carve()
     bufs = [_LoRABufs(m, n, H, I, planes, mem) if m is not None else None for m, n, I in sets]
     if any(b is not None for b in bufs):
         mem.alloc(dev)
-        _prep_sets(bufs, st)
     return bufs
 
 
 def _prep_sets(bufs, st) -> None:
     """smel_lora_prep_sets: the bf16 layouts of one or two LoRA sets (same shapes and planes) in one launch."""
     bufs = [b for b in bufs if b is not None]
+    if not bufs:
+        return
     arr = (L.LoraSet * len(bufs))(*[b.lora_set() for b in bufs])
     b0 = bufs[0]
     L.call("smel_lora_prep_sets", arr, len(bufs), b0.planes, b0.H, b0.I, st, tag="smel_lora_prep")
@@ -517,13 +520,11 @@ def _token_tiles(T: int, E: int, dev):
     return cache[key]
 
 
-def _shared_lora_ext(x, K: int, E: int, bufs, dev, st):
+def _shared_lora_ext(x, K: int, E: int, lb_sh, ext, dev, st):
     """The gate_up LoRA projection of the fused shared expert's rows [TK, TK + T) (x in token order, no routing
-    needed) into a new ext buffer of all TK + T rows; the routed rows are filled after the dispatch."""
-    lb_ex, lb_sh = bufs
+    needed) into the ext buffer of all TK + T rows; the routed rows are filled after the dispatch."""
     T, H = x.shape
-    planes = (lb_ex or lb_sh).planes
-    ext = torch.empty(T * K + T, EXT * planes, dtype=torch.bfloat16, device=dev)
+    planes = lb_sh.planes
     return _lora_ext(_token_tiles(T, E, dev), x, H, T, 0, None, 0, 1, None, lb_sh, "a_gu", H, planes, ext, st,
                      row0=T * K)
 
@@ -801,15 +802,15 @@ def _expert_I(ex: LayerExperts) -> int:
     return (ex.frozen.dn["q"].shape[2] * 2) if isinstance(ex.frozen, Int4Experts) else ex.frozen.down.shape[2]
 
 
-def _prep_lora(ex: LayerExperts, lora_ex, lora_sh, with_shared: bool, H: int, dev, st):
-    """The bf16 LoRA layouts of the selected experts and the shared MLP (a lora_prep launch on stream ``st``), with the
-    gate_up planes both sets need."""
+def _prep_lora(ex: LayerExperts, lora_ex, lora_sh, with_shared: bool, H: int, dev):
+    """The bf16 LoRA layouts of the selected experts and the shared MLP (_lora_bufs), with the gate_up planes both sets
+    need."""
     I = _expert_I(ex)
     has_sel = ex.sel_ids is not None and len(ex._slot)
     use_ex = lora_ex if (lora_ex is not None and has_sel) else None
     use_sh = lora_sh if (lora_sh is not None and with_shared) else None
     planes = _lora_planes(use_ex, use_sh)
-    return _lora_bufs([(use_ex, len(ex._slot), I), (use_sh, 1, I)], H, planes, dev, st)
+    return _lora_bufs([(use_ex, len(ex._slot), I), (use_sh, 1, I)], H, planes, dev)
 
 
 def _tile_rows(TK: int, E: int, lora: bool) -> int:
@@ -844,9 +845,10 @@ def _forward_pipeline(x, ex: LayerExperts, K: int, topv, topi_ids, ids_i64: bool
     fz = ex.frozen
     merge = mt == M_TILE and _MERGE_SHORT and isinstance(fz, Int4Experts) and H % 64 == 0 and fz.fast_dq("gu")
     if prep is None:   # LoRA layouts on a side stream, overlapping the dispatch
+        bufs = _prep_lora(ex, lora_ex, lora_sh, shared is not None, H, dev)
         fork = _Fork(dev, 2)
-        with fork:
-            bufs = _prep_lora(ex, lora_ex, lora_sh, shared is not None, H, dev, fork.st)
+        with fork as sst:
+            _prep_sets(bufs, sst)
         prep = (fork, bufs)
     fork, (lb_ex, lb_sh) = prep
     any_lora = lb_ex is not None or lb_sh is not None
@@ -1152,12 +1154,15 @@ class _MoELayerFn(torch.autograd.Function):
         sgw = plan["shared"][2] if has_sh else None
         # LoRA layouts (and the shared rows' LoRA projection) overlap the router and the dispatch
         side_ext = _FWD_EXT_SIDE and fuse and plan["lora_sh"] is not None
-        fork = _Fork(dev, 2, on=True if side_ext else None)
+        bufs = _prep_lora(plan["ex"], plan["lora_ex"], plan["lora_sh"] if fuse else None, fuse, H, dev)
         ext_pre = None
+        if side_ext:
+            ext_pre = torch.empty(T * K + T, EXT * bufs[1].planes, dtype=torch.bfloat16, device=dev)
+        fork = _Fork(dev, 2, on=True if side_ext else None)
         with fork as sst:
-            bufs = _prep_lora(plan["ex"], plan["lora_ex"], plan["lora_sh"] if fuse else None, fuse, H, dev, sst)
-            if side_ext and bufs[1] is not None:
-                ext_pre = _shared_lora_ext(x, K, E, bufs, dev, sst)
+            _prep_sets(bufs, sst)
+            if ext_pre is not None:
+                _shared_lora_ext(x, K, E, bufs[1], ext_pre, dev, sst)
         L.call("smel_route_counted", L.ptr(x), L.ptr(plan["gate_w"]), L.ptr(sgw), T, H, E, K, L.ptr(probs),
                L.ptr(topv), L.ptr(topv32), L.ptr(topi), L.ptr(topi32), L.ptr(sgate), L.ptr(lg), L.ptr(dws), L.stream(),
                tag="smel_route")
@@ -1169,7 +1174,8 @@ class _MoELayerFn(torch.autograd.Function):
         if split:
             pgu, pdn, _, Is, pgu_t, pdn_t = plan["shared"]
             lsh = plan["lora_sh"]
-            lb_sh = _lora_bufs([(lsh, 1, Is)], H, _lora_planes(lsh), dev, L.stream())[0]
+            lb_sh = _lora_bufs([(lsh, 1, Is)], H, _lora_planes(lsh), dev)[0]
+            _prep_sets([lb_sh], L.stream())
             ysh, sv = _dense_mlp_fwd(x, pgu, pdn, lb_sh, "silu", tag="gemm_shared")
             shared_rows = (sgate, ysh)
             c.split = (sv, pgu_t, pdn_t, lsh, sgate)
@@ -1427,7 +1433,8 @@ class _MLPFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w_gu2, w_dn2, lora, act_name, *leaves):
-        lb = _lora_bufs([(lora, 1, w_dn2[0].C)], x.shape[1], _lora_planes(lora), x.device, L.stream())[0]
+        lb = _lora_bufs([(lora, 1, w_dn2[0].C)], x.shape[1], _lora_planes(lora), x.device)[0]
+        _prep_sets([lb], L.stream())
         y, sv = _dense_mlp_fwd(x, w_gu2[0], w_dn2[0], lb, act_name)
         ctx.sv, ctx.w, ctx.lora, ctx.act_name = sv, (w_gu2[1], w_dn2[1]), lora, act_name
         return y

@@ -686,6 +686,34 @@ def test_shared_lora_rows_on_side_stream_bitwise(name, monkeypatch):
         assert torch.equal(a["grads"][k], b["grads"][k]), k
 
 
+@pytest.mark.parametrize("ext_side", [False, True])
+@pytest.mark.parametrize("form", ["bf16", "strided"])
+def test_converted_factors_on_side_stream_bitwise(form, ext_side, monkeypatch):
+    """LoRA factors that are converted on the way in (bf16, or fp32 that is not contiguous) reach the layouts launched on
+    side stream 2 (with the shared rows' projection, or alone): bitwise the result of everything on one stream."""
+    import smel.moe as M
+    _say(f"converted factors on the side stream {form} {ext_side}")
+    to_layer = to_device_layer
+
+    def converted(*args):
+        W, ex, lora = to_layer(*args)
+        for m in (lora.experts, lora.shared):
+            for p in m.parameters():
+                p.data = p.data.bfloat16() if form == "bf16" else p.data.transpose(-1, -2).contiguous().transpose(-1, -2)
+        return W, ex, lora
+
+    monkeypatch.setitem(globals(), "to_device_layer", converted)
+    b = run_layer("r16", seed=9)
+    monkeypatch.setattr(M, "_FWD_EXT_SIDE", ext_side)
+    monkeypatch.setattr(M, "_SIDE_ON", frozenset((0, 1, 2)))
+    for _ in range(4):
+        a = run_layer("r16", seed=9)
+        assert torch.equal(a["y"].view(torch.int16), b["y"].view(torch.int16))
+        assert torch.equal(a["dx"].view(torch.int16), b["dx"].view(torch.int16))
+        for k in b["grads"]:
+            assert torch.equal(a["grads"][k], b["grads"][k]), k
+
+
 @pytest.mark.parametrize("name", ["r16", "r32", "shared_wide", "r24_mixed"])
 def test_bwd_lora_rows_against_projection(name, monkeypatch):
     """The gate_up backward's LoRA rows from the down backward's per-column-block partials (smel_gmm_bwd_lr +

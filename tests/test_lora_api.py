@@ -6,6 +6,7 @@ import json
 import math
 import os
 
+import pytest
 import torch
 
 from smel.lora import BlockLoRA, ExpertsLoRA, LayerLoRA, MLPLoRA, lora_gate_up, lora_linear
@@ -167,3 +168,45 @@ def test_layer_reads_factors_of_any_lora_object():
             return 2 * w
     torch.nn.utils.parametrize.register_parametrization(sh, "B_up", Double())
     assert [torch.equal(a, getattr(sh, n)) for a, n in zip(_lora_leaves(sh), _LORA_NAMES)] == [True] * 6
+
+
+class _Stop(Exception):
+    pass
+
+
+@pytest.mark.parametrize("entry", ["layer", "routed"])
+@pytest.mark.parametrize("form", ["bf16", "strided"])
+def test_factors_are_converted_before_the_side_stream_waits(entry, form, monkeypatch):
+    """A side stream waits for the current stream where its fork is made, so a factor's conversion to contiguous fp32 (on
+    the current stream) has to be queued before that."""
+    import smel.moe as M
+    E, H, I, K, T = 4, 64, 32, 2, 3
+    ids = [0, 2]
+    lora = ExpertsLoRA(ids, H, I, r=4)
+    for p in lora.parameters():
+        p.data = p.data.bfloat16() if form == "bf16" else p.data.transpose(-1, -2).contiguous().transpose(-1, -2)
+    bf = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)
+    ex = M.LayerExperts(M.BF16Experts(bf(E, 2 * I, H), bf(E, H, I)), ids, bf(2, 2 * I, H), bf(2, H, I))
+    made = []
+    init = M._LoRABufs.__init__
+
+    def record(self, *a, **k):
+        init(self, *a, **k)
+        made.append(self)
+
+    def fork(*a, **k):
+        assert len(made) == 1
+        assert all(f.dtype == torch.float32 and f.is_contiguous() for f in made[0].factors)
+        raise _Stop
+
+    monkeypatch.setattr(M._LoRABufs, "__init__", record)
+    monkeypatch.setattr(M, "_Fork", fork)
+    monkeypatch.setattr(M.L, "stream", lambda: 0)
+    with pytest.raises(_Stop):
+        if entry == "layer":
+            plan = {"ex": ex, "top_k": K, "shared": None, "split_shared": False, "gate_w": bf(E, H), "lora_ex": lora,
+                    "lora_sh": None, "need_grad": False}
+            M._MoELayerFn.forward(None, bf(T, H), plan, None)
+        else:
+            M._forward_pipeline(bf(T, H), ex, K, torch.ones(T, K), torch.zeros(T, K, dtype=torch.int32), False, None, lora,
+                                None, False, M._Ctx())
