@@ -318,28 +318,41 @@ def _bf16(t: torch.Tensor) -> torch.Tensor:
     return t.contiguous()
 
 
-_dense_tiles_cache = {}
+_DENSE_HEIGHTS = (M_TILE, 96, 64, M_SHORT)   # rows per tile of a dense group's lists
+_dense_cache = {}
+
+
+def _dense_entry(T: int, device):
+    """What the launches over one dense group of T rows (group 0) read: ({rows per tile: tile list}, two zeros). All lists
+    of a row count are made together, in one buffer (about T bytes) and one copy, so that neither a new row count nor the
+    first backward after a forward costs more than that."""
+    key = (T, str(device))
+    got = _dense_cache.get(key)
+    if got is None:
+        kind = L.KIND_SHARED << 16
+        v, at = [kind, 0, 0, 0], {}   # the group's kind and the zeros, the lists' lengths, then the lists
+        v += [-(-T // h) for h in _DENSE_HEIGHTS]
+        for h in _DENSE_HEIGHTS:
+            n = -(-T // h)
+            t = [0] * (4 * n)
+            t[1::4], t[2::4], t[3::4] = range(0, T, h), [*range(h, T, h), T][:n], [kind] * n
+            at[h] = len(v)
+            v += t or [0] * 4
+        b = torch.tensor(v, dtype=torch.int32).to(device)
+        lists = {h: (b[at[h]:], b[4 + i:5 + i], -(-T // h), b[:1]) for i, h in enumerate(_DENSE_HEIGHTS)}
+        got = _dense_cache[key] = (lists, b[1:3])
+    return got
 
 
 def _dense_tiles(T: int, device, rows: int = M_TILE):
-    """Tile list of one dense group of T rows (group 0) in tiles of ``rows`` rows, for the router-backward GEMM and the
-    dense MLP."""
-    key = (T, str(device), rows)
-    if key not in _dense_tiles_cache:
-        n = (T + rows - 1) // rows
-        t = torch.zeros(max(n, 1), 4, dtype=torch.int32)
-        for i in range(n):
-            t[i, 0], t[i, 1], t[i, 2], t[i, 3] = 0, i * rows, min(T, (i + 1) * rows), L.KIND_SHARED << 16
-        _dense_tiles_cache[key] = (t.reshape(-1).to(device), torch.tensor([n], dtype=torch.int32, device=device),
-                                   n, torch.tensor([L.KIND_SHARED << 16], dtype=torch.int32, device=device),
-                                   torch.zeros(2, dtype=torch.int32).to(device))
-    return _dense_tiles_cache[key][:4]
+    """Tile list of one dense group of T rows in tiles of ``rows`` rows, for the router-backward GEMM and the dense MLP:
+    (tiles, n_tiles, max_tiles, gkind)."""
+    return _dense_entry(T, device)[0][rows]
 
 
 def _dense_zeros(T: int, device) -> torch.Tensor:
-    """Two zeros kept with the tile list of the same rows."""
-    _dense_tiles(T, device)
-    return _dense_tiles_cache[(T, str(device), M_TILE)][4]
+    """Two zeros kept with the tile lists of the same rows."""
+    return _dense_entry(T, device)[1]
 
 
 def _router_ext_weight(gate_w: torch.Tensor, sg_w: torch.Tensor | None, store: dict | None = None) -> PackedW:
@@ -1299,7 +1312,7 @@ class _DenseSaved:
 
 
 # (rows of a tile, a lone block's time against the 128-row tile's forward and backward, blocks that share a CU)
-_DENSE_TILES = ((128, 1.0, 1.0, 2), (96, 0.86, 0.86, 2), (64, 0.73, 0.73, 2), (M_SHORT, 0.75, 0.64, 4))
+_DENSE_TILES = tuple(zip(_DENSE_HEIGHTS, (1.0, 0.86, 0.73, 0.75), (1.0, 0.86, 0.73, 0.64), (2, 2, 2, 4)))
 
 
 def _dense_rows(T: int, nblk: int, fwd: bool) -> int:

@@ -210,3 +210,23 @@ def test_factors_are_converted_before_the_side_stream_waits(entry, form, monkeyp
         else:
             M._forward_pipeline(bf(T, H), ex, K, torch.ones(T, K), torch.zeros(T, K, dtype=torch.int32), False, None, lora,
                                 None, False, M._Ctx())
+
+
+@pytest.mark.parametrize("T", [0, 1, 31, 32, 33, 64, 96, 97, 128, 129, 517, 1531, 4096])
+def test_dense_tile_lists(T, monkeypatch):
+    """The tile lists of a dense group of T rows: every height's tiles are [0, first row, end row, kind] in row order, and
+    all of a row count come from one copy to the device."""
+    import smel.moe as M
+    monkeypatch.setattr(M, "_dense_cache", {})
+    copies = []
+    to = torch.Tensor.to
+    monkeypatch.setattr(torch.Tensor, "to", lambda self, *a, **k: copies.append(1) or to(self, *a, **k))
+    kind = M.L.KIND_SHARED << 16
+    for rows in M._DENSE_HEIGHTS:
+        tiles, n_tiles, n, gk = M._dense_tiles(T, torch.device("cpu"), rows)
+        want = [[0, r, min(T, r + rows), kind] for r in range(0, T, rows)]
+        assert n == len(want) == n_tiles.item() and gk.tolist() == [kind]
+        assert tiles[:4 * n].reshape(n, 4).tolist() == want
+        assert tiles.numel() >= 4 and tiles.storage_offset() % 4 == 0   # read as 16-byte entries
+    assert M._dense_zeros(T, torch.device("cpu")).tolist() == [0, 0]
+    assert len(copies) == 1
