@@ -1,7 +1,11 @@
 /* C-ABI of the fp32 path of the MoE layer: the reference run on fp32 tensors (its fp32 models; _gmm falls to its
  * per-group matmul loop for any non-bf16 tensor, smel/moe.py:58-72, and the tests compare at 1e-5,
- * tests/test_moe.py:10-36). Every product is an fp32 MFMA (v_mfma_f32_16x16x4_f32) with fp32 accumulation; int4 banks
- * are dequantized to fp32 inside the GEMM (the reference's fp32 Int4Experts: w = q s + z in fp32, smel/quant.py:51-84).
+ * tests/test_moe.py:10-36). Products are fp32, sums fp32 (v_mfma_f32_16x16x4_f32); int4 banks are dequantized to fp32
+ * inside the GEMM (the reference's fp32 Int4Experts: w = q s + z in fp32, smel/quant.py:51-84). int4 tiles with groups
+ * of a multiple of 32 over K of a multiple of 32 (16-byte aligned rows, launches that fill the GPU) form the same
+ * products from bf16 parts that add up to the fp32 values exactly (v_mfma_f32_16x16x32_bf16), with fp32 sums of every
+ * 32 of them; rows with values whose parts would leave bf16's range (below 2^-72, infinities, NaN) and weights that
+ * are no sum of two bf16 values take the fp32 instruction.
  * Rows are in the sorted row space of smel_dispatch (include/smel_moe.h): the tile list {group, row0, row1, gk} and
  * the group kinds are the same as the bf16 GEMMs'. All pointers are device pointers; all matrices are row-major fp32
  * unless stated. Results are deterministic (fixed summation order, no atomics). Entry points return 0 or an error

@@ -1,6 +1,7 @@
 // fp32 path of the MoE layer (include/smel_f32.h): the reference's layer on fp32 tensors, whose _gmm falls to a
-// per-group matmul loop for any non-bf16 tensor (smel/moe.py:58-72). Grouped GEMMs on v_mfma_f32_16x16x4_f32 over the
-// same tile lists and group kinds as the bf16 GEMMs, LoRA weight gradients as row-group reductions on the same MFMA,
+// per-group matmul loop for any non-bf16 tensor (smel/moe.py:58-72). Grouped GEMMs on v_mfma_f32_16x16x4_f32 (int4 tiles
+// also as exact bf16 parts on v_mfma_f32_16x16x32_bf16, Split below) over the same tile lists and group kinds as the bf16
+// GEMMs, LoRA weight gradients as row-group reductions on the same MFMA,
 // and the fp32 element-wise steps around them (gather, act-gate, combine, dX reduce, router selection and backward,
 // the Gemma router input, the shared-expert gate). Everything sums in a fixed order: no atomics.
 #include <math.h>
@@ -163,12 +164,15 @@ struct Gemm {
   static_assert(RB * FK == 8 * 256 && NT * FK == 16 * 256, "staging split");
   static_assert(KS == 1 || KS * RB * (NT + 4) <= LDS_FLOATS, "reduction buffer");
 
-  // NRF: the 16-row slices computed (those of the tile's rows; the others' rows are zeros in LDS)
+  // NRF: the 16-row slices computed (those of the tile's rows; the others' rows are zeros in LDS); only: the rows stored
+  // (bit r: row mr0 + r)
   template <int MODE, int NRF>
   SMEL_DEV static void tile(float* __restrict__ lds, const GemmArgs& G, const WMat& m, int N, int K, int n0, int mr0,
-                            int mr1) {
+                            int mr1, uint64_t only = ~0ull) {
     constexpr bool INT4 = MODE == W_INT4 || MODE == W_INT4R;
-    const int t = threadIdx.x, l = lane_id(), wv = t >> 6, i = l & 15, kq = l >> 4;
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));   // the addresses made from it belong to this tile: kept over a loop of tiles they would spill
+    const int l = t & 63, wv = t >> 6, i = l & 15, kq = l >> 4;
     const int wn = wv % NWN, wk = wv / NWN;
     const int nk = (K + FK - 1) / FK;
     // load coordinates: A row t / (FK / 8), 8 k; W: a run of 16 along the matrix's rows
@@ -298,7 +302,7 @@ struct Gemm {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int row = mr0 + 16 * rf + 4 * kq + r;
-          if (row >= mr1) continue;
+          if (row >= mr1 || !(only >> (row - mr0) & 1)) continue;
           float* const p = G.C + (int64_t)row * G.ldc;
 #pragma unroll
           for (int f = 0; f < NF; ++f) {
@@ -318,7 +322,7 @@ struct Gemm {
       for (int e = t; e < RB * NT; e += 256) {
         const int rr = e / NT, cc = e % NT;
         const int row = mr0 + rr, col = n0 + cc;
-        if (row >= mr1 || col >= N) continue;   // rows past NRF slices are past mr1
+        if (row >= mr1 || col >= N || !(only >> rr & 1)) continue;   // rows past NRF slices are past mr1
         float v = lds[rr * PR + cc];
 #pragma unroll
         for (int q = 1; q < KS; ++q) v += lds[(q * RB + rr) * PR + cc];
@@ -331,21 +335,29 @@ struct Gemm {
 };
 
 // ---------------------------------------------------------------------------------------------- int4 tiles on bf16 MFMAs
-// fp32 products of int4 tiles from 16-bit matrix instructions without losing bits: every fp32 value is the sum of three
-// bf16 values (x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1); the differences are exact and 3 x 8 bits hold
-// all 24), a bf16 x bf16 product is exact in fp32, and of the nine products the three below 2^-25 of the largest are
-// left out: x w = x0 w0 + (x0 w1 + x1 w0) + (x0 w2 + x1 w1 + x2 w0). Six v_mfma_f32_16x16x32_bf16 take 96 cycles for the
-// 32 k that eight v_mfma_f32_16x16x4_f32 take 256 for, and they round the sum six times instead of eight to 32 times, so
-// the error against 64 bits is smaller than the fp32 instruction's. Weights rounded to bf16 (RBF) are one value: three products.
-// Values that do not split (infinities, NaN, numbers that round up to infinity) leave a non-finite sum: such a tile is
-// computed again by the fp32 instruction, which decides what the result is.
-// What bounds it: the VALU work of dequant and splitting, about 8 instructions per weight and pass (with every load of
-// the loop out of range 255 of gate_up's 315 us remain; a cheaper-looking split by two-term dot products, two
-// instructions less per value, took the same time). So no weight is split twice in a pass of up to 48 rows: a wave takes
-// all 128 columns of the block for its quarter of the k-steps (every fourth step of 32), straight from global memory into
+// fp32 products of int4 tiles from 16-bit matrix instructions without losing bits: an fp32 value is the sum of three bf16
+// values (x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1); the differences are exact and 3 x 8 bits hold all 24),
+// a weight q s + z of a group whose scale and zero are of similar size the sum of two (its bits lie in 16 places, see
+// splits()), and a bf16 x bf16 product is exact in fp32: x w = x0 w0 + (x0 w1 + x1 w0 + x1 w1 + x2 w0 + x2 w1), all six
+// products kept. Weights rounded to bf16 (RBF) are one value: three products. Six v_mfma_f32_16x16x32_bf16 take 96 cycles
+// for the 32 k that eight v_mfma_f32_16x16x4_f32 take 256 for.
+// The sums: that instruction loses up to a unit in the last place of what it adds to (an fp32 addition half of one), so
+// no sum runs through it from step to step: per 32 k the products x0 w0 and the small ones each start from zero, and fp32
+// additions bring them together and onto the running sum. Error against 64 bits relative to sum |x w| (1024 to 2048
+// columns, all int4; fp32 instruction -> here), largest / rms: one non-zero term 5.96e-8 / 2.51e-8 -> 5.98e-8 / 2.51e-8,
+// two terms 1.17e-7 / 2.59e-8 -> 1.17e-7 / 3.05e-8 (each rounded before they meet, as in any sum by parts), eight 2.4e-7
+// / 2.7e-8 -> 2.2e-7 / 2.8e-8, 64 3.2e-7 / 2.8e-8 -> 1.3e-7 / 1.5e-8, full rows 3.6e-7 / 2.8e-8 -> 3.4e-8 / 3.7e-9.
+// What the parts cannot hold is computed by the fp32 instruction, in rows of their own (a row's bits depend on that row and
+// the weights alone): rows with a non-zero value below 2^-72 (the parts of smaller values, or their products with the
+// smallest weights, come near the end of the exponent range) and rows with an infinite or NaN sum (infinities, NaN,
+// numbers that round up to infinity); all rows where a weight of the block is no sum of two.
+// What bounds it: the VALU work of dequant and splitting, about 6 instructions per weight and pass, and 6 per row value
+// (48 rows: 888 for 144 MFMAs a step). So no weight is split twice in a pass of up to 48 rows: a wave takes all 128
+// columns of the block for its quarter of the k-steps (every fourth step of 32), straight from global memory into
 // registers without a barrier, and the waves' sums are added through LDS in wave order. Only the block's scales and
-// zeros (packed) wait in LDS. Measured (1021 tokens top-8 of 256 experts, H 2048, I 512; fp32 instruction -> split):
-// gate_up 450 -> 310 us, down 243 -> 186, down backward 276 -> 183, gate_up backward 496 -> 321.
+// zeros (packed) wait in LDS. Measured (8168 rows over 256 int4 experts, H 2048, I 512; the six largest of nine products
+// of three-part weights, summed in the instruction -> here): gate_up 309 -> 302 us, down 166 -> 166, down backward 158 ->
+// 146, gate_up backward 288 -> 272 (the fp32 instruction: 445, 240, 274, 485).
 // x and y as three bf16 values each, packed (the differences are exact).
 SMEL_DEV void split3(float x, float y, uint32_t& p0, uint32_t& p1, uint32_t& p2) {
   p0 = pack2bf(x, y);
@@ -376,10 +388,25 @@ struct Split {
     return K % 32 == 0 && m.group % 32 == 0 && (int64_t)panel_groups(m, N, n0) * (TRANS ? K : NT) <= GM::LDS_FLOATS;
   }
 
+  // A weight q s + z is two bf16 values exactly when all its bits lie in 16 consecutive places: the last bits of s and z
+  // are 2^(exponent - 7) each, the weight is below 2^(1 + max(exponent of s + 4, exponent of z)). Zero or exponents of at
+  // least -40 (what is left of a weight after cancellation is then a normal bf16 value), finite.
+  template <bool RBF>
+  SMEL_DEV static bool splits(uint32_t s, uint32_t z) {
+    const int es = s >> 7 & 0xff, ez = z >> 7 & 0xff;
+    const bool zs = (s & 0x7fffu) == 0, zz = (z & 0x7fffu) == 0;
+    const bool in = (zs | ((unsigned)(es - (127 - 40)) < 168u)) & (zz | ((unsigned)(ez - (127 - 40)) < 168u));
+    return in & (RBF | zs | zz | ((unsigned)(ez - es + 4) <= 12u));
+  }
+
+  // Returns the rows that are still to be computed (bit r: row mr0 + r), the same for the whole block.
   template <int NRF, bool RBF>
-  SMEL_DEV static void tile(float* __restrict__ lds, const GemmArgs& G, const WMat& m, int N, int K, int n0, int mr0,
-                            int mr1) {
-    const int t = threadIdx.x, l = lane_id(), i = l & 15, kq = l >> 4;
+  SMEL_DEV static uint64_t tile(float* __restrict__ lds, const GemmArgs& G, const WMat& m, int N, int K, int n0, int mr0,
+                                int mr1) {
+    __shared__ uint32_t again[2];   // rows to compute again (48 bits)
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));   // as in Gemm
+    const int l = t & 63, i = l & 15, kq = l >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int nk = K / 32, nfw = min(NT, N - n0);
     const int half = m.C >> 1, WR = TRANS ? K : N;
@@ -396,28 +423,34 @@ struct Split {
                               : (uint32_t)((n0 + 8 * i) * half + 4 * kq);
     u32x4_t araw[NRF][2];   // 8 k of the lane's row per 16-row slice
     uint32_t q[8], qn[8];   // 64 nibbles
+    // OOB plus any offset inside a matrix stays out of range; steps past the last one load it again
     auto load_a = [&](int step) {
+      uint32_t at = 128u * min(step, nk - 1);
+      asm("" : "+s"(at));
 #pragma unroll
       for (int rf = 0; rf < NRF; ++rf)
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-          araw[rf][h] = ld16(ra, step < nk && arow[rf] != OOB ? arow[rf] + 128u * step + 16 * h : OOB);
+        for (int h = 0; h < 2; ++h) araw[rf][h] = ld16(ra, arow[rf] + at + 16 * h);
     };
     auto load_q = [&](uint32_t* o, int step) {
+      const uint32_t at = (uint32_t)min(step, nk - 1) * (TRANS ? 32u * half : 16u);
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        o[j] = ld4(rw, step < nk && wb != OOB
-                           ? wb + (uint32_t)(j * half) + (TRANS ? (uint32_t)(32 * step * half) : 16u * step)
-                           : OOB);
+      for (int j = 0; j < 8; ++j) {
+        uint32_t aj = at + (uint32_t)(j * half);
+        asm("" : "+s"(aj));   // one vector add per load, not eight addresses kept over the loop
+        o[j] = ld4(rw, wb + aj);
+      }
     };
     load_a(wv);
     load_q(q, wv);
+    if (t < 2) again[t] = 0;
     // scale | zero << 16 of the block's weights: [group][column] or, TRANS, [group][k]
     uint32_t* const P = reinterpret_cast<uint32_t*>(lds);
     const int ng = panel_groups(m, N, n0), g0 = TRANS ? n0 / m.group : 0;
     const int outer = TRANS ? K : NT;
+    const int gs = ng <= 1 ? 0 : 32 - __builtin_clz((unsigned)(ng - 1));   // consecutive threads: a row's groups
+    uint32_t range = 0, apart = 0;
     {
-      const int gs = ng <= 1 ? 0 : 32 - __builtin_clz((unsigned)(ng - 1));   // consecutive threads: a row's groups
       const rsrc_t rs = make_rsrc(m.s, (uint64_t)WR * m.gpr * 2), rz = make_rsrc(m.z, (uint64_t)WR * m.gpr * 2);
 #pragma unroll 8
       for (int e = t; e < outer << gs; e += 256) {
@@ -425,31 +458,35 @@ struct Split {
         const uint32_t off = 2u * (uint32_t)((TRANS ? o : n0 + o) * m.gpr + g0 + g);
         const uint32_t s = ld2(rs, off), z = ld2(rz, off);
         if (g < ng) P[g * outer + o] = s | (z << 16);
+        // the common case of splits() without its exceptions: exponents in range and apart by no more than it allows
+        const uint32_t s1 = (s & 0x7fffu) - (87u << 7), z1 = (z & 0x7fffu) - (87u << 7);
+        range = max(range, max(s1, z1));
+        if constexpr (!RBF) apart = max(apart, z1 - s1 + 512u);
       }
     }
     lds_barrier();
     const uint32_t* const pl = P + (TRANS ? ((n0 + min(8 * i, nfw - 1)) / m.group - g0) * K + 8 * kq : 8 * i);
     f32v4 acc[NRF][NF] = {};
+    uint32_t least[NRF];   // smallest of 2 |bits| - 1 (zeros wrap to the largest)
+#pragma unroll
+    for (int rf = 0; rf < NRF; ++rf) least[rf] = ~0u;
     for (int step = wv; step < nk; step += 4) {   // no barrier: each wave its own steps
       u32x4_t a0[NRF], a1[NRF], a2[NRF];
 #pragma unroll
       for (int rf = 0; rf < NRF; ++rf)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+          const uint32_t x = araw[rf][j >> 1][2 * (j & 1)], y = araw[rf][j >> 1][2 * (j & 1) + 1];
+          least[rf] = min(least[rf], min(2 * x - 1, 2 * y - 1));
           uint32_t p0, p1, p2;
-          split3(__uint_as_float(araw[rf][j >> 1][2 * (j & 1)]), __uint_as_float(araw[rf][j >> 1][2 * (j & 1) + 1]), p0,
-                 p1, p2);
+          split3(__uint_as_float(x), __uint_as_float(y), p0, p1, p2);
           a0[rf][j] = p0, a1[rf][j] = p1, a2[rf][j] = p2;
         }
-      __builtin_amdgcn_sched_barrier(0);
-      load_a(step + 4);
-      load_q(qn, step + 4);
-      __builtin_amdgcn_sched_barrier(0);
       const uint32_t* const sp = pl + (TRANS ? 32 * step : 32 * step / m.group * NT);
       const u32x4_t z0 = *reinterpret_cast<const u32x4_t*>(sp), z1 = *reinterpret_cast<const u32x4_t*>(sp + 4);
       // TRANS: nibble f of every row's word; the even ones first, then the odd ones shifted into their bytes
       uint32_t nib8[8];
-      u32x4_t b[2][3];
+      u32x4_t b[2][2];
       auto weights = [&](int f, u32x4_t* o) {   // fragment f's 8 weights, split
         float w[8];
 #pragma unroll
@@ -463,10 +500,9 @@ struct Split {
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          uint32_t p0, p1 = 0, p2 = 0;
-          if constexpr (RBF) p0 = pack2bf(w[2 * j], w[2 * j + 1]);
-          else split3(w[2 * j], w[2 * j + 1], p0, p1, p2);
-          o[0][j] = p0, o[1][j] = p1, o[2][j] = p2;
+          const uint32_t p0 = pack2bf(w[2 * j], w[2 * j + 1]);
+          o[0][j] = p0;
+          if constexpr (!RBF) o[1][j] = pack2bf(w[2 * j] - bf_lo(p0), w[2 * j + 1] - bf_hi(p0));
         }
       };
       // fragments in the order 0 2 4 6 1 3 5 7; the next one's weights are made between this one's MFMAs, and the fence
@@ -476,37 +512,65 @@ struct Split {
       for (int o = 0; o < NF; ++o) {
         const int f = o < 4 ? 2 * o : 2 * o - 7, fn = o + 1 < 4 ? 2 * o + 2 : 2 * o - 5;
         __builtin_amdgcn_sched_barrier(0);
-        auto mm = [&](const u32x4_t* a, const u32x4_t& bb) {
-#pragma unroll
-          for (int rf = 0; rf < NRF; ++rf) acc[rf][f] = mfma32b(a[rf], bb, acc[rf][f]);
-        };
+        if (o == 4) load_q(qn, step + 4);
+        if (o == 5) load_a(step + 4);
+        f32v4 big[NRF], small[NRF];   // a0 w0, and the other products, the smallest first
         const u32x4_t* const c = b[o & 1];
-        mm(a2, c[0]);   // the small products first
-        if constexpr (!RBF) {
-          mm(a1, c[1]);
-          mm(a0, c[2]);
-        }
-        mm(a1, c[0]);
-        if constexpr (!RBF) mm(a0, c[1]);
-        mm(a0, c[0]);
+        auto mm = [&](f32v4* d, const u32x4_t* a, const u32x4_t& bb, bool first) {
+#pragma unroll
+          for (int rf = 0; rf < NRF; ++rf) d[rf] = mfma32b(a[rf], bb, first ? f32v4{} : d[rf]);
+        };
+        if constexpr (!RBF) mm(small, a2, c[1], true);
+        mm(small, a2, c[0], RBF);
+        if constexpr (!RBF) mm(small, a1, c[1], false);
+        mm(small, a1, c[0], false);
+        if constexpr (!RBF) mm(small, a0, c[1], false);
+        mm(big, a0, c[0], true);
         if (o + 1 < NF) weights(fn, b[(o + 1) & 1]);
+#pragma unroll
+        for (int rf = 0; rf < NRF; ++rf) acc[rf][f] += big[rf] + small[rf];
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 8; ++j) q[j] = qn[j];
     }
-    float bad = 0.f;   // NaN once any sum is infinite or NaN
+    // rows of a value below 2^-72 that is not zero, and rows with an infinite or NaN sum
+    constexpr uint32_t LEAST = 2u * ((127u - 72u) << 23) - 1u;
+    float bad = 0.f;   // NaN once a sum is infinite or NaN
+    uint32_t low = ~0u;
 #pragma unroll
-    for (int rf = 0; rf < NRF; ++rf)
+    for (int rf = 0; rf < NRF; ++rf) {
+      low = min(low, least[rf]);
 #pragma unroll
       for (int f = 0; f < NF; ++f)
 #pragma unroll
         for (int r = 0; r < 4; ++r) bad = fmaf(acc[rf][f][r], 0.f, bad);
-    if (__syncthreads_or(bad != 0.f)) {
-      GM::template tile<RBF ? W_INT4R : W_INT4, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
-      lds_barrier();
-      return;
     }
+    bool odd = range >= 168u << 7 || apart > 1536u;   // (a group past the block's counts too)
+    if (__builtin_amdgcn_ballot_w64(bad != 0.f || low < LEAST || odd)) {
+      if (odd) {
+        odd = false;
+        for (int e = t; e < outer << gs; e += 256) {
+          const int o = e >> gs, g = e & ((1 << gs) - 1);
+          if (g < ng) odd |= !splits<RBF>(P[g * outer + o] & 0xffffu, P[g * outer + o] >> 16);
+        }
+        if (odd) atomicOr(&again[0], ~0u), atomicOr(&again[1], ~0u);
+      }
+#pragma unroll
+      for (int rf = 0; rf < NRF; ++rf) {
+        if (least[rf] < LEAST) atomicOr(&again[rf >> 1], 1u << (16 * (rf & 1) + i));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float v = 0.f;
+#pragma unroll
+          for (int f = 0; f < NF; ++f) v = fmaf(acc[rf][f][r], 0.f, v);
+          if (v != 0.f) atomicOr(&again[rf >> 1], 1u << (16 * (rf & 1) + 4 * kq + r));
+        }
+      }
+    }
+    lds_barrier();   // every wave is done with the scales
+    const uint32_t redo[2] = {(uint32_t)__builtin_amdgcn_readfirstlane(again[0]),
+                              (uint32_t)__builtin_amdgcn_readfirstlane(again[1])};
 #pragma unroll
     for (int rf = 0; rf < NRF; ++rf) {
 #pragma unroll
@@ -517,19 +581,21 @@ struct Split {
               f32v4{acc[rf][4 * h][r], acc[rf][4 * h + 1][r], acc[rf][4 * h + 2][r], acc[rf][4 * h + 3][r]};
       lds_barrier();
       const int cc = t & (NT - 1), row0 = mr0 + 16 * rf;
+      const uint32_t skip = redo[rf >> 1] >> (16 * (rf & 1) + (t >> 7));
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int rr = (t >> 7) + 2 * j;
         float v = lds[rr * PR + cc];
 #pragma unroll
         for (int q = 1; q < 4; ++q) v += lds[(16 * q + rr) * PR + cc];
-        if (row0 + rr < mr1 && cc < nfw) {
+        if (row0 + rr < mr1 && cc < nfw && !(skip >> 2 * j & 1)) {
           float* const p = G.C + (int64_t)(row0 + rr) * G.ldc + n0 + cc;
           *p = G.beta1 ? *p + G.alpha * v : G.alpha * v;
         }
       }
       lds_barrier();
     }
+    return redo[0] | (uint64_t)redo[1] << 32;
   }
 };
 
@@ -559,10 +625,15 @@ __global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const 
       for (int p = blockIdx.z; p < np; p += gridDim.z) {
         const int s0 = p * ns / np, s1 = (p + 1) * ns / np;
         const int mr0 = r0 + 16 * s0, mr1 = min(r1, r0 + 16 * s1);
-        if (m.rbf) Split<TRANS>::template tile<3, true>(lds, G, m, N, K, n0, mr0, mr1);
-        else if (s1 - s0 == 1) Split<TRANS>::template tile<1, false>(lds, G, m, N, K, n0, mr0, mr1);
-        else if (s1 - s0 == 2) Split<TRANS>::template tile<2, false>(lds, G, m, N, K, n0, mr0, mr1);
-        else Split<TRANS>::template tile<3, false>(lds, G, m, N, K, n0, mr0, mr1);
+        uint64_t redo;
+        if (m.rbf) redo = Split<TRANS>::template tile<3, true>(lds, G, m, N, K, n0, mr0, mr1);
+        else if (s1 - s0 == 1) redo = Split<TRANS>::template tile<1, false>(lds, G, m, N, K, n0, mr0, mr1);
+        else if (s1 - s0 == 2) redo = Split<TRANS>::template tile<2, false>(lds, G, m, N, K, n0, mr0, mr1);
+        else redo = Split<TRANS>::template tile<3, false>(lds, G, m, N, K, n0, mr0, mr1);
+        if (!redo) continue;
+        if (m.rbf) GM::template tile<W_INT4R, GM::RF>(lds, G, m, N, K, n0, mr0, mr1, redo);
+        else GM::template tile<W_INT4, GM::RF>(lds, G, m, N, K, n0, mr0, mr1, redo);
+        lds_barrier();
       }
       return;
     }

@@ -3,8 +3,9 @@ per-group matmul loop for any non-bf16 tensor, smel/moe.py:58-72, and whose own 
 tests/test_moe.py:10-36). ``smel.moe`` enters it when the activations are float32; the functions keep the reference's
 arguments and results.
 
-Every product is an fp32 MFMA of libsmel_moe.so (``smel_gmm_f32`` over the dispatch's tile list, ``smel_wgrad_f32``
-for the LoRA weight gradients) and every element-wise step a HIP kernel of the same library (include/smel_f32.h). The
+Every product is an fp32 one of libsmel_moe.so (``smel_gmm_f32`` over the dispatch's tile list, ``smel_wgrad_f32`` for
+the LoRA weight gradients), on the fp32 MFMA or, for int4 tiles, as exact bf16 parts of both operands (include/smel_f32.h),
+and every element-wise step a HIP kernel of the same library (include/smel_f32.h). The
 structure follows the reference's composition: route -> stats -> routed experts (dispatch, gather, gate_up with the
 LoRA terms added as ``addmm(base, xa, B^T, alpha=s)``, act(g) u, down with its LoRA term, combine) -> shared expert
 (``mlp_lora``) times its sigmoid gate, added to the routed output. int4 banks are dequantized to fp32 inside the GEMM

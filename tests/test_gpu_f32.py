@@ -185,6 +185,137 @@ def test_gmm_f32_split_int4_tiles(trans, N, K, group, kind):
         off += c
 
 
+def _split_case(trans, kind, N=1024, K=256, group=64, seed=11, bank=None):
+    """(weight set, tile list, rows, expert of each row, dequantized fp64 weights as [E][K][N]) of a bank whose tiles run as
+    bf16 parts; ``bank`` changes the quantized bank first."""
+    from smel import _lib as L
+    from smel import moe_f32 as F
+    counts, Rw, Cw = SPLIT_COUNTS, (K if trans else N), (N if trans else K)
+    q = _int4_bank(len(counts), Rw, Cw, group, seed)
+    if bank is not None:
+        bank(q)
+    W = R.dequant_int4(q["q"], q["scale"], q["zero"],
+                       torch.bfloat16 if kind == "int4_bf16" else torch.float32).double()
+    dq = {k: v.to(DEV) for k, v in q.items()}
+    w = F._ws(Rw, Cw, 1 << L.KIND_INT4, q4=L.ptr(dq["q"]), scale=L.ptr(dq["scale"]), zero=L.ptr(dq["zero"]))
+    w.group, w.q4_round_bf16, w._keep = group, int(kind == "int4_bf16"), dq
+    tl, _ = F.count_tiles(counts, L.KIND_INT4, DEV)
+    return w, tl, sum(counts), torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts)), \
+        (W if trans else W.transpose(1, 2)).to(DEV)
+
+
+def _split_run(w, trans, tl, A, N):
+    from smel import moe_f32 as F
+    C = torch.full((A.shape[0], N), 7.0, device=DEV)
+    F.gmm(w, trans, tl, A, A.shape[1], C, N)
+    return C
+
+
+def _split_ref(A, W, expert):
+    ref, size = (torch.empty(A.shape[0], W.shape[2], dtype=torch.float64, device=DEV) for _ in range(2))
+    for e in expert.unique().tolist():
+        r = (expert == e).to(DEV)
+        ref[r] = A[r].double() @ W[e]
+        size[r] = A[r].double().abs() @ W[e].abs()
+    return ref, size
+
+
+@pytest.mark.parametrize("kind", ["int4", "int4_bf16"])
+@pytest.mark.parametrize("trans", [0, 1])
+@pytest.mark.parametrize("terms", [1, 2, 8])
+def test_gmm_f32_split_few_terms(terms, trans, kind):
+    """Results that one, two or eight products carry. A product's parts are exact; its largest and the sum of the others
+    (2^-8 of it, a few roundings of 2^-24 each) meet in one fp32 addition: 2^-24 (1 + 2^-6) of a lone product. Two terms
+    in one k-step: the instruction's sum of the largest parts loses up to 2^-23, the addition of the others 2^-24; terms in
+    different steps round once each and once more per addition: n + 1 units of 2^-24 of sum |x w| for n terms."""
+    N, K = 1024, 256
+    w, tl, rows, expert, W = _split_case(trans, kind, N, K)
+    g = torch.Generator(device=DEV).manual_seed(terms)
+    A = torch.randn(rows, K, generator=g, device=DEV)
+    keep = torch.rand(rows, K, generator=g, device=DEV).argsort(1)[:, :terms]
+    A = A * torch.zeros_like(A).scatter_(1, keep, 1.0)
+    ref, size = _split_ref(A, W, expert)
+    err = ((_split_run(w, trans, tl, A, N).double() - ref).abs() / size)[size > 0].max().item()
+    assert err <= 2.0 ** -24 * (1 + 2.0 ** -6) * (1 if terms == 1 else terms + 1), err
+
+
+@pytest.mark.parametrize("kind", ["int4", "int4_bf16"])
+@pytest.mark.parametrize("trans", [0, 1])
+def test_gmm_f32_split_small_values(trans, kind):
+    """Rows near the small end of the exponent range (whole rows, and single values in ordinary rows whose other weights'
+    products cancel to nothing against them): no parts are lost. Bound as for ordinary rows: K = 256 roundings of 2^-24 at
+    worst, adding as their square root, times 4 for the largest of a million results."""
+    N, K = 1024, 256
+    w, tl, rows, expert, W = _split_case(trans, kind, N, K)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    A = torch.randn(rows, K, generator=g, device=DEV)
+    A = torch.where(A.abs() < 2.0 ** -4, torch.full_like(A, 0.3), A)   # results stay above the subnormal numbers
+    scale = torch.tensor([0, -60, -71, -73, -90, -100, -108, -112, -114], device=DEV)
+    A = torch.ldexp(A, scale[torch.arange(rows, device=DEV) % len(scale)][:, None])
+    A[::7, 5:] = 0.0                                                      # few terms, and rows that hold zeros
+    ref, size = _split_ref(A, W, expert)
+    err = ((_split_run(w, trans, tl, A, N).double() - ref).abs() / size)[size > 0]
+    assert err.max().item() <= 4 * 16 * 2.0 ** -24, err.max().item()
+    # one value at 2^-100 beside zeros: the product itself, to one rounding
+    A = torch.zeros_like(A)
+    A[:, 9] = torch.ldexp(torch.rand(rows, generator=g, device=DEV) + 1.0, torch.tensor(-100, device=DEV))
+    ref, size = _split_ref(A, W, expert)
+    err = ((_split_run(w, trans, tl, A, N).double() - ref).abs() / size)[size > 0].max().item()
+    assert err <= 2.0 ** -24, err
+
+
+@pytest.mark.parametrize("kind", ["int4", "int4_bf16"])
+@pytest.mark.parametrize("trans", [0, 1])
+def test_gmm_f32_split_rows_are_independent(trans, kind):
+    """A row's bits do not depend on its tile's other rows, whatever those hold."""
+    N, K = 1024, 256
+    w, tl, rows, expert, W = _split_case(trans, kind, N, K)
+    A = torch.randn(rows, K, generator=torch.Generator(device=DEV).manual_seed(5), device=DEV)
+    base = _split_run(w, trans, tl, A, N)
+    odd = torch.arange(0, rows, 5, device=DEV)
+    rest = torch.ones(rows, dtype=torch.bool, device=DEV)
+    rest[odd] = False
+    for v in (float("inf"), float("nan"), 3.4028234e38, 1e-30):
+        B = A.clone()
+        B[odd, 17] = v
+        assert torch.equal(_split_run(w, trans, tl, B, N)[rest], base[rest]), v
+
+
+@pytest.mark.parametrize("kind", ["int4", "int4_bf16"])
+@pytest.mark.parametrize("trans", [0, 1])
+@pytest.mark.parametrize("form", ["zero_bank", "no_zero", "no_scale", "small_zero", "large_zero", "tiny", "one_group"])
+def test_gmm_f32_split_weights(form, trans, kind):
+    """Banks with groups whose weights are a sum of two bf16 values in other ways (all zero, scale or zero missing) or are
+    not (a zero far below or above the scale, values near the small end), everywhere or in one group: one product's
+    rounding in rows of one term (2^-24 for the fp32 instruction, (1 + 2^-6) of it in parts), and ordinary rows."""
+    def bank(q):
+        s, z = q["scale"], q["zero"]
+        if form == "zero_bank":
+            s.fill_(1e-8), z.zero_()
+        elif form == "no_zero":
+            z.zero_()
+        elif form == "no_scale":
+            s.zero_()
+        elif form == "small_zero":
+            z.copy_(s.float() * 2.0 ** -9)
+        elif form == "large_zero":
+            z.copy_(s.float() * 1021.0)
+        elif form == "tiny":
+            s.copy_(s.float() * 2.0 ** -60), z.copy_(z.float() * 2.0 ** -60)
+        else:
+            z[3, 5, 0] = 1e-7
+
+    N, K = 1024, 256
+    w, tl, rows, expert, W = _split_case(trans, kind, N, K, bank=bank)
+    g = torch.Generator(device=DEV).manual_seed(7)
+    A = torch.randn(rows, K, generator=g, device=DEV)
+    A[::2] *= torch.zeros_like(A[::2]).scatter_(1, torch.randint(0, K, (A[::2].shape[0], 1), generator=g, device=DEV), 1.0)
+    ref, size = _split_ref(A, W, expert)
+    err = (_split_run(w, trans, tl, A, N).double() - ref).abs() / size.clamp_min(1e-300)
+    assert err[::2].max().item() <= 2.0 ** -24 * (1 + 2.0 ** -6)
+    assert err[1::2].max().item() <= 4 * 16 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("M,N", [(16, 200), (200, 16), (8, 36), (36, 33), (1, 64), (17, 65)])
 def test_wgrad_f32_shapes_against_fp64(M, N):
     """smel_wgrad_f32 with either side the narrower one, sides off the block sizes, and row counts around the waves'
