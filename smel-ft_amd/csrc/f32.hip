@@ -6,6 +6,8 @@
 // the Gemma router input, the shared-expert gate). Everything sums in a fixed order: no atomics.
 #include <math.h>
 
+#include <type_traits>
+
 #include "../../include/smel_f32.h"
 #include "abi_util.h"
 #include "common.h"
@@ -32,12 +34,13 @@ struct WMat {
   int gpr;      // groups per row, C / group
   int group;
   int gshift;   // log2(group), or -1
-  uint32_t gmul;   // ceil(2^32 / group): col / group as one high product (while col group < 2^32)
+  uint32_t gmul;   // ceil(2^32 / group): col / group as one high product (0: some col group is 2^32 or more)
   int rbf;
 };
 
 SMEL_DEV int gidx(const WMat& m, int row, int col) {
-  return row * m.gpr + (m.gshift >= 0 ? col >> m.gshift : col / m.group);
+  return row * m.gpr +
+         (m.gshift >= 0 ? col >> m.gshift : m.gmul ? (int)__umulhi((uint32_t)col, m.gmul) : col / m.group);
 }
 
 SMEL_DEV float dq(const WMat& m, uint32_t q, int gi) {
@@ -79,7 +82,7 @@ SMEL_DEV bool resolve(const smel_wset_f32& w, int kind, int idx, WMat& m) {
   m.group = w.group > 0 ? w.group : 1;
   m.gpr = (int)(w.C / m.group);
   m.gshift = (m.group & (m.group - 1)) == 0 ? __builtin_ctz((unsigned)m.group) : -1;
-  m.gmul = 0xffffffffu / (uint32_t)m.group + 1u;
+  m.gmul = (int64_t)m.C * m.group < (1ll << 32) ? 0xffffffffu / (uint32_t)m.group + 1u : 0u;
   m.rbf = w.q4_round_bf16;
   m.f = nullptr;
   m.q = nullptr;
@@ -132,9 +135,10 @@ SMEL_DEV void dq8(uint32_t w, float sc, float ze, int rbf, float* v) {
 // waiting for global loads, or its load and store code behind branches, the same tiles took 560-620 us.
 // One k-step's operands of a thread on their way from global memory to LDS.
 struct StageRegs {
-  u32x4_t a[2];   // 8 values of an A row
-  u32x4_t b[4];   // a run of 16 weights: fp32 values, or the raw nibbles in b[0]
-  uint32_t bs, bz;   // and their bf16 scale and zero
+  u32x4_t a[2];   // 8 values of A
+  u32x4_t b[4];   // 16 weights: fp32 values, or the raw nibbles in b[0] (b[0..1]: pairs)
+  uint32_t bs, bz;   // scale and zero of a run of 16
+  uint32_t ms[8], mz[8];   // of each quad or pair
 };
 
 struct GemmArgs {
@@ -146,10 +150,18 @@ struct GemmArgs {
   int64_t ldc;
 };
 
-// How a block reads its weights: runs of 16 nibbles (8 bytes, one scale / zero pair), fp32 in 16-byte loads, or element
-// by element (any alignment, any group; A too).
-// W_INT4R: W_INT4 with the dequantized values rounded to bf16.
-enum { W_INT4 = 0, W_F32 = 1, W_ANY = 2, W_INT4R = 3 };
+// How a block reads its operands.
+//   W_INT4   A in 16-byte loads, runs of 16 nibbles (8 bytes, one scale / zero pair); W_INT4R: rounded to bf16
+//   W_F32    A and fp32 weights in 16-byte loads
+// and the forms for any alignment and any group, whose threads take neighbouring elements of the stage instead of runs:
+//   W_QUAD   A in 16-byte loads, four nibbles with a scale / zero pair of their own (W_QUAD1: A element by element)
+//   W_PAIR   A element by element, two nibbles with a pair of their own
+//   W_ELEM   A and fp32 weights element by element
+// All of them keep their loads two k-steps ahead. Measured (64 experts of 32 rows, 1024 x 2048; quads one step ahead on
+// 32x32 MFMAs -> element by element without loads ahead -> here): groups of 8 306 -> 1199 -> 155 us, transposed 230 ->
+// 545 -> 147, A of an odd pitch 253 -> 811 -> 147; fp32 matrices of 2046 columns (16 of 64 rows) 167 -> 190 -> 70,
+// transposed 93 -> 220 -> 77.
+enum { W_INT4 = 0, W_F32 = 1, W_INT4R = 2, W_QUAD = 3, W_QUAD1 = 4, W_PAIR = 5, W_ELEM = 6 };
 
 template <int TRANS, int RB, int NT, int KS, int FK>
 struct Gemm {
@@ -164,12 +176,29 @@ struct Gemm {
   static_assert(RB * FK == 8 * 256 && NT * FK == 16 * 256, "staging split");
   static_assert(KS == 1 || KS * RB * (NT + 4) <= LDS_FLOATS, "reduction buffer");
 
+  // The forms for any alignment: thread t takes units x = 256 e + t of U weights, in the order of the W stage (SW weights a
+  // row of it). Matrix row and column of a unit, held inside the matrix, and whether it is inside.
+  static constexpr int SW = TRANS ? NT : FK;
+  template <int U>
+  SMEL_DEV static int wrow(int x, int k0, int n0, int WR) {
+    return min((TRANS ? k0 : n0) + x / (SW / U), WR - 1);
+  }
+  template <int U>
+  SMEL_DEV static int wcol(int x, int k0, int n0, int WC) {
+    return min((TRANS ? n0 : k0) + x % (SW / U) * U, WC - U);
+  }
+  template <int U>
+  SMEL_DEV static bool wok(int x, int k0, int n0, int WR, int WC) {
+    return (TRANS ? k0 : n0) + x / (SW / U) < WR && (TRANS ? n0 : k0) + x % (SW / U) * U < WC;
+  }
+
   // NRF: the 16-row slices computed (those of the tile's rows; the others' rows are zeros in LDS); only: the rows stored
   // (bit r: row mr0 + r)
   template <int MODE, int NRF>
   SMEL_DEV static void tile(float* __restrict__ lds, const GemmArgs& G, const WMat& m, int N, int K, int n0, int mr0,
                             int mr1, uint64_t only = ~0ull) {
-    constexpr bool INT4 = MODE == W_INT4 || MODE == W_INT4R;
+    constexpr bool INT4 = MODE == W_INT4 || MODE == W_INT4R, RUNS = INT4 || MODE == W_F32;
+    constexpr bool AVEC = RUNS || MODE == W_QUAD;
     int t = threadIdx.x;
     asm volatile("" : "+v"(t));   // the addresses made from it belong to this tile: kept over a loop of tiles they would spill
     const int l = t & 63, wv = t >> 6, i = l & 15, kq = l >> 4;
@@ -190,10 +219,34 @@ struct Gemm {
       const int k = k0 + ak;
       const int wr = TRANS ? k0 + bo : n0 + bo;   // matrix row and first column of the run
       const int wc = TRANS ? n0 + br : k0 + br;
-      if (MODE == W_ANY) return;                  // loaded where it is stored
+      if (AVEC) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) S.a[h] = ld16(ra, (arow != OOB && k + 4 * h < K) ? 4 * (arow + k + 4 * h) : OOB);
-      if (INT4) {   // C a multiple of 16, so a run is inside the matrix or past it
+        for (int h = 0; h < 2; ++h) S.a[h] = ld16(ra, (arow != OOB && k + 4 * h < K) ? 4 * (arow + k + 4 * h) : OOB);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int x = 256 * e + t;
+          S.a[e >> 2][e & 3] = __float_as_uint(ab[min(x / FK, mr1 - mr0 - 1) * G.lda + min(k0 + x % FK, K - 1)]);
+        }
+      }
+      // elements past the edges: the last one's value here, zero where it is stored
+      if (MODE == W_ELEM) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int x = 256 * e + t;
+          S.b[e >> 2][e & 3] = __float_as_uint(m.f[wrow<1>(x, k0, n0, WR) * (int64_t)m.C + wcol<1>(x, k0, n0, WC)]);
+        }
+      } else if (!RUNS) {
+        constexpr int U = MODE == W_PAIR ? 2 : 4;
+#pragma unroll
+        for (int e = 0; e < 16 / U; ++e) {
+          const int x = 256 * e + t, r = wrow<U>(x, k0, n0, WR), c = wcol<U>(x, k0, n0, WC);
+          const uint8_t* const p = m.q + (int64_t)r * (m.C >> 1) + (c >> 1);
+          S.b[e >> 2][e & 3] = U == 4 ? *reinterpret_cast<const uint16_t*>(p) : *p;
+          const int gi = gidx(m, r, c);
+          S.ms[e] = m.s[gi], S.mz[e] = m.z[gi];
+        }
+      } else if (INT4) {   // C a multiple of 16, so a run is inside the matrix or past it
         const bool ok = wr < WR && wc < WC;
         const u32x2_t q = ld8(rw, ok ? (uint32_t)(wr * (m.C >> 1) + (wc >> 1)) : OOB);
         S.b[0][0] = q[0], S.b[0][1] = q[1];
@@ -211,19 +264,45 @@ struct Gemm {
       float* const Bs = As + SA;
       float* const ap = As + am * PA + ak;
       float* const bp = Bs + bo * PB + br;
-      if (MODE == W_ANY) {
-        const int wr = TRANS ? k0 + bo : n0 + bo, wc = TRANS ? n0 + br : k0 + br;
-#pragma unroll 1
+      if (!AVEC) {
+#pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int k = k0 + ak + e;
-          ap[e] = (am < mr1 - mr0 && k < K) ? ab[am * G.lda + k] : 0.f;
+          const int x = 256 * e + t;
+          const bool ok = x / FK < mr1 - mr0 && k0 + x % FK < K;
+          As[x / FK * PA + x % FK] = ok ? __uint_as_float(S.a[e >> 2][e & 3]) : 0.f;
         }
-#pragma unroll 1
-        for (int e = 0; e < 16; ++e) bp[e] = (wr < WR && wc + e < WC) ? w_at(m, wr, wc + e) : 0.f;
+      }
+      if (MODE == W_ELEM) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int x = 256 * e + t;
+          Bs[x / SW * PB + x % SW] = wok<1>(x, k0, n0, WR, WC) ? __uint_as_float(S.b[e >> 2][e & 3]) : 0.f;
+        }
         return;
+      }
+      if (!RUNS) {
+        constexpr int U = MODE == W_PAIR ? 2 : 4;
+#pragma unroll
+        for (int e = 0; e < 16 / U; ++e) {
+          const int x = 256 * e + t;
+          const bool ok = wok<U>(x, k0, n0, WR, WC);
+          const uint32_t n4 = S.b[e >> 2][e & 3];
+          float v[U];
+#pragma unroll
+          for (int j = 0; j < U; ++j) {
+            v[j] = fmaf((float)(n4 >> (4 * j) & 0xfu), bf2f(S.ms[e]), bf2f(S.mz[e]));
+            if (m.rbf) v[j] = bf2f(f2bf(v[j]));
+            v[j] = ok ? v[j] : 0.f;
+          }
+          float* const d = Bs + x / (SW / U) * PB + x % (SW / U) * U;
+          if (U == 4) *reinterpret_cast<float4*>(d) = make_float4(v[0], v[1], v[2 % U], v[3 % U]);
+          else *reinterpret_cast<float2*>(d) = make_float2(v[0], v[1]);
+        }
+        if (!AVEC) return;
       }
 #pragma unroll
       for (int h = 0; h < 2; ++h) *reinterpret_cast<u32x4_t*>(ap + 4 * h) = S.a[h];
+      if (!RUNS) return;
       if (INT4) {
         float v[16];
         const float sc = __uint_as_float(S.bs << 16), ze = __uint_as_float(S.bz << 16);
@@ -599,7 +678,9 @@ struct Split {
   }
 };
 
-template <int TRANS, int RB, int NT, int KS, int FK>
+// ANY: the forms for any alignment and group, in kernels of their own (their registers would cost the others a block per
+// CU); a launch takes it when one of its kinds needs it.
+template <int TRANS, int RB, int NT, int KS, int FK, bool ANY>
 __global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const int32_t* __restrict__ gkind,
                                                          const int32_t* __restrict__ tiles,
                                                          const int32_t* __restrict__ n_tiles, int vec, int qvec,
@@ -618,8 +699,8 @@ __global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const 
   if (!((w.kinds >> kind) & 1)) return;
   WMat m;
   if (!resolve(w, kind, idx, m)) return;
-  if constexpr (NT == Split<TRANS>::NT) {
-    if (!m.f && (vec & 1) && qvec && Split<TRANS>::fits(m, N, K, n0)) {
+  if constexpr (!ANY && NT == Split<TRANS>::NT) {
+    if (!m.f && Split<TRANS>::fits(m, N, K, n0)) {
       // the tile's 16-row slices in passes of up to three, as even as they go
       const int ns = (r1 - r0 + 15) >> 4, np = (ns + Split<TRANS>::MAXRF - 1) / Split<TRANS>::MAXRF;
       for (int p = blockIdx.z; p < np; p += gridDim.z) {
@@ -642,19 +723,26 @@ __global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const 
   for (int mr0 = r0 + RB * (int)blockIdx.z; mr0 < r1; mr0 += RB * (int)gridDim.z) {
     const int mr1 = min(r1, mr0 + RB);
     const int nrf = (mr1 - mr0 + 15) >> 4;
-    if (!m.f && (vec & 1) && qvec && m.rbf) {
+    if constexpr (ANY) {
+      auto run = [&](auto mode) {
+        if (nrf <= 2) GM::template tile<mode.value, 2>(lds, G, m, N, K, n0, mr0, mr1);
+        else if constexpr (GM::RF > 2) GM::template tile<mode.value, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
+      };
+      if (m.f) run(std::integral_constant<int, W_ELEM>{});
+      else if (qvec == 0) run(std::integral_constant<int, W_PAIR>{});
+      else if (vec & 1) run(std::integral_constant<int, W_QUAD>{});
+      else run(std::integral_constant<int, W_QUAD1>{});
+    } else if (m.f) {
+      if (nrf == 1) GM::template tile<W_F32, 1>(lds, G, m, N, K, n0, mr0, mr1);
+      else if (nrf == 2) GM::template tile<W_F32, 2>(lds, G, m, N, K, n0, mr0, mr1);
+      else GM::template tile<W_F32, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
+    } else if (m.rbf) {
       GM::template tile<W_INT4R, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
-    } else if (!m.f && (vec & 1) && qvec) {
+    } else {
       if (nrf == 1) GM::template tile<W_INT4, 1>(lds, G, m, N, K, n0, mr0, mr1);
       else if (nrf == 2) GM::template tile<W_INT4, 2>(lds, G, m, N, K, n0, mr0, mr1);
       else if (GM::RF > 2 && nrf == 3) GM::template tile<W_INT4, GM::RF - 1>(lds, G, m, N, K, n0, mr0, mr1);
       else GM::template tile<W_INT4, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
-    } else if (m.f && vec == 3) {
-      if (nrf == 1) GM::template tile<W_F32, 1>(lds, G, m, N, K, n0, mr0, mr1);
-      else if (nrf == 2) GM::template tile<W_F32, 2>(lds, G, m, N, K, n0, mr0, mr1);
-      else GM::template tile<W_F32, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
-    } else {
-      GM::template tile<W_ANY, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
     }
     lds_barrier();
   }
@@ -1207,9 +1295,10 @@ extern "C" int smel_gmm_f32(const smel_wset_f32* w, int32_t trans, const int32_t
                            (!w->wsh || aligned16(w->wsh))
                        ? 2
                        : 0);
-  // 16 nibbles in one 8-byte load under one scale / zero pair
-  const int qvec = w->q4 && w->C % 16 == 0 && w->group % 16 == 0 && w->C * w->group < (1LL << 32) &&
+  // nibbles under one scale / zero pair in one load: 2: 16 (8 bytes), 1: 4 (2 bytes), 0: 2
+  const bool q16 = w->q4 && w->C % 16 == 0 && w->group % 16 == 0 && w->C * w->group < (1LL << 32) &&
                    ((uintptr_t)w->q4 & 7) == 0 && ((uintptr_t)w->scale & 1) == 0 && ((uintptr_t)w->zero & 1) == 0;
+  const int qvec = q16 ? 2 : w->C % 4 == 0 && w->group % 4 == 0 && ((uintptr_t)w->q4 & 1) == 0;
   const int b1 = beta != 0.f;
   const unsigned mt = (unsigned)max_tiles;
   if (N <= 64) {   // at most one column block of the staged kernel: the whole K of a row tile in one block is the latency
@@ -1235,9 +1324,14 @@ extern "C" int smel_gmm_f32(const smel_wset_f32* w, int32_t trans, const int32_t
   const int64_t blocks = (max_tiles + 7) / 8 * 8 * ncol;
   SMEL_REQUIRE(blocks < (1LL << 31), SMEL_EUNSUPPORTED, "smel_gmm_f32: too many blocks");
   const dim3 grid((unsigned)blocks, 1, small ? 2 : 1);
-#define STAGED(TR, RB, NT, KS, FK)                                                                                \
-  gmm_f32_kernel<TR, RB, NT, KS, FK>                                                                              \
-      <<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, vec, qvec, GemmArgs{A, lda, alpha, b1, C, ldc})
+  const bool q4 = w->kinds & (1 << SMEL_KIND_INT4), f32 = w->kinds & ~(1 << SMEL_KIND_INT4);
+  const bool any = !(vec & 1) || (q4 && qvec != 2) || (f32 && !(vec & 2));
+#define STAGED(TR, RB, NT, KS, FK)                                                                                 \
+  do {                                                                                                             \
+    const GemmArgs G{A, lda, alpha, b1, C, ldc};                                                                   \
+    if (any) gmm_f32_kernel<TR, RB, NT, KS, FK, true><<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, vec, qvec, G); \
+    else gmm_f32_kernel<TR, RB, NT, KS, FK, false><<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, vec, qvec, G); \
+  } while (0)
   if (trans == 0) {
     if (small) STAGED(0, 32, 64, 4, 64);
     else STAGED(0, 64, 128, 1, 32);

@@ -139,6 +139,59 @@ def test_gmm_f32_shapes_against_fp64(shape, trans, kind):
         assert torch.equal(got[:, N:], C0[:, N:]) and torch.equal(got[rows], C0[rows])
 
 
+# (N, K, group or 0 for fp32 weights, extra A columns) that need the forms for any alignment (quads with aligned rows and
+# not, pairs, single elements), and short K (LoRA factors); enough tiles for the 64 x 128 blocks, and (counts of one group)
+# the 32 x 64 ones
+GMM_ANY = [(704, 104, 8, 0), (704, 100, 4, 1), (700, 74, 2, 0), (690, 70, 10, 3), (701, 77, 0, 0), (704, 80, 0, 1),
+           (704, 192, 64, 1), (701, 16, 0, 0), (704, 48, 0, 0), (706, 32, 0, 0), (704, 8, 0, 0), (702, 96, 0, 0)]
+
+
+@pytest.mark.parametrize("counts", [_MANY, [70, 3, 40]])
+@pytest.mark.parametrize("trans", [0, 1])
+@pytest.mark.parametrize("shape", GMM_ANY)
+def test_gmm_f32_any_alignment(shape, trans, counts):
+    """The load forms of smel_gmm_f32 for any alignment and any group, and K of one or two steps, against the fp64 product:
+    forward and transposed, beta 0 and 1, result rows on 8 bytes and not. K <= 192 fp32 products: inside 1e-6."""
+    from smel import _lib as L
+    from smel import moe_f32 as F
+    N, K, group, pad = shape
+    if group and trans:   # the group divides the matrix's columns, which are N here
+        N = N // group * group
+    Rw, Cw = (K, N) if trans else (N, K)
+    E, rows = len(counts), sum(counts)
+    g = torch.Generator().manual_seed(N + K)
+    forms = [("fp32", 0)] if group == 0 else [("int4", 0), ("int4", 1)]
+    for kind, rbf in forms:
+        if kind == "int4":
+            q = _int4_bank(E, Rw, Cw, group, K)
+            W = R.dequant_int4(q["q"], q["scale"], q["zero"], torch.bfloat16 if rbf else torch.float32).double()
+            dq = {k: v.to(DEV) for k, v in q.items()}
+            w = F._ws(Rw, Cw, 1 << L.KIND_INT4, q4=L.ptr(dq["q"]), scale=L.ptr(dq["scale"]), zero=L.ptr(dq["zero"]))
+            w.group, w.q4_round_bf16 = group, rbf
+        else:
+            Wf = torch.randn(E, Rw, Cw, generator=g) * 0.05
+            W, Wd = Wf.double(), Wf.to(DEV)
+            w = F._ws(Rw, Cw, 1 << L.KIND_BF16, wf=L.ptr(Wd))
+        tl, _ = F.count_tiles(counts, L.KIND_INT4 if kind == "int4" else L.KIND_BF16, DEV)
+        A = torch.randn(rows, K + pad, generator=g)
+        A[:, K:] = float("nan")   # never read
+        Ad = A.to(DEV)
+        for beta in (0.0, 1.0):
+            for extra in (2, 3):
+                C0 = torch.randn(rows + 1, N + extra, generator=g)
+                Cd = C0.to(DEV)
+                F.gmm(w, trans, tl, Ad, K + pad, Cd, N + extra, alpha=0.5, beta=beta)
+                ref = C0.double().clone()
+                ref[:rows, :N] *= beta
+                r = 0
+                for e, c in enumerate(counts):
+                    ref[r:r + c, :N] += 0.5 * (A[r:r + c, :K].double() @ (W[e] if trans else W[e].t()))
+                    r += c
+                got = Cd.cpu()
+                _check(got[:rows, :N], ref[:rows, :N], "C", tol=1e-6)
+                assert torch.equal(got[:, N:], C0[:, N:]) and torch.equal(got[rows], C0[rows])
+
+
 # (output columns, K, int4 group) of the tiles whose fp32 products run as bf16 parts: K of one step of 32 to more than a
 # round of four waves, columns over an edge of 128, one to many groups; counts over every number of 16-row slices of a pass
 SPLIT_COUNTS = [1, 16, 17, 33, 48, 49, 64, 65, 97, 128, 130, 0] * 6
