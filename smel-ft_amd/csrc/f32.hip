@@ -148,6 +148,7 @@ struct GemmArgs {
   int beta1;
   float* C;
   int64_t ldc;
+  int c2;   // columns of C in aligned pairs
 };
 
 // How a block reads its operands.
@@ -317,11 +318,10 @@ struct Gemm {
       }
     };
     f32v4 acc[NRF][NF] = {};
-    auto compute = [&](int buf) {
+    auto compute16 = [&](int buf, int k16) {
       const float* const As = lds + buf * (SA + SB);
       const float* const Bs = As + SA;
-#pragma unroll
-      for (int k16 = 0; k16 < KW; k16 += 16) {
+      {
         const int kk = wk * KW + k16 + 4 * kq;
         float b[4][NF];   // [k in the quad][fragment]
         if (TRANS) {
@@ -357,6 +357,10 @@ struct Gemm {
         }
       }
     };
+    auto compute = [&](int buf) {
+#pragma unroll
+      for (int k16 = 0; k16 < KW; k16 += 16) compute16(buf, k16);
+    };
     // Global loads run two k-steps ahead of their use, in two register sets; the barriers wait for LDS only. One
     // branch-free block per step, so that the next stage's dequant is issued between the MFMAs (two waves of a SIMD
     // reach their MFMA and VALU phases together: apart, the phases would add up). Steps past K load and add zeros.
@@ -365,7 +369,8 @@ struct Gemm {
     load(S1, FK);
     store(S0, 0, 0);
     lds_barrier();
-    for (int kt = 0; kt < nk; kt += 2) {
+    int kt = 0;
+    for (; (kt + 2) * FK <= K; kt += 2) {
       load(S0, (kt + 2) * FK);
       compute(0);
       store(S1, 1, (kt + 1) * FK);
@@ -375,6 +380,19 @@ struct Gemm {
       store(S0, 0, (kt + 2) * FK);
       lds_barrier();
     }
+    // up to two steps left, the last one for the k it has: all of a LoRA factor's rank (12 groups of 600 rows, N 2048: K 16
+    // 41 -> 23 us, transposed 42 -> 21; K 48 41 -> 34, 44 -> 32; whole steps of zeros before, results in single columns)
+    auto rest = [&](int buf, int step) {
+#pragma unroll 1
+      for (int k16 = 0; k16 < KW && step * FK + wk * KW + k16 < K; k16 += 16) compute16(buf, k16);
+    };
+    if (kt < nk) rest(0, kt);
+    if (kt + 1 < nk) {
+      store(S1, 1, (kt + 1) * FK);
+      lds_barrier();
+      rest(1, kt + 1);
+    }
+    if constexpr (KS > 1) lds_barrier();   // the stages become the reduction buffer
     if constexpr (KS == 1) {
 #pragma unroll
       for (int rf = 0; rf < NRF; ++rf)
@@ -383,6 +401,15 @@ struct Gemm {
           const int row = mr0 + 16 * rf + 4 * kq + r;
           if (row >= mr1 || !(only >> (row - mr0) & 1)) continue;
           float* const p = G.C + (int64_t)row * G.ldc;
+          if (NF == 2 && G.c2) {   // a lane's two columns in one access
+            const int col = n0 + 16 * NF * wn + NF * i;
+            if (col >= N) continue;
+            float2* const p2 = reinterpret_cast<float2*>(p + col);
+            const float2 o = G.beta1 ? *p2 : make_float2(0.f, 0.f);
+            const float v0 = G.alpha * acc[rf][0][r], v1 = G.alpha * acc[rf][NF - 1][r];
+            *p2 = G.beta1 ? make_float2(o.x + v0, o.y + v1) : make_float2(v0, v1);
+            continue;
+          }
 #pragma unroll
           for (int f = 0; f < NF; ++f) {
             const int col = n0 + 16 * NF * wn + NF * i + f;
@@ -678,10 +705,12 @@ struct Split {
   }
 };
 
-// ANY: the forms for any alignment and group, in kernels of their own (their registers would cost the others a block per
-// CU); a launch takes it when one of its kinds needs it.
-template <int TRANS, int RB, int NT, int KS, int FK, bool ANY>
-__global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const int32_t* __restrict__ gkind,
+// FORMS: what a launch's kinds need of the forms above, in kernels of their own (the registers of one cost the others a
+// block per CU): fp32 weights in 16-byte loads only (dense weights, LoRA factors), those and runs of nibbles, or any
+// alignment and group.
+enum { FORMS_F32 = 0, FORMS_RUNS = 1, FORMS_ANY = 2 };
+template <int TRANS, int RB, int NT, int KS, int FK, int FORMS>
+__global__ __launch_bounds__(256, FORMS == FORMS_F32 && TRANS ? 3 : 2) void gmm_f32_kernel(smel_wset_f32 w, const int32_t* __restrict__ gkind,
                                                          const int32_t* __restrict__ tiles,
                                                          const int32_t* __restrict__ n_tiles, int vec, int qvec,
                                                          GemmArgs G) {
@@ -699,7 +728,7 @@ __global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const 
   if (!((w.kinds >> kind) & 1)) return;
   WMat m;
   if (!resolve(w, kind, idx, m)) return;
-  if constexpr (!ANY && NT == Split<TRANS>::NT) {
+  if constexpr (FORMS == FORMS_RUNS && NT == Split<TRANS>::NT) {
     if (!m.f && Split<TRANS>::fits(m, N, K, n0)) {
       // the tile's 16-row slices in passes of up to three, as even as they go
       const int ns = (r1 - r0 + 15) >> 4, np = (ns + Split<TRANS>::MAXRF - 1) / Split<TRANS>::MAXRF;
@@ -723,7 +752,7 @@ __global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const 
   for (int mr0 = r0 + RB * (int)blockIdx.z; mr0 < r1; mr0 += RB * (int)gridDim.z) {
     const int mr1 = min(r1, mr0 + RB);
     const int nrf = (mr1 - mr0 + 15) >> 4;
-    if constexpr (ANY) {
+    if constexpr (FORMS == FORMS_ANY) {
       auto run = [&](auto mode) {
         if (nrf <= 2) GM::template tile<mode.value, 2>(lds, G, m, N, K, n0, mr0, mr1);
         else if constexpr (GM::RF > 2) GM::template tile<mode.value, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
@@ -732,7 +761,7 @@ __global__ __launch_bounds__(256, 2) void gmm_f32_kernel(smel_wset_f32 w, const 
       else if (qvec == 0) run(std::integral_constant<int, W_PAIR>{});
       else if (vec & 1) run(std::integral_constant<int, W_QUAD>{});
       else run(std::integral_constant<int, W_QUAD1>{});
-    } else if (m.f) {
+    } else if (FORMS == FORMS_F32 || m.f) {
       if (nrf == 1) GM::template tile<W_F32, 1>(lds, G, m, N, K, n0, mr0, mr1);
       else if (nrf == 2) GM::template tile<W_F32, 2>(lds, G, m, N, K, n0, mr0, mr1);
       else GM::template tile<W_F32, GM::RF>(lds, G, m, N, K, n0, mr0, mr1);
@@ -1317,20 +1346,26 @@ extern "C" int smel_gmm_f32(const smel_wset_f32* w, int32_t trans, const int32_t
 #undef SKINNY
     return smel::launch_status();
   }
-  // two 64 x 128 blocks fit a CU: below that count the quarter tiles (32 x 64) fill more of the chip
+  // two 64 x 128 blocks fit a CU: below that count the quarter tiles (32 x 64) fill more of the chip, where there is more
+  // than one of their k-steps of 64 to share among the waves (12 groups of 600 rows, K 16, N 512: 16 us in quarter tiles,
+  // 9 in whole ones; 1021 rows, K 16, N 2048: 11 and 8)
   const int64_t wide = max_tiles * ((N + 127) / 128);
-  const bool small = wide < 512;
+  const bool small = wide < 512 && K > 64;
   const int64_t ncol = small ? (N + 63) / 64 : (N + 127) / 128;
   const int64_t blocks = (max_tiles + 7) / 8 * 8 * ncol;
   SMEL_REQUIRE(blocks < (1LL << 31), SMEL_EUNSUPPORTED, "smel_gmm_f32: too many blocks");
   const dim3 grid((unsigned)blocks, 1, small ? 2 : 1);
+  const int c2 = N % 2 == 0 && ldc % 2 == 0 && ((uintptr_t)C & 7) == 0;
   const bool q4 = w->kinds & (1 << SMEL_KIND_INT4), f32 = w->kinds & ~(1 << SMEL_KIND_INT4);
   const bool any = !(vec & 1) || (q4 && qvec != 2) || (f32 && !(vec & 2));
-#define STAGED(TR, RB, NT, KS, FK)                                                                                 \
-  do {                                                                                                             \
-    const GemmArgs G{A, lda, alpha, b1, C, ldc};                                                                   \
-    if (any) gmm_f32_kernel<TR, RB, NT, KS, FK, true><<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, vec, qvec, G); \
-    else gmm_f32_kernel<TR, RB, NT, KS, FK, false><<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, vec, qvec, G); \
+  const GemmArgs G{A, lda, alpha, b1, C, ldc, c2};
+#define STAGED_F(TR, RB, NT, KS, FK, FORMS) \
+  gmm_f32_kernel<TR, RB, NT, KS, FK, FORMS><<<grid, 256, 0, stream>>>(*w, gkind, tiles, n_tiles, vec, qvec, G)
+#define STAGED(TR, RB, NT, KS, FK)                            \
+  do {                                                        \
+    if (any) STAGED_F(TR, RB, NT, KS, FK, FORMS_ANY);         \
+    else if (q4) STAGED_F(TR, RB, NT, KS, FK, FORMS_RUNS);    \
+    else STAGED_F(TR, RB, NT, KS, FK, FORMS_F32);             \
   } while (0)
   if (trans == 0) {
     if (small) STAGED(0, 32, 64, 4, 64);
@@ -1340,6 +1375,7 @@ extern "C" int smel_gmm_f32(const smel_wset_f32* w, int32_t trans, const int32_t
     else STAGED(1, 64, 128, 1, 32);
   }
 #undef STAGED
+#undef STAGED_F
   return smel::launch_status();
 }
 
