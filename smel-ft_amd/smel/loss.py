@@ -45,13 +45,21 @@ TOKEN_CHUNK_DEFAULT = _DefaultTokenChunk(1024)
 
 def _max_rows(token_chunk) -> int:
     """Token rows a pass may take: at most ``token_chunk`` (it bounds a pass's buffers, the softmax terms
-    [rows][vocab_chunk] and about 12 H bytes per row), or up to ROWS_PER_PASS when the caller left the default."""
+    [rows][vocab_chunk] and the accumulators of _grad_splits), or up to ROWS_PER_PASS when the caller left the default."""
     tc = int(token_chunk)
     if tc <= 0:
         raise ValueError(f"chunked_ce: token_chunk must be positive, got {tc}")
     if isinstance(token_chunk, _DefaultTokenChunk):
         tc = max(tc, ROWS_PER_PASS)
     return tc
+
+
+def _grad_splits(n: int, H: int, vcp: int, dtype) -> int:
+    """Parts of the gradient GEMM's contraction for a pass of ``n`` rows over chunks of ``vcp`` columns, each with an fp32
+    accumulator of 4 H bytes a row: three at most (12 H bytes a row), more only while they take no more than twice the
+    bytes of the pass's softmax terms, so that token_chunk x vocab_chunk bounds the pass whatever H is."""
+    terms = vcp * dtype.itemsize
+    return min(L.load().smel_ce_grad_splits(n, H, vcp, _DT[dtype]), max(3, 2 * terms // (4 * H)))
 
 
 def _round_up(x: int, m: int) -> int:
@@ -229,7 +237,7 @@ class _Pass:
         self.win_e, self.win_s = f(nwin, n), f(nwin, n)
         self.shift = torch.empty(nwin, n, dtype=torch.uint8, device=device)
         self.P = torch.empty(n, vcp, dtype=dtype, device=device) if need_grad else None
-        self.splits = L.load().smel_ce_grad_splits(n, H, vcp, _DT[dtype])
+        self.splits = _grad_splits(n, H, vcp, dtype)
         self.acc = f(self.splits, n, H) if need_grad else None
 
 

@@ -370,6 +370,35 @@ def test_token_chunk_bounds_pass_memory(lm):
     assert d <= 2**-7 * g_dflt.float().abs().max().item(), d
 
 
+@pytest.mark.parametrize("tc,vc", [(128, 4096), (256, 4096), (64, 32768), (640, 8192)])
+def test_accumulators_stay_in_the_pass_bound(lm, tc, vc):
+    """A hidden size whose accumulators are most of a pass: 12 H bytes a row, or twice the bytes of its terms, beside the
+    terms themselves and the row state."""
+    loss_mod, _ = lm
+    torch.manual_seed(tc)
+    H, V = 2048, 2 * vc
+    W = (torch.randn(V, H, device="cuda") * 0.05).bfloat16()
+    tgt = torch.randint(0, V, (tc,), device="cuda")
+    x = torch.randn(tc, H, device="cuda").bfloat16().requires_grad_(True)
+    head = loss_mod.LMHead(weight=W, vocab_chunk=vc)
+
+    def run():   # the head's transposed copy is made in the first one
+        loss_mod.chunked_ce(x, head, tgt, denom=float(tc), token_chunk=tc).backward()
+        x.grad = None
+        torch.cuda.synchronize()
+
+    run()
+    torch.cuda.reset_peak_memory_stats()
+    base = torch.cuda.memory_allocated()
+    run()
+    peak = torch.cuda.max_memory_allocated() - base
+    terms = tc * vc * 2
+    bound = terms + max(tc * H * 12, 2 * terms) + (2 * (vc // 128) * 4 + vc // 128 + 24) * tc
+    bound += 2 * tc * H * 2 + (1 << 18)   # gradients, small tensors
+    print(f"CE peak at H {H}: {peak / 2**20:.1f} MiB (bound {bound / 2**20:.1f})", flush=True)
+    assert peak <= bound
+
+
 def test_qwen_head_full_size(lm):
     """The bench's shape (4092 rows, hidden 2048, vocabulary 248320, chunks of 32768, bf16): loss and gradient of
     chunked_ce against the rounded full-logit comparator run in fp32 torch on the GPU (the [4092, 248320] logits fit
