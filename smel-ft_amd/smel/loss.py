@@ -207,7 +207,8 @@ class LMHead:
         passes fill the GPU; a head converted chunk by chunk stays at vocab_chunk, which bounds the converted rows."""
         cols = self.vocab_chunk
         if self._src.native(dtype) is not None:
-            cols = min(self.vocab, cols * max(1, max_rows // max(1, rows)))
+            most = ((1 << 23) - 1) // dtype.itemsize // TILE_V * TILE_V   # a tile of 256 rows of terms is below 2 GiB
+            cols = min(self.vocab, cols * max(1, max_rows // max(1, rows)), max(most, cols))
         return self._kernel_chunks(cols)
 
     def _transposed(self, w: torch.Tensor) -> torch.Tensor:

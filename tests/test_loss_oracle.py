@@ -67,3 +67,19 @@ def test_ce_entry_points_reject_bad_arguments():
     assert L.smel_ce_transpose(fake, 4, 64, 32, fake, 8, 0, None) == EINVAL                    # pitch < columns
     assert L.smel_ce_scale(fake, 8, 3, fake, None) == EINVAL
     assert L.smel_ce_loss_sum(fake, 4, 1.0, 0, None, None) == EINVAL
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [1, 7, 777, 4096])
+def test_wide_chunks_stay_in_the_kernels_offsets(rows, dtype, monkeypatch):
+    """A short pass takes wider chunks of a head read in place: never more terms than a full pass, and never a pitch of the
+    terms past the kernels' 31-bit tile offsets, up to the largest vocabulary whose transposed head they take."""
+    from smel.loss import LMHead
+    e = dtype.itemsize
+    for V in (1000, 151936, (1 << 23) // e - 8):
+        head = LMHead(weight=torch.empty(V, 8, dtype=dtype, device="meta"))
+        monkeypatch.setattr(head._src, "native", lambda dt: head._src.w)
+        chunks, step = head._pass_chunks(rows, 4096, dtype)
+        assert (V + 7) // 8 * 8 * e * 256 < 1 << 31 and step * e * 256 < 1 << 31
+        assert rows * step <= 4096 * 32768 + 256 * rows
+        assert chunks[0][0] == 0 and chunks[-1][1] == V and all(a[1] == b[0] for a, b in zip(chunks, chunks[1:]))
