@@ -20,6 +20,8 @@
 //  * vmcnt retires in issue order: each step issues its weight loads before its LDS-DMAs and waits for exactly the
 //    loads of the step it is about to use.
 
+#include <type_traits>
+
 #include "abi_util.h"
 #include "common.h"
 
@@ -310,6 +312,13 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
       issue_lds(j + 3, (st + 3) & 3, qs[(st + 3) & 3]);
       compute(st, qs[st]);
     };
+    // The steps after the whole rounds issue nothing (what they would load lies past K): weight words that no step uses
+    // are loads the compiler drops, and the waits count on every load of a group.
+    auto last = [&](auto in_flight, int st) {   // groups that may be in flight while it computes
+      wait_vm_lds<decltype(in_flight)::value * CF::vm_q4(SZ2)>();
+      __builtin_amdgcn_s_barrier();
+      compute(st, qs[st]);
+    };
     issue_lds(0, 0, qa);
     issue_lds(1, 1, qb);
     issue_lds(2, 2, qc);
@@ -321,10 +330,10 @@ SMEL_DEV void run_tile(const BwdArgs& a, int kind, int idx, int row0, int nrows,
       step(i + 3, 3);
     }
     if (i < nk) {
-      step(i, 0);
+      last(std::integral_constant<int, 2>{}, 0);
       if (i + 1 < nk) {
-        step(i + 1, 1);
-        if (i + 2 < nk) step(i + 2, 2);
+        last(std::integral_constant<int, 1>{}, 1);
+        if (i + 2 < nk) last(std::integral_constant<int, 0>{}, 2);
       }
     }
   } else {

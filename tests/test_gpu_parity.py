@@ -686,6 +686,43 @@ def test_shared_lora_rows_on_side_stream_bitwise(name, monkeypatch):
         assert torch.equal(a["grads"][k], b["grads"][k]), k
 
 
+@pytest.mark.parametrize("H,I,group", [(2816, 704, 64), (2880, 736, 32), (1984, 544, 32), (1152, 96, 32), (2752, 576, 64)])
+def test_backward_steps_past_whole_rounds_repeat(H, I, group, monkeypatch):
+    """int4 backward GEMMs whose contraction is 1, 2 or 3 k-steps of 64 past whole rounds of four, on tiles of 32 and 128
+    rows: the same bits in every pass, with the weights in no cache (each step waits for all of its loads, also where no
+    later step's are behind them), and within the bf16 bar of the fp32 path on the same bank."""
+    import smel.moe as M
+    _say(f"backward remainders H{H} I{I} g{group}")
+    E, K, T = 48, 4, 180
+    g = torch.Generator(device=DEV).manual_seed(H)
+    rn = lambda *s, std=0.02: (torch.randn(*s, generator=g, device=DEV) * std).to(torch.bfloat16)
+    bank = M.Int4Experts.from_bf16(rn(E, 2 * I, H), rn(E, H, I), group)
+    ex = M.LayerExperts(bank, act="gelu_tanh")
+    x, gy = rn(T, H, std=1.0), rn(T, H, std=1.0)
+    topi = torch.rand(T, E, generator=g, device=DEV).argsort(1)[:, :K]
+    topv = torch.rand(T, K, generator=g, device=DEV)
+    cold = torch.empty(1 << 29, dtype=torch.uint8, device=DEV)
+
+    def run(e, xin):
+        xg, tv = xin.clone().requires_grad_(True), topv.clone().requires_grad_(True)
+        y = M.routed_experts(xg, tv, topi, e)
+        cold.zero_()
+        y.backward(gy.to(y.dtype))
+        return y.detach(), xg.grad, tv.grad
+
+    runs = []
+    for mt in (M.M_SHORT, M.M_TILE):
+        monkeypatch.setattr(M, "_tile_rows", lambda *a, mt=mt: mt)
+        runs += [run(ex, x) for _ in range(5)]
+    for other in runs[1:]:
+        for a, b in zip(runs[0], other):
+            assert torch.equal(a, b)
+    bank32 = M.Int4Experts(bank.gu, bank.dn, dtype=torch.bfloat16)   # weights rounded to bf16, fp32 products
+    ref = run(M.LayerExperts(bank32, act="gelu_tanh"), x.float())
+    for a, b, n in zip(runs[0], ref, ("y", "dx", "dtopv")):
+        assert_close_bf16(a.cpu(), b.cpu(), n)
+
+
 @pytest.mark.parametrize("ext_side", [False, True])
 @pytest.mark.parametrize("form", ["bf16", "strided"])
 def test_converted_factors_on_side_stream_bitwise(form, ext_side, monkeypatch):
