@@ -46,7 +46,8 @@ int smel_ce_stats(const float* win_e, const float* win_s, int64_t nwin, int64_t 
  * are split in two halves: acc [n][H] fp32 = (chunk == 0 ? 0 : r acc) + sum over the first half of (P[v] 2^-shift) W[v],
  * and part[chunk % 2] = (chunk == 0 ? 0 : r part[(chunk - 1) % 2]) + the same sum over the second half (part:
  * [2][n][H] fp32; the gradient sum after the last chunk is acc + part[last % 2]). smel/loss.py:83-85
- * (`acc * r + p.to(h.dtype) @ W`), the product on MFMA. */
+ * (`acc * r + p.to(h.dtype) @ W`), the product on MFMA. With smel_ce_finish the interface of callers that keep this
+ * buffer layout; smel/loss.py takes the forms in parts below (two halves there give the same bits). */
 int smel_ce_grad(const void* WT, int64_t ldwt, int64_t H, const void* P, int64_t ldp, int64_t vc,
                  const uint8_t* shift, int64_t ldn, const float* r, int64_t n, int32_t dtype, int32_t chunk,
                  float* acc, float* part, hipStream_t stream);

@@ -449,8 +449,8 @@ def test_targets_outside_the_vocabulary(lm):
 
 @pytest.mark.parametrize("n", [1, 128, 129, 256, 257, 384, 385, 512])
 def test_tail_tile_edges(n):
-    """Row counts at the edges of the short last token tile (its own kernel): each row's loss and gradient equal those of
-    the row in a pass of whole tiles within the rounding of sums in another order, and the fp64 formula."""
+    """Row counts at the edges of the short last token tile (its own kernel) through the public call: mean loss and gradient
+    against the fp64 formula (the rows one by one: test_tail_tile_rows_against_whole_tiles)."""
     g = torch.Generator().manual_seed(n)
     H, V = 64, 700
     h = torch.randn(n, H, generator=g).to(torch.bfloat16)
@@ -466,3 +466,29 @@ def test_tail_tile_edges(n):
     # logits are rounded to bf16 (2^-9 of values of about 1.6, V of them averaged), gradients once more
     assert abs(loss.item() - ref.item()) < 1e-2 * abs(ref.item())
     assert (hd.grad.cpu().double() - h64.grad).norm() < 1.5e-2 * h64.grad.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 255, 256, 257, 384, 385])
+def test_tail_tile_rows_against_whole_tiles(lm, n, dtype):
+    """The same row edges over several hidden tiles, rotated parts and a last window of one k-step: every row's loss and
+    fp32 gradient against those of the row in a pass padded to whole 256-row tiles. The two passes take their fp32 sums
+    (about V / 2 terms of a row) in other orders: 1e-5 of the row's size; the terms themselves are the same."""
+    loss_mod, _ = lm
+    torch.manual_seed(n)
+    H, V, m = 776, 5003, (n + 255) // 256 * 256
+    h = torch.randn(m, H, device="cuda").to(dtype)
+    W = (torch.randn(V, H, device="cuda") * 0.1).to(dtype)
+    tgt = torch.randint(0, V, (m,), device="cuda")
+    head = loss_mod.LMHead(weight=W)
+
+    def rows(k):
+        x, t = loss_mod._prep(h[:k], tgt[:k])
+        ps = loss_mod._Pass(k, H, head._kernel_chunks(), dtype, True, x.device)
+        loss_mod._sweep(x, head, t, True, ps)
+        return loss_mod._finish(x, head, t, ps, True), ps.loss
+
+    g, l = rows(n)
+    gw, lw = rows(m)
+    assert ((l - lw[:n]).abs() <= 1e-5 * lw[:n].abs()).all()
+    assert ((g - gw[:n]).abs().amax(1) <= 1e-5 * gw[:n].norm(dim=1)).all()
