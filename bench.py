@@ -484,7 +484,7 @@ def run_c3f32(args, dev):
         log("timing the CPU baseline (the oracle, fp32: 1 warmup + median of 5 full passes) ...")
         cpu = cpu_baseline(x, W, ex, lora, gy, cfg)
     emit("MoE layer fwd+bwd tokens/s with fp32 activations (Qwen3.6 shape, T=4092)", T, args, timing,
-         "C3 in fp32: the C3 layer with float32 activations and weights, int4 bank dequantized to fp32, fp32 MFMA",
+         "C3 in fp32: the C3 layer with float32 activations and weights, int4 bank dequantized to fp32, fp32 products",
          {"selected_slots": S}, roof, bd, cpu, dtype="f32")
 
 
